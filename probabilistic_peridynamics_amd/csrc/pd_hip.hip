@@ -41,19 +41,20 @@
 //   tnode[N]   caller's node id of internal node p; halo: ascending internal
 //              ids per tile.
 //   bond slots, in chunks of 4: chunk (c, l) of a tile with n nodes is
-//              chunk_off + c*n + l and holds bonds 4c..4c+3 of its l-th node,
+//              chunk_off + c*n + l and holds four bonds of its l-th node
 //              rows sorted ascending by j; a wavefront reads its nodes' c-th
 //              chunks contiguously.  A tile has as many chunk rows as its
 //              longest row needs (at least one); the kernel's look-ahead
 //              chunk loads are clamped to the last of them.
-//     loc   u16  1 + halo-local index of j; 0: broken or empty (hot loop;
-//                entry 0 of a staged halo is a zero record)
+//     loc   u16  16 * (1 + halo-local index of j), the LDS offset of the
+//                record's first piece; 0: broken or empty (hot loop; entry 0
+//                of a staged halo is a far node of weight 0)
 //     gidx  i32  j, with bit 31 DEAD and bit 30 NEW (broken in this step,
 //                compact layout) -- read only on breaks and exports
 //     pos   u16  reference column of the slot (exports)
-//     corr  f64, state u16 (bond type << 8 | regime): optional
-//   chunk0[N], stride[N]: node p's chunk 0 and its tile's node count, so
-//              slot(p, k) = (chunk0 + (k/4)*stride)*4 + k%4
+//     corr  f64, state u16 (16 * (bond type * nregimes + regime)): optional
+//   chunk0[N], stride[N]: node p's chunk 0 and its tile's node count, from
+//              which slot_of gives the slot of its k-th bond
 //   u, ud, udd, force, body_force (N,3) f64 in the reference's layout
 //   flags[N]   bit d: displacement BC on DOF d; bit 3+d: force BC on DOF d
 //   bcv, fbcv, dens (N,3) f64, read only for flagged DOFs / dynamic
@@ -92,6 +93,7 @@
 #include <string>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pd_hip.h"
@@ -138,6 +140,10 @@ constexpr int XCDS = 8;
 constexpr int LDS_CAP_PMB = 1280;
 constexpr int LDS_CAP_NLIN = 1152;
 constexpr unsigned LDS_BYTES = 81920;
+// Slots that loc, state and corr are longer than the tiles need: the step
+// kernel requests chunk rows up to two rounds ahead, at most 3 rounds of
+// tile_nodes * lanes_per_node <= 1024 chunks past a tile's last.
+constexpr size_t LOC_SLACK = 3 * 1024 * 4;
 
 // damage models of the step kernel
 constexpr int DM_PMB = 0;    // scalar stiffness
@@ -160,7 +166,8 @@ struct StepArgs {
     int integrator, layout, has_corr;
     unsigned absmask;  // 0x7fffffff: break on |s|; 0xffffffff: on s
     int nregimes, ntab;
-    double dt, damping, s0h, s0h_guard;
+    double dt, damping, s0h;
+    double lim;  // bound of bond_fast's stretch test (n-linear: its sign)
     const NodeRec *rec_old;
     NodeRec *rec_new;
     const TileInfo *tiles;
@@ -192,15 +199,43 @@ struct StepArgs {
     double kx;
 };
 
+// Slot of a row's k-th bond.  Sixteen bonds take four chunks; chunk q of the
+// four holds bonds 2q, 2q+1 and 8+2q, 8+2q+1 of them, so that four lanes that
+// take the four chunks run the first eight bonds before the second, and a
+// row that ends in the first eight leaves the second half of its last round
+// empty for all of them.
 __host__ __device__ __forceinline__ size_t slot_of(long long chunk0,
                                                    int stride, int k)
 {
-    return (size_t)(chunk0 + (long long)(k >> 2) * stride) * 4 + (k & 3);
+    const int chunk = ((k >> 4) << 2) + ((k >> 1) & 3);
+    return (size_t)(chunk0 + (long long)chunk * stride) * 4 +
+           (((k >> 2) & 2) | (k & 1));
+}
+
+// Chunk rows of a row of cnt bonds.
+__host__ __device__ __forceinline__ int chunks_of(int cnt)
+{
+    const int half = ((cnt & 15) + 1) >> 1;
+    return ((cnt >> 4) << 2) + (half < 4 ? half : 4);
 }
 
 // ---------------------------------------------------------------------------
 // device helpers
 // ---------------------------------------------------------------------------
+
+// A 16-byte piece as the compiler's own vector (an array of HIP's double2
+// that is only copied through stays in scratch).
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// f(0), f(1), ..., f(N - 1) with constant arguments.
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F f)
+{
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
 
 // sqrt(q) rounded to nearest for q in [2^-767, inf): the rsq seed, one
 // Goldschmidt step for (g ~ sqrt q, h ~ 0.5/sqrt q) and two residual
@@ -423,6 +458,15 @@ constexpr unsigned piece_bytes()
     return 16u * (DM == DM_NLIN ? LDS_CAP_NLIN : LDS_CAP_PMB);
 }
 
+// Where the halo begins in LDS: after the n-linear tables (two of MAX_TAB
+// 16-byte entries), so that every read of the bond loop has an immediate
+// offset below 2^16.
+template <int DM>
+constexpr unsigned halo_base()
+{
+    return DM == DM_NLIN ? 2u * 16u * MAX_TAB : 0u;
+}
+
 // Squared length of (x, y, z): spatial.pyx's ((x*x + y*y) + z*z), uncontracted
 // (CLA false), or cl/peridynamics.cl:72-73's as contracted,
 // fma(z, z, fma(x, x, y*y)) (CLA true).
@@ -434,210 +478,228 @@ __device__ __forceinline__ double sq3(double x, double y, double z)
     return (x * x + y * y) + z * z;
 }
 
-// W bonds of node i at slots s0 .. s0+W-1: ev their halo indices (LOC_DEAD:
-// broken or empty), st their (bond type << 8 | regime) for DM_NLIN, ci node
-// i's stiffness for DM_FIELD.  Compile-time switches, so that the common
-// runs spend no instruction on what they do not use: CORR, the per-slot
-// stiffness corrections multiply the force (bond_force2/4); TENS, a PMB bond
-// breaks on !(s < s0) (cl/peridynamics.cl:78) instead of !(|s| < s0)
+// A bond as the force needs it: the bond vector, s/2, 0.5/l and the weight.
+struct Bond {
+    double dx, dy, dz, sh, hl, w;
+};
+
+// The model's halved thresholds with a margin of GUARD: a stretch strictly
+// inside (lo, hi) is away from every threshold and from lengths at which
+// sqrt_core is not exact, so the bond neither breaks nor changes its regime.
+// Anything else, NaN included, goes through bond_exact.
+//
+// Why the lengths need no test of their own: coordinates are zero or in
+// [2^-290, 2^300] (else the host sets hi so that every bond takes the exact
+// path), so q0 is 0 (its core value is NaN) or at least 2^-686 and below
+// 2^603.  s/2 > -1/4 then means l > l0/2, so q is at least 2^-690, and a q
+// that is infinite, NaN or 0 gives a NaN; a q in between but below the
+// core's range gives an l of at most 2^-383, whose s/2 is -1/2.
+
+// Compile-time switches of the step kernel, so that the common runs spend no
+// instruction on what they do not use: CORR, the per-slot stiffness
+// corrections multiply the force (bond_force2/4); TENS, a PMB bond breaks on
+// !(s < s0) (cl/peridynamics.cl:78) instead of !(|s| < s0)
 // (peridynamics.pyx:133); CLA, the OpenCL stretch (records hold u; the bond
 // vector is (u_j - u_i) + xi) instead of the Cython one (records hold
 // r0 + u; the bond vector is r_j - r_i).
-template <int DM, int W, bool CORR, bool TENS, bool CLA>
-__device__ __forceinline__ void bonds(const StepArgs &a, const char *ldsb,
-                                      const double4 &r0i, const double4 &ri,
-                                      double ci,
-                                      const unsigned *ev,
-                                      const unsigned short *st, size_t s0,
-                                      const double *ts, const double *tk,
-                                      const double *tp, double &fx,
-                                      double &fy, double &fz, int &nbroken)
+
+// The fast evaluation of the bond to halo entry `ev` (byte offset of its
+// piece 0); for DM_NLIN st is the byte offset of the bond's (type, regime) in
+// the LDS tables.  Returns whether the result stands.
+//
+// A dead or empty slot (ev 0) needs no test here: entry 0 is a node at
+// (2^300, 2^300, 2^300) of weight 0, so that l == l0 and the force is zero.
+template <int DM, bool TENS, bool CLA>
+__device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
+                                          const double4 &r0i,
+                                          const double4 &ri, double ci,
+                                          unsigned ev, unsigned st,
+                                          Bond &o, double &kb, double &pb)
 {
     constexpr unsigned PB = piece_bytes<DM>();
-    // per bond, what the force needs: dr, 0.5/l, s/2 and the weight
-    double dx[W], dy[W], dz[W], hl[W], sh[W], w[W];
-    bool live[W], slow[W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        live[q] = ev[q] != LOC_DEAD;
-        // a dead slot reads the zero record at entry 0 (weight 0)
-        const char *pe = ldsb + 16u * ev[q];
+    const char *pe = ldsb + halo_base<DM>() + ev;
+    const double2 p0 = *reinterpret_cast<const double2 *>(pe);
+    const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
+    const double2 p2 = *reinterpret_cast<const double2 *>(pe + 2 * PB);
+    // c_j is read only by the node-field model
+    double2 p3;
+    if (DM == DM_FIELD) {
+        p3 = *reinterpret_cast<const double2 *>(pe + 3 * PB);
+    } else {
+        p3.x = *reinterpret_cast<const double *>(pe + 3 * PB);
+        p3.y = 0.0;
+    }
+    const double ex = p0.x - r0i.x;
+    const double ey = p0.y - r0i.y;
+    const double ez = p1.x - r0i.z;
+    if (CLA) {
+        // cl/peridynamics.cl:65-71: xi_eta = (u_j - u_i) + xi
+        o.dx = (p2.x - ri.x) + ex;
+        o.dy = (p2.y - ri.y) + ey;
+        o.dz = (p3.x - ri.z) + ez;
+    } else {
+        // spatial.pyx:20-31 with r = r0 + u: dr = r_j - r_i
+        o.dx = p2.x - ri.x;
+        o.dy = p2.y - ri.y;
+        o.dz = p3.x - ri.z;
+    }
+    const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
+    const double q0 = sq3<CLA>(ex, ey, ez);
+    double l, l0, h0;
+    sqrt_core(qq, l, o.hl);
+    sqrt_core(q0, l0, h0);
+    o.sh = (l - l0) * h0;  // s/2, from h0 ~ 0.5/l0
+    // k = (c_i + c_j)/2 for a field: s k/l V_j = (s/2)(0.5/l) w with
+    // w = 2(c_i+c_j)V_j = c_i (2 V_j) + (2 c_j V_j), the staged pair
+    o.w = DM == DM_FIELD ? __builtin_fma(ci, p1.y, p3.y) : p1.y;
+    if constexpr (DM == DM_NLIN) {
+        const double2 c = *reinterpret_cast<const double2 *>(ldsb + st);
+        const double2 k = *reinterpret_cast<const double2 *>(
+            ldsb + 16 * MAX_TAB + st);
+        kb = k.x;
+        pb = k.y;
+        return (o.sh < c.y) & (o.sh > c.x);
+    } else if constexpr (TENS) {
+        return (o.sh < a.lim) & (o.sh > -0.25);
+    } else {
+        return fabs(o.sh) < a.lim;
+    }
+}
+
+// The bond at slot `slot` with IEEE square roots and division
+// (spatial.pyx:87-97, cl/peridynamics.cl:72-74): decides whether it breaks or
+// changes its regime, writes that, and leaves in `o` (and kb, pb for
+// DM_NLIN) what the force needs, zero for a broken or empty slot.
+template <int DM, bool TENS, bool CLA>
+__device__ __forceinline__ void bond_exact(const StepArgs &a,
+                                           const char *ldsb,
+                                           const double4 &r0i, unsigned ev,
+                                           unsigned st, size_t slot, Bond &o,
+                                           double &kb, double &pb,
+                                           int &nbroken)
+{
+    constexpr unsigned PB = piece_bytes<DM>();
+    bool live = ev != LOC_DEAD;
+    if (live) {
+        const char *pe = ldsb + halo_base<DM>() + ev;
         const double2 p0 = *reinterpret_cast<const double2 *>(pe);
         const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
-        const double2 p2 = *reinterpret_cast<const double2 *>(pe + 2 * PB);
-        // c_j is read only by the node-field model
-        double2 p3;
-        if (DM == DM_FIELD) {
-            p3 = *reinterpret_cast<const double2 *>(pe + 3 * PB);
-        } else {
-            p3.x = *reinterpret_cast<const double *>(pe + 3 * PB);
-            p3.y = 0.0;
-        }
+        const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
         const double ex = p0.x - r0i.x;
         const double ey = p0.y - r0i.y;
         const double ez = p1.x - r0i.z;
-        if (CLA) {
-            // cl/peridynamics.cl:65-71: xi_eta = (u_j - u_i) + xi
-            dx[q] = (p2.x - ri.x) + ex;
-            dy[q] = (p2.y - ri.y) + ey;
-            dz[q] = (p3.x - ri.z) + ez;
-        } else {
-            // spatial.pyx:20-31 with r = r0 + u: dr = r_j - r_i
-            dx[q] = p2.x - ri.x;
-            dy[q] = p2.y - ri.y;
-            dz[q] = p3.x - ri.z;
-        }
-        const double qq = sq3<CLA>(dx[q], dy[q], dz[q]);
         const double q0 = sq3<CLA>(ex, ey, ez);
-        double l, l0, h0;
-        sqrt_core(qq, l, hl[q]);
-        sqrt_core(q0, l0, h0);
-        sh[q] = (l - l0) * h0;  // s/2, from h0 ~ 0.5/l0
-        // k = (c_i + c_j)/2 for a field: s k/l V_j = (s/2)(0.5/l) w with
-        // w = 2(c_i+c_j)V_j = c_i (2 V_j) + (2 c_j V_j), the staged pair
-        w[q] = DM == DM_FIELD ? __builtin_fma(ci, p1.y, p3.y) : p1.y;
-        // sqrt_core is exact on [2^-767, inf).  With !(|s| < s0) as the
-        // break test, one compare covers both lengths: with q >= 2^-700, a
-        // q0 below 2^-767 (l0 < 2^-383.5, zero included) gives s > 2^33 or
-        // NaN and an infinite or NaN q0 gives NaN, so the bond breaks here
-        // as in the reference (unless s0 > 2^33); an infinite q gives NaN
-        // here and an infinite s there, both breaking.  q below 2^-700, or
-        // NaN, takes the exact path.  The tension test and the regime walk
-        // check both lengths.
-        bool fast;
-        if constexpr (DM != DM_NLIN && !TENS)
-            fast = qq >= 0x1p-700;
-        else
-            fast = core_range(qq) & core_range(q0);
-        bool near;
-        if (DM != DM_NLIN) {
-            near = fabs((TENS ? sh[q] : fabs(sh[q])) - a.s0h) <= a.s0h_guard;
-        } else {
-            // (lower, upper) thresholds of the bond's regime; regime 0's
-            // lower one is -DBL_MAX, which no stretch is near
-            const double2 c = reinterpret_cast<const double2 *>(
-                ts)[(st[q] >> 8) * a.nregimes + (st[q] & 0xff)];
-            near = fabs(sh[q] - c.y) <= GUARD * fabs(c.y) ||
-                   fabs(sh[q] - c.x) <= GUARD * fabs(c.x);
-        }
-        slow[q] = live[q] & (!fast | near);
-    }
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        if (slow[q]) {
-            // rare: near a threshold, or a square root outside the core's
-            // range: IEEE square roots and division (spatial.pyx:87-97,
-            // cl/peridynamics.cl:72-74)
-            const char *pe = ldsb + 16u * ev[q];
-            const double2 p0 = *reinterpret_cast<const double2 *>(pe);
-            const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
-            const double qq = sq3<CLA>(dx[q], dy[q], dz[q]);
-            const double ex = p0.x - r0i.x;
-            const double ey = p0.y - r0i.y;
-            const double ez = p1.x - r0i.z;
-            const double q0 = sq3<CLA>(ex, ey, ez);
-            const double l = sqrt(qq), l0 = sqrt(q0);
-            if (!(core_range(qq) & core_range(q0)))
-                hl[q] = 0.5 / l;
-            sh[q] = ((l - l0) / l0) * 0.5;
-        }
-    }
-    double cr[W];
-#pragma unroll
-    for (int q = 0; q < W; ++q)
-        cr[q] = CORR ? a.corr[s0 + q] : 1.0;
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        if (!live[q])
-            continue;
-        double g;
-        if (DM != DM_NLIN) {
-            if (!((TENS ? sh[q] : fabs(sh[q])) < a.s0h)) {
-                a.loc[s0 + q] = LOC_DEAD;
-                if (a.brk)
-                    a.brk[s0 + q] = a.step;
-                a.gidx[s0 + q] |=
-                    (int)(DEAD | (a.layout == PD_LAYOUT_COMPACT ? NEWB : 0u));
-                ++nbroken;
-                continue;
-            }
-            // s k/l V_j = (s/2)(0.5/l)(4 k V_j)
-            g = sh[q] * hl[q] * w[q];
+        const double l = sqrt(qq), l0 = sqrt(q0);
+        if (!(core_range(qq) & core_range(q0)))
+            o.hl = 0.5 / l;
+        o.sh = ((l - l0) / l0) * 0.5;
+        if constexpr (DM != DM_NLIN) {
+            live = (TENS ? o.sh : fabs(o.sh)) < a.s0h;
         } else {
             // cl/peridynamics.cl:326-378 (bond_force3/4), thresholds halved
-            const int t = st[q] >> 8;
-            const int reg = st[q] & 0xff;
+            const int t = (int)(st >> 4) / a.nregimes;
+            const int reg = (int)(st >> 4) - t * a.nregimes;
             const int base = t * a.nregimes;
-            const double2 c =
-                reinterpret_cast<const double2 *>(ts)[base + reg];
-            const double c_hi = c.y, c_lo = c.x;
             int nreg = reg;
-            if (sh[q] < c_hi) {
-                if (reg > 0 && sh[q] < c_lo)
+            if (o.sh < a.s_tab[base + reg] * 0.5) {
+                if (reg > 0 && o.sh < a.s_tab[base + reg - 1] * 0.5)
                     nreg = reg - 1;
             } else {
                 nreg = reg + 1;
             }
-            if (nreg != reg)
-                a.state[s0 + q] = (unsigned short)((t << 8) | nreg);
-            if (nreg >= a.nregimes) {
-                a.loc[s0 + q] = LOC_DEAD;
-                if (a.brk)
-                    a.brk[s0 + q] = a.step;
-                a.gidx[s0 + q] |= (int)DEAD;
-                ++nbroken;
-                continue;
+            live = nreg < a.nregimes;
+            if (live) {
+                if (nreg != reg)
+                    a.state[slot] = (unsigned short)((base + nreg) << 4);
+                kb = 4.0 * a.k_tab[base + nreg];
+                pb = 2.0 * a.pc_tab[base + nreg];
             }
-            // (bond stiffness, plus_cs) of the new regime
-            const double2 kp =
-                reinterpret_cast<const double2 *>(tk)[base + nreg];
-            const double fn = __builtin_fma(sh[q] + sh[q], kp.x, kp.y);
-            g = fn * (hl[q] + hl[q]) * w[q];
         }
-        if (CORR)
-            g *= cr[q];
-        fx = __builtin_fma(g, dx[q], fx);
-        fy = __builtin_fma(g, dy[q], fy);
-        fz = __builtin_fma(g, dz[q], fz);
+        if (!live) {
+            a.loc[slot] = LOC_DEAD;
+            if (a.brk)
+                a.brk[slot] = a.step;
+            a.gidx[slot] |=
+                (int)(DEAD | (a.layout == PD_LAYOUT_COMPACT ? NEWB : 0u));
+            ++nbroken;
+        }
+    }
+    if (!live) {
+        // a displacement that is not finite must not reach the sum either
+        o.dx = o.dy = o.dz = o.sh = o.hl = o.w = 0.0;
+        kb = pb = 0.0;
     }
 }
 
-// A chunk's bond data: the halo indices and, for DM_NLIN, the bond states.
+// A chunk's bond data: the halo entries and, for DM_NLIN, the bond states,
+// with CORR the corrections.
+template <bool CORR>
 struct Chunk {
-    ushort4 loc, st;
+    uint2 loc, st;
+    double2 ca, cb;
 };
 
-// A chunk of four bonds of node i, slots s0 .. s0+3.  The pieces of halo
-// entry h are (r0x, r0y) (r0z, w) (rx, ry) (rz, v), as the records: w =
-// 4 k V for DM_PMB, 2 V for DM_FIELD and V for DM_NLIN; v = 2 c V for
-// DM_FIELD.  The bonds go two at a time: their reads are
-// issued first and the arithmetic is straight-line code (a dead slot
-// computes on the zero record and is masked), so the two chains interleave.
-// (Four at a time is no faster and needs 40 more registers, which the
-// field and n-linear models would spill.)  Only the exact-division path -- a stretch
-// near a threshold, or a square root outside the core's range -- and
-// breaking branch.
+template <>
+struct Chunk<false> {
+    uint2 loc, st;
+};
+
+// Two bonds of node i, at slots s0 and s0 + 1: `lw` their halo entries, `sw`
+// their states, `cr` their corrections.  The two are straight-line code whose
+// chains interleave; only a bond near a threshold (or broken by this step)
+// leaves it.
 template <int DM, bool CORR, bool TENS, bool CLA>
-__device__ __forceinline__ void chunk4(const StepArgs &a, const char *ldsb,
-                                       const double4 &r0i, const double4 &ri,
-                                       double ci,
-                                       const Chunk &ch, size_t s0,
-                                       const double *ts, const double *tk,
-                                       const double *tp, double &fx,
-                                       double &fy, double &fz, int &nbroken)
+__device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
+                                          const double4 &r0i,
+                                          const double4 &ri, double ci,
+                                          unsigned lw, unsigned sw, double2 cr,
+                                          size_t s0, double &fx, double &fy,
+                                          double &fz, int &nbroken)
 {
-    const unsigned ev[4] = {ch.loc.x, ch.loc.y, ch.loc.z, ch.loc.w};
-    const unsigned short st[4] = {ch.st.x, ch.st.y, ch.st.z, ch.st.w};
-    bonds<DM, 2, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, ev, st, s0, ts, tk,
-                                  tp, fx, fy, fz, nbroken);
-    bonds<DM, 2, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, ev + 2, st + 2,
-                                  s0 + 2, ts, tk, tp, fx, fy, fz, nbroken);
+    Bond o[2];
+    double kb[2], pb[2];
+    const unsigned ev[2] = {lw & 0xffffu, lw >> 16};
+    const unsigned st[2] = {sw & 0xffffu, sw >> 16};
+    const bool ok0 = bond_fast<DM, TENS, CLA>(a, ldsb, r0i, ri, ci, ev[0],
+                                              st[0], o[0], kb[0], pb[0]);
+    const bool ok1 = bond_fast<DM, TENS, CLA>(a, ldsb, r0i, ri, ci, ev[1],
+                                              st[1], o[1], kb[1], pb[1]);
+    if (__builtin_expect(!(ok0 & ok1), 0)) {
+        if (!ok0)
+            bond_exact<DM, TENS, CLA>(a, ldsb, r0i, ev[0], st[0], s0, o[0],
+                                      kb[0], pb[0], nbroken);
+        if (!ok1)
+            bond_exact<DM, TENS, CLA>(a, ldsb, r0i, ev[1], st[1], s0 + 1,
+                                      o[1], kb[1], pb[1], nbroken);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        // s k/l V_j = (s/2)(0.5/l)(4 k V_j); n-linear (s k + plus_cs)/l V_j
+        // = ((s/2)(4 k) + 2 plus_cs)(0.5/l) V_j, the tables scaled
+        double g = DM == DM_NLIN ? __builtin_fma(o[q].sh, kb[q], pb[q])
+                                 : o[q].sh;
+        g = g * o[q].hl * o[q].w;
+        if (CORR)
+            g *= q ? cr.y : cr.x;
+        fx = __builtin_fma(g, o[q].dx, fx);
+        fy = __builtin_fma(g, o[q].dy, fy);
+        fz = __builtin_fma(g, o[q].dz, fz);
+    }
 }
 
+// What bounds it: the VALU, busy ~75 % of the cycles on the 1,038,230-node
+// beam (1.16e8 wave instructions per launch before, mostly FP64 at 4 cycles
+// and more; the clock gives way under that load).  So the bond loop has one
+// compare per bond for everything that is rare, dead slots cost no test, LDS
+// offsets come ready from loc, chunk loads step one 32-bit offset, and a row
+// runs half rounds: 305 -> 270 us a step there, 113 -> 77 on the 263k-node
+// composite bar (its state now is the LDS offset of the bond's table entry),
+// 57 -> 48 on a 141k-node bar with corrections (requested with the chunk).
+//
 // DM: DM_PMB, DM_NLIN or DM_FIELD.  One workgroup per tile, LPN lanes per
 // node taking its 4-bond chunks round-robin and reducing with cross-lane
-// shuffles.  LDS (static, LDS_BYTES): the halo, four pieces of
-// piece_bytes<DM>() each, then for DM_NLIN the three damage-model tables.
+// shuffles.  LDS (static, LDS_BYTES): for DM_NLIN the
+// damage-model tables, then the halo, four pieces of piece_bytes<DM>() each.
 // CLA: the slot layout's OpenCL arithmetic (records hold u, updates
 // contracted); otherwise the Cython path's (records hold r0 + u).
 template <int DM, int LPN, bool CORR, bool TENS, bool CLA>
@@ -652,27 +714,53 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
     const TileInfo ti = a.tiles[tile];
     char *ldsb = reinterpret_cast<char *>(lds);
 
-    // node state and the first DEPTH chunks of halo indices are requested
-    // before the halo is staged, so their latency overlaps the staging; the
-    // bond loop then keeps DEPTH chunk loads in flight.  Chunk rows are
-    // clamped to the tile's longest row (a node's surplus loads are unused).
-    constexpr int DEPTH = 4;
     const int l = threadIdx.x / LPN;
     const int sub = threadIdx.x % LPN;
     const bool valid = l < ti.nodes;
-    const ushort4 *L4 = reinterpret_cast<const ushort4 *>(a.loc);
-    const long long c0 = ti.chunk_off + (valid ? l : 0);
-    const int last_row = max(ti.nch, 1) - 1;
-    const ushort4 *S4 = reinterpret_cast<const ushort4 *>(a.state);
-    auto chunk_at = [&](int c) {
-        const long long k = c0 + (long long)min(c, last_row) * ti.nodes;
-        Chunk ch;
-        ch.loc = L4[k];
-        ch.st = DM == DM_NLIN ? S4[k] : make_ushort4(0, 0, 0, 0);
+
+    // the halo's node indices first: the records they name are the longest
+    // chain of this kernel.  Thread x copies 16-byte piece x%4 of records
+    // x/4, x/4 + blockDim/4, ...
+    constexpr int SP = 10;
+    constexpr unsigned PB = piece_bytes<DM>();
+    const int *H = a.halo + ti.halo_off;
+    const unsigned e0 = threadIdx.x >> 2;
+    const unsigned piece = threadIdx.x & 3u;
+    const unsigned eper = blockDim.x >> 2;
+    const unsigned elast = (unsigned)ti.halo - 1u;
+    unsigned hi[SP];
+    unsigned hx = e0;
+    static_for<SP>([&](auto k) {
+        hi[k] = (unsigned)H[min(hx, elast)];
+        hx += eper;
+    });
+
+    // node state and the first chunks of halo entries are requested before
+    // the halo is staged, so their latency overlaps the staging.  Chunk rows
+    // past the node's last are never used (their loads stay inside loc's
+    // allocation, which is LOC_SLACK slots longer than the tiles need).
+    const char *L = reinterpret_cast<const char *>(a.loc + 4 * ti.chunk_off);
+    const char *S = reinterpret_cast<const char *>(a.state + 4 * ti.chunk_off);
+    const char *C = reinterpret_cast<const char *>(a.corr + 4 * ti.chunk_off);
+    const unsigned cstep = 8u * LPN * (unsigned)ti.nodes;
+    unsigned coff = 8u * ((valid ? (unsigned)l : 0u) +
+                          (unsigned)sub * (unsigned)ti.nodes);
+    auto chunk_at = [&](unsigned off) {
+        Chunk<CORR> ch;
+        ch.loc = *reinterpret_cast<const uint2 *>(L + off);
+        if constexpr (DM == DM_NLIN)
+            ch.st = *reinterpret_cast<const uint2 *>(S + off);
+        else
+            ch.st = make_uint2(0u, 0u);
+        if constexpr (CORR) {
+            const double2 *c =
+                reinterpret_cast<const double2 *>(C + 4ull * off);
+            ch.ca = c[0];
+            ch.cb = c[1];
+        }
         return ch;
     };
-    Chunk q0 = chunk_at(sub), q1 = chunk_at(sub + LPN),
-          q2 = chunk_at(sub + 2 * LPN), q3 = chunk_at(sub + 3 * LPN);
+    Chunk<CORR> qa = chunk_at(coff), qb = chunk_at(coff + cstep);
     int cnt = 0;
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     double4 r0i = make_double4(0.0, 0.0, 0.0, 0.0), ri = r0i;
@@ -701,63 +789,103 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         }
     }
 
-    // stage the halo: piece x copies 16-byte piece x%4 of record x/4 into
-    // entry x/4 + 1, SP pieces per thread in flight at once (loads clamped in
-    // bounds, stores predicated)
-    constexpr int SP = 10;
-    constexpr unsigned PB = piece_bytes<DM>();
-    const int np = 4 * ti.halo;
-    for (int x0 = threadIdx.x; x0 < np; x0 += SP * blockDim.x) {
-        double2 v[SP];
-#pragma unroll
-        for (int k = 0; k < SP; ++k) {
-            const int x = min(x0 + k * (int)blockDim.x, np - 1);
-            const int g = a.halo[ti.halo_off + (x >> 2)];
-            v[k] = reinterpret_cast<const double2 *>(a.rec_old + g)[x & 3];
-        }
-#pragma unroll
-        for (int k = 0; k < SP; ++k) {
-            const int x = x0 + k * (int)blockDim.x;
-            if (x < np) {
-                const double2 w = v[k];
-                *reinterpret_cast<double2 *>(
-                    ldsb + (x & 3) * PB + 16u * (unsigned)((x >> 2) + 1)) = w;
-            }
-        }
+    // stage the halo, SP pieces per thread in flight at once (a block of
+    // 512 threads needs one pass).  Pieces past the last entry store that
+    // entry again: a condition would move each load next to its store.
+    const char *R = reinterpret_cast<const char *>(a.rec_old);
+    char *D = ldsb + halo_base<DM>() + piece * PB + 16u;
+    {
+        v2d v[SP];
+        static_for<SP>([&](auto k) {
+            v[k] = *reinterpret_cast<const v2d *>(
+                R + (hi[k] * 64u + piece * 16u));
+        });
+        unsigned x = e0;
+        static_for<SP>([&](auto k) {
+            *reinterpret_cast<v2d *>(D + 16u * min(x, elast)) = v[k];
+            x += eper;
+        });
     }
-    if (threadIdx.x < 4)  // entry 0: the zero record dead slots read
-        *reinterpret_cast<double2 *>(ldsb + threadIdx.x * PB) =
-            make_double2(0.0, 0.0);
+    for (unsigned x0 = hx; x0 - e0 <= elast; x0 += 4 * eper) {
+        v2d v[4];
+        unsigned x = x0;
+        static_for<4>([&](auto k) {
+            v[k] = *reinterpret_cast<const v2d *>(
+                R + ((unsigned)H[min(x, elast)] * 64u + piece * 16u));
+            x += eper;
+        });
+        x = x0;
+        static_for<4>([&](auto k) {
+            *reinterpret_cast<v2d *>(D + 16u * min(x, elast)) = v[k];
+            x += eper;
+        });
+    }
+    if (threadIdx.x < 4) {  // entry 0: what dead slots read
+        constexpr double FAR = 0x1p300;
+        double2 z = make_double2(0.0, 0.0);
+        if (threadIdx.x == 0 || (!CLA && threadIdx.x == 2))
+            z = make_double2(FAR, FAR);
+        else if (threadIdx.x == 1 || (!CLA && threadIdx.x == 3))
+            z.x = FAR;
+        *reinterpret_cast<double2 *>(ldsb + halo_base<DM>() +
+                                     threadIdx.x * PB) = z;
+    }
     // n-linear tables, one 16-byte read each: (lower, upper) halved
-    // thresholds of regime r of type t, and (stiffness, plus_cs)
-    double2 *tsp = reinterpret_cast<double2 *>(ldsb + 4 * PB);
-    double2 *tkp = tsp + MAX_TAB;
-    const double *ts = reinterpret_cast<const double *>(tsp);
-    const double *tk = reinterpret_cast<const double *>(tkp);
-    const double *tp = nullptr;
+    // thresholds of regime r of type t with their margin, and (4 stiffness,
+    // 2 plus_cs)
     if (DM == DM_NLIN) {
+        double2 *tsp = reinterpret_cast<double2 *>(ldsb);
+        double2 *tkp = tsp + MAX_TAB;
         for (int t = threadIdx.x; t < a.ntab; t += blockDim.x) {
-            const bool first = t % a.nregimes == 0;
-            tsp[t] = make_double2(first ? -__DBL_MAX__ : a.s_tab[t - 1] * 0.5,
-                                  a.s_tab[t] * 0.5);
-            tkp[t] = make_double2(a.k_tab[t], a.pc_tab[t]);
+            const double up = a.s_tab[t] * 0.5;
+            double lo = -0.25;
+            if (t % a.nregimes != 0) {
+                const double c = a.s_tab[t - 1] * 0.5;
+                lo = fmax(lo, c + GUARD * fabs(c));
+            }
+            tsp[t] = make_double2(
+                lo, a.lim > 0.0 ? up - GUARD * fabs(up) : -__DBL_MAX__);
+            tkp[t] = make_double2(4.0 * a.k_tab[t], 2.0 * a.pc_tab[t]);
         }
     }
     __syncthreads();
 
     double fx = 0.0, fy = 0.0, fz = 0.0;
     int nbroken = 0;
+    // nodes are sorted by descending bond count, so the wavefront's first
+    // node has its longest row: every lane runs that row's rounds (surplus
+    // slots are empty).  Round k's chunks hold 2-bond groups 8 apart
+    // (slot_of), so a row's last round of at most 8 bonds runs half of it.
+    const int cmax = __builtin_amdgcn_readfirstlane(cnt);
+    const unsigned cend = 8u * (unsigned)ti.nodes * (unsigned)ti.nch;
+    auto round = [&](const Chunk<CORR> &ch, int k, unsigned off) {
+        if (off >= cend)
+            return;  // past the tile's rows (LPN does not divide them)
+        const size_t s0 =
+            4 * ((size_t)ti.chunk_off + (off >> 3));
+        double2 ca = make_double2(1.0, 1.0), cb = ca;
+        if constexpr (CORR) {
+            ca = ch.ca;
+            cb = ch.cb;
+        }
+        bond_pair<DM, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, ch.loc.x,
+                                       ch.st.x, ca, s0, fx, fy, fz, nbroken);
+        if (16 * (LPN * k / 4) + 8 < cmax)
+            bond_pair<DM, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, ch.loc.y,
+                                           ch.st.y, cb, s0 + 2, fx, fy, fz,
+                                           nbroken);
+    };
+    const int rounds = (chunks_of(cmax) + LPN - 1) / LPN;
     if (valid) {
-        const int nch = (cnt + 3) >> 2;
-        for (int c = sub; c < nch; c += LPN) {
-            const Chunk nx = chunk_at(c + DEPTH * LPN);
-            const size_t s0 = (size_t)(c0 + (long long)c * ti.nodes) * 4;
-            chunk4<DM, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, q0, s0, ts, tk,
-                                        tp, fx, fy, fz, nbroken);
-            q0 = q1;
-            q1 = q2;
-            q2 = q3;
-            q3 = nx;
+        for (int k = 0; k < rounds; k += 2) {
+            round(qa, k, coff);
+            coff += cstep;
+            qa = chunk_at(coff + cstep);
+            if (k + 1 >= rounds)
+                break;
+            round(qb, k + 1, coff);
+            coff += cstep;
+            qb = chunk_at(coff + cstep);
         }
     }
 
@@ -1071,7 +1199,8 @@ __global__ void k_export_regimes(int n, int K, const int *tnode,
                                  const int *cnt, const long long *chunk0,
                                  const int *stride,
                                  const unsigned short *pos,
-                                 const unsigned short *state, int *out)
+                                 const unsigned short *state,
+                                 const int *gidx, int nregimes, int *out)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n)
@@ -1080,7 +1209,9 @@ __global__ void k_export_regimes(int n, int K, const int *tnode,
     const int c = cnt[p];
     for (int k = 0; k < c; ++k) {
         const size_t s = slot_of(chunk0[p], stride[p], k);
-        out[row + pos[s]] = state[s] & 0xff;
+        // a broken bond has walked past its last regime
+        out[row + pos[s]] =
+            gidx[s] < 0 ? nregimes : (state[s] >> 4) % nregimes;
     }
 }
 
@@ -1187,7 +1318,7 @@ __device__ __forceinline__ ExactTerm exact_term(const char *ldsb, unsigned e,
                                                 const double4 &rm, double k)
 {
     constexpr unsigned PB = 16u * EXACT_CAP;
-    const char *pe = ldsb + 16u * e;
+    const char *pe = ldsb + e;
     const double2 p0 = *reinterpret_cast<const double2 *>(pe);
     const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
     const double2 p2 = *reinterpret_cast<const double2 *>(pe + 2 * PB);
@@ -1595,7 +1726,7 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     const int4 *B4 = reinterpret_cast<const int4 *>(a.brk);
     const double2 *I2 = reinterpret_cast<const double2 *>(a.il0);
     const long long c0 = ti.chunk_off + l;
-    const int nch = (cnt + 3) >> 2;
+    const int nch = chunks_of(cnt);
     for (int c = sub; c < nch; c += LPN) {
         const long long k = c0 + (long long)c * ti.nodes;
         const ushort4 lc = L4[k];
@@ -1608,7 +1739,7 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
         for (int q = 0; q < 4; ++q) {
             if (ev[q] == LOC_DEAD || br[q] <= a.step)
                 continue;  // empty, or broken before or in this step
-            const char *pe = ldsb + 16u * ev[q];
+            const char *pe = ldsb + ev[q];
             const double2 p0 = *reinterpret_cast<const double2 *>(pe);
             const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
             const double2 p2 =
@@ -1727,6 +1858,8 @@ struct pd_sim {
     int hstride = 0;        // largest halo of the current tiles
     size_t lds_budget = 0;  // bytes of LDS a workgroup may use
     int ntiles = 0;
+    size_t nslots = 0;  // bond slots of the tiles (loc holds LOC_SLACK more)
+    bool coords_core = false;  // coordinates in bond_fast's range
     bool retile_pending = false;  // tile_nodes changed since the tiling
     bool has_buffers = false, has_corr = false, has_btypes = false,
          has_cnode = false;
@@ -1881,7 +2014,11 @@ StepArgs make_args(pd_sim *s)
     a.dt = s->dt;
     a.damping = s->damping;
     a.s0h = s->s0 * 0.5;
-    a.s0h_guard = GUARD * a.s0h;
+    // coordinates outside the range that bond_fast relies on: every bond
+    // takes the exact path
+    a.lim = !s->coords_core ? -1.0
+            : dm_of(s) == DM_NLIN ? 1.0
+                                  : std::min(a.s0h * (1.0 - GUARD), 0.25);
     a.rec_old = s->rec[s->cur].p;
     a.rec_new = s->rec[1 - s->cur].p;
     a.tiles = s->tiles.p;
@@ -2186,7 +2323,7 @@ std::vector<int> spread_halo(const std::vector<std::vector<int>> &rows,
         const int q1 = std::min(q0 + 16, lanes);
         int rounds = 0;
         for (int t = q0; t < q1; ++t) {
-            const int nch = ((int)rows[t / lpn].size() + 3) / 4;
+            const int nch = chunks_of((int)rows[t / lpn].size());
             rounds = std::max(rounds, (nch - t % lpn + lpn - 1) / lpn);
         }
         for (int k = 0; k < rounds; ++k)
@@ -2194,7 +2331,9 @@ std::vector<int> spread_halo(const std::vector<std::vector<int>> &rows,
                 const int g = ngroups++;
                 for (int t = q0; t < q1; ++t) {
                     const std::vector<int> &row = rows[t / lpn];
-                    const int p = 4 * (t % lpn + lpn * k) + b;
+                    const int c = t % lpn + lpn * k;
+                    const int p = 16 * (c >> 2) + 8 * (b >> 1) +
+                                  2 * (c & 3) + (b & 1);
                     if (p < (int)row.size() && seen[row[p]] != g) {
                         seen[row[p]] = g;
                         memb[row[p]].push_back(g);
@@ -2385,6 +2524,11 @@ int pd_build(pd_sim **out, int device, int integrator, int layout, double dt,
     s->hmax = LDS_CAP_PMB - 1;
     const size_t N = (size_t)nnodes;
     s->h_coords.assign(coords, coords + 3 * N);
+    s->coords_core = true;
+    for (size_t q = 0; q < 3 * N && s->coords_core; ++q) {
+        const double x = std::fabs(coords[q]);
+        s->coords_core = x == 0.0 || (x >= 0x1p-290 && x <= 0x1p300);
+    }
 
     std::vector<int> flags(N);
     for (size_t i = 0; i < N; ++i) {
@@ -2635,7 +2779,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         halo_total += t.halo;
         int nch = 0;
         for (int l = 0; l < t.nodes; ++l)
-            nch = std::max(nch, (cnt[tnode[t.node_off + l]] + 3) >> 2);
+            nch = std::max(nch, chunks_of(cnt[tnode[t.node_off + l]]));
         t.nch = nch;
         t.pad = 0;
         t.chunk_off = chunk_total;
@@ -2646,15 +2790,15 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         return fail(PD_E_LIMIT, "total halo size exceeds 2^31");
     const size_t S = (size_t)chunk_total * 4;
     std::vector<int> halo(halo_total);
-    std::vector<unsigned short> loc(S, LOC_DEAD);
+    std::vector<unsigned short> loc(S + LOC_SLACK, LOC_DEAD);
     std::vector<int> gidx(S, (int)DEAD);
     std::vector<unsigned short> pos(S, 0);
     std::vector<double> corr;
     std::vector<unsigned short> state;
     if (s->has_corr)
-        corr.assign(S, 0.0);
+        corr.assign(S + LOC_SLACK, 0.0);
     if (nlin)
-        state.assign(S, 0);
+        state.assign(S + LOC_SLACK, 0);
     std::vector<long long> chunk0(N);
     std::vector<int> stride(N);
     const bool compact = s->layout == PD_LAYOUT_COMPACT;
@@ -2704,7 +2848,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                     const int j = rj[rstart[i] + k];
                     const int p = rp[rstart[i] + k];
                     const size_t sl = slot_of(ti.chunk_off + l, ti.nodes, k);
-                    loc[sl] = (unsigned short)(lmap[inv[j]] + 1);
+                    loc[sl] = (unsigned short)(16 * (lmap[inv[j]] + 1));
                     gidx[sl] = j;
                     pos[sl] = (unsigned short)p;
                     const size_t src = (size_t)i * K + p;
@@ -2712,7 +2856,8 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                         corr[sl] = s->h_corr[src];
                     if (nlin)
                         state[sl] = (unsigned short)(
-                            (s->h_btypes[src] << 8) | (regimes ? regimes[src] : 0));
+                            16 * (s->h_btypes[src] * nregimes +
+                                  (regimes ? regimes[src] : 0)));
                 }
                 if (compact) {
                     // row position -> slot, then the exact step's lists:
@@ -2758,6 +2903,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
             rc = fail(PD_E_HIP, std::string(what) + ": " + hipGetErrorString(e));
     };
     s->ntiles = ntiles;
+    s->nslots = S;
     s->hstride = 1;
     for (const auto &t : tiles)
         s->hstride = std::max(s->hstride, t.halo);
@@ -3268,7 +3414,7 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
     if (nsteps < 1 || checkpoint_every < 1)
         return fail(PD_E_ARG, "nsteps and checkpoint_every must be >= 1");
     adjoint_release(s);
-    const size_t S = s->loc.n, N = (size_t)s->n, B = 3 * N;
+    const size_t S = s->nslots, N = (size_t)s->n, B = 3 * N;
     const int nck = (nsteps + checkpoint_every - 1) / checkpoint_every;
     std::vector<int> inv(N);
     for (size_t q = 0; q < N; ++q)
@@ -3596,7 +3742,8 @@ int pd_get_regimes(pd_sim *s, int *regimes)
     const int blocks = (s->n + 255) / 256;
     hipLaunchKernelGGL(k_export_regimes, dim3(blocks), dim3(256), 0,
                        s->stream, s->n, s->K, s->tnode.p, s->cnt.p,
-                       s->chunk0.p, s->stride.p, s->pos.p, s->state.p, out.p);
+                       s->chunk0.p, s->stride.p, s->pos.p, s->state.p,
+                       s->gidx.p, s->nregimes, out.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->stream));
     HIPCHK(hipMemcpy(regimes, out.p, NK * sizeof(int), hipMemcpyDeviceToHost));
@@ -3651,7 +3798,7 @@ int pd_tile_stats(pd_sim *s, int *ntiles, int *hmax, int *hstride,
     if (halo_total)
         *halo_total = (long long)s->halo.n;
     if (slots)
-        *slots = (long long)s->loc.n;
+        *slots = (long long)s->nslots;
     return PD_OK;
 }
 
