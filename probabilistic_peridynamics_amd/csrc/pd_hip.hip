@@ -1055,42 +1055,80 @@ __global__ void k_records(int n, double wscale, int ucla, const double *r0,
     rec1[i] = r;
 }
 
+// Lanes per node of the kernels that walk every row once.  Over the chunks of
+// the rows (live counts, recordings) four: a wavefront then reads 128
+// contiguous bytes of loc in each of four chunk rows, and each lane's loads
+// are independent.  Over the caller's rows (lists) sixteen: 64 contiguous
+// bytes of a row at a time.
+constexpr int CHUNK_LANES = 4;
+constexpr int ROW_LANES = 16;
+
+// Live slots of a node, counted by its LANES lanes (every lane gets the sum):
+// loc is 0 in a broken or empty slot.
+template <int LANES>
+__device__ __forceinline__ int live_slots(const unsigned short *loc,
+                                          long long chunk0, int stride,
+                                          int cnt, int sub)
+{
+    const uint2 *L = reinterpret_cast<const uint2 *>(loc) + chunk0;
+    const int nch = chunks_of(cnt);
+    int live = 0;
+#pragma unroll 4
+    for (int c = sub; c < nch; c += LANES) {
+        const uint2 v = L[(long long)c * stride];
+        live += ((v.x & 0xffffu) != 0) + ((v.x >> 16) != 0) +
+                ((v.y & 0xffffu) != 0) + ((v.y >> 16) != 0);
+    }
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1)
+        live += __shfl_xor(live, off, LANES);
+    return live;
+}
+
 // Live-slot count per node, the damage (family - n)/family
 // (peridynamics.pyx:29), and, for the slot layout, the reference-layout
-// neighbour list: -1 everywhere but at the live slots' columns.  Thread p
-// handles internal node p and writes row tnode[p] of the outputs.
+// neighbour list: -1 everywhere but at the live slots' columns.  LANES
+// lanes handle internal node p and write row tnode[p] of the outputs.
 // rows == 0 counts the live bonds without rebuilding the slot-layout rows.
-__global__ void k_export(int n, int K, int layout, int rows, const int *tnode,
-                         const int *cnt, const long long *chunk0,
-                         const int *stride, const int *gidx,
-                         const unsigned short *pos, const int *family,
-                         const int *n_neigh_c, int *nlist_out,
-                         int *n_neigh_out, double *damage)
+// Without rows it reads 2 B per slot (loc): 3.8 us on a 2560-node bar and 83
+// on 1,038,230 nodes, where one lane per node walking gidx took 23 and 243.
+template <int LANES>
+__global__ void __launch_bounds__(256)
+    k_export(int n, int K, int layout, int rows, const int *tnode,
+             const int *cnt, const long long *chunk0, const int *stride,
+             const unsigned short *loc, const int *gidx,
+             const unsigned short *pos, const int *family,
+             const int *n_neigh_c, int *nlist_out, int *n_neigh_out,
+             double *damage)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n)
-        return;
-    const int i = tnode[p];
-    int live;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int p = t / LANES, sub = t % LANES;
+    const bool valid = p < n;
+    const int i = valid ? tnode[p] : 0;
+    int live = 0;
     if (layout == PD_LAYOUT_SLOT) {
-        int *row = nlist_out + (size_t)i * K;
-        if (rows)
-            for (int q = 0; q < K; ++q)
-                row[q] = -1;
-        live = 0;
-        const int c = cnt[p];
-        for (int k = 0; k < c; ++k) {
-            const size_t s = slot_of(chunk0[p], stride[p], k);
-            const int e = gidx[s];
-            if (e >= 0) {
-                if (rows)
+        const int c = valid ? cnt[p] : 0;
+        const long long c0 = valid ? chunk0[p] : 0;
+        const int st = valid ? stride[p] : 0;
+        live = live_slots<LANES>(loc, c0, st, c, sub);
+        if (rows) {
+            int *row = nlist_out + (size_t)i * K;
+            if (valid)
+                for (int q = sub; q < K; q += LANES)
+                    row[q] = -1;
+            __syncthreads();  // the row is cleared before its bonds are set
+            for (int k = sub; k < c; k += LANES) {
+                const size_t s = slot_of(c0, st, k);
+                const int e = gidx[s];
+                if (e >= 0)
                     row[pos[s]] = e;
-                ++live;
             }
         }
-    } else {
+    } else if (valid) {
         live = n_neigh_c[i];
     }
+    if (!valid || sub != 0)
+        return;
     n_neigh_out[i] = live;
     const double f = (double)family[i];
     damage[i] = (f - (double)live) / f;
@@ -1100,17 +1138,19 @@ __global__ void k_export(int n, int K, int layout, int rows, const int *tnode,
 // positions below the row's count at set-up list their slots' keys (live
 // ones first, then what swap-with-last left behind); the others keep the
 // caller's values (uploaded into nlist_ref at set-up).
-__global__ void k_export_rows(int n, int K, const int *tnode, const int *cnt,
-                              const long long *chunk0, const int *stride,
-                              const int *gidx, const unsigned short *rslot,
-                              int *nlist_ref)
+__global__ void __launch_bounds__(256)
+    k_export_rows(int n, int K, const int *tnode, const int *cnt,
+                  const long long *chunk0, const int *stride,
+                  const int *gidx, const unsigned short *rslot,
+                  int *nlist_ref)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int p = t / ROW_LANES, sub = t % ROW_LANES;
     if (p >= n)
         return;
     const size_t row = (size_t)tnode[p] * K;
     const int c = cnt[p];
-    for (int q = 0; q < c; ++q)
+    for (int q = sub; q < c; q += ROW_LANES)
         nlist_ref[row + q] =
             (int)((uint32_t)gidx[slot_of(chunk0[p], stride[p],
                                          rslot[row + q])] & KEYM);
@@ -1215,27 +1255,26 @@ __global__ void k_export_regimes(int n, int K, const int *tnode,
     }
 }
 
-__global__ void k_live(int n, const int *cnt, const long long *chunk0,
-                       const int *stride, const int *gidx,
-                       unsigned long long *total)
+__global__ void __launch_bounds__(256)
+    k_live(int n, const int *cnt, const long long *chunk0, const int *stride,
+           const unsigned short *loc, unsigned long long *total)
 {
-    __shared__ unsigned long long part[256];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long live = 0;
-    if (i < n) {
-        const int c = cnt[i];
-        for (int k = 0; k < c; ++k)
-            live += gidx[slot_of(chunk0[i], stride[i], k)] >= 0;
-    }
-    part[threadIdx.x] = live;
+    __shared__ int part[256 / CHUNK_LANES];
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int p = t / CHUNK_LANES, sub = t % CHUNK_LANES;
+    const bool valid = p < n;
+    const int live =
+        live_slots<CHUNK_LANES>(loc, valid ? chunk0[p] : 0, valid ? stride[p] : 0,
+                   valid ? cnt[p] : 0, sub);
+    if (sub == 0)
+        part[threadIdx.x / CHUNK_LANES] = live;
     __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s)
-            part[threadIdx.x] += part[threadIdx.x + s];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+        for (int k = 0; k < 256 / CHUNK_LANES; ++k)
+            sum += (unsigned long long)part[k];
+        atomicAdd(total, sum);
     }
-    if (threadIdx.x == 0)
-        atomicAdd(total, part[0]);
 }
 
 // --- exact-order Euler step of the Cython path ----------------------------
@@ -1543,22 +1582,35 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
 //   dL/dc_m += dt/2 sum_j (1/l0 - 1/l)_mj d_mj . (V_j mu_m - V_m mu_j).
 
 // Bond state at the start of step n0: alive iff it broke at a step >= n0.
-__global__ void k_adj_restore(int n, int n0, const int *cnt,
-                              const long long *chunk0, const int *stride,
-                              const int *brk, const unsigned short *loc0,
-                              unsigned short *loc, int *gidx)
+// Slots are taken four at a time, whatever node they belong to (an empty slot
+// has brk -1), and gidx is written only where it changes.
+__global__ void __launch_bounds__(256)
+    k_adj_restore(long long nchunks, int n0, const int *brk,
+                  const unsigned short *loc0, unsigned short *loc, int *gidx)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n)
+    const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (c >= nchunks)
         return;
-    const int c = cnt[p];
-    for (int k = 0; k < c; ++k) {
-        const size_t s = slot_of(chunk0[p], stride[p], k);
-        const bool alive = brk[s] >= n0;
-        loc[s] = alive ? loc0[s] : LOC_DEAD;
-        const uint32_t e = (uint32_t)gidx[s] & ~(DEAD | NEWB);
-        gidx[s] = (int)(alive ? e : (e | DEAD));
+    const int4 b = reinterpret_cast<const int4 *>(brk)[c];
+    ushort4 l = reinterpret_cast<const ushort4 *>(loc0)[c];
+    const int4 g = reinterpret_cast<const int4 *>(gidx)[c];
+    const int bv[4] = {b.x, b.y, b.z, b.w}, gv[4] = {g.x, g.y, g.z, g.w};
+    unsigned short lv[4] = {l.x, l.y, l.z, l.w};
+    int w[4];
+    bool changed = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool alive = bv[q] >= n0;
+        if (!alive)
+            lv[q] = LOC_DEAD;
+        const uint32_t e = (uint32_t)gv[q] & ~(DEAD | NEWB);
+        w[q] = (int)(alive ? e : (e | DEAD));
+        changed |= w[q] != gv[q];
     }
+    reinterpret_cast<ushort4 *>(loc)[c] =
+        make_ushort4(lv[0], lv[1], lv[2], lv[3]);
+    if (changed)
+        reinterpret_cast<int4 *>(gidx)[c] = make_int4(w[0], w[1], w[2], w[3]);
 }
 
 // A per-node array in the caller's node order: dst[tnode[p]] = src[p], w
@@ -1587,19 +1639,21 @@ __global__ void k_perm(int n, int w, const int *tnode, const double *src,
         dst[q + d] = src[c + d];
 }
 
-// brk at the start of a recording: -1 for bonds already broken, else "never".
-__global__ void k_adj_init(int n, const int *cnt, const long long *chunk0,
-                           const int *stride, const unsigned short *loc,
-                           int *brk)
+// loc0 and brk at the start of a recording: brk -1 for bonds already broken
+// and empty slots, else "never".
+__global__ void __launch_bounds__(256)
+    k_adj_init(long long nchunks, const unsigned short *loc,
+               unsigned short *loc0, int *brk)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n)
+    const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (c >= nchunks)
         return;
-    const int c = cnt[p];
-    for (int k = 0; k < c; ++k) {
-        const size_t s = slot_of(chunk0[p], stride[p], k);
-        brk[s] = loc[s] == LOC_DEAD ? -1 : 0x7fffffff;
-    }
+    const ushort4 l = reinterpret_cast<const ushort4 *>(loc)[c];
+    reinterpret_cast<ushort4 *>(loc0)[c] = l;
+    constexpr int NEVER = 0x7fffffff;
+    reinterpret_cast<int4 *>(brk)[c] =
+        make_int4(l.x == LOC_DEAD ? -1 : NEVER, l.y == LOC_DEAD ? -1 : NEVER,
+                  l.z == LOC_DEAD ? -1 : NEVER, l.w == LOC_DEAD ? -1 : NEVER);
 }
 
 // 1/sqrt(q) for q in [2^-767, 2^767]: the hardware estimate and two Newton
@@ -1614,27 +1668,45 @@ __device__ __forceinline__ double rsqrt_newton(double q)
 }
 
 // 1/l0 of every slot's bond, once per recording (inv: caller id -> internal
-// id); the slots past a node's count keep the 0 they were cleared to.  The
-// same reciprocal square root of the same squared length as the backward
-// kernel's 1/l, so that a bond with l == l0 (bitwise, e.g. both ends at
-// rest) gets 1/l0 - 1/l = 0 exactly, as its stretch is 0 in the forward
-// step: a one-ulp difference there, times k dt, is not small.
-__global__ void k_adj_il0(int n, const int *cnt, const long long *chunk0,
-                          const int *stride, const int *gidx, const int *inv,
-                          const double *r0, double *il0)
+// id), 0 where there is none.  The same reciprocal square root
+// of the same squared length as the backward kernel's 1/l, so that a bond
+// with l == l0 (bitwise, e.g. both ends at rest) gets 1/l0 - 1/l = 0 exactly,
+// as its stretch is 0 in the forward step: a one-ulp difference there, times
+// k dt, is not small.  Bound by the neighbours' coordinates (four scattered
+// reads per bond): 105 us on the 50,820-node bar with one lane per node, 61
+// with 4 lanes, 50 with 16.
+__global__ void __launch_bounds__(256)
+    k_adj_il0(int n, const int *cnt, const long long *chunk0,
+              const int *stride, const int *gidx, const unsigned short *loc0,
+              const int *inv, const double *r0, double *il0)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int p = t / ROW_LANES, sub = t % ROW_LANES;
     if (p >= n)
         return;
-    const int c = cnt[p];
+    const int nch = chunks_of(cnt[p]);
     const size_t b = 3 * (size_t)p;
-    for (int k = 0; k < c; ++k) {
-        const size_t s = slot_of(chunk0[p], stride[p], k);
-        const size_t bj = 3 * (size_t)inv[(uint32_t)gidx[s] & KEYM];
-        const double ex = r0[bj] - r0[b];
-        const double ey = r0[bj + 1] - r0[b + 1];
-        const double ez = r0[bj + 2] - r0[b + 2];
-        il0[s] = rsqrt_newton((ex * ex + ey * ey) + ez * ez);
+    const double x = r0[b], y = r0[b + 1], z = r0[b + 2];
+    for (int c = sub; c < nch; c += ROW_LANES) {
+        const size_t k = (size_t)(chunk0[p] + (long long)c * stride[p]);
+        const int4 g = reinterpret_cast<const int4 *>(gidx)[k];
+        const ushort4 l = reinterpret_cast<const ushort4 *>(loc0)[k];
+        const int gv[4] = {g.x, g.y, g.z, g.w};
+        const unsigned short lv[4] = {l.x, l.y, l.z, l.w};
+        double v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const size_t bj = 3 * (size_t)inv[(uint32_t)gv[q] & KEYM];
+            const double ex = r0[bj] - x;
+            const double ey = r0[bj + 1] - y;
+            const double ez = r0[bj + 2] - z;
+            v[q] = lv[q] == LOC_DEAD
+                       ? 0.0
+                       : rsqrt_newton((ex * ex + ey * ey) + ez * ez);
+        }
+        double2 *o = reinterpret_cast<double2 *>(il0) + 2 * k;
+        o[0] = make_double2(v[0], v[1]);
+        o[1] = make_double2(v[2], v[3]);
     }
 }
 
@@ -1980,6 +2052,37 @@ int download_caller(pd_sim *s, double *dst, const double *src, int w)
                           hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     return PD_OK;
+}
+
+// Blocks of 256 threads for that many lanes per node.
+unsigned row_blocks(int n, int lanes)
+{
+    return (unsigned)(((long long)n * lanes + 255) / 256);
+}
+
+// Blocks of 256 threads for one thread per chunk of slots.
+unsigned chunk_blocks(const pd_sim *s)
+{
+    return (unsigned)((s->nslots / 4 + 255) / 256);
+}
+
+hipError_t launch_export(pd_sim *s, int rows)
+{
+    const auto go = [&](auto kernel, int lanes) {
+        hipLaunchKernelGGL(kernel, dim3(row_blocks(s->n, lanes)), dim3(256),
+                           0, s->stream, s->n, s->K, s->layout, rows,
+                           s->tnode.p, s->cnt.p, s->chunk0.p, s->stride.p,
+                           s->loc.p, s->gidx.p, s->pos.p, s->family.p,
+                           s->n_neigh.p, s->out_nlist.p, s->out_nneigh.p,
+                           s->damage.p);
+    };
+    if (s->layout == PD_LAYOUT_COMPACT)
+        go(k_export<1>, 1);  // counts are kept: one lane per node
+    else if (rows)
+        go(k_export<ROW_LANES>, ROW_LANES);
+    else
+        go(k_export<CHUNK_LANES>, CHUNK_LANES);
+    return hipGetLastError();
 }
 
 int check_sim(pd_sim *s)
@@ -3075,12 +3178,7 @@ int pd_monitor(pd_sim *s, double *model, double *tips)
     if (s->mon_out.n < nout) {
         HIPCHK(s->mon_out.alloc(nout));
     }
-    hipLaunchKernelGGL(k_export, dim3((N + 255) / 256), dim3(256), 0,
-                       s->stream, N, s->K, s->layout, 0, s->tnode.p,
-                       s->cnt.p, s->chunk0.p, s->stride.p, s->gidx.p,
-                       s->pos.p, s->family.p, s->n_neigh.p, s->out_nlist.p,
-                       s->out_nneigh.p, s->damage.p);
-    HIPCHK(hipGetLastError());
+    HIPCHK(launch_export(s, 0));
     hipLaunchKernelGGL(k_monitor_part, dim3(MON_BLOCKS), dim3(256), 0,
                        s->stream, N, s->u.p, s->ud.p, s->udd.p, s->force.p,
                        s->body_force.p, s->flags.p, s->vol.p, s->damage.p,
@@ -3153,12 +3251,7 @@ int pd_monitor_noalloc(pd_sim *s, double *model, double *tips)
     double *part = sp;
     double *staged = sp + (size_t)MON_BLOCKS * MON_SUMS;
     const int N = s->n;
-    hipLaunchKernelGGL(k_export, dim3((N + 255) / 256), dim3(256), 0,
-                       s->stream, N, s->K, s->layout, 0, s->tnode.p,
-                       s->cnt.p, s->chunk0.p, s->stride.p, s->gidx.p,
-                       s->pos.p, s->family.p, s->n_neigh.p, s->out_nlist.p,
-                       s->out_nneigh.p, s->damage.p);
-    HIPCHK(hipGetLastError());
+    HIPCHK(launch_export(s, 0));
     hipLaunchKernelGGL(k_monitor_part, dim3(MON_BLOCKS), dim3(256), 0,
                        s->stream, N, s->u.p, s->ud.p, s->udd.p, s->force.p,
                        s->body_force.p, s->flags.p, s->vol.p, s->damage.p,
@@ -3434,19 +3527,13 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
     HIPCHK(s->fin_u.alloc(B));
     HIPCHK(s->fin_force.alloc(B));
     HIPCHK(s->fin_bforce.alloc(B));
-    HIPCHK(hipMemcpyAsync(s->loc0.p, s->loc.p, S * sizeof(unsigned short),
-                          hipMemcpyDeviceToDevice, s->stream));
-    // slots past a node's count: brk -1 (all bytes set), 1/l0 zero
-    HIPCHK(hipMemsetAsync(s->brk.p, 0xff, S * sizeof(int), s->stream));
-    HIPCHK(hipMemsetAsync(s->il0.p, 0, S * sizeof(double), s->stream));
-    const int blocks = (s->n + 255) / 256;
-    hipLaunchKernelGGL(k_adj_init, dim3(blocks), dim3(256), 0, s->stream,
-                       s->n, s->cnt.p, s->chunk0.p, s->stride.p, s->loc.p,
+    hipLaunchKernelGGL(k_adj_init, dim3(chunk_blocks(s)), dim3(256), 0,
+                       s->stream, (long long)(S / 4), s->loc.p, s->loc0.p,
                        s->brk.p);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_adj_il0, dim3(blocks), dim3(256), 0, s->stream,
-                       s->n, s->cnt.p, s->chunk0.p, s->stride.p, s->gidx.p,
-                       inv_d.p, s->r0.p, s->il0.p);
+    hipLaunchKernelGGL(k_adj_il0, dim3(row_blocks(s->n, ROW_LANES)),
+                       dim3(256), 0, s->stream, s->n, s->cnt.p, s->chunk0.p, s->stride.p,
+                       s->gidx.p, s->loc0.p, inv_d.p, s->r0.p, s->il0.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(s->ckpt.p, s->u.p, B * sizeof(double),
                           hipMemcpyDeviceToDevice, s->stream));
@@ -3464,10 +3551,9 @@ namespace {
 // states from brk, records from u.
 int adjoint_restore(pd_sim *s, int n0)
 {
-    const int blocks = (s->n + 255) / 256;
-    hipLaunchKernelGGL(k_adj_restore, dim3(blocks), dim3(256), 0, s->stream,
-                       s->n, n0, s->cnt.p, s->chunk0.p, s->stride.p,
-                       s->brk.p, s->loc0.p, s->loc.p, s->gidx.p);
+    hipLaunchKernelGGL(k_adj_restore, dim3(chunk_blocks(s)), dim3(256), 0,
+                       s->stream, (long long)(s->nslots / 4), n0, s->brk.p,
+                       s->loc0.p, s->loc.p, s->gidx.p);
     HIPCHK(hipGetLastError());
     return refresh_records(s);
 }
@@ -3626,12 +3712,7 @@ int pd_write_device(pd_sim *s, double *u, double *damage)
     const int N = s->n;
     const int blocks = (N + 255) / 256;
     if (damage) {
-        hipLaunchKernelGGL(k_export, dim3(blocks), dim3(256), 0, s->stream,
-                           N, s->K, s->layout, 0, s->tnode.p, s->cnt.p,
-                           s->chunk0.p, s->stride.p, s->gidx.p, s->pos.p,
-                           s->family.p, s->n_neigh.p, s->out_nlist.p,
-                           s->out_nneigh.p, s->damage.p);
-        HIPCHK(hipGetLastError());
+        HIPCHK(launch_export(s, 0));
         HIPCHK(hipMemcpyAsync(damage, s->damage.p, (size_t)N * sizeof(double),
                               hipMemcpyDeviceToDevice, s->stream));
     }
@@ -3664,15 +3745,10 @@ int pd_write(pd_sim *s, double *u, double *ud, double *udd, double *force,
         return fail(PD_E_STATE, "pd_create_buffers has not been called");
     const int N = s->n;
     const int blocks = (N + 255) / 256;
-    hipLaunchKernelGGL(k_export, dim3(blocks), dim3(256), 0, s->stream, N,
-                       s->K, s->layout, nlist ? 1 : 0, s->tnode.p, s->cnt.p,
-                       s->chunk0.p,
-                       s->stride.p, s->gidx.p, s->pos.p, s->family.p,
-                       s->n_neigh.p, s->out_nlist.p, s->out_nneigh.p,
-                       s->damage.p);
-    HIPCHK(hipGetLastError());
+    HIPCHK(launch_export(s, nlist ? 1 : 0));
     if (nlist && s->layout == PD_LAYOUT_COMPACT) {
-        hipLaunchKernelGGL(k_export_rows, dim3(blocks), dim3(256), 0,
+        hipLaunchKernelGGL(k_export_rows, dim3(row_blocks(N, ROW_LANES)),
+                           dim3(256), 0,
                            s->stream, N, s->K, s->tnode.p, s->cnt.p,
                            s->chunk0.p, s->stride.p, s->gidx.p, s->rslot.p,
                            s->nlist_ref.p);
@@ -3761,10 +3837,10 @@ int pd_live_bonds(pd_sim *s, long long *count)
         return fail(PD_E_STATE, "pd_create_buffers has not been called");
     HIPCHK(hipMemsetAsync(s->counter.p, 0, sizeof(unsigned long long),
                           s->stream));
-    const int blocks = (s->n + 255) / 256;
-    hipLaunchKernelGGL(k_live, dim3(blocks), dim3(256), 0, s->stream, s->n,
-                       s->cnt.p, s->chunk0.p, s->stride.p, s->gidx.p,
-                       s->counter.p);
+    hipLaunchKernelGGL(k_live, dim3(row_blocks(s->n, CHUNK_LANES)),
+                       dim3(256), 0,
+                       s->stream, s->n, s->cnt.p, s->chunk0.p, s->stride.p,
+                       s->loc.p, s->counter.p);
     HIPCHK(hipGetLastError());
     unsigned long long h = 0;
     HIPCHK(hipMemcpyAsync(&h, s->counter.p, sizeof(h), hipMemcpyDeviceToHost,
