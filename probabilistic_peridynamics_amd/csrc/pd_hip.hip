@@ -191,12 +191,13 @@ struct StepArgs {
     const double *cnode;  // node stiffness c (DM_FIELD)
     int *brk;  // if set: the step at which each slot's bond broke
     int step;  // index of this step (for brk)
-    // exact-order step: lower-slot counts, upper-list lengths and the upper
-    // lists (slot index << 16 | halo loc), the scalar stiffness
+    // exact-order step: lower-slot counts, upper-list lengths and the fold
+    // lists (slot index << 16 | halo loc), the scalar stiffness, and the
+    // stretches strictly between which a bond takes the fast evaluation
     const int *nlow;
     int *nup;
-    unsigned *uord;
-    double kx;
+    unsigned *ford;
+    double kx, xlo, xhi;
 };
 
 // Slot of a row's k-th bond.  Sixteen bonds take four chunks; chunk q of the
@@ -210,6 +211,18 @@ __host__ __device__ __forceinline__ size_t slot_of(long long chunk0,
     const int chunk = ((k >> 4) << 2) + ((k >> 1) & 3);
     return (size_t)(chunk0 + (long long)chunk * stride) * 4 +
            (((k >> 2) & 2) | (k & 1));
+}
+
+// Index of position pos of a node's fold list (exact-order step): round
+// pos/8, in which lane pos%4 takes positions pos%4 and 4 + pos%4 with one
+// 8-byte load; chunk0 and stride as in slot_of (a tile's lists take the place
+// of its slots, two rows of pairs for a row of chunks).
+__host__ __device__ __forceinline__ size_t fold_of(long long tile_chunk0,
+                                                   int stride, int l, int pos)
+{
+    const int row = ((pos >> 3) << 2) + (pos & 3);
+    return 2 * (size_t)(2 * tile_chunk0 + (long long)row * stride + l) +
+           ((pos >> 2) & 1);
 }
 
 // Chunk rows of a row of cnt bonds.
@@ -367,8 +380,8 @@ __host__ __device__ constexpr unsigned compact_row_bytes(int K)
 // node's count of bonds broken in this step (the same in all its lanes).  The
 // rows of the nodes that lost bonds are staged in `scratch` (`bytes` of LDS
 // the block no longer reads once every thread is here), compacted by one
-// lane each, and written back; with EXACT, the node's upper list (uord, nup)
-// is rebuilt in the new row order.  NEW flags are cleared.  Nodes take
+// lane each, and written back; with EXACT, the upper part of the node's fold
+// list (ford, nup) is rebuilt in the new row order.  NEW flags are cleared.  Nodes take
 // scratch regions in groups when they do not all fit.  The first 64 bytes
 // hold each wave's count of such nodes, from which every node's region
 // follows without atomics.
@@ -429,15 +442,19 @@ __device__ void compact_tile(const StepArgs &a, const TileInfo &ti,
                                             a.nlow[i], m, rs, fl, n, nhi);
             a.n_neigh[m] = n1;
             if (EXACT) {
-                int c = 0;
+                int pos = a.nlow[i];
+                const int end = pos + a.nup[i];
                 for (int p = 0; p < n1; ++p) {
                     const int k = rs[p];
                     if (k >= nhi)
-                        a.uord[slot_of(c0, ti.nodes, c++)] =
+                        a.ford[fold_of(ti.chunk_off, ti.nodes, l, pos++)] =
                             ((unsigned)k << 16) |
                             a.loc[slot_of(c0, ti.nodes, k)];
                 }
-                a.nup[i] = c;
+                a.nup[i] = pos - a.nlow[i];
+                for (; pos < end; ++pos)
+                    a.ford[fold_of(ti.chunk_off, ti.nodes, l, pos)] =
+                        LOC_DEAD;
             }
         }
         __syncthreads();
@@ -476,6 +493,74 @@ __device__ __forceinline__ double sq3(double x, double y, double z)
     if (CLA)
         return __builtin_fma(z, z, __builtin_fma(x, x, y * y));
     return (x * x + y * y) + z * z;
+}
+
+// Staging of a tile's halo records into LDS, piece-major: piece q of the
+// record of entry x at D + q*PB + 16*(x + 1).  Thread t copies piece t%4 of
+// entries t/4, t/4 + blockDim/4, ...; the node indices are requested as early
+// as possible (they head the longest chain of dependent loads), the records
+// SP pieces per thread in flight at once (a block of 512 threads needs one
+// pass).  Pieces past the last entry store that entry again: a condition
+// would move each load next to its store.
+struct HaloLoads {
+    static constexpr int SP = 10;
+    unsigned hi[SP];
+
+    __device__ __forceinline__ void request(const int *H, unsigned halo)
+    {
+        const unsigned last = halo - 1u;
+        unsigned x = threadIdx.x >> 2;
+        static_for<SP>([&](auto k) {
+            hi[k] = (unsigned)H[min(x, last)];
+            x += blockDim.x >> 2;
+        });
+    }
+
+    __device__ __forceinline__ void stage(const NodeRec *rec, const int *H,
+                                          unsigned halo, char *D, unsigned PB)
+    {
+        const unsigned last = halo - 1u, per = blockDim.x >> 2;
+        const unsigned e0 = threadIdx.x >> 2, piece = threadIdx.x & 3u;
+        const char *R = reinterpret_cast<const char *>(rec);
+        D += piece * PB + 16u;
+        unsigned x = e0;
+        {
+            v2d v[SP];
+            static_for<SP>([&](auto k) {
+                v[k] = *reinterpret_cast<const v2d *>(
+                    R + (hi[k] * 64u + piece * 16u));
+            });
+            static_for<SP>([&](auto k) {
+                *reinterpret_cast<v2d *>(D + 16u * min(x, last)) = v[k];
+                x += per;
+            });
+        }
+        while (x - e0 <= last) {  // the same in every thread
+            v2d v[4];
+            unsigned y = x;
+            static_for<4>([&](auto k) {
+                v[k] = *reinterpret_cast<const v2d *>(
+                    R + ((unsigned)H[min(y, last)] * 64u + piece * 16u));
+                y += per;
+            });
+            static_for<4>([&](auto k) {
+                *reinterpret_cast<v2d *>(D + 16u * min(x, last)) = v[k];
+                x += per;
+            });
+        }
+    }
+};
+
+// Entry 0 of a staged halo, what dead and empty slots read: a far node of
+// weight 0 (CLA: records hold u, which is 0).  Threads 0-3.
+template <bool CLA>
+__device__ __forceinline__ void far_entry(char *D, unsigned PB)
+{
+    constexpr double FAR = 0x1p300;
+    const unsigned t = threadIdx.x;
+    const bool r = t < 2 || !CLA;
+    *reinterpret_cast<double2 *>(D + t * PB) =
+        make_double2(r ? FAR : 0.0, r && !(t & 1) ? FAR : 0.0);
 }
 
 // A bond as the force needs it: the bond vector, s/2, 0.5/l and the weight.
@@ -719,21 +804,10 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
     const bool valid = l < ti.nodes;
 
     // the halo's node indices first: the records they name are the longest
-    // chain of this kernel.  Thread x copies 16-byte piece x%4 of records
-    // x/4, x/4 + blockDim/4, ...
-    constexpr int SP = 10;
+    // chain of this kernel
     constexpr unsigned PB = piece_bytes<DM>();
-    const int *H = a.halo + ti.halo_off;
-    const unsigned e0 = threadIdx.x >> 2;
-    const unsigned piece = threadIdx.x & 3u;
-    const unsigned eper = blockDim.x >> 2;
-    const unsigned elast = (unsigned)ti.halo - 1u;
-    unsigned hi[SP];
-    unsigned hx = e0;
-    static_for<SP>([&](auto k) {
-        hi[k] = (unsigned)H[min(hx, elast)];
-        hx += eper;
-    });
+    HaloLoads hl;
+    hl.request(a.halo + ti.halo_off, (unsigned)ti.halo);
 
     // node state and the first chunks of halo entries are requested before
     // the halo is staged, so their latency overlaps the staging.  Chunk rows
@@ -789,47 +863,10 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         }
     }
 
-    // stage the halo, SP pieces per thread in flight at once (a block of
-    // 512 threads needs one pass).  Pieces past the last entry store that
-    // entry again: a condition would move each load next to its store.
-    const char *R = reinterpret_cast<const char *>(a.rec_old);
-    char *D = ldsb + halo_base<DM>() + piece * PB + 16u;
-    {
-        v2d v[SP];
-        static_for<SP>([&](auto k) {
-            v[k] = *reinterpret_cast<const v2d *>(
-                R + (hi[k] * 64u + piece * 16u));
-        });
-        unsigned x = e0;
-        static_for<SP>([&](auto k) {
-            *reinterpret_cast<v2d *>(D + 16u * min(x, elast)) = v[k];
-            x += eper;
-        });
-    }
-    for (unsigned x0 = hx; x0 - e0 <= elast; x0 += 4 * eper) {
-        v2d v[4];
-        unsigned x = x0;
-        static_for<4>([&](auto k) {
-            v[k] = *reinterpret_cast<const v2d *>(
-                R + ((unsigned)H[min(x, elast)] * 64u + piece * 16u));
-            x += eper;
-        });
-        x = x0;
-        static_for<4>([&](auto k) {
-            *reinterpret_cast<v2d *>(D + 16u * min(x, elast)) = v[k];
-            x += eper;
-        });
-    }
-    if (threadIdx.x < 4) {  // entry 0: what dead slots read
-        constexpr double FAR = 0x1p300;
-        double2 z = make_double2(0.0, 0.0);
-        if (threadIdx.x == 0 || (!CLA && threadIdx.x == 2))
-            z = make_double2(FAR, FAR);
-        else if (threadIdx.x == 1 || (!CLA && threadIdx.x == 3))
-            z.x = FAR;
-        *reinterpret_cast<double2 *>(ldsb + halo_base<DM>() +
-                                     threadIdx.x * PB) = z;
-    }
+    hl.stage(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo,
+             ldsb + halo_base<DM>(), PB);
+    if (threadIdx.x < 4)
+        far_entry<CLA>(ldsb + halo_base<DM>(), PB);
     // n-linear tables, one 16-byte read each: (lower, upper) halved
     // thresholds of regime r of type t with their margin, and (4 stiffness,
     // 2 plus_cs)
@@ -1290,21 +1327,21 @@ __global__ void __launch_bounds__(256)
 // negated, as r_m - r_k is the exact negation of r_k - r_m.  The fold order
 // depends only on node m's own row, so each tile folds its own nodes.
 //
-// A node's fold list is its lower slots in ascending order (slot order:
-// rows are sorted by caller id; a dead slot adds nothing), then its upper
-// neighbours in current row order (uord: slot index << 16 | halo loc,
-// rebuilt by compact_tile after every break of the node).  The node's four
-// lanes take four consecutive positions per round: each evaluates its bond
-// with the reference's operations -- bitwise square roots, IEEE divisions,
-// no contraction -- decides the break from that exact stretch
-// (peridynamics.pyx:133), and writes its three force terms to the node's
-// 96-byte LDS window; lanes 0-2 then add the four terms of their component
-// in order.  Breaking is applied before the force, as in Euler.__call__: a
-// bond that breaks adds nothing, and when any bond of the node breaks the
-// row is compacted (peridynamics.pyx:102-156) and the upper part, whose
-// order the compaction may change, is folded again from the sum of the
-// lower part.  Assumes symmetric neighbour lists without repeats, as the
-// model builds them.
+// A node's fold list (ford) is its lower slots in ascending order (slot
+// order: rows are sorted by caller id; a dead slot adds nothing), then its
+// upper neighbours in current row order (slot index << 16 | halo loc, rebuilt
+// by compact_tile after every break of the node).  The node's four lanes take
+// eight consecutive positions per round, two each, whose evaluations
+// interleave: with the reference's operations -- bitwise square roots, IEEE
+// divisions, no contraction -- each gives its three force terms and decides
+// the break from that exact stretch (peridynamics.pyx:133).  The terms pass
+// through the node's 96-byte LDS window, four positions at a time; lanes 0-2
+// add the terms of their component in order.  Breaking is applied before the
+// force, as in Euler.__call__: a bond that breaks adds nothing, and when any
+// bond of the node breaks the row is compacted (peridynamics.pyx:102-156) and
+// the part of the list whose order the compaction may change is folded again
+// from the sum before it.  Assumes symmetric neighbour lists without repeats,
+// as the model builds them.
 
 // LDS of the exact step: the halo (pieces of EXACT_CAP entries), then the
 // fold windows (12 doubles per node, tiles of up to EXACT_NODES nodes).
@@ -1323,38 +1360,38 @@ struct ExactTerm {
     double t0, t1, t2, s;
 };
 
-// a / b rounded to nearest by the compiler's f64 division sequence (rcp, two
-// Newton steps, the quotient and one residual correction) without its
-// v_div_scale / v_div_fixup steps.  Those change nothing -- the result is
-// the IEEE quotient -- when a is zero, or when a, b and a/b are normal, a >=
-// 2^-969, 1/b is normal and a's exponent exceeds b's by less than 768.
-__device__ __forceinline__ double div_core(double a, double b)
+// a / b rounded to nearest, given h ~ 0.5/b (sqrt_core's, relative error
+// below 2^-46): one Newton step makes y the reciprocal to within its rounding
+// and 2^-92, as the compiler's f64 division does in two from the hardware's
+// estimate; then its quotient and residual correction, without its scaling
+// steps, which change nothing when a is zero, or when a, b and a/b are
+// normal, a >= 2^-969, 1/b is normal and a's exponent exceeds b's by less
+// than 768.
+__device__ __forceinline__ double div_core(double a, double b, double h)
 {
-    double y = __builtin_amdgcn_rcp(b);
-    double e = __builtin_fma(-b, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-b, y, 1.0);
+    double y = h + h;
+    const double e = __builtin_fma(-b, y, 1.0);
     y = __builtin_fma(y, e, y);
     const double q = a * y;
     const double r = __builtin_fma(-b, q, a);
     return __builtin_fma(r, y, q);
 }
 
-// The exact bond evaluation.  With q and q0 at least 2^-700, l and l0 come
-// from sqrt_core (exact there, and l, l0 lie in [2^-350, 2^512]).  With the
-// stiffness k in [2^-100, 2^100] and s0 below 2^300 (SAFE, checked by the
-// host) both quotients come from div_core: s = (l - l0)/l0 is 0 or at least
-// 2^-54 in magnitude (l - l0 is 0 or at least an ulp of the shorter), and for a
-// bond that does not break it is below s0, so every operand and quotient is
-// normal, numerators exceed 2^-969 and no exponent gap reaches 768; a bond
-// that breaks only needs its stretch on the right side of s0, which a huge
-// (or NaN: l0 from a q0 outside the range) value is, as the reference's
-// infinite or NaN one is.  The rest take the library's square roots and
-// divisions.
-template <bool SAFE>
-__device__ __forceinline__ ExactTerm exact_term(const char *ldsb, unsigned e,
+// The terms of halo entry e, exactly the reference's while the stretch lies
+// strictly in (a.xlo, a.xhi); the caller takes exact_slow otherwise.  The
+// interval is empty unless the stiffness is in [2^-100, 2^100], s0 below
+// 2^300 and the coordinates in bond_fast's range.  Then q0 is 0 (NaN stretch)
+// or in [2^-686, 2^603], s > -1/2 gives q at least 2^-690 (see bond_fast), so
+// l and l0 come from sqrt_core exactly and lie in [2^-346, 2^512]; s is 0 or
+// at least 2^-54 in magnitude (l - l0 is 0 or at least an ulp of the
+// shorter), so every operand and quotient is normal, numerators exceed
+// 2^-969 and no exponent gap reaches 768: both quotients are div_core's.  A
+// dead or empty position reads entry 0, a far node of volume 0: its terms
+// are zero.
+__device__ __forceinline__ ExactTerm exact_fast(const StepArgs &a,
+                                                const char *ldsb, unsigned e,
                                                 const double4 &r0m,
-                                                const double4 &rm, double k)
+                                                const double4 &rm)
 {
     constexpr unsigned PB = 16u * EXACT_CAP;
     const char *pe = ldsb + e;
@@ -1367,30 +1404,59 @@ __device__ __forceinline__ ExactTerm exact_term(const char *ldsb, unsigned e,
     const double q = (dx * dx + dy * dy) + dz * dz;
     const double ex = p0.x - r0m.x, ey = p0.y - r0m.y, ez = p1.x - r0m.z;
     const double q0 = (ex * ex + ey * ey) + ez * ez;
-    const bool fast = (q >= 0x1p-700) & (q0 >= 0x1p-700);
-    double l, l0, h;
+    double l, l0, h, h0;
     sqrt_core(q, l, h);
-    sqrt_core(q0, l0, h);
+    sqrt_core(q0, l0, h0);
     ExactTerm t;
-    double fn;
     // spatial.pyx:87-97, peridynamics.pyx:75-89
-    if (SAFE && fast) {
-        t.s = div_core(l - l0, l0);
-        fn = div_core(t.s * k, l);
-    } else {
-        if (!fast) {
-            l = sqrt(q);
-            l0 = sqrt(q0);
-        }
-        t.s = (l - l0) / l0;
-        fn = t.s * k;
-        fn = fn / l;
-    }
+    t.s = div_core(l - l0, l0, h0);
+    const double fn = div_core(t.s * a.kx, l, h);
     const double v = p1.y;  // V_j
     t.t0 = (fn * dx) * v;
     t.t1 = (fn * dy) * v;
     t.t2 = (fn * dz) * v;
     return t;
+}
+
+// The same with the library's square roots and divisions, and the break
+// (peridynamics.pyx:133) of the bond at slot `slot`, position `fold` of its
+// node's list; `check` false only evaluates.
+__device__ __forceinline__ void exact_slow(const StepArgs &a,
+                                           const char *ldsb, unsigned e,
+                                           const double4 &r0m,
+                                           const double4 &rm, bool check,
+                                           size_t slot, size_t fold,
+                                           ExactTerm &t, int &nbroken)
+{
+    if (e == LOC_DEAD) {
+        t.t0 = t.t1 = t.t2 = 0.0;
+        return;
+    }
+    constexpr unsigned PB = 16u * EXACT_CAP;
+    const char *pe = ldsb + e;
+    const double2 p0 = *reinterpret_cast<const double2 *>(pe);
+    const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
+    const double2 p2 = *reinterpret_cast<const double2 *>(pe + 2 * PB);
+    const double p3 = *reinterpret_cast<const double *>(pe + 3 * PB);
+    const double dx = p2.x - rm.x, dy = p2.y - rm.y, dz = p3 - rm.z;
+    const double ex = p0.x - r0m.x, ey = p0.y - r0m.y, ez = p1.x - r0m.z;
+    const double l = sqrt((dx * dx + dy * dy) + dz * dz);
+    const double l0 = sqrt((ex * ex + ey * ey) + ez * ez);
+    t.s = (l - l0) / l0;
+    if (check && !(sign_mask(t.s, a.absmask) < 2.0 * a.s0h)) {
+        a.loc[slot] = LOC_DEAD;
+        a.ford[fold] = LOC_DEAD;
+        a.gidx[slot] |= (int)(DEAD | NEWB);
+        ++nbroken;
+        t.t0 = t.t1 = t.t2 = 0.0;
+        return;
+    }
+    double fn = t.s * a.kx;
+    fn = fn / l;
+    const double v = p1.y;
+    t.t0 = (fn * dx) * v;
+    t.t1 = (fn * dy) * v;
+    t.t2 = (fn * dz) * v;
 }
 
 // The fold window of a node: [component][position of the round].
@@ -1415,7 +1481,15 @@ __device__ __forceinline__ void window_done()
 // One workgroup per tile of at most EXACT_NODES nodes, four lanes per node
 // (block 4 * tile_nodes), on k_step's tiles and halo staging.  Records hold
 // (r0, V | r0 + u, 0).
-template <bool SAFE>
+//
+// What bounds it: the VALU on large meshes, and on small ones a round's
+// latency (gather, two square roots, two divisions, window, ordered adds:
+// one chain).  Two positions per lane and round halve the chain's rounds and
+// interleave two evaluations; with the list's entries in one array (one
+// 8-byte load per lane and round), div_core seeded from the square roots and
+// one interval test for everything rare, a bond takes 65 wave instructions
+// where it took 115: 150 -> 104 us a step on 270,000 nodes, 20.7 -> 14 on
+// the 2560-node bar.
 __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
                                                     double fmag)
 {
@@ -1431,124 +1505,110 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
     const int l = threadIdx.x / LPN;
     const int sub = threadIdx.x % LPN;
     const bool valid = l < ti.nodes;
+    HaloLoads hl;
+    hl.request(a.halo + ti.halo_off, (unsigned)ti.halo);
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     const long long c0 = ti.chunk_off + (valid ? l : 0);
+    // the node's pair of list entries in round r is r * fstep further on
+    const char *L = reinterpret_cast<const char *>(a.ford + 4 * ti.chunk_off);
+    const unsigned fstep = 8u * LPN * (unsigned)ti.nodes;
+    unsigned foff = 8u * ((valid ? (unsigned)l : 0u) +
+                          (unsigned)sub * (unsigned)ti.nodes);
+    auto pair_at = [&](unsigned off) {
+        return *reinterpret_cast<const uint2 *>(L + off);
+    };
+    uint2 qa = pair_at(foff), qb = pair_at(foff + fstep);
     double4 r0m = make_double4(0.0, 0.0, 0.0, 0.0), rm = r0m;
-    int cnt = 0, nlow = 0, nup = 0, fl = 0;
+    int cnt = 0, nlow = 0, fl = 0;
     double pu = 0.0;
     if (valid) {
         r0m = a.rec_old[i].a;
         rm = a.rec_old[i].b;
         cnt = a.cnt[i];
         nlow = a.nlow[i];
-        nup = a.nup[i];
         if (sub < 3) {
             fl = a.flags[i];
             pu = a.u[3 * (size_t)i + sub];
         }
     }
-    // stage the halo (as k_step)
-    constexpr int SP = 10;
-    const int np = 4 * ti.halo;
-    for (int x0 = threadIdx.x; x0 < np; x0 += SP * blockDim.x) {
-        double2 v[SP];
-#pragma unroll
-        for (int k = 0; k < SP; ++k) {
-            const int x = min(x0 + k * (int)blockDim.x, np - 1);
-            const int g = a.halo[ti.halo_off + (x >> 2)];
-            v[k] = reinterpret_cast<const double2 *>(a.rec_old + g)[x & 3];
-        }
-#pragma unroll
-        for (int k = 0; k < SP; ++k) {
-            const int x = x0 + k * (int)blockDim.x;
-            if (x < np)
-                *reinterpret_cast<double2 *>(
-                    ldsb + (x & 3) * PB + 16u * (unsigned)((x >> 2) + 1)) =
-                    v[k];
-        }
-    }
+    hl.stage(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb, PB);
     if (threadIdx.x < 4)
-        *reinterpret_cast<double2 *>(ldsb + threadIdx.x * PB) =
-            make_double2(0.0, 0.0);
+        far_entry<false>(ldsb, PB);
     __syncthreads();
 
     double *win = reinterpret_cast<double *>(ldsb + 4 * PB) + 12 * l;
-    const double s0 = 2.0 * a.s0h;
     double F = 0.0, Flow = 0.0;  // lane d < 3: component d
     int nbroken = 0;
-    if (valid) {
-        const int total = nlow + nup;
-        // fold position -> slot index << 16 | halo loc (lower positions are
-        // the slots themselves, upper ones come from uord), requested two
-        // rounds ahead of their use
-        auto entry = [&](int pos) -> unsigned {
-            if (pos < nlow)
-                return ((unsigned)pos << 16) |
-                       a.loc[slot_of(c0, ti.nodes, pos)];
-            if (pos < total)
-                return a.uord[slot_of(c0, ti.nodes, pos - nlow)];
-            return LOC_DEAD;
-        };
-        unsigned ahead0 = entry(sub), ahead1 = entry(sub + LPN);
-        for (int r = 0; r < total; r += LPN) {
-            const unsigned cur = ahead0;
-            ahead0 = ahead1;
-            ahead1 = entry(r + 2 * LPN + sub);
-            const unsigned e = cur & 0xffffu;
-            const size_t slot = slot_of(c0, ti.nodes, (int)(cur >> 16));
-            ExactTerm t = {0.0, 0.0, 0.0, 0.0};
-            if (e != LOC_DEAD) {
-                t = exact_term<SAFE>(ldsb, e, r0m, rm, a.kx);
-                const double as = sign_mask(t.s, a.absmask);
-                if (!(as < s0)) {  // peridynamics.pyx:133
-                    a.loc[slot] = LOC_DEAD;
-                    a.gidx[slot] |= (int)(DEAD | NEWB);
-                    ++nbroken;
-                    t.t0 = t.t1 = t.t2 = 0.0;
-                }
-            }
-            window_put(win, sub, t);
-            if (sub < 3) {
+    // four terms of every lane's component, in order
+    auto fold4 = [&](const ExactTerm &t) {
+        window_put(win, sub, t);
+        if (sub < 3) {
 #pragma unroll
-                for (int q = 0; q < LPN; ++q) {
-                    if (r + q == nlow)
-                        Flow = F;
-                    F = F + win[4 * sub + q];
-                }
-            }
-            window_done();
+            for (int q = 0; q < LPN; ++q)
+                F = F + win[4 * sub + q];
         }
-        if (nlow >= total)
-            Flow = F;
+        window_done();
+    };
+    auto round = [&](uint2 en, int r, bool check) {
+        ExactTerm t0 = exact_fast(a, ldsb, en.x & 0xffffu, r0m, rm);
+        ExactTerm t1 = exact_fast(a, ldsb, en.y & 0xffffu, r0m, rm);
+        const bool ok0 = (t0.s > a.xlo) & (t0.s < a.xhi);
+        const bool ok1 = (t1.s > a.xlo) & (t1.s < a.xhi);
+        if (__builtin_expect(!(ok0 & ok1), 0)) {
+            const int pos = 8 * r + sub;
+            if (!ok0)
+                exact_slow(a, ldsb, en.x & 0xffffu, r0m, rm, check,
+                           slot_of(c0, ti.nodes, (int)(en.x >> 16)),
+                           fold_of(ti.chunk_off, ti.nodes, l, pos), t0,
+                           nbroken);
+            if (!ok1)
+                exact_slow(a, ldsb, en.y & 0xffffu, r0m, rm, check,
+                           slot_of(c0, ti.nodes, (int)(en.y >> 16)),
+                           fold_of(ti.chunk_off, ti.nodes, l, pos + 4), t1,
+                           nbroken);
+        }
+        fold4(t0);
+        fold4(t1);
+    };
+    // the wavefront's first node has its longest list (nodes are sorted by
+    // bond count); positions past a list's end are dead
+    const int rounds = (__builtin_amdgcn_readfirstlane(cnt) + 7) >> 3;
+    const int rlow = nlow >> 3;  // the first round with an upper position
+    if (valid) {
+        for (int r = 0; r < rounds; r += 2) {
+            if (r <= rlow)
+                Flow = F;
+            round(qa, r, true);
+            foff += fstep;
+            qa = pair_at(foff + fstep);
+            if (r + 1 >= rounds)
+                break;
+            if (r + 1 <= rlow)
+                Flow = F;
+            round(qb, r + 1, true);
+            foff += fstep;
+            qb = pair_at(foff + fstep);
+        }
+        if (rlow >= rounds)
+            Flow = F;  // no upper part
     }
 #pragma unroll
     for (int off = LPN / 2; off > 0; off >>= 1)
         nbroken += __shfl_xor(nbroken, off, LPN);
     // the fold windows are free: they hold the rows being compacted, and
-    // the upper lists of those nodes are rebuilt in the new row order
+    // the lists of those nodes are rebuilt in the new row order
     compact_tile<LPN, true>(a, ti, ldsb + 4 * PB, EXACT_NODES * 96u, valid, l,
                             sub, i, cnt, nbroken);
     if (!valid)
         return;
     if (nbroken > 0) {
-        // the upper part again, in the new row order
-        const int nup2 = ld_slot(&a.nup[i]);
+        // again from the round in which the upper part begins
         F = Flow;
-        for (int r = 0; r < nup2; r += LPN) {
-            const int pos = r + sub;
-            ExactTerm t = {0.0, 0.0, 0.0, 0.0};
-            if (pos < nup2) {
-                const unsigned u = ld_slot(reinterpret_cast<const int *>(
-                    &a.uord[slot_of(c0, ti.nodes, pos)]));
-                t = exact_term<SAFE>(ldsb, u & 0xffffu, r0m, rm, a.kx);
-            }
-            window_put(win, sub, t);
-            if (sub < 3) {
-#pragma unroll
-                for (int q = 0; q < LPN; ++q)
-                    F = F + win[4 * sub + q];
-            }
-            window_done();
+        const int total = nlow + (int)ld_slot(&a.nup[i]);
+        for (int r = rlow; 8 * r < total; ++r) {
+            const int *e = reinterpret_cast<const int *>(a.ford) +
+                           fold_of(ti.chunk_off, ti.nodes, l, 8 * r + sub);
+            round(make_uint2(ld_slot(e), ld_slot(e + 1)), r, false);
         }
     }
     if (sub < 3) {
@@ -1566,6 +1626,41 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         const double r0d = sub == 0 ? r0m.x : (sub == 1 ? r0m.y : r0m.z);
         reinterpret_cast<double *>(&a.rec_new[i].b)[sub] = r0d + u;
     }
+}
+
+// The fold lists of every node from its row and live bonds (set-up, and when
+// the exact order is turned on: the fast step does not keep them).
+__global__ void __launch_bounds__(256)
+    k_fold_lists(int n, int K, const int *tnode, const int *cnt,
+                 const long long *chunk0, const int *stride,
+                 const long long *tile0, const int *gidx,
+                 const unsigned short *loc, const unsigned short *rslot,
+                 const int *n_neigh, const int *nlow, int *nup,
+                 unsigned *ford)
+{
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= n)
+        return;
+    const int i = tnode[p], st = stride[p], low = nlow[p];
+    const long long c0 = chunk0[p];
+    const long long t0 = tile0[p];
+    const int l = (int)(c0 - t0);
+    int pos = 0;
+    for (int k = 0; k < low; ++k) {
+        const unsigned e = loc[slot_of(c0, st, k)];
+        ford[fold_of(t0, st, l, pos++)] =
+            e == LOC_DEAD ? LOC_DEAD : ((unsigned)k << 16) | e;
+    }
+    const int live = n_neigh[i];
+    for (int q = 0; q < live; ++q) {
+        const int k = rslot[(size_t)i * K + q];
+        const size_t s = slot_of(c0, st, k);
+        if ((int)((uint32_t)gidx[s] & KEYM) > i)
+            ford[fold_of(t0, st, l, pos++)] = ((unsigned)k << 16) | loc[s];
+    }
+    nup[p] = pos - low;
+    for (; pos < cnt[p]; ++pos)
+        ford[fold_of(t0, st, l, pos)] = LOC_DEAD;
 }
 
 // --- adjoint of the Euler step with a recorded break mask -------------------
@@ -1943,7 +2038,8 @@ struct pd_sim {
     const double *u_in = nullptr;
     double *u_out = nullptr;
     DevBuf<int> nlow, nup;  // exact step: lower slots, upper-list length
-    DevBuf<unsigned> uord;  // exact step: upper lists in row order
+    DevBuf<unsigned> ford;  // exact step: fold lists
+    DevBuf<long long> tile0;  // compact layout: first chunk of a node's tile
     DevBuf<double> wbuf;  // a per-node array reordered for download
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -2155,8 +2251,14 @@ StepArgs make_args(pd_sim *s)
     a.step = s->step_counter;
     a.nlow = s->nlow.p;
     a.nup = s->nup.p;
-    a.uord = s->uord.p;
+    a.ford = s->ford.p;
     a.kx = s->k;
+    // exact_fast's interval; empty where its range does not hold
+    const double ak = std::fabs(s->k);
+    const bool core = s->coords_core && ak >= 0x1p-100 && ak <= 0x1p100 &&
+                      s->s0 < 0x1p300;
+    a.xhi = core ? s->s0 : -1.0;
+    a.xlo = s->tension_only ? -0.5 : std::max(-s->s0, -0.5);
     return a;
 }
 
@@ -2308,7 +2410,7 @@ int launch_step(pd_sim *s, double dmag, double fmag)
                                 "scalar stiffness model only");
     if (s->exact && (s->layout != PD_LAYOUT_COMPACT ||
                      s->integrator != PD_EULER || dm_of(s) != DM_PMB ||
-                     s->has_corr || !s->uord.p))
+                     s->has_corr || !s->ford.p))
         return fail(PD_E_STATE, "the exact-order step needs the compact "
                                 "layout, the Euler integrator and the scalar "
                                 "model without corrections");
@@ -2321,18 +2423,9 @@ int launch_step(pd_sim *s, double dmag, double fmag)
     const StepArgs a = make_args(s);
     hipError_t e;
     if (s->exact) {
-        // the stiffness range in which div_core is the IEEE division
-        const double ak = std::fabs(s->k);
-        if (ak >= 0x1p-100 && ak <= 0x1p100 && s->s0 < 0x1p300)
-            hipLaunchKernelGGL(k_exact_step<true>,
-                               dim3(XCDS * a.tiles_per_xcd),
-                               dim3(4 * s->tile_nodes), 0, s->stream, a, dmag,
-                               fmag);
-        else
-            hipLaunchKernelGGL(k_exact_step<false>,
-                               dim3(XCDS * a.tiles_per_xcd),
-                               dim3(4 * s->tile_nodes), 0, s->stream, a, dmag,
-                               fmag);
+        hipLaunchKernelGGL(k_exact_step, dim3(XCDS * a.tiles_per_xcd),
+                           dim3(4 * s->tile_nodes), 0, s->stream, a, dmag,
+                           fmag);
         e = hipGetLastError();
     } else {
         switch (dm_of(s)) {
@@ -2387,6 +2480,20 @@ int refresh_records(pd_sim *s)
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->stream));
     s->cur = 0;
+    return PD_OK;
+}
+
+// The compact layout's fold lists from its rows and live bonds.
+int fold_lists(pd_sim *s)
+{
+    if (s->layout != PD_LAYOUT_COMPACT)
+        return PD_OK;
+    hipLaunchKernelGGL(k_fold_lists, dim3((s->n + 255) / 256), dim3(256), 0,
+                       s->stream, s->n, s->K, s->tnode.p, s->cnt.p,
+                       s->chunk0.p, s->stride.p, s->tile0.p, s->gidx.p,
+                       s->loc.p, s->rslot.p, s->n_neigh.p, s->nlow.p,
+                       s->nup.p, s->ford.p);
+    HIPCHK(hipGetLastError());
     return PD_OK;
 }
 
@@ -2883,6 +2990,10 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         int nch = 0;
         for (int l = 0; l < t.nodes; ++l)
             nch = std::max(nch, chunks_of(cnt[tnode[t.node_off + l]]));
+        // the exact step's fold lists take the place of the slots: two rows
+        // of pairs per row of chunks, four per round of eight positions
+        if (s->layout == PD_LAYOUT_COMPACT && t.nodes > 0)
+            nch = std::max(nch, 2 * ((cnt[tnode[t.node_off]] + 7) >> 3));
         t.nch = nch;
         t.pad = 0;
         t.chunk_off = chunk_total;
@@ -2905,8 +3016,8 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     std::vector<long long> chunk0(N);
     std::vector<int> stride(N);
     const bool compact = s->layout == PD_LAYOUT_COMPACT;
-    std::vector<int> nlow_h(compact ? N : 0), nup_h(compact ? N : 0);
-    std::vector<unsigned> uord_h(compact ? S : 0, 0u);
+    std::vector<int> nlow_h(compact ? N : 0);
+    std::vector<long long> tile0_h(compact ? N : 0);
     std::vector<unsigned short> rslot_h(compact ? (size_t)N * K : 0, 0);
     std::atomic<int> halo_mismatch{0};
     run_parallel(ntiles, [&](int lo, int hi) {
@@ -2963,27 +3074,14 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                                   (regimes ? regimes[src] : 0)));
                 }
                 if (compact) {
-                    // row position -> slot, then the exact step's lists:
-                    // lower slots, and the upper neighbours in row order
+                    // row position -> slot; the lower slots
                     for (int k = 0; k < cnt[i]; ++k)
                         rslot_h[(size_t)i * K + rp[rstart[i] + k]] =
                             (unsigned short)k;
                     const int p = ti.node_off + l;
                     const int *rb = rj.data() + rstart[i];
                     nlow_h[p] = (int)(std::lower_bound(rb, rb + cnt[i], i) - rb);
-                    const int *row = nlist + (size_t)i * K;
-                    int c = 0;
-                    for (int q = 0; q < cnt[i]; ++q) {
-                        const int j = row[q];
-                        if (j <= i)
-                            continue;
-                        const int k =
-                            (int)(std::lower_bound(rb, rb + cnt[i], j) - rb);
-                        uord_h[slot_of(ti.chunk_off + l, ti.nodes, c++)] =
-                            ((unsigned)k << 16) |
-                            loc[slot_of(ti.chunk_off + l, ti.nodes, k)];
-                    }
-                    nup_h[p] = c;
+                    tile0_h[p] = ti.chunk_off;
                 }
             }
             for (int h : hl)
@@ -3067,15 +3165,22 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         chk(upload(s->rslot, rslot_h.data(), rslot_h.size()), "nlist");
         chk(upload(s->n_neigh, n_neigh, (size_t)N), "n_neigh");
         chk(upload(s->nlow, nlow_h.data(), nlow_h.size()), "exact lists");
-        chk(upload(s->nup, nup_h.data(), nup_h.size()), "exact lists");
-        chk(upload(s->uord, uord_h.data(), uord_h.size()), "exact lists");
+        chk(upload(s->tile0, tile0_h.data(), tile0_h.size()), "exact lists");
+        chk(s->nup.alloc((size_t)N), "exact lists");
+        // the rounds' look-ahead reads past a tile's lists, and positions
+        // past a list's end are dead
+        chk(s->ford.alloc(S + LOC_SLACK), "exact lists");
+        if (rc == PD_OK)
+            chk(hipMemset(s->ford.p, 0, (S + LOC_SLACK) * sizeof(unsigned)),
+                "exact lists");
     } else {
         s->nlist_ref.release();
         s->rslot.release();
         s->n_neigh.release();
         s->nlow.release();
         s->nup.release();
-        s->uord.release();
+        s->ford.release();
+        s->tile0.release();
     }
     chk(s->out_nlist.alloc(s->layout == PD_LAYOUT_SLOT ? (size_t)N * K : 0),
         "nlist export");
@@ -3108,6 +3213,9 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         s->k = bond_stiffness[0];
         s->s0 = critical_stretch[0];
     }
+    if (rc)
+        return rc;
+    rc = fold_lists(s);
     if (rc)
         return rc;
     rc = refresh_records(s);
@@ -3347,9 +3455,16 @@ int pd_set_exact_order(pd_sim *s, int on)
                                 "neighbours per node");
     const bool was = s->exact;
     s->exact = on != 0;
-    // the records carry V (exact) or 4kV (default): rewrite them
-    if (s->has_buffers && was != s->exact)
+    // the records carry V (exact) or 4kV (default): rewrite them; the fast
+    // step does not keep the fold lists
+    if (s->has_buffers && was != s->exact) {
+        if (s->exact) {
+            const int rc2 = fold_lists(s);
+            if (rc2)
+                return rc2;
+        }
         return refresh_records(s);
+    }
     return PD_OK;
 }
 

@@ -126,3 +126,46 @@ def test_rows_of_every_length(model, lanes, scale):
         assert pc.rel_l2(force, ref.force) < 1e-9
         broken = int(fam.sum() - np.sum(nn))
     assert 0 < broken < fam.sum() / 2
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-92])
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("fast_first", [False, True])
+def test_exact_order_rows_of_every_length(fast_first, tile, scale):
+    """The exact-order step on the same stars, bitwise: fold lists of every
+    length, split anywhere between lower and upper neighbours (the numbering
+    is random), with bonds breaking in both parts.  ``fast_first`` runs the
+    first, breaking step in the fast order, whose broken bonds the fold lists
+    made for the exact order must leave out."""
+    x, u0, fam, nl = _stars(scale, True, seed=8)
+    n, k = nl.shape
+    vol = np.random.default_rng(9).uniform(0.5, 1.5, n)
+    bct = np.zeros((n, 3), np.int32)
+    bcv = np.zeros((n, 3))
+    dt = 2e-4 * scale
+    z = np.zeros((n, 3))
+    integ = it.Euler(dt, exact_order=not fast_first)
+    integ.build(n, 3, k, x, vol, fam, bct, bcv, bct, bcv, None, None, None)
+    integ.set_launch(4, tile)
+    integ.create_buffers(nl, fam.copy(), 1.0, S0, None, u0, z, z, z, z,
+                         np.zeros(n), None, 1, 1)
+    ref = oracle.CythonEuler(dt, x, vol, fam, bct, bcv, bct, bcv, nl, fam,
+                             1.0, S0, u=u0)
+    for s in range(3):
+        integ(0.0, 0.0)
+        ref(0.0, 0.0)
+        if fast_first and s == 0:
+            integ.set_exact_order(True)
+            continue
+        u, _, _, force, _, dmg, lists, nn = integ.write(
+            None, None, None, None, None, None, None, None)
+        np.testing.assert_array_equal(lists, ref.nlist)
+        np.testing.assert_array_equal(nn, ref.n_neigh)
+        np.testing.assert_array_equal(dmg, ref.damage())
+        if fast_first:
+            assert pc.rel_l2(u / scale, ref.u / scale) < 1e-10
+            assert pc.rel_l2(force, ref.force) < 1e-9
+        else:
+            np.testing.assert_array_equal(u, ref.u)
+            np.testing.assert_array_equal(force, ref.force)
+    assert 0 < int(fam.sum() - nn.sum()) < fam.sum() / 2
