@@ -101,7 +101,11 @@ int pd_build(pd_sim **sim, int device, int integrator, int layout, double dt,
  *   plus_cs from model.py:941-1091, and regimes (N,K) i32 or NULL (zeros);
  *   bond_types must then have been given to pd_build (all zeros allowed).
  *   u, ud, udd: (N,3) f64 or NULL (zeros).
- * May be called again to restart from new state (Model.simulate does). */
+ * May be called again to restart from new state (Model.simulate does): with
+ * the same nlist and n_neigh (compared value by value with a host copy, kept
+ * while N*K is at most 2^28), launch shape and table shape, and no starting
+ * regimes but zeros, the tiles and bond slots are kept and only the state is
+ * set anew. */
 int pd_create_buffers(pd_sim *sim, const int *nlist, const int *n_neigh,
                       const double *bond_stiffness,
                       const double *critical_stretch, const double *plus_cs,
@@ -201,7 +205,8 @@ int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
  * Device memory: 14 bytes per bond slot, and per node 256 bytes plus 24
  * per checkpoint and per step of a segment.  Requires PD_EULER,
  * PD_LAYOUT_SLOT and pd_set_node_stiffness.  pd_create_buffers or
- * pd_adjoint_stop ends a recording. */
+ * pd_adjoint_stop ends a recording; its memory is kept for the next one until
+ * pd_adjoint_stop, a pd_create_buffers that tiles anew, or pd_destroy. */
 int pd_adjoint_start(pd_sim *sim, int nsteps, int checkpoint_every);
 
 /* dL_du (N,3) f64: dL/du after the recorded steps.  dL_dc (N) f64 receives

@@ -90,6 +90,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <string>
 #include <mutex>
 #include <thread>
@@ -1708,6 +1709,58 @@ __global__ void __launch_bounds__(256)
         reinterpret_cast<int4 *>(gidx)[c] = make_int4(w[0], w[1], w[2], w[3]);
 }
 
+// The bonds back to their state at set-up: loc and the n-linear state from
+// their copies, gidx without its marks (a slot that never held a bond has
+// loc_init 0 and keeps its own).  One thread per chunk, a stream of 2 + 4 B
+// read and at most 2 + 4 written per slot.
+__global__ void __launch_bounds__(256)
+    k_reset_bonds(long long nchunks, const unsigned short *loc_init,
+                  const unsigned short *state_init, unsigned short *loc,
+                  unsigned short *state, int *gidx)
+{
+    const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (c >= nchunks)
+        return;
+    const ushort4 l = reinterpret_cast<const ushort4 *>(loc_init)[c];
+    const int4 g = reinterpret_cast<const int4 *>(gidx)[c];
+    const unsigned short lv[4] = {l.x, l.y, l.z, l.w};
+    const int gv[4] = {g.x, g.y, g.z, g.w};
+    int w[4];
+    bool changed = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        w[q] = lv[q] == LOC_DEAD ? gv[q]
+                                 : (int)((uint32_t)gv[q] & KEYM);
+        changed |= w[q] != gv[q];
+    }
+    reinterpret_cast<ushort4 *>(loc)[c] = l;
+    if (changed)
+        reinterpret_cast<int4 *>(gidx)[c] = make_int4(w[0], w[1], w[2], w[3]);
+    if (state)
+        reinterpret_cast<ushort4 *>(state)[c] =
+            reinterpret_cast<const ushort4 *>(state_init)[c];
+}
+
+// The compact layout's rows as given at set-up: position pos[s] of the
+// caller's row lists slot s, and every bond counts.
+__global__ void __launch_bounds__(256)
+    k_row_slots(int n, int K, const int *tnode, const int *cnt,
+                const long long *chunk0, const int *stride,
+                const unsigned short *pos, unsigned short *rslot,
+                int *n_neigh)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int p = t / ROW_LANES, sub = t % ROW_LANES;
+    if (p >= n)
+        return;
+    const int i = tnode[p], c = cnt[p];
+    for (int k = sub; k < c; k += ROW_LANES)
+        rslot[(size_t)i * K + pos[slot_of(chunk0[p], stride[p], k)]] =
+            (unsigned short)k;
+    if (sub == 0)
+        n_neigh[i] = c;
+}
+
 // A per-node array in the caller's node order: dst[tnode[p]] = src[p], w
 // values per node.
 __global__ void k_unperm(int n, int w, const int *tnode, const double *src,
@@ -2029,6 +2082,11 @@ struct DevBuf {
             return hipSuccess;
         return hipMalloc(reinterpret_cast<void **>(&p), count * sizeof(T));
     }
+    // room for count values; what is there is kept if it suffices
+    hipError_t reserve(size_t count)
+    {
+        return p && n >= count ? hipSuccess : alloc(count);
+    }
 };
 
 }  // namespace
@@ -2059,7 +2117,7 @@ struct pd_sim {
     DevBuf<int> nlow, nup;  // exact step: lower slots, upper-list length
     DevBuf<unsigned> ford;  // exact step: fold lists
     DevBuf<long long> tile0;  // compact layout: first chunk of a node's tile
-    DevBuf<double> wbuf;  // a per-node array reordered for download
+    DevBuf<double> wbuf;  // a per-node array on its way to or from the host
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 
@@ -2070,6 +2128,14 @@ struct pd_sim {
     std::vector<double> h_corr;    // (N,K) as given to build
     std::vector<int> h_btypes;     // (N,K)
     std::vector<int> perm;         // internal node p -> caller's node id
+    // the tiling's inputs: a later pd_create_buffers with the same ones
+    // (compared value by value) keeps the tiles and slots
+    bool plan = false, plan_nlin = false;
+    int plan_tile_nodes = 0, plan_lpn = 0, plan_nregimes = 0, plan_types = 0;
+    std::unique_ptr<int[]> plan_nlist;  // (N,K)
+    std::vector<int> plan_nneigh;       // compact layout
+    DevBuf<unsigned short> loc_init, state_init;  // per slot, as set up
+    DevBuf<int> inv;  // caller's node id -> internal node (adjoint)
     std::vector<int> h_group;      // tiling groups (empty: one group)
 
     DevBuf<NodeRec> rec[2];
@@ -2368,12 +2434,18 @@ hipError_t launch_adjoint(pd_sim *s, const AdjArgs &a)
     return hipGetLastError();
 }
 
-void adjoint_release(pd_sim *s)
+// Ends a recording; its memory stays for the next one.
+void adjoint_end(pd_sim *s)
 {
     s->adj_recording = s->adj_ready = s->adj_replay = false;
     s->adj_nsteps = s->adj_every = s->step_counter = 0;
     s->adj_dmag.clear();
     s->adj_fmag.clear();
+}
+
+void adjoint_release(pd_sim *s)
+{
+    adjoint_end(s);
     s->brk.release();
     s->loc0.release();
     s->il0.release();
@@ -2516,6 +2588,144 @@ int fold_lists(pd_sim *s)
     return PD_OK;
 }
 
+// Rows of w values given in the caller's order into tile order on the device
+// (through wbuf); null clears.  On the library's stream: h is read until the
+// next synchronization.
+int upload_caller(pd_sim *s, DevBuf<double> &d, const double *h, int w)
+{
+    const size_t count = (size_t)s->n * w;
+    HIPCHK(d.reserve(count));
+    if (!h) {
+        HIPCHK(hipMemsetAsync(d.p, 0, count * sizeof(double), s->stream));
+        return PD_OK;
+    }
+    HIPCHK(s->wbuf.reserve(count));
+    HIPCHK(hipMemcpyAsync(s->wbuf.p, h, count * sizeof(double),
+                          hipMemcpyHostToDevice, s->stream));
+    hipLaunchKernelGGL(k_perm, dim3((s->n + 255) / 256), dim3(256), 0,
+                       s->stream, s->n, w, s->tnode.p, s->wbuf.p, d.p);
+    HIPCHK(hipGetLastError());
+    return PD_OK;
+}
+
+// The state of a (re)start once the bonds are set up: u, ud, udd, the fold
+// lists and the records.  Synchronizes.
+int start_state(pd_sim *s, const double *u, const double *ud,
+                const double *udd)
+{
+    int rc = upload_caller(s, s->u, u, 3);
+    if (rc == PD_OK)
+        rc = upload_caller(s, s->ud, ud, 3);
+    if (rc == PD_OK)
+        rc = upload_caller(s, s->udd, udd, 3);
+    if (rc == PD_OK)
+        rc = fold_lists(s);
+    return rc == PD_OK ? refresh_records(s) : rc;
+}
+
+// Whether a[0, count) and b[0, count) hold the same values, on as many
+// threads as their size is worth.
+bool same_values(const int *a, const int *b, size_t count)
+{
+    constexpr size_t PIECE = (size_t)1 << 19;
+    const int pieces = (int)((count + PIECE - 1) / PIECE);
+    std::atomic<int> differ{0};
+    run_parallel(pieces, [&](int lo, int hi) {
+        for (int c = lo; c < hi && !differ; ++c) {
+            const size_t first = (size_t)c * PIECE;
+            const size_t m = std::min(PIECE, count - first);
+            if (std::memcmp(a + first, b + first, m * sizeof(int)) != 0)
+                differ = 1;
+        }
+    }, 2);
+    return !differ;
+}
+
+// Most values of a neighbour list that are kept for comparison (1 GiB).
+constexpr size_t PLAN_MOST = (size_t)1 << 28;
+
+void keep_plan(pd_sim *s, const int *nlist, const int *n_neigh, bool nlin,
+               bool regimes_given)
+{
+    const size_t count = (size_t)s->n * s->K;
+    s->plan = false;
+    if (count > PLAN_MOST || (nlin && regimes_given))
+        return;
+    s->plan_nlist.reset(new (std::nothrow) int[count]);
+    if (!s->plan_nlist)
+        return;
+    int *dst = s->plan_nlist.get();
+    run_parallel(s->n, [&](int lo, int hi) {
+        std::memcpy(dst + (size_t)lo * s->K, nlist + (size_t)lo * s->K,
+                    (size_t)(hi - lo) * s->K * sizeof(int));
+    });
+    s->plan_nneigh.clear();
+    if (s->layout == PD_LAYOUT_COMPACT)
+        s->plan_nneigh.assign(n_neigh, n_neigh + s->n);
+    s->plan_nlin = nlin;
+    s->plan_nregimes = s->nregimes;
+    s->plan_types = s->nbond_types;
+    s->plan_tile_nodes = s->tile_nodes;
+    s->plan_lpn = s->lpn;
+    s->plan = true;
+}
+
+// Whether the tiles and slots made by the last pd_create_buffers serve these
+// arguments too: the same bonds, launch shape and damage-model tables' shape
+// (node arrays, corrections, bond types and groups cannot have changed).
+bool plan_holds(const pd_sim *s, const int *nlist, const int *n_neigh,
+                bool nlin, int nregimes, int nbond_types, bool regimes_given)
+{
+    return s->plan && s->has_buffers && !regimes_given &&
+           s->plan_nlin == nlin && s->plan_nregimes == nregimes &&
+           s->plan_types == nbond_types &&
+           s->plan_tile_nodes == s->tile_nodes && s->plan_lpn == s->lpn &&
+           (s->layout != PD_LAYOUT_COMPACT ||
+            same_values(s->plan_nneigh.data(), n_neigh, (size_t)s->n)) &&
+           same_values(s->plan_nlist.get(), nlist, (size_t)s->n * s->K);
+}
+
+// pd_create_buffers on the tiles and slots that are there: every bond live
+// again, new state and damage-model values.  What bounds it is PCIe (u, ud,
+// udd) and the comparison of the lists; tiling the 50,820-node bar anew took
+// 47 ms.
+int restart(pd_sim *s, const double *bond_stiffness,
+            const double *critical_stretch, const double *plus_cs,
+            const double *u, const double *ud, const double *udd)
+{
+    HIPCHK(hipStreamSynchronize(s->stream));
+    s->has_buffers = false;  // until the state is whole again
+    adjoint_end(s);
+    hipLaunchKernelGGL(k_reset_bonds, dim3(chunk_blocks(s)), dim3(256), 0,
+                       s->stream, (long long)(s->nslots / 4), s->loc_init.p,
+                       s->state_init.p, s->loc.p, s->state.p, s->gidx.p);
+    HIPCHK(hipGetLastError());
+    if (s->layout == PD_LAYOUT_COMPACT) {
+        hipLaunchKernelGGL(k_row_slots, dim3(row_blocks(s->n, ROW_LANES)),
+                           dim3(256), 0, s->stream, s->n, s->K, s->tnode.p,
+                           s->cnt.p, s->chunk0.p, s->stride.p, s->pos.p,
+                           s->rslot.p, s->n_neigh.p);
+        HIPCHK(hipGetLastError());
+    }
+    if (s->plan_nlin) {
+        const size_t T = (size_t)s->nregimes * s->nbond_types;
+        HIPCHK(upload(s->k_tab, bond_stiffness, T));
+        HIPCHK(upload(s->s_tab, critical_stretch, T));
+        HIPCHK(upload(s->pc_tab, plus_cs, T));
+    } else {
+        s->k = bond_stiffness[0];
+        s->s0 = critical_stretch[0];
+    }
+    int rc = start_state(s, u, ud, udd);
+    if (rc == PD_OK && !s->tip_q.p)
+        rc = upload_tips(s);
+    if (rc)
+        return rc;
+    s->has_buffers = true;
+    s->retile_pending = false;
+    return PD_OK;
+}
+
 uint64_t spread3(uint64_t v)
 {
     v &= 0x1fffff;
@@ -2631,26 +2841,42 @@ std::vector<int> morton_order(int n, const double *x, const int *group)
     if (!(h > 0.0))
         h = 1.0;
     std::vector<uint64_t> code(n);
-    for (int i = 0; i < n; ++i) {
-        uint64_t c = 0;
-        for (int d = 0; d < 3; ++d) {
-            double v = std::floor((x[3 * (size_t)i + d] - lo[d]) / h);
-            v = std::min(std::max(v, 0.0), 2097151.0);
-            c |= spread3((uint64_t)v) << d;
+    run_parallel(n, [&](int first, int end) {
+        for (int i = first; i < end; ++i) {
+            uint64_t c = 0;
+            for (int d = 0; d < 3; ++d) {
+                double v = std::floor((x[3 * (size_t)i + d] - lo[d]) / h);
+                v = std::min(std::max(v, 0.0), 2097151.0);
+                c |= spread3((uint64_t)v) << d;
+            }
+            code[i] = c;
         }
-        code[i] = c;
-    }
-    std::vector<int> order(n);
+    });
+    std::vector<int> order(n), other(n);
     for (int i = 0; i < n; ++i)
         order[i] = i;
-    if (group)
-        std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-            return group[a] != group[b] ? group[a] < group[b]
-                                        : code[a] < code[b];
+    // stable counting sort, 11 bits of the key at a time from the lowest:
+    // by code, then by group
+    const auto sort_by = [&](auto key) {
+        uint64_t top = 0;
+        for (int i = 0; i < n; ++i)
+            top |= key(i);
+        for (int shift = 0; shift < 64 && (top >> shift) != 0; shift += 11) {
+            std::vector<int> at(2049, 0);
+            for (int i = 0; i < n; ++i)
+                ++at[((key(i) >> shift) & 2047) + 1];
+            for (int b = 0; b < 2048; ++b)
+                at[b + 1] += at[b];
+            for (int q = 0; q < n; ++q)
+                other[at[(key(order[q]) >> shift) & 2047]++] = order[q];
+            order.swap(other);
+        }
+    };
+    sort_by([&](int i) { return code[i]; });
+    if (group)  // signed values in order
+        sort_by([&](int i) {
+            return (uint64_t)((uint32_t)group[i] ^ 0x80000000u);
         });
-    else
-        std::stable_sort(order.begin(), order.end(),
-                         [&](int a, int b) { return code[a] < code[b]; });
     return order;
 }
 
@@ -2849,18 +3075,37 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
             return fail(PD_E_LIMIT, "damage model table too large");
     }
     const int N = s->n, K = s->K;
+    std::atomic<int> given{0};  // some bond starts past its first regime
     if (nlin) {
-        for (size_t q = 0; q < (size_t)N * K; ++q) {
-            if (nlist[q] == -1)
-                continue;
-            const int t = s->h_btypes[q];
-            if (t < 0 || t >= nbond_types)
-                return fail(PD_E_ARG, "bond_types value out of range");
-            if (regimes && (regimes[q] < 0 || regimes[q] >= nregimes))
-                return fail(PD_E_ARG, "regimes value out of range for a "
-                                      "live bond");
-        }
+        std::atomic<int> bad{0};
+        run_parallel(N, [&](int lo, int hi) {
+            int found = 0, past = 0;
+            for (size_t q = (size_t)lo * K; q < (size_t)hi * K; ++q) {
+                if (nlist[q] == -1)
+                    continue;
+                const int t = s->h_btypes[q];
+                if (t < 0 || t >= nbond_types)
+                    found = 1;
+                if (regimes) {
+                    if (regimes[q] < 0 || regimes[q] >= nregimes)
+                        found = found == 1 ? 1 : 2;
+                    past |= regimes[q];
+                }
+            }
+            if (found)
+                bad = bad == 1 ? 1 : found;
+            if (past)
+                given = 1;
+        });
+        if (bad == 1)
+            return fail(PD_E_ARG, "bond_types value out of range");
+        if (bad == 2)
+            return fail(PD_E_ARG, "regimes value out of range for a "
+                                  "live bond");
     }
+    if (plan_holds(s, nlist, n_neigh, nlin, nregimes, nbond_types, given))
+        return restart(s, bond_stiffness, critical_stretch, plus_cs, u, ud,
+                       udd);
 
     // bond rows: live entries (j, reference column), sorted ascending by j
     std::vector<int> cnt(N);
@@ -2924,80 +3169,82 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         }
     });
 
-    // tiles: greedy over the Morton order, capped by tile_nodes and by the
-    // LDS halo capacity
+    // tiles: runs of the Morton order, capped by tile_nodes and by the LDS
+    // halo capacity
     // entry 0 of a staged halo is the zero record of dead slots
     // the compact layout's tiles leave room for the exact step's windows
     s->hmax = (nlin ? LDS_CAP_NLIN
                     : (s->layout == PD_LAYOUT_COMPACT ? EXACT_CAP
                                                       : LDS_CAP_PMB)) -
               1;
-    const std::vector<int> order = morton_order(
+    std::vector<int> tnode = morton_order(
         N, s->h_coords.data(), s->h_group.empty() ? nullptr : s->h_group.data());
-    std::vector<int> stamp(N, -1), probe(N, -1);
-    std::vector<TileInfo> tiles;
-    std::vector<int> tnode;
-    tnode.reserve(N);
-    {
-        int cur_nodes = 0, cur_halo = 0, tid = 0, nprobe = 0;
-        // distinct nodes of i's neighbourhood not yet in tile t (a row may
-        // list a neighbour more than once)
-        auto count_new = [&](int i, int t) {
-            ++nprobe;
-            int c = 0;
-            auto visit = [&](int j) {
-                if (stamp[j] != t && probe[j] != nprobe) {
-                    probe[j] = nprobe;
-                    ++c;
+    // blocks: runs of tile_nodes nodes of one group.  A block is one tile, or
+    // several where the halo capacity cuts it; blocks do not depend on each
+    // other, so threads take them side by side.
+    const int cap = s->tile_nodes;
+    std::vector<int> bstart;
+    for (int q = 0; q < N; ++q)
+        if (q == 0 || q - bstart.back() == cap ||
+            (!s->h_group.empty() &&
+             s->h_group[tnode[q]] != s->h_group[tnode[q - 1]]))
+            bstart.push_back(q);
+    const int nblocks = (int)bstart.size();
+    bstart.push_back(N);
+    std::vector<std::vector<TileInfo>> cuts(nblocks);
+    std::atomic<int> wide{0};
+    run_parallel(nblocks, [&](int lo, int hi) {
+        std::vector<int> stamp(N, -1);
+        int tid = 0;
+        for (int bl = lo; bl < hi; ++bl) {
+            TileInfo t{};
+            t.node_off = bstart[bl];
+            ++tid;
+            for (int q = bstart[bl]; q < bstart[bl + 1]; ++q) {
+                const int i = tnode[q];
+                if (1 + cnt[i] > s->hmax) {
+                    wide = 1;
+                    return;
                 }
-            };
-            visit(i);
-            for (long long q = rstart[i]; q < rstart[i + 1]; ++q)
-                visit(rj[q]);
-            return c;
-        };
-        for (int q = 0; q < N; ++q) {
-            const int i = order[q];
-            if (1 + cnt[i] > s->hmax)
-                return fail(PD_E_LIMIT, "a node's neighbourhood exceeds the "
-                                        "LDS halo capacity");
-            int add = count_new(i, tid);
-            const bool new_group =
-                cur_nodes > 0 && !s->h_group.empty() &&
-                s->h_group[i] != s->h_group[tnode.back()];
-            if (cur_nodes > 0 && (cur_nodes == s->tile_nodes || new_group ||
-                                  cur_halo + add > s->hmax)) {
-                TileInfo t;
-                t.node_off = (int)tnode.size() - cur_nodes;
-                t.nodes = cur_nodes;
-                t.halo = cur_halo;
-                tiles.push_back(t);
-                ++tid;
-                cur_nodes = 0;
-                cur_halo = 0;
-                add = count_new(i, tid);
+                // the distinct nodes that i and its neighbours add (a row
+                // may list a neighbour more than once)
+                auto add = [&]() {
+                    int c = 0;
+                    auto visit = [&](int j) {
+                        c += stamp[j] != tid;
+                        stamp[j] = tid;
+                    };
+                    visit(i);
+                    for (long long r = rstart[i]; r < rstart[i + 1]; ++r)
+                        visit(rj[r]);
+                    return c;
+                };
+                int c = add();
+                if (t.nodes > 0 && t.halo + c > s->hmax) {
+                    cuts[bl].push_back(t);
+                    t = TileInfo{};
+                    t.node_off = q;
+                    ++tid;
+                    c = add();
+                }
+                t.halo += c;
+                ++t.nodes;
             }
-            stamp[i] = tid;
-            for (long long r = rstart[i]; r < rstart[i + 1]; ++r)
-                stamp[rj[r]] = tid;
-            cur_halo += add;
-            ++cur_nodes;
-            tnode.push_back(i);
+            cuts[bl].push_back(t);
+            // within a tile, nodes by descending bond count: the nodes
+            // sharing a wavefront then run loops of nearly equal length
+            for (const auto &x : cuts[bl])
+                std::stable_sort(tnode.begin() + x.node_off,
+                                 tnode.begin() + x.node_off + x.nodes,
+                                 [&](int y, int z) { return cnt[y] > cnt[z]; });
         }
-        if (cur_nodes > 0) {
-            TileInfo t;
-            t.node_off = (int)tnode.size() - cur_nodes;
-            t.nodes = cur_nodes;
-            t.halo = cur_halo;
-            tiles.push_back(t);
-        }
-    }
-    // within a tile, nodes by descending bond count: the nodes sharing a
-    // wavefront then run loops of nearly equal length
-    for (const auto &t : tiles)
-        std::stable_sort(tnode.begin() + t.node_off,
-                         tnode.begin() + t.node_off + t.nodes,
-                         [&](int x, int y) { return cnt[x] > cnt[y]; });
+    }, 16);
+    if (wide)
+        return fail(PD_E_LIMIT, "a node's neighbourhood exceeds the "
+                                "LDS halo capacity");
+    std::vector<TileInfo> tiles;
+    for (const auto &c : cuts)
+        tiles.insert(tiles.end(), c.begin(), c.end());
     std::vector<int> inv(N);  // caller's node id -> internal id
     for (int q = 0; q < N; ++q)
         inv[tnode[q]] = q;
@@ -3037,7 +3284,6 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     const bool compact = s->layout == PD_LAYOUT_COMPACT;
     std::vector<int> nlow_h(compact ? N : 0);
     std::vector<long long> tile0_h(compact ? N : 0);
-    std::vector<unsigned short> rslot_h(compact ? (size_t)N * K : 0, 0);
     std::atomic<int> halo_mismatch{0};
     run_parallel(ntiles, [&](int lo, int hi) {
         std::vector<int> lmap(N, -1);  // internal id -> halo position
@@ -3093,10 +3339,6 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                                   (regimes ? regimes[src] : 0)));
                 }
                 if (compact) {
-                    // row position -> slot; the lower slots
-                    for (int k = 0; k < cnt[i]; ++k)
-                        rslot_h[(size_t)i * K + rp[rstart[i] + k]] =
-                            (unsigned short)k;
                     const int p = ti.node_off + l;
                     const int *rb = rj.data() + rstart[i];
                     nlow_h[p] = (int)(std::lower_bound(rb, rb + cnt[i], i) - rb);
@@ -3117,7 +3359,9 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     // from here the device state is replaced: until it is whole again no
     // step may run (a failure below leaves the simulation without buffers)
     s->has_buffers = false;
+    s->plan = false;
     adjoint_release(s);
+    s->inv.release();
     auto chk = [&](hipError_t e, const char *what) {
         if (e != hipSuccess && rc == PD_OK)
             rc = fail(PD_E_HIP, std::string(what) + ": " + hipGetErrorString(e));
@@ -3179,10 +3423,31 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         chk(upload(s->state, state.data(), state.size()), "state");
     else
         s->state.release();
+    chk(s->loc_init.alloc(S), "loc");
+    if (rc == PD_OK)
+        chk(hipMemcpyAsync(s->loc_init.p, s->loc.p, S * sizeof(unsigned short),
+                           hipMemcpyDeviceToDevice, s->stream),
+            "loc");
+    s->state_init.release();
+    if (nlin && !given) {
+        chk(s->state_init.alloc(S), "state");
+        if (rc == PD_OK)
+            chk(hipMemcpyAsync(s->state_init.p, s->state.p,
+                               S * sizeof(unsigned short),
+                               hipMemcpyDeviceToDevice, s->stream),
+                "state");
+    }
     if (s->layout == PD_LAYOUT_COMPACT) {
         chk(upload(s->nlist_ref, nlist, (size_t)N * K), "nlist");
-        chk(upload(s->rslot, rslot_h.data(), rslot_h.size()), "nlist");
-        chk(upload(s->n_neigh, n_neigh, (size_t)N), "n_neigh");
+        chk(s->rslot.alloc((size_t)N * K), "nlist");
+        chk(s->n_neigh.alloc((size_t)N), "n_neigh");
+        if (rc == PD_OK) {
+            hipLaunchKernelGGL(k_row_slots, dim3(row_blocks(N, ROW_LANES)),
+                               dim3(256), 0, s->stream, N, K, s->tnode.p,
+                               s->cnt.p, s->chunk0.p, s->stride.p, s->pos.p,
+                               s->rslot.p, s->n_neigh.p);
+            chk(hipGetLastError(), "nlist");
+        }
         chk(upload(s->nlow, nlow_h.data(), nlow_h.size()), "exact lists");
         chk(upload(s->tile0, tile0_h.data(), tile0_h.size()), "exact lists");
         chk(s->nup.alloc((size_t)N), "exact lists");
@@ -3190,7 +3455,8 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         // past a list's end are dead
         chk(s->ford.alloc(S + LOC_SLACK), "exact lists");
         if (rc == PD_OK)
-            chk(hipMemset(s->ford.p, 0, (S + LOC_SLACK) * sizeof(unsigned)),
+            chk(hipMemsetAsync(s->ford.p, 0,
+                               (S + LOC_SLACK) * sizeof(unsigned), s->stream),
                 "exact lists");
     } else {
         s->nlist_ref.release();
@@ -3203,19 +3469,6 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     }
     chk(s->out_nlist.alloc(s->layout == PD_LAYOUT_SLOT ? (size_t)N * K : 0),
         "nlist export");
-    const size_t B = 3 * (size_t)N * sizeof(double);
-    if (u)
-        chk(upload_perm(s->u, s->perm, u, 3), "u");
-    else
-        chk(hipMemset(s->u.p, 0, B), "u");
-    if (ud)
-        chk(upload_perm(s->ud, s->perm, ud, 3), "ud");
-    else
-        chk(hipMemset(s->ud.p, 0, B), "ud");
-    if (udd)
-        chk(upload_perm(s->udd, s->perm, udd, 3), "udd");
-    else
-        chk(hipMemset(s->udd.p, 0, B), "udd");
     s->nregimes = nregimes;
     s->nbond_types = nbond_types;
     if (nlin) {
@@ -3234,10 +3487,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     }
     if (rc)
         return rc;
-    rc = fold_lists(s);
-    if (rc)
-        return rc;
-    rc = refresh_records(s);
+    rc = start_state(s, u, ud, udd);
     if (rc)
         return rc;
     rc = upload_tips(s);
@@ -3245,7 +3495,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         return rc;
     s->has_buffers = true;
     s->retile_pending = false;
-    adjoint_release(s);  // slot arrays were rebuilt
+    keep_plan(s, nlist, n_neigh, nlin, given);
     return PD_OK;
 }
 
@@ -3640,27 +3890,29 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
                               "slot layout and a node stiffness field");
     if (nsteps < 1 || checkpoint_every < 1)
         return fail(PD_E_ARG, "nsteps and checkpoint_every must be >= 1");
-    adjoint_release(s);
+    adjoint_end(s);
     const size_t S = s->nslots, N = (size_t)s->n, B = 3 * N;
     const int nck = (nsteps + checkpoint_every - 1) / checkpoint_every;
-    std::vector<int> inv(N);
-    for (size_t q = 0; q < N; ++q)
-        inv[s->perm[q]] = (int)q;
-    DevBuf<int> inv_d;
-    HIPCHK(upload(inv_d, inv.data(), N));
-    HIPCHK(s->brk.alloc(S));
-    HIPCHK(s->il0.alloc(S));
-    HIPCHK(s->arec[0].alloc(N));
-    HIPCHK(s->arec[1].alloc(N));
-    HIPCHK(s->loc0.alloc(S));
-    HIPCHK(s->ckpt.alloc((size_t)nck * B));
-    HIPCHK(s->seg.alloc((size_t)checkpoint_every * B));
-    HIPCHK(s->lam[0].alloc(B));
-    HIPCHK(s->lam[1].alloc(B));
-    HIPCHK(s->gradc.alloc(N));
-    HIPCHK(s->fin_u.alloc(B));
-    HIPCHK(s->fin_force.alloc(B));
-    HIPCHK(s->fin_bforce.alloc(B));
+    if (!s->inv.p) {
+        std::vector<int> inv(N);
+        for (size_t q = 0; q < N; ++q)
+            inv[s->perm[q]] = (int)q;
+        HIPCHK(upload(s->inv, inv.data(), N));
+    }
+    // a recording after one of the same size allocates nothing
+    HIPCHK(s->brk.reserve(S));
+    HIPCHK(s->il0.reserve(S));
+    HIPCHK(s->arec[0].reserve(N));
+    HIPCHK(s->arec[1].reserve(N));
+    HIPCHK(s->loc0.reserve(S));
+    HIPCHK(s->ckpt.reserve((size_t)nck * B));
+    HIPCHK(s->seg.reserve((size_t)checkpoint_every * B));
+    HIPCHK(s->lam[0].reserve(B));
+    HIPCHK(s->lam[1].reserve(B));
+    HIPCHK(s->gradc.reserve(N));
+    HIPCHK(s->fin_u.reserve(B));
+    HIPCHK(s->fin_force.reserve(B));
+    HIPCHK(s->fin_bforce.reserve(B));
     // rows past a node's own, up to its tile's longest: finite
     HIPCHK(hipMemsetAsync(s->il0.p, 0, S * sizeof(double), s->stream));
     hipLaunchKernelGGL(k_adj_init, dim3(chunk_blocks(s)), dim3(256), 0,
@@ -3669,11 +3921,10 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_adj_il0, dim3(row_blocks(s->n, ROW_LANES)),
                        dim3(256), 0, s->stream, s->n, s->cnt.p, s->chunk0.p, s->stride.p,
-                       s->gidx.p, s->loc0.p, inv_d.p, s->r0.p, s->il0.p);
+                       s->gidx.p, s->loc0.p, s->inv.p, s->r0.p, s->il0.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(s->ckpt.p, s->u.p, B * sizeof(double),
                           hipMemcpyDeviceToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
     s->adj_nsteps = nsteps;
     s->adj_every = checkpoint_every;
     s->step_counter = 0;
