@@ -1127,7 +1127,9 @@ __device__ __forceinline__ int live_slots(const unsigned short *loc,
 // (peridynamics.pyx:29), and, for the slot layout, the reference-layout
 // neighbour list: -1 everywhere but at the live slots' columns.  LANES
 // lanes handle internal node p and write row tnode[p] of the outputs.
-// rows == 0 counts the live bonds without rebuilding the slot-layout rows.
+// rows == 0 counts the live bonds without rebuilding the slot-layout rows;
+// with u_out, u goes along into the caller's node order (one launch for the
+// read-out of u and damage that every write interval makes).
 // Without rows it reads 2 B per slot (loc): 3.8 us on a 2560-node bar and 83
 // on 1,038,230 nodes, where one lane per node walking gidx took 23 and 243.
 template <int LANES>
@@ -1137,12 +1139,15 @@ __global__ void __launch_bounds__(256)
              const unsigned short *loc, const int *gidx,
              const unsigned short *pos, const int *family,
              const int *n_neigh_c, int *nlist_out, int *n_neigh_out,
-             double *damage)
+             double *damage, const double *u, double *u_out)
 {
     const int t = blockIdx.x * 256 + threadIdx.x;
     const int p = t / LANES, sub = t % LANES;
     const bool valid = p < n;
     const int i = valid ? tnode[p] : 0;
+    if (u_out && valid)
+        for (int d = sub; d < 3; d += LANES)
+            u_out[3 * (size_t)i + d] = u[3 * (size_t)p + d];
     int live = 0;
     if (layout == PD_LAYOUT_SLOT) {
         const int c = valid ? cnt[p] : 0;
@@ -2247,7 +2252,8 @@ unsigned chunk_blocks(const pd_sim *s)
     return (unsigned)((s->nslots / 4 + 255) / 256);
 }
 
-hipError_t launch_export(pd_sim *s, int rows)
+hipError_t launch_export(pd_sim *s, int rows, double *damage,
+                         double *u_out = nullptr)
 {
     const auto go = [&](auto kernel, int lanes) {
         hipLaunchKernelGGL(kernel, dim3(row_blocks(s->n, lanes)), dim3(256),
@@ -2255,7 +2261,7 @@ hipError_t launch_export(pd_sim *s, int rows)
                            s->tnode.p, s->cnt.p, s->chunk0.p, s->stride.p,
                            s->loc.p, s->gidx.p, s->pos.p, s->family.p,
                            s->n_neigh.p, s->out_nlist.p, s->out_nneigh.p,
-                           s->damage.p);
+                           damage, s->u.p, u_out);
     };
     if (s->layout == PD_LAYOUT_COMPACT)
         go(k_export<1>, 1);  // counts are kept: one lane per node
@@ -2741,8 +2747,8 @@ uint64_t spread3(uint64_t v)
 // reads together fall into different banks.  One ds_read_b128 over 16
 // consecutive lanes reads a 16-byte piece of each lane's neighbour record;
 // records whose entries are equal modulo HALO_BANK_GROUPS share banks, and
-// distinct records in one bank are read one after another.  rows[l] lists
-// the tile's node l's neighbours as halo indices in slot order; lane
+// distinct records in one bank are read one after another.  A row lists its
+// node's neighbours as halo indices in slot order; lane
 // t = l * lpn + sub takes the chunks of four slots sub, sub + lpn, ...  Read
 // groups are (16 lanes, round, bond of the chunk).  Greedy: records in the
 // most groups first, each to the residue least loaded over its groups among
@@ -2750,73 +2756,92 @@ uint64_t spread3(uint64_t v)
 // halo index; the order changes no result.
 constexpr int HALO_BANK_GROUPS = 16;
 
-std::vector<int> spread_halo(const std::vector<std::vector<int>> &rows,
-                             int lpn, int H)
-{
-    constexpr int NB = HALO_BANK_GROUPS;
-    std::vector<std::vector<int>> memb(H);
-    std::vector<int> seen(H, -1);
-    const int lanes = (int)rows.size() * lpn;
-    int ngroups = 0;
-    for (int q0 = 0; q0 < lanes; q0 += 16) {
-        const int q1 = std::min(q0 + 16, lanes);
-        int rounds = 0;
-        for (int t = q0; t < q1; ++t) {
-            const int nch = chunks_of((int)rows[t / lpn].size());
-            rounds = std::max(rounds, (nch - t % lpn + lpn - 1) / lpn);
-        }
-        for (int k = 0; k < rounds; ++k)
-            for (int b = 0; b < 4; ++b) {
-                const int g = ngroups++;
-                for (int t = q0; t < q1; ++t) {
-                    const std::vector<int> &row = rows[t / lpn];
-                    const int c = t % lpn + lpn * k;
-                    const int p = 16 * (c >> 2) + 8 * (b >> 1) +
-                                  2 * (c & 3) + (b & 1);
-                    if (p < (int)row.size() && seen[row[p]] != g) {
-                        seen[row[p]] = g;
-                        memb[row[p]].push_back(g);
+// Its scratch, kept from tile to tile of one thread.
+struct HaloSpread {
+    std::vector<int> seen, first, pairs, order, pos, rank;
+    std::vector<std::pair<int, int>> found;  // (record, group)
+    std::vector<unsigned short> load;
+
+    // off[l], off[l + 1]: node l's row in nb
+    const std::vector<int> &place(const std::vector<int> &off,
+                                  const std::vector<int> &nb, int lpn, int H)
+    {
+        constexpr int NB = HALO_BANK_GROUPS;
+        seen.assign(H, -1);
+        first.assign(H + 1, 0);
+        found.clear();
+        const int lanes = ((int)off.size() - 1) * lpn;
+        int ngroups = 0;
+        for (int q0 = 0; q0 < lanes; q0 += 16) {
+            const int q1 = std::min(q0 + 16, lanes);
+            int rounds = 0;
+            for (int t = q0; t < q1; ++t) {
+                const int l = t / lpn;
+                const int nch = chunks_of(off[l + 1] - off[l]);
+                rounds = std::max(rounds, (nch - t % lpn + lpn - 1) / lpn);
+            }
+            for (int k = 0; k < rounds; ++k)
+                for (int b = 0; b < 4; ++b) {
+                    const int g = ngroups++;
+                    for (int t = q0; t < q1; ++t) {
+                        const int l = t / lpn, c = t % lpn + lpn * k;
+                        const int p = off[l] + 16 * (c >> 2) + 8 * (b >> 1) +
+                                      2 * (c & 3) + (b & 1);
+                        if (p < off[l + 1] && seen[nb[p]] != g) {
+                            seen[nb[p]] = g;
+                            found.emplace_back(nb[p], g);
+                            ++first[nb[p] + 1];
+                        }
                     }
                 }
-            }
-    }
-    std::vector<int> avail(NB, 0);
-    for (int e = 1; e <= H; ++e)
-        ++avail[e % NB];
-    std::vector<int> order(H);
-    for (int h = 0; h < H; ++h)
-        order[h] = h;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        return memb[x].size() > memb[y].size();
-    });
-    std::vector<unsigned short> load((size_t)ngroups * NB, 0);
-    std::vector<int> res(H);
-    int score[NB];
-    for (int h : order) {
-        for (int r = 0; r < NB; ++r)
-            score[r] = 0;
-        for (int g : memb[h])
+        }
+        int most = 0;
+        for (int h = 0; h < H; ++h) {
+            most = std::max(most, first[h + 1]);
+            first[h + 1] += first[h];
+        }
+        pairs.resize(found.size());
+        pos.assign(first.begin(), first.end() - 1);
+        for (const auto &f : found)
+            pairs[pos[f.first]++] = f.second;
+        // records by descending number of groups, in index order where equal
+        rank.assign(most + 2, 0);
+        for (int h = 0; h < H; ++h)
+            ++rank[most - (first[h + 1] - first[h]) + 1];
+        for (int r = 0; r <= most; ++r)
+            rank[r + 1] += rank[r];
+        order.resize(H);
+        for (int h = 0; h < H; ++h)
+            order[rank[most - (first[h + 1] - first[h])]++] = h;
+        int avail[NB] = {}, next[NB];
+        for (int e = 1; e <= H; ++e)
+            ++avail[e % NB];
+        load.assign((size_t)ngroups * NB, 0);
+        pos.resize(H);
+        for (int h : order) {
+            int score[NB] = {};
+            for (int m = first[h]; m < first[h + 1]; ++m)
+                for (int r = 0; r < NB; ++r)
+                    score[r] += load[(size_t)pairs[m] * NB + r];
+            int best = -1;
             for (int r = 0; r < NB; ++r)
-                score[r] += load[(size_t)g * NB + r];
-        int best = -1;
+                if (avail[r] > 0 && (best < 0 || score[r] < score[best]))
+                    best = r;
+            pos[h] = best;
+            --avail[best];
+            for (int m = first[h]; m < first[h + 1]; ++m)
+                ++load[(size_t)pairs[m] * NB + best];
+        }
         for (int r = 0; r < NB; ++r)
-            if (avail[r] > 0 && (best < 0 || score[r] < score[best]))
-                best = r;
-        res[h] = best;
-        --avail[best];
-        for (int g : memb[h])
-            ++load[(size_t)g * NB + best];
+            next[r] = r == 0 ? NB : r;
+        for (int h = 0; h < H; ++h) {
+            const int r = pos[h];
+            pos[h] = next[r] - 1;
+            next[r] += NB;
+        }
+        return pos;
     }
-    int next[NB];
-    for (int r = 0; r < NB; ++r)
-        next[r] = r == 0 ? NB : r;
-    std::vector<int> pos(H);
-    for (int h = 0; h < H; ++h) {
-        pos[h] = next[res[h]] - 1;
-        next[res[h]] += NB;
-    }
-    return pos;
-}
+};
 
 // Node order for tiling: Morton order of the initial coordinates on a grid
 // whose cell holds about one node.
@@ -3157,11 +3182,12 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                     if (row[p] != -1)
                         ent.emplace_back(row[p], p);
             }
-            std::stable_sort(ent.begin(), ent.end(),
-                             [](const std::pair<int, int> &x,
-                                const std::pair<int, int> &y) {
-                                 return x.first < y.first;
-                             });
+            const auto by_key = [](const std::pair<int, int> &x,
+                                   const std::pair<int, int> &y) {
+                return x.first < y.first;
+            };
+            if (!std::is_sorted(ent.begin(), ent.end(), by_key))
+                std::stable_sort(ent.begin(), ent.end(), by_key);
             for (size_t k = 0; k < ent.size(); ++k) {
                 rj[rstart[i] + k] = ent[k].first;
                 rp[rstart[i] + k] = (unsigned short)ent[k].second;
@@ -3288,33 +3314,40 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     run_parallel(ntiles, [&](int lo, int hi) {
         std::vector<int> lmap(N, -1);  // internal id -> halo position
         std::vector<int> hl;
-        std::vector<std::vector<int>> rows;
+        std::vector<int> roff, rows;
+        HaloSpread spread;
         for (int t = lo; t < hi; ++t) {
             const TileInfo &ti = tiles[t];
             hl.clear();
+            auto visit = [&](int h) {
+                if (lmap[h] == -1) {
+                    lmap[h] = 0;
+                    hl.push_back(h);
+                }
+            };
             for (int l = 0; l < ti.nodes; ++l) {
                 const int i = tnode[ti.node_off + l];
-                hl.push_back(ti.node_off + l);
+                visit(ti.node_off + l);
                 for (long long r = rstart[i]; r < rstart[i + 1]; ++r)
-                    hl.push_back(inv[rj[r]]);
+                    visit(inv[rj[r]]);
             }
             std::sort(hl.begin(), hl.end());
-            hl.erase(std::unique(hl.begin(), hl.end()), hl.end());
             if ((int)hl.size() != ti.halo) {
                 halo_mismatch = 1;
-                continue;
+                break;
             }
             for (size_t h = 0; h < hl.size(); ++h)
                 lmap[hl[h]] = (int)h;
-            rows.resize(ti.nodes);
+            rows.clear();
+            roff.assign(1, 0);
             for (int l = 0; l < ti.nodes; ++l) {
                 const int i = tnode[ti.node_off + l];
-                rows[l].clear();
                 for (int k = 0; k < cnt[i]; ++k)
-                    rows[l].push_back(lmap[inv[rj[rstart[i] + k]]]);
+                    rows.push_back(lmap[inv[rj[rstart[i] + k]]]);
+                roff.push_back((int)rows.size());
             }
-            const std::vector<int> hpos =
-                spread_halo(rows, s->lpn, (int)hl.size());
+            const std::vector<int> &hpos =
+                spread.place(roff, rows, s->lpn, (int)hl.size());
             for (size_t h = 0; h < hl.size(); ++h) {
                 lmap[hl[h]] = hpos[h];
                 halo[ti.halo_off + hpos[h]] = hl[h];
@@ -3555,7 +3588,7 @@ int pd_monitor(pd_sim *s, double *model, double *tips)
     if (s->mon_out.n < nout) {
         HIPCHK(s->mon_out.alloc(nout));
     }
-    HIPCHK(launch_export(s, 0));
+    HIPCHK(launch_export(s, 0, s->damage.p));
     hipLaunchKernelGGL(k_monitor_part, dim3(MON_BLOCKS), dim3(256), 0,
                        s->stream, N, s->u.p, s->ud.p, s->udd.p, s->force.p,
                        s->body_force.p, s->flags.p, s->vol.p, s->damage.p,
@@ -3628,7 +3661,7 @@ int pd_monitor_noalloc(pd_sim *s, double *model, double *tips)
     double *part = sp;
     double *staged = sp + (size_t)MON_BLOCKS * MON_SUMS;
     const int N = s->n;
-    HIPCHK(launch_export(s, 0));
+    HIPCHK(launch_export(s, 0, s->damage.p));
     hipLaunchKernelGGL(k_monitor_part, dim3(MON_BLOCKS), dim3(256), 0,
                        s->stream, N, s->u.p, s->ud.p, s->udd.p, s->force.p,
                        s->body_force.p, s->flags.p, s->vol.p, s->damage.p,
@@ -4096,16 +4129,11 @@ int pd_write_device(pd_sim *s, double *u, double *damage)
         return rc;
     if (!s->has_buffers)
         return fail(PD_E_STATE, "pd_create_buffers has not been called");
-    const int N = s->n;
-    const int blocks = (N + 255) / 256;
     if (damage) {
-        HIPCHK(launch_export(s, 0));
-        HIPCHK(hipMemcpyAsync(damage, s->damage.p, (size_t)N * sizeof(double),
-                              hipMemcpyDeviceToDevice, s->stream));
-    }
-    if (u) {
-        hipLaunchKernelGGL(k_unperm, dim3(blocks), dim3(256), 0, s->stream, N,
-                           3, s->tnode.p, s->u.p, u);
+        HIPCHK(launch_export(s, 0, damage, u));
+    } else if (u) {
+        hipLaunchKernelGGL(k_unperm, dim3((s->n + 255) / 256), dim3(256), 0,
+                           s->stream, s->n, 3, s->tnode.p, s->u.p, u);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -4131,8 +4159,10 @@ int pd_write(pd_sim *s, double *u, double *ud, double *udd, double *force,
     if (!s->has_buffers)
         return fail(PD_E_STATE, "pd_create_buffers has not been called");
     const int N = s->n;
-    const int blocks = (N + 255) / 256;
-    HIPCHK(launch_export(s, nlist ? 1 : 0));
+    if (u)
+        HIPCHK(s->wbuf.reserve(3 * (size_t)N));
+    HIPCHK(launch_export(s, nlist ? 1 : 0, s->damage.p,
+                         u ? s->wbuf.p : nullptr));
     if (nlist && s->layout == PD_LAYOUT_COMPACT) {
         hipLaunchKernelGGL(k_export_rows, dim3(row_blocks(N, ROW_LANES)),
                            dim3(256), 0,
@@ -4141,11 +4171,17 @@ int pd_write(pd_sim *s, double *u, double *ud, double *udd, double *force,
                            s->nlist_ref.p);
         HIPCHK(hipGetLastError());
     }
+    if (u)
+        HIPCHK(hipMemcpyAsync(u, s->wbuf.p, 3 * (size_t)N * sizeof(double),
+                              hipMemcpyDeviceToHost, s->stream));
+    if (damage)
+        HIPCHK(hipMemcpyAsync(damage, s->damage.p, (size_t)N * sizeof(double),
+                              hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     const struct {
         double *dst;
         const double *src;
-    } fields[] = {{u, s->u.p}, {ud, s->ud.p}, {udd, s->udd.p},
+    } fields[] = {{ud, s->ud.p}, {udd, s->udd.p},
                   {force, s->force.p}, {body_force, s->body_force.p}};
     for (const auto &f : fields) {
         if (f.dst) {
@@ -4169,9 +4205,6 @@ int pd_write(pd_sim *s, double *u, double *ud, double *udd, double *force,
             if (!((s->h_flags[q / 3] >> (3 + (int)(q % 3))) & 1))
                 body_force[q] = f[q];
     }
-    if (damage)
-        HIPCHK(hipMemcpy(damage, s->damage.p, (size_t)N * sizeof(double),
-                         hipMemcpyDeviceToHost));
     if (nlist) {
         const size_t NB = (size_t)N * s->K * sizeof(int);
         if (s->layout == PD_LAYOUT_SLOT)
