@@ -1338,7 +1338,7 @@ __global__ void __launch_bounds__(256)
 // upper neighbours in current row order (slot index << 16 | halo loc, rebuilt
 // by compact_tile after every break of the node).  The node's four lanes take
 // eight consecutive positions per round, two each, whose evaluations
-// interleave: with the reference's operations -- bitwise square roots, IEEE
+// interleave (eight lanes, one each): with the reference's operations -- bitwise square roots, IEEE
 // divisions, no contraction -- each gives its three force terms and decides
 // the break from that exact stretch (peridynamics.pyx:133).  The terms pass
 // through the node's 96-byte LDS window, four positions at a time; lanes 0-2
@@ -1353,6 +1353,9 @@ __global__ void __launch_bounds__(256)
 // fold windows (12 doubles per node, tiles of up to EXACT_NODES nodes).
 constexpr int EXACT_NODES = 128;
 constexpr int EXACT_CAP = (int)((LDS_BYTES - EXACT_NODES * 96u) / 64u);
+// Tiles of at most that many nodes run eight lanes per node: they are small
+// because the mesh is (tile_cap_of), so that a round's latency bounds it.
+constexpr int EXACT_WIDE_NODES = 64;
 
 // Rows of K slots fit compact_tile's groups in the exact step's fold
 // windows (its 64 bytes of counts, then at least one row).
@@ -1465,27 +1468,26 @@ __device__ __forceinline__ void exact_slow(const StepArgs &a,
     t.t2 = (fn * dz) * v;
 }
 
-// The fold window of a node: [component][position of the round].
-__device__ __forceinline__ void window_put(double *win, int sub,
+// The fold window of a node: [component][position of four].
+__device__ __forceinline__ void window_put(double *win, int q,
                                           const ExactTerm &t)
 {
-    win[sub] = t.t0;
-    win[4 + sub] = t.t1;
-    win[8 + sub] = t.t2;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    win[q] = t.t0;
+    win[4 + q] = t.t1;
+    win[8 + q] = t.t2;
 }
 
-__device__ __forceinline__ void window_done()
+// Between a wavefront's writes of its windows and their reads.
+__device__ __forceinline__ void window_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// One workgroup per tile of at most EXACT_NODES nodes, four lanes per node
-// (block 4 * tile_nodes), on k_step's tiles and halo staging.  Records hold
+// One workgroup per tile of at most EXACT_NODES nodes, four lanes per node or
+// eight (small meshes; the same results, as the fold's order does not depend
+// on who evaluates a position), on k_step's tiles and halo staging.  Records hold
 // (r0, V | r0 + u, 0).
 //
 // What bounds it: the VALU on large meshes, and on small ones a round's
@@ -1496,11 +1498,12 @@ __device__ __forceinline__ void window_done()
 // one interval test for everything rare, a bond takes 65 wave instructions
 // where it took 115: 150 -> 104 us a step on 270,000 nodes, 20.7 -> 14 on
 // the 2560-node bar.
+template <int LPN>
 __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
                                                     double fmag)
 {
+    static_assert(LPN == 4 || LPN == 8, "two or one positions per lane");
     __shared__ double2 lds[LDS_BYTES / sizeof(double2)];
-    constexpr int LPN = 4;
     constexpr unsigned PB = 16u * EXACT_CAP;
     const int b = blockIdx.x;
     const int tile = (b % XCDS) * a.tiles_per_xcd + b / XCDS;
@@ -1515,13 +1518,19 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
     hl.request(a.halo + ti.halo_off, (unsigned)ti.halo);
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     const long long c0 = ti.chunk_off + (valid ? l : 0);
-    // the node's pair of list entries in round r is r * fstep further on
+    // the lane's list entries of round r are r * fstep further on; with
+    // eight lanes, lanes 4-7 take the second of the pairs
     const char *L = reinterpret_cast<const char *>(a.ford + 4 * ti.chunk_off);
-    const unsigned fstep = 8u * LPN * (unsigned)ti.nodes;
+    const unsigned fstep = 8u * 4u * (unsigned)ti.nodes;
     unsigned foff = 8u * ((valid ? (unsigned)l : 0u) +
-                          (unsigned)sub * (unsigned)ti.nodes);
+                          (unsigned)(sub & 3) * (unsigned)ti.nodes) +
+                    (LPN == 8 ? (unsigned)(sub & 4) : 0u);
     auto pair_at = [&](unsigned off) {
-        return *reinterpret_cast<const uint2 *>(L + off);
+        if constexpr (LPN == 8)
+            return make_uint2(*reinterpret_cast<const unsigned *>(L + off),
+                              0u);
+        else
+            return *reinterpret_cast<const uint2 *>(L + off);
     };
     uint2 qa = pair_at(foff), qb = pair_at(foff + fstep);
     double4 r0m = make_double4(0.0, 0.0, 0.0, 0.0), rm = r0m;
@@ -1545,18 +1554,31 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
     double *win = reinterpret_cast<double *>(ldsb + 4 * PB) + 12 * l;
     double F = 0.0, Flow = 0.0;  // lane d < 3: component d
     int nbroken = 0;
-    // four terms of every lane's component, in order
-    auto fold4 = [&](const ExactTerm &t) {
-        window_put(win, sub, t);
+    // four terms of every lane's component, in order: those of lanes from,
+    // from + 1, ...
+    auto fold4 = [&](const ExactTerm &t, int from) {
+        if (LPN == 4 || (sub & 4) == from)
+            window_put(win, sub & 3, t);
+        window_sync();
         if (sub < 3) {
 #pragma unroll
-            for (int q = 0; q < LPN; ++q)
+            for (int q = 0; q < 4; ++q)
                 F = F + win[4 * sub + q];
         }
-        window_done();
+        window_sync();
     };
     auto round = [&](uint2 en, int r, bool check) {
         ExactTerm t0 = exact_fast(a, ldsb, en.x & 0xffffu, r0m, rm);
+        if constexpr (LPN == 8) {
+            if (__builtin_expect(!((t0.s > a.xlo) & (t0.s < a.xhi)), 0))
+                exact_slow(a, ldsb, en.x & 0xffffu, r0m, rm, check,
+                           slot_of(c0, ti.nodes, (int)(en.x >> 16)),
+                           fold_of(ti.chunk_off, ti.nodes, l, 8 * r + sub),
+                           t0, nbroken);
+            fold4(t0, 0);
+            fold4(t0, 4);
+            return;
+        }
         ExactTerm t1 = exact_fast(a, ldsb, en.y & 0xffffu, r0m, rm);
         const bool ok0 = (t0.s > a.xlo) & (t0.s < a.xhi);
         const bool ok1 = (t1.s > a.xlo) & (t1.s < a.xhi);
@@ -1573,8 +1595,8 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
                            fold_of(ti.chunk_off, ti.nodes, l, pos + 4), t1,
                            nbroken);
         }
-        fold4(t0);
-        fold4(t1);
+        fold4(t0, 0);
+        fold4(t1, 0);
     };
     // the wavefront's first node has its longest list (nodes are sorted by
     // bond count); positions past a list's end are dead
@@ -1614,7 +1636,8 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         for (int r = rlow; 8 * r < total; ++r) {
             const int *e = reinterpret_cast<const int *>(a.ford) +
                            fold_of(ti.chunk_off, ti.nodes, l, 8 * r + sub);
-            round(make_uint2(ld_slot(e), ld_slot(e + 1)), r, false);
+            round(make_uint2(ld_slot(e), LPN == 8 ? 0u : ld_slot(e + 1)), r,
+                  false);
         }
     }
     if (sub < 3) {
@@ -2102,7 +2125,11 @@ struct pd_sim {
     double dt = 0.0, damping = 0.0;
     int n = 0, K = 0;
     int tension_only = 0;
-    int lpn = 4, tile_nodes = 128;
+    int lpn = 4, tile_nodes = 128;  // pd_set_launch's values
+    bool launch_given = false;      // pd_set_launch was called
+    int lanes = 4;      // lanes per node of the steps (lpn, unless not given)
+    int tile_cap = 128; // most nodes of a tile of the current tiling
+    int cus = 256;
     int hmax = 0;           // halo capacity of a tile (LDS budget)
     int hstride = 0;        // largest halo of the current tiles
     size_t lds_budget = 0;  // bytes of LDS a workgroup may use
@@ -2353,11 +2380,17 @@ StepArgs make_args(pd_sim *s)
     return a;
 }
 
+// Threads of a workgroup: the tiles' nodes, in whole wavefronts.
+unsigned block_of(const pd_sim *s, int lanes)
+{
+    return ((unsigned)(s->tile_cap * lanes) + 63u) & ~63u;
+}
+
 template <int DM, int LPN, bool CLA>
 hipError_t launch_cla(pd_sim *s, const StepArgs &a, double dmag, double fmag)
 {
     const unsigned grid = (unsigned)XCDS * a.tiles_per_xcd;
-    const unsigned block = (unsigned)(s->tile_nodes * LPN);
+    const unsigned block = block_of(s, LPN);
     // the n-linear model breaks by regimes, not by the sign mode
     const bool tens = DM != DM_NLIN && a.absmask == 0xffffffffu;
     if (a.has_corr && tens)
@@ -2385,7 +2418,7 @@ hipError_t launch_one(pd_sim *s, const StepArgs &a, double dmag, double fmag)
     if (a.layout == PD_LAYOUT_SLOT)
         return launch_cla<DM, LPN, true>(s, a, dmag, fmag);
     const unsigned grid = (unsigned)XCDS * a.tiles_per_xcd;
-    const unsigned block = (unsigned)(s->tile_nodes * LPN);
+    const unsigned block = block_of(s, LPN);
     if (DM != DM_PMB || a.has_corr)
         return hipErrorInvalidValue;  // rejected before launch
     if (a.absmask == 0xffffffffu)
@@ -2402,7 +2435,7 @@ hipError_t launch_one(pd_sim *s, const StepArgs &a, double dmag, double fmag)
 template <int DM>
 hipError_t launch_dm(pd_sim *s, const StepArgs &a, double dmag, double fmag)
 {
-    switch (s->lpn) {
+    switch (s->lanes) {
     case 1:
         return launch_one<DM, 1>(s, a, dmag, fmag);
     case 2:
@@ -2419,22 +2452,19 @@ hipError_t launch_dm(pd_sim *s, const StepArgs &a, double dmag, double fmag)
 hipError_t launch_adjoint(pd_sim *s, const AdjArgs &a)
 {
     const unsigned grid = (unsigned)XCDS * a.tiles_per_xcd;
-    switch (s->lpn) {
+    const dim3 block(block_of(s, s->lanes));
+    switch (s->lanes) {
     case 1:
-        hipLaunchKernelGGL(k_adj_tile<1>, dim3(grid), dim3(s->tile_nodes), 0,
-                           s->stream, a);
+        hipLaunchKernelGGL(k_adj_tile<1>, dim3(grid), block, 0, s->stream, a);
         break;
     case 2:
-        hipLaunchKernelGGL(k_adj_tile<2>, dim3(grid),
-                           dim3(2 * s->tile_nodes), 0, s->stream, a);
+        hipLaunchKernelGGL(k_adj_tile<2>, dim3(grid), block, 0, s->stream, a);
         break;
     case 4:
-        hipLaunchKernelGGL(k_adj_tile<4>, dim3(grid),
-                           dim3(4 * s->tile_nodes), 0, s->stream, a);
+        hipLaunchKernelGGL(k_adj_tile<4>, dim3(grid), block, 0, s->stream, a);
         break;
     default:
-        hipLaunchKernelGGL(k_adj_tile<8>, dim3(grid),
-                           dim3(8 * s->tile_nodes), 0, s->stream, a);
+        hipLaunchKernelGGL(k_adj_tile<8>, dim3(grid), block, 0, s->stream, a);
         break;
     }
     return hipGetLastError();
@@ -2520,9 +2550,13 @@ int launch_step(pd_sim *s, double dmag, double fmag)
     const StepArgs a = make_args(s);
     hipError_t e;
     if (s->exact) {
-        hipLaunchKernelGGL(k_exact_step, dim3(XCDS * a.tiles_per_xcd),
-                           dim3(4 * s->tile_nodes), 0, s->stream, a, dmag,
-                           fmag);
+        const dim3 grid(XCDS * a.tiles_per_xcd);
+        if (s->tile_cap <= EXACT_WIDE_NODES)
+            hipLaunchKernelGGL(k_exact_step<8>, grid, dim3(block_of(s, 8)), 0,
+                               s->stream, a, dmag, fmag);
+        else
+            hipLaunchKernelGGL(k_exact_step<4>, grid, dim3(block_of(s, 4)), 0,
+                               s->stream, a, dmag, fmag);
         e = hipGetLastError();
     } else {
         switch (dm_of(s)) {
@@ -2592,6 +2626,28 @@ int fold_lists(pd_sim *s)
                        s->nup.p, s->ford.p);
     HIPCHK(hipGetLastError());
     return PD_OK;
+}
+
+// The launch shape of the next tiling.  On a mesh of fewer nodes than one
+// workgroup per CU takes, a step is one workgroup's latency, most of it the
+// issue of its rounds, so the nodes are spread: tiles as small as give every
+// CU one (no smaller than 32 nodes at eight lanes, 48 at four: their halos
+// then cost more), and eight lanes per node where the caller set no shape and
+// the tiles are that small.  Tiles change no result; lanes change the order
+// of a node's sum.  us a step, scalar model, tiles of 128 / the rule, four
+// lanes, and the rule with eight: 2,560 nodes 10.6 / 8.4, 6.7; 5,000 nodes
+// 11.6 / 9.1, 6.8; 20,655 nodes 12.4 / 12.0, 12.4 (not taken).  From two
+// workgroups per CU on, 128 nodes are the fastest (50,820 nodes: 19.5; with
+// 96, 23.1).
+void set_shape(pd_sim *s)
+{
+    if (!s->launch_given)
+        s->lanes = s->n <= 48 * s->cus ? 8 : s->lpn;
+    const int least = s->lanes == 8 ? 32 : 48;
+    const int even = ((s->n + s->cus - 1) / s->cus + 15) & ~15;
+    s->tile_cap = std::min(std::max(even, least), s->tile_nodes);
+    if (s->n > s->cus * s->tile_nodes)
+        s->tile_cap = s->tile_nodes;
 }
 
 // Rows of w values given in the caller's order into tile order on the device
@@ -2672,7 +2728,7 @@ void keep_plan(pd_sim *s, const int *nlist, const int *n_neigh, bool nlin,
     s->plan_nregimes = s->nregimes;
     s->plan_types = s->nbond_types;
     s->plan_tile_nodes = s->tile_nodes;
-    s->plan_lpn = s->lpn;
+    s->plan_lpn = s->lanes;
     s->plan = true;
 }
 
@@ -2685,7 +2741,7 @@ bool plan_holds(const pd_sim *s, const int *nlist, const int *n_neigh,
     return s->plan && s->has_buffers && !regimes_given &&
            s->plan_nlin == nlin && s->plan_nregimes == nregimes &&
            s->plan_types == nbond_types &&
-           s->plan_tile_nodes == s->tile_nodes && s->plan_lpn == s->lpn &&
+           s->plan_tile_nodes == s->tile_nodes && s->plan_lpn == s->lanes &&
            (s->layout != PD_LAYOUT_COMPACT ||
             same_values(s->plan_nneigh.data(), n_neigh, (size_t)s->n)) &&
            same_values(s->plan_nlist.get(), nlist, (size_t)s->n * s->K);
@@ -2989,8 +3045,12 @@ int pd_build(pd_sim **out, int device, int integrator, int layout, double dt,
     HIPCHK(hipDeviceGetAttribute(&lds_max,
                                  hipDeviceAttributeMaxSharedMemoryPerBlock,
                                  device));
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(
+        &cus, hipDeviceAttributeMultiprocessorCount, device));
     pd_sim *s = new pd_sim();
     s->device = device;
+    s->cus = std::max(cus, 1);
     s->integrator = integrator;
     s->layout = layout;
     s->dt = dt;
@@ -3205,10 +3265,11 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
               1;
     std::vector<int> tnode = morton_order(
         N, s->h_coords.data(), s->h_group.empty() ? nullptr : s->h_group.data());
-    // blocks: runs of tile_nodes nodes of one group.  A block is one tile, or
+    // blocks: runs of tile_cap nodes of one group.  A block is one tile, or
     // several where the halo capacity cuts it; blocks do not depend on each
     // other, so threads take them side by side.
-    const int cap = s->tile_nodes;
+    set_shape(s);
+    const int cap = s->tile_cap;
     std::vector<int> bstart;
     for (int q = 0; q < N; ++q)
         if (q == 0 || q - bstart.back() == cap ||
@@ -3347,7 +3408,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                 roff.push_back((int)rows.size());
             }
             const std::vector<int> &hpos =
-                spread.place(roff, rows, s->lpn, (int)hl.size());
+                spread.place(roff, rows, s->lanes, (int)hl.size());
             for (size_t h = 0; h < hl.size(); ++h) {
                 lmap[hl[h]] = hpos[h];
                 halo[ti.halo_off + hpos[h]] = hl[h];
@@ -3786,8 +3847,9 @@ int pd_set_launch(pd_sim *s, int lanes_per_node, int tile_nodes)
     // then the current tiles (of the old size) cannot be stepped
     if (s->has_buffers && tile_nodes != s->tile_nodes)
         s->retile_pending = true;
-    s->lpn = lanes_per_node;
+    s->lpn = s->lanes = lanes_per_node;
     s->tile_nodes = tile_nodes;
+    s->launch_given = true;
     return PD_OK;
 }
 

@@ -129,15 +129,18 @@ def test_rows_of_every_length(model, lanes, scale):
 
 
 @pytest.mark.parametrize("scale", [1.0, 1e-92])
+@pytest.mark.parametrize("most", [40, 185])
 @pytest.mark.parametrize("tile", [64, 128])
 @pytest.mark.parametrize("fast_first", [False, True])
-def test_exact_order_rows_of_every_length(fast_first, tile, scale):
+def test_exact_order_rows_of_every_length(fast_first, tile, most, scale):
     """The exact-order step on the same stars, bitwise: fold lists of every
     length, split anywhere between lower and upper neighbours (the numbering
     is random), with bonds breaking in both parts.  ``fast_first`` runs the
     first, breaking step in the fast order, whose broken bonds the fold lists
-    made for the exact order must leave out."""
-    x, u0, fam, nl = _stars(scale, True, seed=8)
+    made for the exact order must leave out.  185 stars (17,390 nodes) take
+    tiles of more than 64 nodes where these are allowed, and with them four
+    lanes per node instead of eight."""
+    x, u0, fam, nl = _stars(scale, True, seed=8, most=most)
     n, k = nl.shape
     vol = np.random.default_rng(9).uniform(0.5, 1.5, n)
     bct = np.zeros((n, 3), np.int32)
