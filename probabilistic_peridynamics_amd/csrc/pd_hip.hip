@@ -9,9 +9,9 @@
 // the step (the break-before-force order of peripy/integrators.py:339-349 and
 // the single bond_force pass of cl/peridynamics.cl both read u_n only).
 //
-// Tiles.  The nodes are cut into tiles: runs of up to `tile_nodes` nodes in
-// Morton order of their initial coordinates, grown while the tile's halo --
-// the tile's nodes and all their neighbours -- fits in LDS (1280 entries,
+// Tiles.  The nodes are cut into tiles of up to `tile_nodes` nodes by
+// recursive bisection of their initial coordinates, such that a tile's halo
+// -- the tile's nodes and all their neighbours -- fits in LDS (1280 entries,
 // 80 KiB, so two workgroups share a CU and one stages its halo while the
 // other computes).  Within a tile the nodes are ordered by descending bond
 // count, so a wavefront's nodes run loops of nearly equal length.  One
@@ -504,49 +504,75 @@ __device__ __forceinline__ double sq3(double x, double y, double z)
 // pass).  Pieces past the last entry store that entry again: a condition
 // would move each load next to its store.
 struct HaloLoads {
-    static constexpr int SP = 10;
+    // passes of all threads over the entries: SP at once; a halo that needs
+    // at most FEW (a plate's) stages no more
+    static constexpr int SP = 10, FEW = 3;
     unsigned hi[SP];
+
+    // byte offsets into H: four times the entry
+    static __device__ __forceinline__ unsigned step()
+    {
+        return blockDim.x & ~3u;
+    }
 
     __device__ __forceinline__ void request(const int *H, unsigned halo)
     {
-        const unsigned last = halo - 1u;
-        unsigned x = threadIdx.x >> 2;
+        const char *h = reinterpret_cast<const char *>(H);
+        const unsigned last = 4u * (halo - 1u);
+        unsigned x = threadIdx.x & ~3u;
         static_for<SP>([&](auto k) {
-            hi[k] = (unsigned)H[min(x, last)];
-            x += blockDim.x >> 2;
+            hi[k] = *reinterpret_cast<const unsigned *>(h + min(x, last));
+            x += step();
         });
     }
 
+    // passes [0, N), their indices in hi
+    template <int N>
+    __device__ __forceinline__ void pass(const char *R, unsigned last,
+                                         char *D) const
+    {
+        v2d v[N];
+        static_for<N>([&](auto k) {
+            v[k] = *reinterpret_cast<const v2d *>(
+                R + (hi[k] * 64u + (threadIdx.x & 3u) * 16u));
+        });
+        unsigned x = threadIdx.x & ~3u;
+        static_for<N>([&](auto k) {
+            *reinterpret_cast<v2d *>(D + 4u * min(x, last)) = v[k];
+            x += step();
+        });
+    }
+
+    // SHORT: with the short form for few passes (401 x 233 plate 14.4 -> 13.1
+    // us a step; the n-linear kernel leaves it out, whose bars it costs 3 %)
+    template <bool SHORT>
     __device__ __forceinline__ void stage(const NodeRec *rec, const int *H,
                                           unsigned halo, char *D, unsigned PB)
     {
-        const unsigned last = halo - 1u, per = blockDim.x >> 2;
-        const unsigned e0 = threadIdx.x >> 2, piece = threadIdx.x & 3u;
+        const char *h = reinterpret_cast<const char *>(H);
+        const unsigned last = 4u * (halo - 1u);
+        const unsigned piece = threadIdx.x & 3u;
         const char *R = reinterpret_cast<const char *>(rec);
         D += piece * PB + 16u;
-        unsigned x = e0;
-        {
-            v2d v[SP];
-            static_for<SP>([&](auto k) {
-                v[k] = *reinterpret_cast<const v2d *>(
-                    R + (hi[k] * 64u + piece * 16u));
-            });
-            static_for<SP>([&](auto k) {
-                *reinterpret_cast<v2d *>(D + 16u * min(x, last)) = v[k];
-                x += per;
-            });
+        if (SHORT && last < FEW * step()) {
+            pass<FEW>(R, last, D);
+            return;
         }
-        while (x - e0 <= last) {  // the same in every thread
-            v2d v[4];
+        pass<SP>(R, last, D);
+        const unsigned e0 = threadIdx.x & ~3u;
+        for (unsigned x = e0 + SP * step(); x - e0 <= last;) {
+            v2d v[4];  // the loop's trips are the same in every thread
             unsigned y = x;
             static_for<4>([&](auto k) {
+                const unsigned g =
+                    *reinterpret_cast<const unsigned *>(h + min(y, last));
                 v[k] = *reinterpret_cast<const v2d *>(
-                    R + ((unsigned)H[min(y, last)] * 64u + piece * 16u));
-                y += per;
+                    R + (g * 64u + piece * 16u));
+                y += step();
             });
             static_for<4>([&](auto k) {
-                *reinterpret_cast<v2d *>(D + 16u * min(x, last)) = v[k];
-                x += per;
+                *reinterpret_cast<v2d *>(D + 4u * min(x, last)) = v[k];
+                x += step();
             });
         }
     }
@@ -562,6 +588,40 @@ __device__ __forceinline__ void far_entry(char *D, unsigned PB)
     const bool r = t < 2 || !CLA;
     *reinterpret_cast<double2 *>(D + t * PB) =
         make_double2(r ? FAR : 0.0, r && !(t & 1) ? FAR : 0.0);
+}
+
+// v of the lane whose number differs in bit OFF (1, 2 or 4).  Inside a quad
+// the exchange is a DPP move of each half: no LDS access to wait for.
+template <int OFF>
+__device__ __forceinline__ int lane_xor(int v)
+{
+    if constexpr (OFF == 1)
+        return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);
+    else if constexpr (OFF == 2)
+        return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);
+    else
+        return __shfl_xor(v, OFF, 2 * OFF);
+}
+
+template <int OFF>
+__device__ __forceinline__ double lane_xor(double v)
+{
+    return __hiloint2double(lane_xor<OFF>(__double2hiint(v)),
+                            lane_xor<OFF>(__double2loint(v)));
+}
+
+// Sum over a node's LPN lanes, the same in each: v + (v of lane ^ LPN/2),
+// then ^ LPN/4, ...
+template <int LPN, typename T>
+__device__ __forceinline__ T node_sum(T v)
+{
+    if constexpr (LPN >= 8)
+        v += lane_xor<4>(v);
+    if constexpr (LPN >= 4)
+        v += lane_xor<2>(v);
+    if constexpr (LPN >= 2)
+        v += lane_xor<1>(v);
+    return v;
 }
 
 // A bond as the force needs it: the bond vector, s/2, 0.5/l and the weight.
@@ -864,8 +924,8 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         }
     }
 
-    hl.stage(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo,
-             ldsb + halo_base<DM>(), PB);
+    hl.stage<DM != DM_NLIN>(a.rec_old, a.halo + ti.halo_off,
+                            (unsigned)ti.halo, ldsb + halo_base<DM>(), PB);
     if (threadIdx.x < 4)
         far_entry<CLA>(ldsb + halo_base<DM>(), PB);
     // n-linear tables, one 16-byte read each: (lower, upper) halved
@@ -927,13 +987,10 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         }
     }
 
-#pragma unroll
-    for (int off = LPN / 2; off > 0; off >>= 1) {
-        fx += __shfl_xor(fx, off, LPN);
-        fy += __shfl_xor(fy, off, LPN);
-        fz += __shfl_xor(fz, off, LPN);
-        nbroken += __shfl_xor(nbroken, off, LPN);
-    }
+    fx = node_sum<LPN>(fx);
+    fy = node_sum<LPN>(fy);
+    fz = node_sum<LPN>(fz);
+    nbroken = node_sum<LPN>(nbroken);
     // the compact layout (the Cython path, launched with !CLA only): once
     // the halo is no longer read, its LDS holds the rows being compacted
     if constexpr (!CLA) {
@@ -1546,7 +1603,8 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
             pu = a.u[3 * (size_t)i + sub];
         }
     }
-    hl.stage(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb, PB);
+    hl.stage<true>(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb,
+                   PB);
     if (threadIdx.x < 4)
         far_entry<false>(ldsb, PB);
     __syncthreads();
@@ -1620,9 +1678,7 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         if (rlow >= rounds)
             Flow = F;  // no upper part
     }
-#pragma unroll
-    for (int off = LPN / 2; off > 0; off >>= 1)
-        nbroken += __shfl_xor(nbroken, off, LPN);
+    nbroken = node_sum<LPN>(nbroken);
     // the fold windows are free: they hold the rows being compacted, and
     // the lists of those nodes are rebuilt in the new row order
     compact_tile<LPN, true>(a, ti, ldsb + 4 * PB, EXACT_NODES * 96u, valid, l,
@@ -1973,7 +2029,7 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     const NodeRec own = a.rec[i];
     const int cnt = valid ? a.cnt[i] : 0;
-    hl.stage(a.rec, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb, PB);
+    hl.stage<true>(a.rec, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb, PB);
     if (threadIdx.x < 4)
         far_entry<true>(ldsb, PB);
     __syncthreads();
@@ -2035,13 +2091,10 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
         }
     }
     gc *= -0.5;
-#pragma unroll
-    for (int off = LPN / 2; off > 0; off >>= 1) {
-        jt[0] += __shfl_xor(jt[0], off, LPN);
-        jt[1] += __shfl_xor(jt[1], off, LPN);
-        jt[2] += __shfl_xor(jt[2], off, LPN);
-        gc += __shfl_xor(gc, off, LPN);
-    }
+    jt[0] = node_sum<LPN>(jt[0]);
+    jt[1] = node_sum<LPN>(jt[1]);
+    jt[2] = node_sum<LPN>(jt[2]);
+    gc = node_sum<LPN>(gc);
     if (!valid)
         return;
     const size_t b = 3 * (size_t)i;
@@ -2788,17 +2841,6 @@ int restart(pd_sim *s, const double *bond_stiffness,
     return PD_OK;
 }
 
-uint64_t spread3(uint64_t v)
-{
-    v &= 0x1fffff;
-    v = (v | v << 32) & 0x1f00000000ffffull;
-    v = (v | v << 16) & 0x1f0000ff0000ffull;
-    v = (v | v << 8) & 0x100f00f00f00f00full;
-    v = (v | v << 4) & 0x10c30c30c30c30c3ull;
-    v = (v | v << 2) & 0x1249249249249249ull;
-    return v;
-}
-
 // LDS entries of a tile's halo, chosen so that the records the bond loop
 // reads together fall into different banks.  One ds_read_b128 over 16
 // consecutive lanes reads a 16-byte piece of each lane's neighbour record;
@@ -2899,65 +2941,119 @@ struct HaloSpread {
     }
 };
 
-// Node order for tiling: Morton order of the initial coordinates on a grid
-// whose cell holds about one node.
-// Node order for tiling: by group (when given), then by Morton code of the
-// coordinates on a grid of about one node per cell.
-std::vector<int> morton_order(int n, const double *x, const int *group)
+// Tiles by recursive bisection of the initial coordinates: the nodes of each
+// group (when given) are halved across their longest extent, in proportion
+// to the tiles of at most `cap` nodes that each half needs, until a part is
+// one tile.  Such tiles are full and nearly cubes, whose halos are smaller
+// and more alike than those of runs of a Morton curve (128 nodes of a
+// jittered 200 x 47 x 47 lattice: 804 entries on average and 973 at most,
+// against 939 and 1283), and parts that are near in the order are near in
+// space.  Returns the order of the nodes; starts gets each tile's first.
+struct TilePoint {
+    double x[3];
+    int id;
+};
+
+struct TileRange {
+    int lo, hi;
+};
+
+// One halving of p[r.lo, r.hi), which needs more than one tile.
+int bisect(TilePoint *p, const TileRange &r, int cap)
 {
-    double lo[3] = {x[0], x[1], x[2]}, hi[3] = {x[0], x[1], x[2]};
-    for (int i = 0; i < n; ++i)
-        for (int d = 0; d < 3; ++d) {
-            lo[d] = std::min(lo[d], x[3 * (size_t)i + d]);
-            hi[d] = std::max(hi[d], x[3 * (size_t)i + d]);
-        }
-    double vol = 1.0;
-    int dims = 0;
+    double lo[3], hi[3];
     for (int d = 0; d < 3; ++d)
-        if (hi[d] > lo[d]) {
-            vol *= hi[d] - lo[d];
-            ++dims;
+        lo[d] = hi[d] = p[r.lo].x[d];
+    for (int q = r.lo + 1; q < r.hi; ++q)
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = std::min(lo[d], p[q].x[d]);
+            hi[d] = std::max(hi[d], p[q].x[d]);
         }
-    double h = dims ? std::pow(vol / n, 1.0 / dims) : 1.0;
-    if (!(h > 0.0))
-        h = 1.0;
-    std::vector<uint64_t> code(n);
-    run_parallel(n, [&](int first, int end) {
-        for (int i = first; i < end; ++i) {
-            uint64_t c = 0;
-            for (int d = 0; d < 3; ++d) {
-                double v = std::floor((x[3 * (size_t)i + d] - lo[d]) / h);
-                v = std::min(std::max(v, 0.0), 2097151.0);
-                c |= spread3((uint64_t)v) << d;
-            }
-            code[i] = c;
-        }
+    int ax[3] = {0, 1, 2};
+    std::stable_sort(ax, ax + 3, [&](int d, int e) {
+        return hi[d] - lo[d] > hi[e] - lo[e];
     });
-    std::vector<int> order(n), other(n);
+    const long long n = r.hi - r.lo, m = (n + cap - 1) / cap;
+    const int cut = r.lo + (int)(n * (m / 2) / m);
+    std::nth_element(p + r.lo, p + cut, p + r.hi,
+                     [&](const TilePoint &a, const TilePoint &b) {
+                         for (int d : ax)
+                             if (a.x[d] != b.x[d])
+                                 return a.x[d] < b.x[d];
+                         return a.id < b.id;
+                     });
+    return cut;
+}
+
+std::vector<int> tile_order(int n, const double *x, const int *group, int cap,
+                            std::vector<int> &starts)
+{
+    std::vector<int> order(n);
     for (int i = 0; i < n; ++i)
         order[i] = i;
-    // stable counting sort, 11 bits of the key at a time from the lowest:
-    // by code, then by group
-    const auto sort_by = [&](auto key) {
-        uint64_t top = 0;
-        for (int i = 0; i < n; ++i)
-            top |= key(i);
-        for (int shift = 0; shift < 64 && (top >> shift) != 0; shift += 11) {
-            std::vector<int> at(2049, 0);
-            for (int i = 0; i < n; ++i)
-                ++at[((key(i) >> shift) & 2047) + 1];
-            for (int b = 0; b < 2048; ++b)
-                at[b + 1] += at[b];
-            for (int q = 0; q < n; ++q)
-                other[at[(key(order[q]) >> shift) & 2047]++] = order[q];
-            order.swap(other);
+    if (group)
+        std::stable_sort(order.begin(), order.end(),
+                         [&](int a, int b) { return group[a] < group[b]; });
+    std::vector<TilePoint> p(n);
+    std::vector<TileRange> parts;
+    for (int q = 0; q < n; ++q) {
+        const int i = order[q];
+        for (int d = 0; d < 3; ++d) {
+            // a coordinate that is not a number has no place in the order
+            const double v = x[3 * (size_t)i + d];
+            p[q].x[d] = std::fabs(v) <= __DBL_MAX__ ? v : 0.0;
         }
-    };
-    sort_by([&](int i) { return code[i]; });
-    if (group)  // signed values in order
-        sort_by([&](int i) {
-            return (uint64_t)((uint32_t)group[i] ^ 0x80000000u);
-        });
+        p[q].id = i;
+        if (q == 0 || (group && group[i] != group[order[q - 1]]))
+            parts.push_back({q, q});
+        parts.back().hi = q + 1;
+    }
+    // the first halvings, each level's side by side, until there is a part
+    // for every thread; then each part to its tiles
+    while (parts.size() < 64) {
+        std::vector<int> cut(parts.size(), -1);
+        run_parallel((int)parts.size(), [&](int lo, int hi) {
+            for (int k = lo; k < hi; ++k)
+                if (parts[k].hi - parts[k].lo > std::max(cap, 2048))
+                    cut[k] = bisect(p.data(), parts[k], cap);
+        }, 2);
+        std::vector<TileRange> next;
+        for (size_t k = 0; k < parts.size(); ++k) {
+            if (cut[k] < 0) {
+                next.push_back(parts[k]);
+            } else {
+                next.push_back({parts[k].lo, cut[k]});
+                next.push_back({cut[k], parts[k].hi});
+            }
+        }
+        const bool done = next.size() == parts.size();
+        parts.swap(next);
+        if (done)
+            break;
+    }
+    std::vector<std::vector<int>> leaves(parts.size());
+    run_parallel((int)parts.size(), [&](int lo, int hi) {
+        std::vector<TileRange> todo;
+        for (int k = lo; k < hi; ++k) {
+            todo.assign(1, parts[k]);
+            while (!todo.empty()) {
+                const TileRange r = todo.back();
+                todo.pop_back();
+                if (r.hi - r.lo <= cap) {
+                    leaves[k].push_back(r.lo);
+                    continue;
+                }
+                const int cut = bisect(p.data(), r, cap);
+                todo.push_back({cut, r.hi});  // the left half first
+                todo.push_back({r.lo, cut});
+            }
+        }
+    }, 2);
+    starts.clear();
+    for (const auto &l : leaves)
+        starts.insert(starts.end(), l.begin(), l.end());
+    for (int q = 0; q < n; ++q)
+        order[q] = p[q].id;
     return order;
 }
 
@@ -3255,27 +3351,22 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         }
     });
 
-    // tiles: runs of the Morton order, capped by tile_nodes and by the LDS
-    // halo capacity
+    // tiles, capped by tile_nodes and by the LDS halo capacity
     // entry 0 of a staged halo is the zero record of dead slots
     // the compact layout's tiles leave room for the exact step's windows
     s->hmax = (nlin ? LDS_CAP_NLIN
                     : (s->layout == PD_LAYOUT_COMPACT ? EXACT_CAP
                                                       : LDS_CAP_PMB)) -
               1;
-    std::vector<int> tnode = morton_order(
-        N, s->h_coords.data(), s->h_group.empty() ? nullptr : s->h_group.data());
-    // blocks: runs of tile_cap nodes of one group.  A block is one tile, or
+    // blocks: the parts of at most tile_cap nodes.  A block is one tile, or
     // several where the halo capacity cuts it; blocks do not depend on each
     // other, so threads take them side by side.
     set_shape(s);
     const int cap = s->tile_cap;
     std::vector<int> bstart;
-    for (int q = 0; q < N; ++q)
-        if (q == 0 || q - bstart.back() == cap ||
-            (!s->h_group.empty() &&
-             s->h_group[tnode[q]] != s->h_group[tnode[q - 1]]))
-            bstart.push_back(q);
+    std::vector<int> tnode = tile_order(
+        N, s->h_coords.data(), s->h_group.empty() ? nullptr : s->h_group.data(),
+        cap, bstart);
     const int nblocks = (int)bstart.size();
     bstart.push_back(N);
     std::vector<std::vector<TileInfo>> cuts(nblocks);
