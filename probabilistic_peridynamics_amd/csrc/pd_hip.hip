@@ -57,6 +57,7 @@
 //              which slot_of gives the slot of its k-th bond
 //   u, ud, udd, force, body_force (N,3) f64 in the reference's layout
 //   flags[N]   bit d: displacement BC on DOF d; bit 3+d: force BC on DOF d
+//   meta[N]    a node's row length and its flags in one word (k_step)
 //   bcv, fbcv, dens (N,3) f64, read only for flagged DOFs / dynamic
 //              integrators
 //   rslot (N,K) u16 + n_neigh: the reference-layout list of the compact
@@ -173,13 +174,16 @@ struct StepArgs {
     NodeRec *rec_new;
     const TileInfo *tiles;
     const int *tnode, *halo;
-    const double *u;  // u_n
+    const double *u;  // u_n (compact layout; the slot layout's is in rec_old)
     double *u_out;    // u_{n+1}: u itself, or the next slot of a replay
+    // whether this step's u (slot layout, whose next step reads the record),
+    // force, body_force and Euler-Cromer udd are stored: the next step does
+    // not read them, so a run stores those of its last step
+    int store;
     double *ud, *udd, *force, *body_force;
-    const int *flags;
     const double *bcv, *fbcv, *dens;
     const double *dens1;  // per-node density when all three DOFs share it
-    const int *cnt;
+    const int *meta;      // row length | flags << 16
     unsigned short *loc;
     int *gidx;
     const double *corr;
@@ -841,6 +845,9 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
 // runs half rounds: 305 -> 270 us a step there, 113 -> 77 on the 263k-node
 // composite bar (its state now is the LDS offset of the bond's table entry),
 // 57 -> 48 on a 141k-node bar with corrections (requested with the chunk).
+// Tiles by bisection and a leaner prologue gave 257 us on the beam, 74.5 and
+// 46.4 on the other two; what a run's inner steps store for nobody (force, the
+// slot layout's u, Euler-Cromer's udd) left out, 250, 72 and 45.5.
 //
 // DM: DM_PMB, DM_NLIN or DM_FIELD.  One workgroup per tile, LPN lanes per
 // node taking its 4-bond chunks round-robin and reducing with cross-lane
@@ -873,7 +880,9 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
     // node state and the first chunks of halo entries are requested before
     // the halo is staged, so their latency overlaps the staging.  Chunk rows
     // past the node's last are never used (their loads stay inside loc's
-    // allocation, which is LOC_SLACK slots longer than the tiles need).
+    // allocation, which is LOC_SLACK slots longer than the tiles need); past
+    // the wavefront's last round the loads repeat it, as a condition around
+    // them would make the loop wait for them at once.
     const char *L = reinterpret_cast<const char *>(a.loc + 4 * ti.chunk_off);
     const char *S = reinterpret_cast<const char *>(a.state + 4 * ti.chunk_off);
     const char *C = reinterpret_cast<const char *>(a.corr + 4 * ti.chunk_off);
@@ -896,26 +905,27 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         return ch;
     };
     Chunk<CORR> qa = chunk_at(coff), qb = chunk_at(coff + cstep);
-    int cnt = 0;
+    int cnt = 0, fl = 0;
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     double4 r0i = make_double4(0.0, 0.0, 0.0, 0.0), ri = r0i;
     if (valid) {
         const NodeRec *pi = a.rec_old + i;
         r0i = pi->a;
         ri = pi->b;
-        cnt = a.cnt[i];
+        const int meta = a.meta[i];
+        cnt = meta & 0xffff;
+        fl = meta >> 16;
     }
     const double ci = DM == DM_FIELD && valid ? a.cnode[i] : 0.0;
     // with 4 or more lanes per node, lane d < 3 updates component d: its
     // inputs are requested now too (the prescribed values, needed only on
     // flagged DOFs, are read at the update)
     constexpr bool PRE = LPN >= 4;
-    int pfl = 0;
     double pu = 0.0, pud = 0.0, pudd = 0.0, pdens = 1.0;
     if (PRE && valid && sub < 3) {
         const size_t k = 3 * (size_t)i + sub;
-        pfl = a.flags[i];
-        pu = a.u[k];
+        if (!CLA)
+            pu = a.u[k];
         if (a.integrator != PD_EULER) {
             pud = a.ud[k];
             pdens = a.dens1 ? a.dens1[i] : a.dens[k];
@@ -978,12 +988,12 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         for (int k = 0; k < rounds; k += 2) {
             round(qa, k, coff);
             coff += cstep;
-            qa = chunk_at(coff + cstep);
+            qa = chunk_at(coff + (k + 2 < rounds ? cstep : 0u));
             if (k + 1 >= rounds)
                 break;
             round(qb, k + 1, coff);
             coff += cstep;
-            qb = chunk_at(coff + cstep);
+            qb = chunk_at(coff + (k + 3 < rounds ? cstep : 0u));
         }
     }
 
@@ -1003,7 +1013,6 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
 
     // the node's lanes share its three components (after the xor reduction
     // every lane holds the sums), so the per-node loads and stores coalesce
-    const int fl = PRE ? pfl : a.flags[i];
     const size_t b3 = 3 * (size_t)i;
     for (int d = sub; d < 3; d += LPN) {
         const size_t k = b3 + d;
@@ -1017,11 +1026,15 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         if (fbc)
             F = CLA ? __builtin_fma(fmag, a.fbcv[k], bf)
                     : bf + fmag * a.fbcv[k];
-        if (fbc)
-            a.body_force[k] = bf;
-        a.force[k] = F;
+        if (a.store) {
+            if (fbc)
+                a.body_force[k] = bf;
+            a.force[k] = F;
+        }
         const bool fixed = (fl >> d) & 1;
-        double u = PRE ? pu : a.u[k];
+        // the slot layout's records hold u
+        double u = CLA ? (d == 0 ? ri.x : (d == 1 ? ri.y : ri.z))
+                       : (PRE ? pu : a.u[k]);
         if (a.integrator == PD_EULER) {
             // peridynamics.pyx:179-185; cl/euler.cl:21-23 (contracted)
             const double un = CLA ? __builtin_fma(a.dt, F, u) : u + a.dt * F;
@@ -1033,7 +1046,8 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
                 PRE ? pdens : (a.dens1 ? a.dens1[i] : a.dens[k]);
             const double udd = __builtin_fma(-a.damping, ud, F) / dens;
             ud = __builtin_fma(udd, a.dt, ud);
-            a.udd[k] = udd;
+            if (a.store)
+                a.udd[k] = udd;
             a.ud[k] = ud;
             u = fixed ? dmag * a.bcv[k] : __builtin_fma(a.dt, ud, u);
         } else {
@@ -1050,7 +1064,8 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
             u = fixed ? dmag * a.bcv[k]
                       : __builtin_fma(a.dt, __builtin_fma(hdt, udd1, ud), u);
         }
-        a.u_out[k] = u;
+        if (!CLA || a.store)
+            a.u_out[k] = u;
         // the bond loop's position for the next step: r0 + u (compact) or
         // u (slot); the record's c (w) is static
         const double r0d = d == 0 ? r0i.x : (d == 1 ? r0i.y : r0i.z);
@@ -1596,12 +1611,12 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
     if (valid) {
         r0m = a.rec_old[i].a;
         rm = a.rec_old[i].b;
-        cnt = a.cnt[i];
+        const int meta = a.meta[i];
+        cnt = meta & 0xffff;
+        fl = meta >> 16;
         nlow = a.nlow[i];
-        if (sub < 3) {
-            fl = a.flags[i];
+        if (sub < 3)
             pu = a.u[3 * (size_t)i + sub];
-        }
     }
     hl.stage<true>(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb,
                    PB);
@@ -1666,14 +1681,14 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
                 Flow = F;
             round(qa, r, true);
             foff += fstep;
-            qa = pair_at(foff + fstep);
+            qa = pair_at(foff + (r + 2 < rounds ? fstep : 0u));
             if (r + 1 >= rounds)
                 break;
             if (r + 1 <= rlow)
                 Flow = F;
             round(qb, r + 1, true);
             foff += fstep;
-            qb = pair_at(foff + fstep);
+            qb = pair_at(foff + (r + 3 < rounds ? fstep : 0u));
         }
         if (rlow >= rounds)
             Flow = F;  // no upper part
@@ -1701,11 +1716,13 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         const size_t k = 3 * (size_t)i + sub;
         const bool fbc = (fl >> (3 + sub)) & 1;
         double Fd = F;
-        if (fbc) {
+        if (fbc)
             Fd = F + fmag * a.fbcv[k];
-            a.body_force[k] = F;
+        if (a.store) {
+            if (fbc)
+                a.body_force[k] = F;
+            a.force[k] = Fd;
         }
-        a.force[k] = Fd;
         const double u = (fl >> sub) & 1 ? dmag * a.bcv[k] : pu + a.dt * Fd;
         a.u_out[k] = u;
         const double r0d = sub == 0 ? r0m.x : (sub == 1 ? r0m.y : r0m.z);
@@ -2229,6 +2246,7 @@ struct pd_sim {
     DevBuf<double> r0, vol, u, ud, udd, force, body_force, bcv, fbcv, dens,
         damage, cnode, corr, k_tab, s_tab, pc_tab;
     DevBuf<double> cnode_caller;  // a field given on the device (caller order)
+    DevBuf<int> meta;  // cnt | flags << 16
     DevBuf<int> flags, family, cnt, tnode, halo, gidx, stride, nlist_ref,
         n_neigh, out_nlist, out_nneigh;
     DevBuf<long long> chunk0;
@@ -2400,12 +2418,11 @@ StepArgs make_args(pd_sim *s)
     a.udd = s->udd.p;
     a.force = s->force.p;
     a.body_force = s->body_force.p;
-    a.flags = s->flags.p;
     a.bcv = s->bcv.p;
     a.fbcv = s->fbcv.p;
     a.dens = s->dens.p;
     a.dens1 = s->dens1.p;
-    a.cnt = s->cnt.p;
+    a.meta = s->meta.p;
     a.loc = s->loc.p;
     a.gidx = s->gidx.p;
     a.corr = s->corr.p;
@@ -2576,7 +2593,8 @@ int after_step(pd_sim *s, double dmag, double fmag)
     return PD_OK;
 }
 
-int launch_step(pd_sim *s, double dmag, double fmag)
+// One step; `last`: the last of its run, whose u and forces are stored.
+int launch_step(pd_sim *s, double dmag, double fmag, bool last)
 {
     if (s->retile_pending)
         return fail(PD_E_STATE, "tile_nodes changed: call pd_create_buffers "
@@ -2600,7 +2618,11 @@ int launch_step(pd_sim *s, double dmag, double fmag)
     if (s->exact && !exact_rows_fit(s->K))
         return fail(PD_E_LIMIT, "the exact-order step takes at most 4074 "
                                 "neighbours per node");
-    const StepArgs a = make_args(s);
+    StepArgs a = make_args(s);
+    // a replay keeps every u, a recording those of its checkpoints
+    a.store = last || s->u_out ||
+              (s->adj_recording &&
+               (s->step_counter + 1) % s->adj_every == 0);
     hipError_t e;
     if (s->exact) {
         const dim3 grid(XCDS * a.tiles_per_xcd);
@@ -3564,6 +3586,12 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     chk(upload_perm(s->r0, s->perm, s->h_coords.data(), 3), "coords");
     chk(upload_perm(s->vol, s->perm, s->h_vol.data(), 1), "volume");
     chk(upload_perm(s->flags, s->perm, s->h_flags.data(), 1), "flags");
+    {
+        std::vector<int> meta(N);
+        for (int i = 0; i < N; ++i)
+            meta[i] = cnt[i] | s->h_flags[i] << 16;
+        chk(upload_perm(s->meta, s->perm, meta.data(), 1), "flags");
+    }
     chk(upload_perm(s->bcv, s->perm, s->h_bcv.data(), 3), "bc_values");
     chk(upload_perm(s->fbcv, s->perm, s->h_fbcv.data(), 3),
         "force_bc_values");
@@ -3966,7 +3994,7 @@ int pd_step(pd_sim *s, double dmag, double fmag)
         return rc;
     if (!s->has_buffers)
         return fail(PD_E_STATE, "pd_create_buffers has not been called");
-    return launch_step(s, dmag, fmag);
+    return launch_step(s, dmag, fmag, true);
 }
 
 int pd_run(pd_sim *s, int nsteps, const double *disp_mags,
@@ -3981,7 +4009,7 @@ int pd_run(pd_sim *s, int nsteps, const double *disp_mags,
         return fail(PD_E_ARG, "nsteps < 0");
     for (int t = 0; t < nsteps; ++t) {
         rc = launch_step(s, disp_mags ? disp_mags[t] : 0.0,
-                         force_mags ? force_mags[t] : 0.0);
+                         force_mags ? force_mags[t] : 0.0, t + 1 == nsteps);
         if (rc)
             return rc;
     }
@@ -4029,7 +4057,7 @@ int pd_run_graph(pd_sim *s, int nsteps, const double *disp_mags,
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     for (int t = 0; t < nsteps && rc == PD_OK; ++t)
         rc = launch_step(s, disp_mags ? disp_mags[t] : 0.0,
-                         force_mags ? force_mags[t] : 0.0);
+                         force_mags ? force_mags[t] : 0.0, t + 1 == nsteps);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(s->stream, &graph);
     if (rc != PD_OK || ec != hipSuccess) {
@@ -4212,7 +4240,7 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
             s->step_counter = n;
             s->u_in = s->seg.p + (size_t)(n - n0) * B;
             s->u_out = s->seg.p + (size_t)(n - n0 + 1) * B;
-            rc = launch_step(s, s->adj_dmag[n], s->adj_fmag[n]);
+            rc = launch_step(s, s->adj_dmag[n], s->adj_fmag[n], false);
         }
         s->u_in = nullptr;
         s->u_out = nullptr;
