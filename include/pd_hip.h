@@ -151,8 +151,8 @@ int pd_set_exact_order(pd_sim *sim, int on);
  * largest number of nodes per tile (a multiple of 64, with
  * tile_nodes * lanes_per_node <= 1024; one workgroup runs one tile).
  * Defaults: 4 and 128; without a call, meshes of at most 48 nodes per CU run
- * 8 lanes per node.  A mesh too small to give every CU a tile of tile_nodes
- * nodes is cut into smaller ones (the tiles change no result).
+ * 8 lanes per node.  A mesh of at most five tiles of tile_nodes nodes per CU
+ * is cut into smaller ones, as many for every CU (the tiles change no result).
  * lanes_per_node takes effect at the next step;
  * tile_nodes at the next pd_create_buffers, which builds the tiles (stepping
  * in between fails with PD_E_STATE).  A tile's

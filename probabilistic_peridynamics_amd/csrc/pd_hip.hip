@@ -91,6 +91,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <memory>
 #include <string>
 #include <mutex>
@@ -1426,7 +1427,7 @@ __global__ void __launch_bounds__(256)
 constexpr int EXACT_NODES = 128;
 constexpr int EXACT_CAP = (int)((LDS_BYTES - EXACT_NODES * 96u) / 64u);
 // Tiles of at most that many nodes run eight lanes per node: they are small
-// because the mesh is (tile_cap_of), so that a round's latency bounds it.
+// because the mesh is (set_shape), so that a round's latency bounds it.
 constexpr int EXACT_WIDE_NODES = 64;
 
 // Rows of K slots fit compact_tile's groups in the exact step's fold
@@ -2703,26 +2704,49 @@ int fold_lists(pd_sim *s)
     return PD_OK;
 }
 
-// The launch shape of the next tiling.  On a mesh of fewer nodes than one
-// workgroup per CU takes, a step is one workgroup's latency, most of it the
-// issue of its rounds, so the nodes are spread: tiles as small as give every
-// CU one (no smaller than 32 nodes at eight lanes, 48 at four: their halos
-// then cost more), and eight lanes per node where the caller set no shape and
-// the tiles are that small.  Tiles change no result; lanes change the order
-// of a node's sum.  us a step, scalar model, tiles of 128 / the rule, four
-// lanes, and the rule with eight: 2,560 nodes 10.6 / 8.4, 6.7; 5,000 nodes
-// 11.6 / 9.1, 6.8; 20,655 nodes 12.4 / 12.0, 12.4 (not taken).  From two
-// workgroups per CU on, 128 nodes are the fastest (50,820 nodes: 19.5; with
-// 96, 23.1).
+// The launch shape of the next tiling.  Up to WAVES_EVEN tiles per CU the tiles
+// are as small as keeps that number, so that every CU gets as many of them: a
+// mesh of less than one workgroup per CU is one workgroup's latency, most of
+// it the issue of its rounds, and of one and a half the latency of two on half
+// of the CUs.  No smaller than 32 nodes at eight lanes, 48 at four (their
+// halos then cost more), and eight lanes per node where the caller set no
+// shape and the tiles are that small.  Tiles change no result; lanes change
+// the order of a node's sum.  us a step, scalar model, tiles of 128 / the
+// rule, four lanes, and the rule with eight: 2,560 nodes 10.6 / 8.4, 6.7;
+// 5,000 nodes 11.6 / 9.1, 6.8; 20,655 nodes 12.4 / 12.0, 12.4 (not taken).
+// Four lanes, 128 / the rule: 35,420 nodes 18.2 / 15.0 (n-linear 19.8 / 15.9,
+// exact order 24.0 / 20.0), 50,820 nodes 19.0 / 18.7, 75,900 nodes 25.5 / 24.2
+// (28.3 / 26.2, 35.1 / 33.0), 111,320 nodes 32.3 / 31.5 (36.8 / 34.3), 141,143
+// nodes 38.9 / 38.7 (43.3 / 41.6, 54.5 / 53.7); from six tiles per CU on
+// nothing is gained, or lost to the halos (170,810 nodes, exact order: 64.5 /
+// 72.2).  A tile more than a multiple of the CUs costs what the multiple
+// gains: 50,820 nodes in 530 tiles 23.1.
+constexpr int WAVES_EVEN = 5;
+
 void set_shape(pd_sim *s)
 {
     if (!s->launch_given)
         s->lanes = s->n <= 48 * s->cus ? 8 : s->lpn;
     const int least = s->lanes == 8 ? 32 : 48;
-    const int even = ((s->n + s->cus - 1) / s->cus + 15) & ~15;
-    s->tile_cap = std::min(std::max(even, least), s->tile_nodes);
-    if (s->n > s->cus * s->tile_nodes)
-        s->tile_cap = s->tile_nodes;
+    // no tile spans two groups
+    std::map<int, int> sizes;
+    if (s->h_group.empty())
+        sizes[0] = s->n;
+    else
+        for (int g : s->h_group)
+            ++sizes[g];
+    auto tiles = [&](int cap) {
+        long long m = 0;
+        for (const auto &g : sizes)
+            m += (g.second + cap - 1) / cap;
+        return m;
+    };
+    const long long per_cu = (tiles(s->tile_nodes) + s->cus - 1) / s->cus;
+    s->tile_cap = s->tile_nodes;
+    if (per_cu > WAVES_EVEN)
+        return;
+    while (s->tile_cap > least && tiles(s->tile_cap - 1) <= per_cu * s->cus)
+        --s->tile_cap;
 }
 
 // Rows of w values given in the caller's order into tile order on the device
