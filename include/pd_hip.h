@@ -201,11 +201,15 @@ int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
  * counterpart in the reference.  Usage: pd_adjoint_start, then nsteps steps
  * by pd_step / pd_run (not pd_run_graph), then pd_adjoint_backward (any
  * number of times).  The recording keeps the step at which each bond broke
- * (the break mask is held fixed in the backward pass) and u every
- * checkpoint_every steps; the backward pass replays each segment from its
- * checkpoint with the step kernel (bitwise the recorded trajectory) and
- * runs the adjoint kernel (on the step kernel's tiles) back through it.
- * Device memory: 14 bytes per bond slot, and per node 256 bytes plus 24
+ * (the break mask is held fixed in the backward pass) and u of every step,
+ * or, where that takes more than 16 times the memory of checkpoints every
+ * checkpoint_every steps and of one segment between two, a 64th of the
+ * device's or a quarter of what is free, u at those checkpoints: the backward
+ * pass then replays each segment from its checkpoint with the step kernel
+ * (bitwise the recorded trajectory; so it does where the stiffness field, the
+ * break mode or the launch shape was set since pd_adjoint_start).  The adjoint
+ * kernel (on the step kernel's tiles) runs back through the steps.  Device
+ * memory: 14 bytes per bond slot, and per node 256 bytes plus 24 per step, or
  * per checkpoint and per step of a segment.  Requires PD_EULER,
  * PD_LAYOUT_SLOT and pd_set_node_stiffness.  pd_create_buffers or
  * pd_adjoint_stop ends a recording; its memory is kept for the next one until

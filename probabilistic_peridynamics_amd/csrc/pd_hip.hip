@@ -164,6 +164,8 @@ struct TileInfo {
     int nch, pad;
 };
 
+constexpr int STORE_U = 1, STORE_F = 2;
+
 struct StepArgs {
     int n, K, hstride, ntiles, tiles_per_xcd;
     int integrator, layout, has_corr;
@@ -177,9 +179,10 @@ struct StepArgs {
     const int *tnode, *halo;
     const double *u;  // u_n (compact layout; the slot layout's is in rec_old)
     double *u_out;    // u_{n+1}: u itself, or the next slot of a replay
-    // whether this step's u (slot layout, whose next step reads the record),
-    // force, body_force and Euler-Cromer udd are stored: the next step does
-    // not read them, so a run stores those of its last step
+    // what this step stores of that which the next one does not read (a run
+    // stores those of its last step): STORE_U u of the slot layout, whose
+    // next step reads the record; STORE_F force, body_force and
+    // Euler-Cromer's udd
     int store;
     double *ud, *udd, *force, *body_force;
     const double *bcv, *fbcv, *dens;
@@ -1027,7 +1030,7 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         if (fbc)
             F = CLA ? __builtin_fma(fmag, a.fbcv[k], bf)
                     : bf + fmag * a.fbcv[k];
-        if (a.store) {
+        if (a.store & STORE_F) {
             if (fbc)
                 a.body_force[k] = bf;
             a.force[k] = F;
@@ -1047,7 +1050,7 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
                 PRE ? pdens : (a.dens1 ? a.dens1[i] : a.dens[k]);
             const double udd = __builtin_fma(-a.damping, ud, F) / dens;
             ud = __builtin_fma(udd, a.dt, ud);
-            if (a.store)
+            if (a.store & STORE_F)
                 a.udd[k] = udd;
             a.ud[k] = ud;
             u = fixed ? dmag * a.bcv[k] : __builtin_fma(a.dt, ud, u);
@@ -1065,7 +1068,7 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
             u = fixed ? dmag * a.bcv[k]
                       : __builtin_fma(a.dt, __builtin_fma(hdt, udd1, ud), u);
         }
-        if (!CLA || a.store)
+        if (!CLA || (a.store & STORE_U))
             a.u_out[k] = u;
         // the bond loop's position for the next step: r0 + u (compact) or
         // u (slot); the record's c (w) is static
@@ -1719,7 +1722,7 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         double Fd = F;
         if (fbc)
             Fd = F + fmag * a.fbcv[k];
-        if (a.store) {
+        if (a.store & STORE_F) {
             if (fbc)
                 a.body_force[k] = F;
             a.force[k] = Fd;
@@ -2214,8 +2217,7 @@ struct pd_sim {
     double k = 0.0, s0 = 0.0;
     int cur = 0;
     bool exact = false;  // exact-order Euler step (k_exact_step)
-    // a replay's u_n and u_{n+1} (slots of the segment buffer); null: u
-    const double *u_in = nullptr;
+    // a replay's u_{n+1} (a slot of the segment buffer); null: u
     double *u_out = nullptr;
     DevBuf<int> nlow, nup;  // exact step: lower slots, upper-list length
     DevBuf<unsigned> ford;  // exact step: fold lists
@@ -2256,6 +2258,10 @@ struct pd_sim {
 
     // adjoint recording (Euler, node field): break steps, checkpoints
     bool adj_recording = false, adj_ready = false, adj_replay = false;
+    bool adj_all = false;  // u of every recorded step is in seg
+    // the model or the launch shape was set anew since the recording began:
+    // its steps are replayed with the new ones
+    bool adj_changed = false;
     int adj_nsteps = 0, adj_every = 0, step_counter = 0;
     std::vector<double> adj_dmag, adj_fmag;
     DevBuf<int> brk;
@@ -2413,7 +2419,7 @@ StepArgs make_args(pd_sim *s)
     a.tiles = s->tiles.p;
     a.tnode = s->tnode.p;
     a.halo = s->halo.p;
-    a.u = s->u_in ? s->u_in : s->u.p;
+    a.u = s->u.p;
     a.u_out = s->u_out ? s->u_out : s->u.p;
     a.ud = s->ud.p;
     a.udd = s->udd.p;
@@ -2545,6 +2551,7 @@ hipError_t launch_adjoint(pd_sim *s, const AdjArgs &a)
 void adjoint_end(pd_sim *s)
 {
     s->adj_recording = s->adj_ready = s->adj_replay = false;
+    s->adj_all = s->adj_changed = false;
     s->adj_nsteps = s->adj_every = s->step_counter = 0;
     s->adj_dmag.clear();
     s->adj_fmag.clear();
@@ -2582,7 +2589,7 @@ int after_step(pd_sim *s, double dmag, double fmag)
     s->adj_fmag.push_back(fmag);
     ++s->step_counter;
     const size_t B = 3 * (size_t)s->n;
-    if (s->step_counter % s->adj_every == 0 &&
+    if (!s->adj_all && s->step_counter % s->adj_every == 0 &&
         s->step_counter < s->adj_nsteps)
         HIPCHK(hipMemcpyAsync(s->ckpt.p + (s->step_counter / s->adj_every) * B,
                               s->u.p, B * sizeof(double),
@@ -2620,10 +2627,19 @@ int launch_step(pd_sim *s, double dmag, double fmag, bool last)
         return fail(PD_E_LIMIT, "the exact-order step takes at most 4074 "
                                 "neighbours per node");
     StepArgs a = make_args(s);
-    // a replay keeps every u, a recording those of its checkpoints
-    a.store = last || s->u_out ||
-              (s->adj_recording &&
-               (s->step_counter + 1) % s->adj_every == 0);
+    a.store = last ? STORE_U | STORE_F : 0;
+    // a replay stores every u, a recording those that it keeps: all, each in
+    // a slot of its own (and the last step's in u), or its checkpoints'
+    double *slot = nullptr;
+    if (s->u_out) {
+        a.store |= STORE_U;
+    } else if (s->adj_recording) {
+        const int next = s->step_counter + 1;
+        if (next % s->adj_every == 0 || s->adj_all)
+            a.store |= STORE_U;
+        if (s->adj_all && next < s->adj_nsteps)
+            a.u_out = slot = s->seg.p + (size_t)next * 3 * s->n;
+    }
     hipError_t e;
     if (s->exact) {
         const dim3 grid(XCDS * a.tiles_per_xcd);
@@ -2651,6 +2667,9 @@ int launch_step(pd_sim *s, double dmag, double fmag, bool last)
         return fail(PD_E_HIP, std::string("step kernel launch: ") +
                                   hipGetErrorString(e));
     s->cur = 1 - s->cur;
+    if (slot && last)
+        HIPCHK(hipMemcpyAsync(s->u.p, slot, 3 * (size_t)s->n * sizeof(double),
+                              hipMemcpyDeviceToDevice, s->stream));
     return after_step(s, dmag, fmag);
 }
 
@@ -3892,6 +3911,7 @@ int pd_set_node_stiffness(pd_sim *s, const double *c)
     if (rc)
         return rc;
     HIPCHK(hipStreamSynchronize(s->stream));
+    s->adj_changed = true;
     s->cnode_caller.release();
     if (!c) {
         s->cnode.release();
@@ -3921,6 +3941,7 @@ int pd_set_node_stiffness_device(pd_sim *s, const double *c)
     if (!c)
         return fail(PD_E_ARG, "c is NULL (pd_set_node_stiffness clears)");
     HIPCHK(hipStreamSynchronize(s->stream));
+    s->adj_changed = true;
     const size_t N = (size_t)s->n;
     HIPCHK(s->cnode_caller.alloc(N));
     HIPCHK(hipMemcpyAsync(s->cnode_caller.p, c, N * sizeof(double),
@@ -3945,6 +3966,7 @@ int pd_set_break_mode(pd_sim *s, int tension_only)
     if (rc)
         return rc;
     s->tension_only = tension_only ? 1 : 0;
+    s->adj_changed = true;
     return PD_OK;
 }
 
@@ -3993,6 +4015,7 @@ int pd_set_launch(pd_sim *s, int lanes_per_node, int tile_nodes)
     s->lpn = s->lanes = lanes_per_node;
     s->tile_nodes = tile_nodes;
     s->launch_given = true;
+    s->adj_changed = true;
     return PD_OK;
 }
 
@@ -4115,6 +4138,35 @@ int pd_run_graph(pd_sim *s, int nsteps, const double *disp_mags,
     return PD_OK;
 }
 
+namespace {
+
+// Whether a recording keeps u of all its steps (room for them is then in
+// seg), where checkpoints and a segment take `slots` arrays: the backward
+// pass then replays nothing (a third of it and of the forward pass together:
+// 200 steps and their gradient on 50,820 nodes 12.3 -> 8.8 ms).  At most
+// KEEP_TIMES the memory that the caller's checkpoint interval asks for, a
+// 64th of the device's and a quarter of what is free.
+constexpr size_t KEEP_TIMES = 16;
+
+bool keep_all(pd_sim *s, int nsteps, size_t slots)
+{
+    const size_t count = (size_t)nsteps * 3 * s->n;
+    if ((size_t)nsteps > KEEP_TIMES * slots)
+        return false;
+    if (s->seg.p && s->seg.n >= count)
+        return true;
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess ||
+        count * sizeof(double) > std::min(total / 64, avail / 4) ||
+        s->seg.alloc(count) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+}  // namespace
+
 int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
 {
     int rc = check_sim(s);
@@ -4143,14 +4195,14 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
     HIPCHK(s->arec[0].reserve(N));
     HIPCHK(s->arec[1].reserve(N));
     HIPCHK(s->loc0.reserve(S));
-    HIPCHK(s->ckpt.reserve((size_t)nck * B));
-    HIPCHK(s->seg.reserve((size_t)checkpoint_every * B));
+    s->adj_all = keep_all(s, nsteps, (size_t)nck + checkpoint_every);
+    if (!s->adj_all) {
+        HIPCHK(s->ckpt.reserve((size_t)nck * B));
+        HIPCHK(s->seg.reserve((size_t)checkpoint_every * B));
+    }
     HIPCHK(s->lam[0].reserve(B));
     HIPCHK(s->lam[1].reserve(B));
     HIPCHK(s->gradc.reserve(N));
-    HIPCHK(s->fin_u.reserve(B));
-    HIPCHK(s->fin_force.reserve(B));
-    HIPCHK(s->fin_bforce.reserve(B));
     // rows past a node's own, up to its tile's longest: finite
     HIPCHK(hipMemsetAsync(s->il0.p, 0, S * sizeof(double), s->stream));
     hipLaunchKernelGGL(k_adj_init, dim3(chunk_blocks(s)), dim3(256), 0,
@@ -4161,8 +4213,9 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
                        dim3(256), 0, s->stream, s->n, s->cnt.p, s->chunk0.p, s->stride.p,
                        s->gidx.p, s->loc0.p, s->inv.p, s->r0.p, s->il0.p);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(s->ckpt.p, s->u.p, B * sizeof(double),
-                          hipMemcpyDeviceToDevice, s->stream));
+    HIPCHK(hipMemcpyAsync(s->adj_all ? s->seg.p : s->ckpt.p, s->u.p,
+                          B * sizeof(double), hipMemcpyDeviceToDevice,
+                          s->stream));
     s->adj_nsteps = nsteps;
     s->adj_every = checkpoint_every;
     s->step_counter = 0;
@@ -4183,9 +4236,34 @@ int adjoint_restore(pd_sim *s, int n0)
     return refresh_records(s);
 }
 
-}  // namespace
-
-namespace {
+// Steps n0 .. n1 - 2 again from u of step n0, the segment's first slot: the
+// same kernel from the same state reproduces the recorded steps (and their
+// breaks) bitwise; step n writes u_{n+1} to slot n + 1 - n0 of the segment.
+int adjoint_replay(pd_sim *s, double *seg, int n0, int n1)
+{
+    const size_t B = 3 * (size_t)s->n;
+    HIPCHK(hipMemcpyAsync(s->u.p, seg, B * sizeof(double),
+                          hipMemcpyDeviceToDevice, s->stream));
+    const int rc0 = adjoint_restore(s, n0);
+    if (rc0)
+        return rc0;
+    struct ReplayGuard {  // the steps below are replays
+        pd_sim *s;
+        ~ReplayGuard()
+        {
+            s->adj_replay = false;
+            s->u_out = nullptr;
+        }
+    } guard{s};
+    s->adj_replay = true;
+    int rc = PD_OK;
+    for (int n = n0; n < n1 - 1 && rc == PD_OK; ++n) {
+        s->step_counter = n;
+        s->u_out = seg + (size_t)(n - n0 + 1) * B;
+        rc = launch_step(s, s->adj_dmag[n], s->adj_fmag[n], false);
+    }
+    return rc;
+}
 
 // pd_adjoint_backward with dL_du and dL_dc in host memory (device false) or
 // in device memory (device true), both in the caller's node order.
@@ -4201,16 +4279,24 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
     if (!dL_du || !dL_dc)
         return fail(PD_E_ARG, "dL_du and dL_dc are required");
     const size_t N = (size_t)s->n, B = 3 * N, BB = B * sizeof(double);
-    const int every = s->adj_every, nsteps = s->adj_nsteps;
+    // with every u kept, the recording is one segment that needs no replay,
+    // and the state is not touched
+    const bool replay = !s->adj_all || s->adj_changed;
+    const int nsteps = s->adj_nsteps, every = replay ? s->adj_every : nsteps;
     const int nck = (nsteps + every - 1) / every;
     hipStream_t st = s->stream;
     HIPCHK(hipStreamSynchronize(st));
-    HIPCHK(hipMemcpyAsync(s->fin_u.p, s->u.p, BB, hipMemcpyDeviceToDevice,
-                          st));
-    HIPCHK(hipMemcpyAsync(s->fin_force.p, s->force.p, BB,
-                          hipMemcpyDeviceToDevice, st));
-    HIPCHK(hipMemcpyAsync(s->fin_bforce.p, s->body_force.p, BB,
-                          hipMemcpyDeviceToDevice, st));
+    if (replay) {
+        HIPCHK(s->fin_u.reserve(B));
+        HIPCHK(s->fin_force.reserve(B));
+        HIPCHK(s->fin_bforce.reserve(B));
+        HIPCHK(hipMemcpyAsync(s->fin_u.p, s->u.p, BB, hipMemcpyDeviceToDevice,
+                              st));
+        HIPCHK(hipMemcpyAsync(s->fin_force.p, s->force.p, BB,
+                              hipMemcpyDeviceToDevice, st));
+        HIPCHK(hipMemcpyAsync(s->fin_bforce.p, s->body_force.p, BB,
+                              hipMemcpyDeviceToDevice, st));
+    }
     if (device) {
         hipLaunchKernelGGL(k_perm, dim3((s->n + 255) / 256), dim3(256), 0, st,
                            s->n, 3, s->tnode.p, dL_du, s->lam[0].p);
@@ -4238,43 +4324,22 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
     aa.loc0 = s->loc0.p;
     aa.il0 = s->il0.p;
     aa.gradc = s->gradc.p;
-    struct ReplayGuard {  // steps below are replays, also on early returns
-        pd_sim *s;
-        ~ReplayGuard()
-        {
-            s->adj_replay = false;
-            s->u_in = nullptr;
-            s->u_out = nullptr;
-        }
-    } guard{s};
-    s->adj_replay = true;
     for (int k = nck - 1; k >= 0 && rc == PD_OK; --k) {
         const int n0 = k * every, n1 = std::min(n0 + every, nsteps);
-        HIPCHK(hipMemcpyAsync(s->u.p, s->ckpt.p + (size_t)k * B, BB,
-                              hipMemcpyDeviceToDevice, st));
-        rc = adjoint_restore(s, n0);
-        if (rc)
-            break;
-        HIPCHK(hipMemcpyAsync(s->seg.p, s->u.p, BB, hipMemcpyDeviceToDevice,
-                              st));
-        // replay the segment: the same kernel from the same state reproduces
-        // the recorded steps (and their breaks) bitwise; step n reads u_n
-        // from slot n - n0 of the segment and writes u_{n+1} to the next
-        for (int n = n0; n < n1 - 1 && rc == PD_OK; ++n) {
-            s->step_counter = n;
-            s->u_in = s->seg.p + (size_t)(n - n0) * B;
-            s->u_out = s->seg.p + (size_t)(n - n0 + 1) * B;
-            rc = launch_step(s, s->adj_dmag[n], s->adj_fmag[n], false);
+        double *seg = s->seg.p + (s->adj_all ? (size_t)n0 * B : 0);
+        if (!s->adj_all)
+            HIPCHK(hipMemcpyAsync(seg, s->ckpt.p + (size_t)k * B, BB,
+                                  hipMemcpyDeviceToDevice, st));
+        if (replay) {
+            rc = adjoint_replay(s, seg, n0, n1);
+            if (rc)
+                break;
         }
-        s->u_in = nullptr;
-        s->u_out = nullptr;
-        if (rc)
-            break;
         // the records of the segment's last step; each backward step then
         // writes those of the step before it, within the segment
         int ra = 0;
         hipLaunchKernelGGL(k_adj_pack, dim3(pblocks), dim3(256), 0, st, s->n,
-                           s->r0.p, s->seg.p + (size_t)(n1 - 1 - n0) * B,
+                           s->r0.p, seg + (size_t)(n1 - 1 - n0) * B,
                            s->vol.p, s->cnode.p, s->flags.p, s->lam[cur].p,
                            s->arec[ra].p);
         HIPCHK(hipGetLastError());
@@ -4283,28 +4348,28 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
             aa.rec = s->arec[ra].p;
             aa.lam_out = s->lam[1 - cur].p;
             aa.rec_next = n > n0 ? s->arec[1 - ra].p : nullptr;
-            aa.u_prev = n > n0 ? s->seg.p + (size_t)(n - 1 - n0) * B
-                               : nullptr;
+            aa.u_prev = n > n0 ? seg + (size_t)(n - 1 - n0) * B : nullptr;
             if (s->ntiles > 0)
                 HIPCHK(launch_adjoint(s, aa));
             cur = 1 - cur;
             ra = 1 - ra;
         }
     }
-    s->adj_replay = false;
     if (rc)
         return rc;
-    // back to the end of the recording
-    HIPCHK(hipMemcpyAsync(s->u.p, s->fin_u.p, BB, hipMemcpyDeviceToDevice,
-                          st));
-    HIPCHK(hipMemcpyAsync(s->force.p, s->fin_force.p, BB,
-                          hipMemcpyDeviceToDevice, st));
-    HIPCHK(hipMemcpyAsync(s->body_force.p, s->fin_bforce.p, BB,
-                          hipMemcpyDeviceToDevice, st));
-    rc = adjoint_restore(s, nsteps);
-    if (rc)
-        return rc;
-    s->step_counter = nsteps;
+    if (replay) {
+        // back to the end of the recording
+        HIPCHK(hipMemcpyAsync(s->u.p, s->fin_u.p, BB, hipMemcpyDeviceToDevice,
+                              st));
+        HIPCHK(hipMemcpyAsync(s->force.p, s->fin_force.p, BB,
+                              hipMemcpyDeviceToDevice, st));
+        HIPCHK(hipMemcpyAsync(s->body_force.p, s->fin_bforce.p, BB,
+                              hipMemcpyDeviceToDevice, st));
+        rc = adjoint_restore(s, nsteps);
+        if (rc)
+            return rc;
+        s->step_counter = nsteps;
+    }
     if (device) {
         hipLaunchKernelGGL(k_unperm, dim3((s->n + 255) / 256), dim3(256), 0,
                            st, s->n, 1, s->tnode.p, s->gradc.p, dL_dc);

@@ -281,9 +281,10 @@ class Integrator(ABC):
 
     def adjoint_start(self, steps, checkpoint_every=100):
         """Record the next ``steps`` steps (run by ``__call__`` / ``run``)
-        for :meth:`adjoint_backward`: break steps and a checkpoint of u
-        every ``checkpoint_every`` steps.  Euler with a node stiffness
-        field only."""
+        for :meth:`adjoint_backward`: break steps and u of every step, or
+        where that takes much memory a checkpoint of u every
+        ``checkpoint_every`` steps.  Euler with a node stiffness field
+        only."""
         self._need_sim()
         check(_lib.lib().pd_adjoint_start(self._sim, int(steps),
                                           int(checkpoint_every)))
