@@ -189,9 +189,9 @@ int pd_run(pd_sim *sim, int nsteps, const double *disp_mags,
 int pd_run_timed(pd_sim *sim, int nsteps, const double *disp_mags,
                  const double *force_mags, float *elapsed_ms);
 
-/* pd_run captured as one hipGraph and launched once (synchronous); if
- * elapsed_ms is not NULL it receives the graph's run time, measured with
- * events on the library's stream.  Replaces the step loop of Model.simulate
+/* pd_run captured as hipGraphs of a few steps, the device running one while
+ * the next is captured (synchronous); if elapsed_ms is not NULL it receives
+ * their run time, measured with events on the library's stream.  Replaces the step loop of Model.simulate
  * (model.py:1295-1301) when the magnitudes of all steps are known. */
 int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
                  const double *force_mags, float *elapsed_ms);

@@ -61,7 +61,7 @@ def autotune(apply, time_steps, cands=None, repeats=1):
 def autotune_batch(batch, steps=10, cands=None, graph=True):
     """:func:`autotune` for a :class:`~.batch.SampleBatch`: each candidate
     re-tiles the batch and is timed over ``steps`` steps from the initial
-    state, captured in one hipGraph (``graph``) as the batch's runs are, or
+    state, captured in hipGraphs (``graph``) as the batch's runs are, or
     as plain launches."""
     def apply(lp, t):
         batch.set_launch(lp, t)

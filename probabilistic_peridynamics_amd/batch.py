@@ -7,7 +7,7 @@ concatenated into one node set (node ids offset per sample, so no bond joins
 two samples), each sample is a tiling group (tiles never span samples), the
 per-node stiffness field ``c`` gives each bond ``k_ij = (c_i + c_j)/2``, and
 all samples advance together: one step kernel launch per step for the whole
-batch, the steps of a run captured into one hipGraph and launched once.
+batch, the steps of a run captured into hipGraphs.
 
 Every node's arithmetic is the same as in a run of its sample alone with the
 same lanes per node, so per-sample results are bitwise those of solo runs.
@@ -118,8 +118,7 @@ class SampleBatch:
     def run(self, steps, graph=True):
         """Advance every sample ``steps`` steps; returns the GPU time (ms)
         of the run (HIP events on the library's stream).  ``graph``: capture
-        the steps into one hipGraph and launch it once, else one launch per
-        step."""
+        the steps into hipGraphs, else one launch per step."""
         d, f = self.magnitudes(steps)
         if graph:
             ms = self.integrator.run_graph(steps, d, f)

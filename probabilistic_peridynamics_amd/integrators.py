@@ -269,8 +269,8 @@ class Integrator(ABC):
 
     def run_graph(self, steps, displacement_bc_magnitudes=None,
                   force_bc_magnitudes=None):
-        """:meth:`run` captured as one hipGraph and launched once; returns
-        the graph's run time in ms (HIP events on the library's stream)."""
+        """:meth:`run` captured as hipGraphs of a few steps; returns
+        their run time in ms (HIP events on the library's stream)."""
         self._need_sim()
         d = self._mags(displacement_bc_magnitudes, steps)
         f = self._mags(force_bc_magnitudes, steps)
