@@ -77,8 +77,9 @@
 // fixtures evaluated them.  The square roots use the correctly rounded
 // rsq-Goldschmidt sequence that the compiler emits for sqrt(double), without
 // its range scaling (taken only for q outside [2^-767, inf), where the
-// library sqrt is called).  Its by-product h ~ 0.5/sqrt(q) (relative error
-// ~1e-13) replaces the two divisions; a stretch within a relative 1e-10 of
+// library sqrt is called); the step in plain order takes it with one
+// residual correction instead of two (sqrt_core<1>).  Its by-product h ~ 0.5/sqrt(q) (relative error
+// ~5e-15) replaces the two divisions; a stretch within a relative 1e-10 of
 // any threshold it is compared with is recomputed with the IEEE division, so
 // every break and regime decision equals the one made with the correctly
 // rounded s.
@@ -264,6 +265,16 @@ __device__ __forceinline__ void static_for(F f)
 // corrections of g -- the sequence LLVM emits for llvm.sqrt.f64 on gfx9,
 // minus the input scaling and the zero/infinity selects it needs outside
 // that range.
+// CORRECTIONS 1 leaves out the second one: the seed's relative error e is at
+// most 6.0e-8 (2^29 ulp), the step's d = 3/2 e^2 <= 5.4e-15, and the first
+// correction's 3/2 d^2 <= 4.4e-29 before its one rounding, so g is within
+// 0.5 + 4e-13 ulp of sqrt(q): the nearest double unless sqrt(q) lies within
+// 4e-13 ulp of the middle between two (of 4.3e9 random q none got another g).
+// The step kernel's fast evaluation, whose lengths need not be the Cython
+// code's to the bit, spends no instruction on the second: 4 of a bond's 51
+// issue slots, 255 -> 242 us a step on the 1,038,230-node beam, 37.1 -> 35.1 on
+// 141,143 nodes, 72.3 -> 69.1 with n-linear tables on 263,407.
+template <int CORRECTIONS = 2>
 __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
 {
     const double y = __builtin_amdgcn_rsq(q);
@@ -272,10 +283,11 @@ __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
     const double r = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, r, g);
     h = __builtin_fma(h, r, h);
-    double d = __builtin_fma(-g, g, q);
-    g = __builtin_fma(d, h, g);
-    d = __builtin_fma(-g, g, q);
-    g = __builtin_fma(d, h, g);
+#pragma unroll
+    for (int c = 0; c < CORRECTIONS; ++c) {
+        const double d = __builtin_fma(-g, g, q);
+        g = __builtin_fma(d, h, g);
+    }
 }
 
 __device__ __forceinline__ bool core_range(double q)
@@ -700,8 +712,8 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
     const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
     const double q0 = sq3<CLA>(ex, ey, ez);
     double l, l0, h0;
-    sqrt_core(qq, l, o.hl);
-    sqrt_core(q0, l0, h0);
+    sqrt_core<1>(qq, l, o.hl);
+    sqrt_core<1>(q0, l0, h0);
     o.sh = (l - l0) * h0;  // s/2, from h0 ~ 0.5/l0
     // k = (c_i + c_j)/2 for a field: s k/l V_j = (s/2)(0.5/l) w with
     // w = 2(c_i+c_j)V_j = c_i (2 V_j) + (2 c_j V_j), the staged pair
@@ -851,7 +863,9 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
 // 57 -> 48 on a 141k-node bar with corrections (requested with the chunk).
 // Tiles by bisection and a leaner prologue gave 257 us on the beam, 74.5 and
 // 46.4 on the other two; what a run's inner steps store for nobody (force, the
-// slot layout's u, Euler-Cromer's udd) left out, 250, 72 and 45.5.
+// slot layout's u, Euler-Cromer's udd) left out, 250, 72 and 45.5; tiles even
+// over the CUs 42.3 on the last, one correction of each square root less, 242,
+// 69 and 40.8.
 //
 // DM: DM_PMB, DM_NLIN or DM_FIELD.  One workgroup per tile, LPN lanes per
 // node taking its 4-bond chunks round-robin and reducing with cross-lane
@@ -1909,15 +1923,16 @@ __global__ void __launch_bounds__(256)
                   l.z == LOC_DEAD ? -1 : NEVER, l.w == LOC_DEAD ? -1 : NEVER);
 }
 
-// 1/sqrt(q) for q in [2^-767, 2^767]: the hardware estimate and two Newton
-// steps y <- y (3/2 - q y^2 / 2).
-__device__ __forceinline__ double rsqrt_newton(double q)
+// 1/sqrt(q) for q in [2^-767, 2^767]: the hardware estimate y and one step of
+// third order, y (1 + r/2 + 3/8 r^2) with r = 1 - q y^2, whose error is of the
+// order of e^3 = 2e-22 for an estimate good to e = 6e-8.  Over 4.3e9 random q
+// the relative error is at most 1.4e-16, 5.3e-17 in the mean square (two
+// Newton steps, of two instructions more: 2.4e-16 and 7.3e-17).
+__device__ __forceinline__ double rsqrt_cubic(double q)
 {
-    double y = __builtin_amdgcn_rsq(q);
-    const double hq = 0.5 * q;
-    y = y * __builtin_fma(-hq * y, y, 1.5);
-    y = y * __builtin_fma(-hq * y, y, 1.5);
-    return y;
+    const double y = __builtin_amdgcn_rsq(q);
+    const double r = __builtin_fma(-(q * y), y, 1.0);
+    return __builtin_fma(y, r * __builtin_fma(r, 0.375, 0.5), y);
 }
 
 // 1/l0 of every slot's bond, once per recording (inv: caller id -> internal
@@ -1955,7 +1970,7 @@ __global__ void __launch_bounds__(256)
             const double ez = r0[bj + 2] - z;
             v[q] = lv[q] == LOC_DEAD
                        ? 0.0
-                       : rsqrt_newton(sq3<true>(ex, ey, ez));
+                       : rsqrt_cubic(sq3<true>(ex, ey, ez));
         }
         double2 *o = reinterpret_cast<double2 *>(il0) + 2 * k;
         o[0] = make_double2(v[0], v[1]);
@@ -2009,7 +2024,8 @@ struct AdjArgs {
 // What bounds it: the chunks' streams (14 B a slot: loc0, brk, 1/l0) and the
 // latency of each, so they are requested two rounds ahead; the arithmetic is
 // contracted (43 issue slots per bond where the plain form took 59): 27.3 ->
-// 23.5 us on the 50,820-node bar, 3.2 TB/s of streams.
+// 23.5 us on the 50,820-node bar, and 19.6 with tiles even over the CUs and
+// 41 slots, 3.8 TB/s of streams.
 template <int LPN>
 __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
 {
@@ -2073,10 +2089,9 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
 #pragma unroll
         for (int d = 0; d < 3; ++d)
             w[d] = __builtin_fma(vm, muj[d], -(vj * mum[d]));
-        // 1/l from the reciprocal square root of the squared length, two
-        // Newton steps (relative error ~1e-16): no square root or division
-        // in the loop
-        const double il = rsqrt_newton(sq3<true>(dd[0], dd[1], dd[2]));
+        // 1/l from the reciprocal square root of the squared length: no
+        // square root or division in the loop
+        const double il = rsqrt_cubic(sq3<true>(dd[0], dd[1], dd[2]));
         const double psi = il0 - il;
         const double kk = cm + p3.y;  // (c_m + c_j)/2
         const double dw = __builtin_fma(
