@@ -144,6 +144,12 @@ constexpr int XCDS = 8;
 constexpr int LDS_CAP_PMB = 1280;
 constexpr int LDS_CAP_NLIN = 1152;
 constexpr unsigned LDS_BYTES = 81920;
+// The narrow form of a halo (scalar stiffness, which has no use for a
+// record's last double): piece 3 holds 8 bytes per entry, at half of the
+// others' offset, and 960 entries take 53,760 bytes, the most (in the LDS's
+// allocation steps of 1,280) that lets three workgroups share a CU.
+constexpr int LDS_CAP_NARROW = 960;
+constexpr unsigned LDS_BYTES_NARROW = 56u * LDS_CAP_NARROW;
 // Slots that loc, state and corr are longer than the tiles need: the step
 // kernel requests chunk rows up to two rounds ahead, at most 3 rounds of
 // tile_nodes * lanes_per_node <= 1024 chunks past a tile's last.
@@ -490,10 +496,11 @@ __device__ void compact_tile(const StepArgs &a, const TileInfo &ti,
 // the step kernel
 // ---------------------------------------------------------------------------
 
-template <int DM>
+template <int DM, bool NARROW = false>
 constexpr unsigned piece_bytes()
 {
-    return 16u * (DM == DM_NLIN ? LDS_CAP_NLIN : LDS_CAP_PMB);
+    return 16u * (NARROW ? LDS_CAP_NARROW
+                         : (DM == DM_NLIN ? LDS_CAP_NLIN : LDS_CAP_PMB));
 }
 
 // Where the halo begins in LDS: after the n-linear tables (two of MAX_TAB
@@ -523,10 +530,12 @@ __device__ __forceinline__ double sq3(double x, double y, double z)
 // SP pieces per thread in flight at once (a block of 512 threads needs one
 // pass).  Pieces past the last entry store that entry again: a condition
 // would move each load next to its store.
+template <bool NARROW = false>
 struct HaloLoads {
-    // passes of all threads over the entries: SP at once; a halo that needs
-    // at most FEW (a plate's) stages no more
-    static constexpr int SP = 10, FEW = 3;
+    // passes of all threads over the entries: SP at once (all of a narrow
+    // halo's in a block of 512); a halo that needs at most FEW (a plate's)
+    // stages no more
+    static constexpr int SP = NARROW ? 8 : 10, FEW = 3;
     unsigned hi[SP];
 
     // byte offsets into H: four times the entry
@@ -546,6 +555,15 @@ struct HaloLoads {
         });
     }
 
+    // this thread's piece of an entry, 4 e bytes of H in, into LDS
+    static __device__ __forceinline__ void put(char *D, unsigned x, v2d v)
+    {
+        if (NARROW && (threadIdx.x & 3u) == 3u)
+            *reinterpret_cast<double *>(D + 2u * x) = v.x;
+        else
+            *reinterpret_cast<v2d *>(D + 4u * x) = v;
+    }
+
     // passes [0, N), their indices in hi
     template <int N>
     __device__ __forceinline__ void pass(const char *R, unsigned last,
@@ -558,7 +576,7 @@ struct HaloLoads {
         });
         unsigned x = threadIdx.x & ~3u;
         static_for<N>([&](auto k) {
-            *reinterpret_cast<v2d *>(D + 4u * min(x, last)) = v[k];
+            put(D, min(x, last), v[k]);
             x += step();
         });
     }
@@ -573,7 +591,7 @@ struct HaloLoads {
         const unsigned last = 4u * (halo - 1u);
         const unsigned piece = threadIdx.x & 3u;
         const char *R = reinterpret_cast<const char *>(rec);
-        D += piece * PB + 16u;
+        D += piece * PB + (NARROW && piece == 3u ? 8u : 16u);
         if (SHORT && last < FEW * step()) {
             pass<FEW>(R, last, D);
             return;
@@ -591,7 +609,7 @@ struct HaloLoads {
                 y += step();
             });
             static_for<4>([&](auto k) {
-                *reinterpret_cast<v2d *>(D + 4u * min(x, last)) = v[k];
+                put(D, min(x, last), v[k]);
                 x += step();
             });
         }
@@ -600,14 +618,17 @@ struct HaloLoads {
 
 // Entry 0 of a staged halo, what dead and empty slots read: a far node of
 // weight 0 (CLA: records hold u, which is 0).  Threads 0-3.
-template <bool CLA>
+template <bool CLA, bool NARROW = false>
 __device__ __forceinline__ void far_entry(char *D, unsigned PB)
 {
     constexpr double FAR = 0x1p300;
     const unsigned t = threadIdx.x;
     const bool r = t < 2 || !CLA;
-    *reinterpret_cast<double2 *>(D + t * PB) =
-        make_double2(r ? FAR : 0.0, r && !(t & 1) ? FAR : 0.0);
+    const double2 v = make_double2(r ? FAR : 0.0, r && !(t & 1) ? FAR : 0.0);
+    if (NARROW && t == 3)
+        *reinterpret_cast<double *>(D + t * PB) = v.x;
+    else
+        *reinterpret_cast<double2 *>(D + t * PB) = v;
 }
 
 // v of the lane whose number differs in bit OFF (1, 2 or 4).  Inside a quad
@@ -675,14 +696,14 @@ struct Bond {
 //
 // A dead or empty slot (ev 0) needs no test here: entry 0 is a node at
 // (2^300, 2^300, 2^300) of weight 0, so that l == l0 and the force is zero.
-template <int DM, bool TENS, bool CLA>
+template <int DM, bool TENS, bool CLA, bool NARROW>
 __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
                                           const double4 &r0i,
                                           const double4 &ri, double ci,
                                           unsigned ev, unsigned st,
                                           Bond &o, double &kb, double &pb)
 {
-    constexpr unsigned PB = piece_bytes<DM>();
+    constexpr unsigned PB = piece_bytes<DM, NARROW>();
     const char *pe = ldsb + halo_base<DM>() + ev;
     const double2 p0 = *reinterpret_cast<const double2 *>(pe);
     const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
@@ -692,7 +713,8 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
     if (DM == DM_FIELD) {
         p3 = *reinterpret_cast<const double2 *>(pe + 3 * PB);
     } else {
-        p3.x = *reinterpret_cast<const double *>(pe + 3 * PB);
+        p3.x = *reinterpret_cast<const double *>(
+            NARROW ? ldsb + 3 * PB + (ev >> 1) : pe + 3 * PB);
         p3.y = 0.0;
     }
     const double ex = p0.x - r0i.x;
@@ -736,7 +758,7 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
 // (spatial.pyx:87-97, cl/peridynamics.cl:72-74): decides whether it breaks or
 // changes its regime, writes that, and leaves in `o` (and kb, pb for
 // DM_NLIN) what the force needs, zero for a broken or empty slot.
-template <int DM, bool TENS, bool CLA>
+template <int DM, bool TENS, bool CLA, bool NARROW>
 __device__ __forceinline__ void bond_exact(const StepArgs &a,
                                            const char *ldsb,
                                            const double4 &r0i, unsigned ev,
@@ -744,7 +766,7 @@ __device__ __forceinline__ void bond_exact(const StepArgs &a,
                                            double &kb, double &pb,
                                            int &nbroken)
 {
-    constexpr unsigned PB = piece_bytes<DM>();
+    constexpr unsigned PB = piece_bytes<DM, NARROW>();
     bool live = ev != LOC_DEAD;
     if (live) {
         const char *pe = ldsb + halo_base<DM>() + ev;
@@ -814,7 +836,7 @@ struct Chunk<false> {
 // their states, `cr` their corrections.  The two are straight-line code whose
 // chains interleave; only a bond near a threshold (or broken by this step)
 // leaves it.
-template <int DM, bool CORR, bool TENS, bool CLA>
+template <int DM, bool CORR, bool TENS, bool CLA, bool NARROW>
 __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
                                           const double4 &r0i,
                                           const double4 &ri, double ci,
@@ -826,17 +848,18 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
     double kb[2], pb[2];
     const unsigned ev[2] = {lw & 0xffffu, lw >> 16};
     const unsigned st[2] = {sw & 0xffffu, sw >> 16};
-    const bool ok0 = bond_fast<DM, TENS, CLA>(a, ldsb, r0i, ri, ci, ev[0],
-                                              st[0], o[0], kb[0], pb[0]);
-    const bool ok1 = bond_fast<DM, TENS, CLA>(a, ldsb, r0i, ri, ci, ev[1],
-                                              st[1], o[1], kb[1], pb[1]);
+    const bool ok0 = bond_fast<DM, TENS, CLA, NARROW>(
+        a, ldsb, r0i, ri, ci, ev[0], st[0], o[0], kb[0], pb[0]);
+    const bool ok1 = bond_fast<DM, TENS, CLA, NARROW>(
+        a, ldsb, r0i, ri, ci, ev[1], st[1], o[1], kb[1], pb[1]);
     if (__builtin_expect(!(ok0 & ok1), 0)) {
         if (!ok0)
-            bond_exact<DM, TENS, CLA>(a, ldsb, r0i, ev[0], st[0], s0, o[0],
-                                      kb[0], pb[0], nbroken);
+            bond_exact<DM, TENS, CLA, NARROW>(a, ldsb, r0i, ev[0], st[0], s0,
+                                              o[0], kb[0], pb[0], nbroken);
         if (!ok1)
-            bond_exact<DM, TENS, CLA>(a, ldsb, r0i, ev[1], st[1], s0 + 1,
-                                      o[1], kb[1], pb[1], nbroken);
+            bond_exact<DM, TENS, CLA, NARROW>(a, ldsb, r0i, ev[1], st[1],
+                                              s0 + 1, o[1], kb[1], pb[1],
+                                              nbroken);
     }
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -865,7 +888,7 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
 // 46.4 on the other two; what a run's inner steps store for nobody (force, the
 // slot layout's u, Euler-Cromer's udd) left out, 250, 72 and 45.5; tiles even
 // over the CUs 42.3 on the last, one correction of each square root less, 242,
-// 69 and 40.8.
+// 69 and 40.8; the narrow form 230 on the beam.
 //
 // DM: DM_PMB, DM_NLIN or DM_FIELD.  One workgroup per tile, LPN lanes per
 // node taking its 4-bond chunks round-robin and reducing with cross-lane
@@ -873,11 +896,19 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
 // damage-model tables, then the halo, four pieces of piece_bytes<DM>() each.
 // CLA: the slot layout's OpenCL arithmetic (records hold u, updates
 // contracted); otherwise the Cython path's (records hold r0 + u).
-template <int DM, int LPN, bool CORR, bool TENS, bool CLA>
-__global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
-                                               double fmag)
+// NARROW: the narrow halo form, blocks of at most 512, and registers for six
+// wavefronts per SIMD, that is three workgroups of 128 nodes per CU instead of
+// two; used where a CU gets more than two tiles (narrow_fits).  The
+// node's state is then read after the bonds: the registers that would hold it
+// are what six wavefronts lack, and there are others to run meanwhile.
+template <int DM, int LPN, bool CORR, bool TENS, bool CLA, bool NARROW>
+__global__ __launch_bounds__(NARROW ? 512 : 1024, NARROW ? 6 : 1) void k_step(
+    StepArgs a, double dmag, double fmag)
 {
-    __shared__ double2 lds[LDS_BYTES / sizeof(double2)];
+    static_assert(!NARROW || (DM == DM_PMB && CLA && !CORR),
+                  "no use of c_j, and no rows to compact in LDS");
+    __shared__ double2
+        lds[(NARROW ? LDS_BYTES_NARROW : LDS_BYTES) / sizeof(double2)];
     const int b = blockIdx.x;
     const int tile = (b % XCDS) * a.tiles_per_xcd + b / XCDS;
     if (tile >= a.ntiles)
@@ -891,8 +922,8 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
 
     // the halo's node indices first: the records they name are the longest
     // chain of this kernel
-    constexpr unsigned PB = piece_bytes<DM>();
-    HaloLoads hl;
+    constexpr unsigned PB = piece_bytes<DM, NARROW>();
+    HaloLoads<NARROW> hl;
     hl.request(a.halo + ti.halo_off, (unsigned)ti.halo);
 
     // node state and the first chunks of halo entries are requested before
@@ -938,7 +969,7 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
     // with 4 or more lanes per node, lane d < 3 updates component d: its
     // inputs are requested now too (the prescribed values, needed only on
     // flagged DOFs, are read at the update)
-    constexpr bool PRE = LPN >= 4;
+    constexpr bool PRE = LPN >= 4 && !NARROW;
     double pu = 0.0, pud = 0.0, pudd = 0.0, pdens = 1.0;
     if (PRE && valid && sub < 3) {
         const size_t k = 3 * (size_t)i + sub;
@@ -952,10 +983,10 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
         }
     }
 
-    hl.stage<DM != DM_NLIN>(a.rec_old, a.halo + ti.halo_off,
+    hl.template stage<DM != DM_NLIN>(a.rec_old, a.halo + ti.halo_off,
                             (unsigned)ti.halo, ldsb + halo_base<DM>(), PB);
     if (threadIdx.x < 4)
-        far_entry<CLA>(ldsb + halo_base<DM>(), PB);
+        far_entry<CLA, NARROW>(ldsb + halo_base<DM>(), PB);
     // n-linear tables, one 16-byte read each: (lower, upper) halved
     // thresholds of regime r of type t with their margin, and (4 stiffness,
     // 2 plus_cs)
@@ -994,12 +1025,13 @@ __global__ __launch_bounds__(1024) void k_step(StepArgs a, double dmag,
             ca = ch.ca;
             cb = ch.cb;
         }
-        bond_pair<DM, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, ch.loc.x,
-                                       ch.st.x, ca, s0, fx, fy, fz, nbroken);
+        bond_pair<DM, CORR, TENS, CLA, NARROW>(a, ldsb, r0i, ri, ci, ch.loc.x,
+                                               ch.st.x, ca, s0, fx, fy, fz,
+                                               nbroken);
         if (16 * (LPN * k / 4) + 8 < cmax)
-            bond_pair<DM, CORR, TENS, CLA>(a, ldsb, r0i, ri, ci, ch.loc.y,
-                                           ch.st.y, cb, s0 + 2, fx, fy, fz,
-                                           nbroken);
+            bond_pair<DM, CORR, TENS, CLA, NARROW>(
+                a, ldsb, r0i, ri, ci, ch.loc.y, ch.st.y, cb, s0 + 2, fx, fy,
+                fz, nbroken);
     };
     const int rounds = (chunks_of(cmax) + LPN - 1) / LPN;
     if (valid) {
@@ -1604,7 +1636,7 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
     const int l = threadIdx.x / LPN;
     const int sub = threadIdx.x % LPN;
     const bool valid = l < ti.nodes;
-    HaloLoads hl;
+    HaloLoads<> hl;
     hl.request(a.halo + ti.halo_off, (unsigned)ti.halo);
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     const long long c0 = ti.chunk_off + (valid ? l : 0);
@@ -1636,8 +1668,8 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         if (sub < 3)
             pu = a.u[3 * (size_t)i + sub];
     }
-    hl.stage<true>(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb,
-                   PB);
+    hl.template stage<true>(a.rec_old, a.halo + ti.halo_off,
+                            (unsigned)ti.halo, ldsb, PB);
     if (threadIdx.x < 4)
         far_entry<false>(ldsb, PB);
     __syncthreads();
@@ -2039,7 +2071,7 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     const int l = threadIdx.x / LPN;
     const int sub = threadIdx.x % LPN;
     const bool valid = l < ti.nodes;
-    HaloLoads hl;
+    HaloLoads<> hl;
     hl.request(a.halo + ti.halo_off, (unsigned)ti.halo);
     // chunk k's streams; chunk rows past the tile's last are not used, and
     // their loads stay at the row before it
@@ -2066,7 +2098,8 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     const NodeRec own = a.rec[i];
     const int cnt = valid ? a.cnt[i] : 0;
-    hl.stage<true>(a.rec, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb, PB);
+    hl.template stage<true>(a.rec, a.halo + ti.halo_off, (unsigned)ti.halo,
+                            ldsb, PB);
     if (threadIdx.x < 4)
         far_entry<true>(ldsb, PB);
     __syncthreads();
@@ -2478,6 +2511,18 @@ unsigned block_of(const pd_sim *s, int lanes)
     return ((unsigned)(s->tile_cap * lanes) + 63u) & ~63u;
 }
 
+// Whether tiles of at most `halo` halo entries run the narrow form at four
+// lanes per node: it takes blocks of at most 512, and pays where a CU has
+// more than two tiles to run (us a step, wide / narrow: 1,038,230-node beam
+// 245 / 230, 93,433-node plate 11.5 / 11.0, bars of three to five tiles per CU
+// the same within the noise; with two or fewer the wide form's early reads of
+// the node's state are worth more).
+bool narrow_fits(const pd_sim *s, int ntiles, int halo)
+{
+    return ntiles > 2 * s->cus && halo < LDS_CAP_NARROW &&
+           block_of(s, 4) <= 512;
+}
+
 template <int DM, int LPN, bool CLA>
 hipError_t launch_cla(pd_sim *s, const StepArgs &a, double dmag, double fmag)
 {
@@ -2485,19 +2530,32 @@ hipError_t launch_cla(pd_sim *s, const StepArgs &a, double dmag, double fmag)
     const unsigned block = block_of(s, LPN);
     // the n-linear model breaks by regimes, not by the sign mode
     const bool tens = DM != DM_NLIN && a.absmask == 0xffffffffu;
+    if constexpr (DM == DM_PMB && LPN == 4 && CLA) {
+        if (!a.has_corr && narrow_fits(s, s->ntiles, s->hstride)) {
+            if (tens)
+                hipLaunchKernelGGL((k_step<DM, LPN, false, true, CLA, true>),
+                                   dim3(grid), dim3(block), 0, s->stream, a,
+                                   dmag, fmag);
+            else
+                hipLaunchKernelGGL((k_step<DM, LPN, false, false, CLA, true>),
+                                   dim3(grid), dim3(block), 0, s->stream, a,
+                                   dmag, fmag);
+            return hipGetLastError();
+        }
+    }
     if (a.has_corr && tens)
-        hipLaunchKernelGGL((k_step<DM, LPN, true, DM != DM_NLIN, CLA>),
+        hipLaunchKernelGGL((k_step<DM, LPN, true, DM != DM_NLIN, CLA, false>),
                            dim3(grid), dim3(block), 0, s->stream, a, dmag,
                            fmag);
     else if (a.has_corr)
-        hipLaunchKernelGGL((k_step<DM, LPN, true, false, CLA>), dim3(grid),
+        hipLaunchKernelGGL((k_step<DM, LPN, true, false, CLA, false>), dim3(grid),
                            dim3(block), 0, s->stream, a, dmag, fmag);
     else if (tens)
-        hipLaunchKernelGGL((k_step<DM, LPN, false, DM != DM_NLIN, CLA>),
+        hipLaunchKernelGGL((k_step<DM, LPN, false, DM != DM_NLIN, CLA, false>),
                            dim3(grid), dim3(block), 0, s->stream, a, dmag,
                            fmag);
     else
-        hipLaunchKernelGGL((k_step<DM, LPN, false, false, CLA>), dim3(grid),
+        hipLaunchKernelGGL((k_step<DM, LPN, false, false, CLA, false>), dim3(grid),
                            dim3(block), 0, s->stream, a, dmag, fmag);
     return hipGetLastError();
 }
@@ -2514,11 +2572,11 @@ hipError_t launch_one(pd_sim *s, const StepArgs &a, double dmag, double fmag)
     if (DM != DM_PMB || a.has_corr)
         return hipErrorInvalidValue;  // rejected before launch
     if (a.absmask == 0xffffffffu)
-        hipLaunchKernelGGL((k_step<DM_PMB, LPN, false, true, false>),
+        hipLaunchKernelGGL((k_step<DM_PMB, LPN, false, true, false, false>),
                            dim3(grid), dim3(block), 0, s->stream, a, dmag,
                            fmag);
     else
-        hipLaunchKernelGGL((k_step<DM_PMB, LPN, false, false, false>),
+        hipLaunchKernelGGL((k_step<DM_PMB, LPN, false, false, false, false>),
                            dim3(grid), dim3(block), 0, s->stream, a, dmag,
                            fmag);
     return hipGetLastError();
@@ -3450,59 +3508,78 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     const int nblocks = (int)bstart.size();
     bstart.push_back(N);
     std::vector<std::vector<TileInfo>> cuts(nblocks);
-    std::atomic<int> wide{0};
-    run_parallel(nblocks, [&](int lo, int hi) {
-        std::vector<int> stamp(N, -1);
-        int tid = 0;
-        for (int bl = lo; bl < hi; ++bl) {
-            TileInfo t{};
-            t.node_off = bstart[bl];
-            ++tid;
-            for (int q = bstart[bl]; q < bstart[bl + 1]; ++q) {
-                const int i = tnode[q];
-                if (1 + cnt[i] > s->hmax) {
-                    wide = 1;
-                    return;
-                }
-                // the distinct nodes that i and its neighbours add (a row
-                // may list a neighbour more than once)
-                auto add = [&]() {
-                    int c = 0;
-                    auto visit = [&](int j) {
-                        c += stamp[j] != tid;
-                        stamp[j] = tid;
+    // each block cut into tiles whose halos hold at most `most` entries;
+    // their number, or -1 where a node's own neighbourhood does not fit
+    auto cut_blocks = [&](int most) {
+        std::atomic<int> wide{0}, count{0};
+        run_parallel(nblocks, [&](int lo, int hi) {
+            std::vector<int> stamp(N, -1);
+            int tid = 0;
+            for (int bl = lo; bl < hi; ++bl) {
+                cuts[bl].clear();
+                TileInfo t{};
+                t.node_off = bstart[bl];
+                ++tid;
+                for (int q = bstart[bl]; q < bstart[bl + 1]; ++q) {
+                    const int i = tnode[q];
+                    if (1 + cnt[i] > most) {
+                        wide = 1;
+                        return;
+                    }
+                    // the distinct nodes that i and its neighbours add (a
+                    // row may list a neighbour more than once)
+                    auto add = [&]() {
+                        int c = 0;
+                        auto visit = [&](int j) {
+                            c += stamp[j] != tid;
+                            stamp[j] = tid;
+                        };
+                        visit(i);
+                        for (long long r = rstart[i]; r < rstart[i + 1]; ++r)
+                            visit(rj[r]);
+                        return c;
                     };
-                    visit(i);
-                    for (long long r = rstart[i]; r < rstart[i + 1]; ++r)
-                        visit(rj[r]);
-                    return c;
-                };
-                int c = add();
-                if (t.nodes > 0 && t.halo + c > s->hmax) {
-                    cuts[bl].push_back(t);
-                    t = TileInfo{};
-                    t.node_off = q;
-                    ++tid;
-                    c = add();
+                    int c = add();
+                    if (t.nodes > 0 && t.halo + c > most) {
+                        cuts[bl].push_back(t);
+                        t = TileInfo{};
+                        t.node_off = q;
+                        ++tid;
+                        c = add();
+                    }
+                    t.halo += c;
+                    ++t.nodes;
                 }
-                t.halo += c;
-                ++t.nodes;
+                cuts[bl].push_back(t);
+                count += (int)cuts[bl].size();
             }
-            cuts[bl].push_back(t);
-            // within a tile, nodes by descending bond count: the nodes
-            // sharing a wavefront then run loops of nearly equal length
-            for (const auto &x : cuts[bl])
-                std::stable_sort(tnode.begin() + x.node_off,
-                                 tnode.begin() + x.node_off + x.nodes,
-                                 [&](int y, int z) { return cnt[y] > cnt[z]; });
-        }
-    }, 16);
-    if (wide)
+        }, 16);
+        return wide ? -1 : (int)count;
+    };
+    // the narrow form's capacity first, where the step may use it and it
+    // costs few more tiles (in 50 at most one: its gain is three times that)
+    int ncut = -1;
+    if (s->layout == PD_LAYOUT_SLOT && s->lanes == 4 && !nlin &&
+        dm_of(s) == DM_PMB && !s->has_corr && narrow_fits(s, nblocks, 0)) {
+        ncut = cut_blocks(LDS_CAP_NARROW - 1);
+        if (ncut > nblocks + nblocks / 50)
+            ncut = -1;
+    }
+    if (ncut < 0 && cut_blocks(s->hmax) < 0)
         return fail(PD_E_LIMIT, "a node's neighbourhood exceeds the "
                                 "LDS halo capacity");
     std::vector<TileInfo> tiles;
     for (const auto &c : cuts)
         tiles.insert(tiles.end(), c.begin(), c.end());
+    // within a tile, nodes by descending bond count: the nodes sharing a
+    // wavefront then run loops of nearly equal length
+    run_parallel((int)tiles.size(), [&](int lo, int hi) {
+        for (int t = lo; t < hi; ++t)
+            std::stable_sort(tnode.begin() + tiles[t].node_off,
+                             tnode.begin() + tiles[t].node_off +
+                                 tiles[t].nodes,
+                             [&](int y, int z) { return cnt[y] > cnt[z]; });
+    }, 16);
     std::vector<int> inv(N);  // caller's node id -> internal id
     for (int q = 0; q < N; ++q)
         inv[tnode[q]] = q;
