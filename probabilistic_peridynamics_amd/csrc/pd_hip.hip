@@ -174,7 +174,7 @@ struct TileInfo {
 constexpr int STORE_U = 1, STORE_F = 2;
 
 struct StepArgs {
-    int n, K, hstride, ntiles, tiles_per_xcd;
+    int K, ntiles, tiles_per_xcd;
     int integrator, layout, has_corr;
     unsigned absmask;  // 0x7fffffff: break on |s|; 0xffffffff: on s
     int nregimes, ntab;
@@ -200,8 +200,6 @@ struct StepArgs {
     const double *corr;
     unsigned short *state;
     const double *k_tab, *s_tab, *pc_tab;
-    const long long *chunk0;
-    const int *stride;
     unsigned short *rslot;  // compact layout: row position -> slot
     int *n_neigh;
     const double *cnode;  // node stiffness c (DM_FIELD)
@@ -876,9 +874,10 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
     }
 }
 
-// What bounds it: the VALU, busy ~75 % of the cycles on the 1,038,230-node
-// beam (1.16e8 wave instructions per launch before, mostly FP64 at 4 cycles
-// and more; the clock gives way under that load).  So the bond loop has one
+// What bounds it on large meshes: the VALU (busy 72 % of the cycles on the
+// 1,038,230-node beam in the wide form; 8.6e7 wave instructions per launch,
+// mostly FP64 at 4 cycles and more, where there were 1.16e8; the clock gives
+// way under that load) and the LDS (63 %).  So the bond loop has one
 // compare per bond for everything that is rare, dead slots cost no test, LDS
 // offsets come ready from loc, chunk loads step one 32-bit offset, and a row
 // runs half rounds: 305 -> 270 us a step there, 113 -> 77 on the 263k-node
@@ -892,8 +891,8 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
 //
 // DM: DM_PMB, DM_NLIN or DM_FIELD.  One workgroup per tile, LPN lanes per
 // node taking its 4-bond chunks round-robin and reducing with cross-lane
-// shuffles.  LDS (static, LDS_BYTES): for DM_NLIN the
-// damage-model tables, then the halo, four pieces of piece_bytes<DM>() each.
+// moves.  LDS (static): for DM_NLIN the damage-model tables, then the
+// halo, pieces of piece_bytes<DM, NARROW>() each.
 // CLA: the slot layout's OpenCL arithmetic (records hold u, updates
 // contracted); otherwise the Cython path's (records hold r0 + u).
 // NARROW: the narrow halo form, blocks of at most 512, and registers for six
@@ -1619,7 +1618,9 @@ __device__ __forceinline__ void window_sync()
 // 8-byte load per lane and round), div_core seeded from the square roots and
 // one interval test for everything rare, a bond takes 65 wave instructions
 // where it took 115: 150 -> 104 us a step on 270,000 nodes, 20.7 -> 14 on
-// the 2560-node bar.
+// the 2560-node bar.  Tiles by bisection and fewer stores 94 on the former;
+// small tiles and eight lanes 9.8 on the latter.  On large meshes the VALU is
+// busy 60 % of the cycles and the LDS (halo reads and windows) 66 %.
 template <int LPN>
 __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
                                                     double fmag)
@@ -1668,8 +1669,8 @@ __global__ __launch_bounds__(512) void k_exact_step(StepArgs a, double dmag,
         if (sub < 3)
             pu = a.u[3 * (size_t)i + sub];
     }
-    hl.template stage<true>(a.rec_old, a.halo + ti.halo_off,
-                            (unsigned)ti.halo, ldsb, PB);
+    hl.stage<true>(a.rec_old, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb,
+                   PB);
     if (threadIdx.x < 4)
         far_entry<false>(ldsb, PB);
     __syncthreads();
@@ -2098,8 +2099,7 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     const uint32_t i = (uint32_t)(ti.node_off + (valid ? l : 0));
     const NodeRec own = a.rec[i];
     const int cnt = valid ? a.cnt[i] : 0;
-    hl.template stage<true>(a.rec, a.halo + ti.halo_off, (unsigned)ti.halo,
-                            ldsb, PB);
+    hl.stage<true>(a.rec, a.halo + ti.halo_off, (unsigned)ti.halo, ldsb, PB);
     if (threadIdx.x < 4)
         far_entry<true>(ldsb, PB);
     __syncthreads();
@@ -2443,9 +2443,7 @@ int dm_of(const pd_sim *s)
 StepArgs make_args(pd_sim *s)
 {
     StepArgs a;
-    a.n = s->n;
     a.K = s->K;
-    a.hstride = s->hstride;
     a.ntiles = s->ntiles;
     a.tiles_per_xcd = (s->ntiles + XCDS - 1) / XCDS;
     a.integrator = s->integrator;
@@ -2485,8 +2483,6 @@ StepArgs make_args(pd_sim *s)
     a.k_tab = s->k_tab.p;
     a.s_tab = s->s_tab.p;
     a.pc_tab = s->pc_tab.p;
-    a.chunk0 = s->chunk0.p;
-    a.stride = s->stride.p;
     a.rslot = s->rslot.p;
     a.n_neigh = s->n_neigh.p;
     a.cnode = s->cnode.p;
