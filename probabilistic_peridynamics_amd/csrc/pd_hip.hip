@@ -694,11 +694,12 @@ struct Bond {
 //
 // A dead or empty slot (ev 0) needs no test here: entry 0 is a node at
 // (2^300, 2^300, 2^300) of weight 0, so that l == l0 and the force is zero.
+// lim: a.lim, or -1 where no bond of the node's may stand.
 template <int DM, bool TENS, bool CLA, bool NARROW>
 __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
                                           const double4 &r0i,
                                           const double4 &ri, double ci,
-                                          unsigned ev, unsigned st,
+                                          double lim, unsigned ev, unsigned st,
                                           Bond &o, double &kb, double &pb)
 {
     constexpr unsigned PB = piece_bytes<DM, NARROW>();
@@ -746,9 +747,9 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
         pb = k.y;
         return (o.sh < c.y) & (o.sh > c.x);
     } else if constexpr (TENS) {
-        return (o.sh < a.lim) & (o.sh > -0.25);
+        return (o.sh < lim) & (o.sh > -0.25);
     } else {
-        return fabs(o.sh) < a.lim;
+        return fabs(o.sh) < lim;
     }
 }
 
@@ -838,7 +839,8 @@ template <int DM, bool CORR, bool TENS, bool CLA, bool NARROW>
 __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
                                           const double4 &r0i,
                                           const double4 &ri, double ci,
-                                          unsigned lw, unsigned sw, double2 cr,
+                                          double lim, unsigned lw,
+                                          unsigned sw, double2 cr,
                                           size_t s0, double &fx, double &fy,
                                           double &fz, int &nbroken)
 {
@@ -847,9 +849,9 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
     const unsigned ev[2] = {lw & 0xffffu, lw >> 16};
     const unsigned st[2] = {sw & 0xffffu, sw >> 16};
     const bool ok0 = bond_fast<DM, TENS, CLA, NARROW>(
-        a, ldsb, r0i, ri, ci, ev[0], st[0], o[0], kb[0], pb[0]);
+        a, ldsb, r0i, ri, ci, lim, ev[0], st[0], o[0], kb[0], pb[0]);
     const bool ok1 = bond_fast<DM, TENS, CLA, NARROW>(
-        a, ldsb, r0i, ri, ci, ev[1], st[1], o[1], kb[1], pb[1]);
+        a, ldsb, r0i, ri, ci, lim, ev[1], st[1], o[1], kb[1], pb[1]);
     if (__builtin_expect(!(ok0 & ok1), 0)) {
         if (!ok0)
             bond_exact<DM, TENS, CLA, NARROW>(a, ldsb, r0i, ev[0], st[0], s0,
@@ -965,6 +967,10 @@ __global__ __launch_bounds__(NARROW ? 512 : 1024, NARROW ? 6 : 1) void k_step(
         fl = meta >> 16;
     }
     const double ci = DM == DM_FIELD && valid ? a.cnode[i] : 0.0;
+    // where c_i is not finite, 0 c_i of a dead slot is not 0: all of the
+    // node's bonds take bond_exact, which leaves dead ones out
+    const double lim =
+        DM == DM_FIELD && !(fabs(ci) < __builtin_inf()) ? -1.0 : a.lim;
     // with 4 or more lanes per node, lane d < 3 updates component d: its
     // inputs are requested now too (the prescribed values, needed only on
     // flagged DOFs, are read at the update)
@@ -1024,13 +1030,13 @@ __global__ __launch_bounds__(NARROW ? 512 : 1024, NARROW ? 6 : 1) void k_step(
             ca = ch.ca;
             cb = ch.cb;
         }
-        bond_pair<DM, CORR, TENS, CLA, NARROW>(a, ldsb, r0i, ri, ci, ch.loc.x,
-                                               ch.st.x, ca, s0, fx, fy, fz,
-                                               nbroken);
+        bond_pair<DM, CORR, TENS, CLA, NARROW>(
+            a, ldsb, r0i, ri, ci, lim, ch.loc.x, ch.st.x, ca, s0, fx, fy, fz,
+            nbroken);
         if (16 * (LPN * k / 4) + 8 < cmax)
             bond_pair<DM, CORR, TENS, CLA, NARROW>(
-                a, ldsb, r0i, ri, ci, ch.loc.y, ch.st.y, cb, s0 + 2, fx, fy,
-                fz, nbroken);
+                a, ldsb, r0i, ri, ci, lim, ch.loc.y, ch.st.y, cb, s0 + 2, fx,
+                fy, fz, nbroken);
     };
     const int rounds = (chunks_of(cmax) + LPN - 1) / LPN;
     if (valid) {
