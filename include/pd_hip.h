@@ -202,7 +202,7 @@ int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
  * by pd_step / pd_run (not pd_run_graph), then pd_adjoint_backward (any
  * number of times).  The recording keeps the step at which each bond broke
  * (the break mask is held fixed in the backward pass) and u of every step,
- * or, where that takes more than 16 times the memory of checkpoints every
+ * or, where that takes more than 32 times the memory of checkpoints every
  * checkpoint_every steps and of one segment between two, a 64th of the
  * device's or a quarter of what is free, u at those checkpoints: the backward
  * pass then replays each segment from its checkpoint with the step kernel

@@ -2550,15 +2550,17 @@ hipError_t launch_cla(pd_sim *s, const StepArgs &a, double dmag, double fmag)
                            dim3(grid), dim3(block), 0, s->stream, a, dmag,
                            fmag);
     else if (a.has_corr)
-        hipLaunchKernelGGL((k_step<DM, LPN, true, false, CLA, false>), dim3(grid),
-                           dim3(block), 0, s->stream, a, dmag, fmag);
+        hipLaunchKernelGGL((k_step<DM, LPN, true, false, CLA, false>),
+                           dim3(grid), dim3(block), 0, s->stream, a, dmag,
+                           fmag);
     else if (tens)
         hipLaunchKernelGGL((k_step<DM, LPN, false, DM != DM_NLIN, CLA, false>),
                            dim3(grid), dim3(block), 0, s->stream, a, dmag,
                            fmag);
     else
-        hipLaunchKernelGGL((k_step<DM, LPN, false, false, CLA, false>), dim3(grid),
-                           dim3(block), 0, s->stream, a, dmag, fmag);
+        hipLaunchKernelGGL((k_step<DM, LPN, false, false, CLA, false>),
+                           dim3(grid), dim3(block), 0, s->stream, a, dmag,
+                           fmag);
     return hipGetLastError();
 }
 
@@ -4255,8 +4257,9 @@ namespace {
 // pass then replays nothing (a third of it and of the forward pass together:
 // 200 steps and their gradient on 50,820 nodes 12.3 -> 8.8 ms).  At most
 // KEEP_TIMES the memory that the caller's checkpoint interval asks for, a
-// 64th of the device's and a quarter of what is free.
-constexpr size_t KEEP_TIMES = 16;
+// 64th of the device's and a quarter of what is free (2000 steps of 50,820
+// nodes with checkpoints every 100: 17 times, 2.4 GB).
+constexpr size_t KEEP_TIMES = 32;
 
 bool keep_all(pd_sim *s, int nsteps, size_t slots)
 {

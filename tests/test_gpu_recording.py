@@ -1,5 +1,5 @@
 """A recording that keeps u of every step and one that keeps checkpoints (more
-steps than 16 times its checkpoints and a segment) give bitwise the same
+steps than 32 times its checkpoints and a segment) give bitwise the same
 gradient and end state, with bonds breaking; a field or a launch shape that is
 set after the recording is the one that the backward pass replays or
 refuses."""
@@ -45,11 +45,11 @@ def _state(integ):
     return integ.write(None, None, None, None, None, None, None, None)
 
 
-@pytest.mark.parametrize("steps,every", [(1100, 32), (1300, 50)])
+@pytest.mark.parametrize("steps,every", [(4200, 64), (4705, 99)])
 def test_checkpoints_equal_every_step(steps, every):
     out = []
     for e in (every, steps):
-        assert (steps > 16 * (-(-steps // e) + e)) == (e == every)
+        assert (steps > 32 * (-(-steps // e) + e)) == (e == every)
         integ, _ = _make(2e-3)
         live = _state(integ)[7].sum()
         integ.adjoint_start(steps, checkpoint_every=e)
