@@ -78,11 +78,11 @@
 // rsq-Goldschmidt sequence that the compiler emits for sqrt(double), without
 // its range scaling (taken only for q outside [2^-767, inf), where the
 // library sqrt is called); the step in plain order takes it with one
-// residual correction instead of two (sqrt_core<1>).  Its by-product h ~ 0.5/sqrt(q) (relative error
-// ~5e-15) replaces the two divisions; a stretch within a relative 1e-10 of
-// any threshold it is compared with is recomputed with the IEEE division, so
-// every break and regime decision equals the one made with the correctly
-// rounded s.
+// residual correction instead of two (sqrt_core<1>).  Its by-product h ~
+// 0.5/sqrt(q) (relative error ~5e-15) replaces the two divisions; a stretch
+// within a relative 1e-10 (and 2^-49) of any threshold it is compared with is
+// recomputed with the library's square roots and the IEEE division, so every
+// break and regime decision equals the one made with the correctly rounded s.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -133,6 +133,8 @@ constexpr uint32_t KEYM = 0x3FFFFFFFu;
 constexpr unsigned short LOC_DEAD = 0;  // loc of a broken or empty slot
 constexpr int MAX_NODES = 1 << 26;
 constexpr double GUARD = 1e-10;
+// and of s/2 itself, above what a root that is an ulp off does to it
+constexpr double GUARD_ABS = 0x1p-50;
 constexpr int MAX_TAB = 256;  // nbond_types * nregimes
 constexpr int MAX_LPN = 8;
 constexpr int XCDS = 8;
@@ -668,10 +670,10 @@ struct Bond {
     double dx, dy, dz, sh, hl, w;
 };
 
-// The model's halved thresholds with a margin of GUARD: a stretch strictly
-// inside (lo, hi) is away from every threshold and from lengths at which
-// sqrt_core is not exact, so the bond neither breaks nor changes its regime.
-// Anything else, NaN included, goes through bond_exact.
+// The model's halved thresholds with margins of GUARD (relative) and
+// GUARD_ABS: a stretch strictly inside (lo, hi) is away from every threshold
+// and from lengths outside sqrt_core's range, so the bond neither breaks nor
+// changes its regime.  Anything else, NaN included, goes through bond_exact.
 //
 // Why the lengths need no test of their own: coordinates are zero or in
 // [2^-290, 2^300] (else the host sets hi so that every bond takes the exact
@@ -1003,10 +1005,11 @@ __global__ __launch_bounds__(NARROW ? 512 : 1024, NARROW ? 6 : 1) void k_step(
             double lo = -0.25;
             if (t % a.nregimes != 0) {
                 const double c = a.s_tab[t - 1] * 0.5;
-                lo = fmax(lo, c + GUARD * fabs(c));
+                lo = fmax(lo, c + (GUARD * fabs(c) + GUARD_ABS));
             }
             tsp[t] = make_double2(
-                lo, a.lim > 0.0 ? up - GUARD * fabs(up) : -__DBL_MAX__);
+                lo, a.lim > 0.0 ? up - (GUARD * fabs(up) + GUARD_ABS)
+                                : -__DBL_MAX__);
             tkp[t] = make_double2(4.0 * a.k_tab[t], 2.0 * a.pc_tab[t]);
         }
     }
@@ -2465,7 +2468,8 @@ StepArgs make_args(pd_sim *s)
     // takes the exact path
     a.lim = !s->coords_core ? -1.0
             : dm_of(s) == DM_NLIN ? 1.0
-                                  : std::min(a.s0h * (1.0 - GUARD), 0.25);
+                                  : std::min(a.s0h * (1.0 - GUARD) - GUARD_ABS,
+                                             0.25);
     a.rec_old = s->rec[s->cur].p;
     a.rec_new = s->rec[1 - s->cur].p;
     a.tiles = s->tiles.p;
