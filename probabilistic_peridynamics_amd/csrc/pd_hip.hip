@@ -758,13 +758,14 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
 // The bond at slot `slot` with IEEE square roots and division
 // (spatial.pyx:87-97, cl/peridynamics.cl:72-74): decides whether it breaks or
 // changes its regime, writes that, and leaves in `o` (and kb, pb for
-// DM_NLIN) what the force needs, zero for a broken or empty slot.
+// DM_NLIN) what the force needs, zero for a broken or empty slot, whose
+// correction `cr` becomes zero too (it may be infinite or NaN).
 template <int DM, bool TENS, bool CLA, bool NARROW>
 __device__ __forceinline__ void bond_exact(const StepArgs &a,
                                            const char *ldsb,
                                            const double4 &r0i, unsigned ev,
                                            unsigned st, size_t slot, Bond &o,
-                                           double &kb, double &pb,
+                                           double &kb, double &pb, double &cr,
                                            int &nbroken)
 {
     constexpr unsigned PB = piece_bytes<DM, NARROW>();
@@ -816,7 +817,7 @@ __device__ __forceinline__ void bond_exact(const StepArgs &a,
     if (!live) {
         // a displacement that is not finite must not reach the sum either
         o.dx = o.dy = o.dz = o.sh = o.hl = o.w = 0.0;
-        kb = pb = 0.0;
+        kb = pb = cr = 0.0;
     }
 }
 
@@ -847,7 +848,7 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
                                           double &fz, int &nbroken)
 {
     Bond o[2];
-    double kb[2], pb[2];
+    double kb[2], pb[2], c[2] = {cr.x, cr.y};
     const unsigned ev[2] = {lw & 0xffffu, lw >> 16};
     const unsigned st[2] = {sw & 0xffffu, sw >> 16};
     const bool ok0 = bond_fast<DM, TENS, CLA, NARROW>(
@@ -857,11 +858,12 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
     if (__builtin_expect(!(ok0 & ok1), 0)) {
         if (!ok0)
             bond_exact<DM, TENS, CLA, NARROW>(a, ldsb, r0i, ev[0], st[0], s0,
-                                              o[0], kb[0], pb[0], nbroken);
+                                              o[0], kb[0], pb[0], c[0],
+                                              nbroken);
         if (!ok1)
             bond_exact<DM, TENS, CLA, NARROW>(a, ldsb, r0i, ev[1], st[1],
                                               s0 + 1, o[1], kb[1], pb[1],
-                                              nbroken);
+                                              c[1], nbroken);
     }
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -871,7 +873,7 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
                                  : o[q].sh;
         g = g * o[q].hl * o[q].w;
         if (CORR)
-            g *= q ? cr.y : cr.x;
+            g *= c[q];
         fx = __builtin_fma(g, o[q].dx, fx);
         fy = __builtin_fma(g, o[q].dy, fy);
         fz = __builtin_fma(g, o[q].dz, fz);
@@ -2267,6 +2269,7 @@ struct pd_sim {
     int ntiles = 0;
     size_t nslots = 0;  // bond slots of the tiles (loc holds LOC_SLACK more)
     bool coords_core = false;  // coordinates in bond_fast's range
+    bool odd_corr = false;     // some bond's correction is not finite
     bool retile_pending = false;  // tile_nodes changed since the tiling
     bool has_buffers = false, has_corr = false, has_btypes = false,
          has_cnode = false;
@@ -2464,9 +2467,10 @@ StepArgs make_args(pd_sim *s)
     a.dt = s->dt;
     a.damping = s->damping;
     a.s0h = s->s0 * 0.5;
-    // coordinates outside the range that bond_fast relies on: every bond
+    // coordinates outside the range that bond_fast relies on, or corrections
+    // whose product with a dead slot's zero force is not zero: every bond
     // takes the exact path
-    a.lim = !s->coords_core ? -1.0
+    a.lim = !s->coords_core || s->odd_corr ? -1.0
             : dm_of(s) == DM_NLIN ? 1.0
                                   : std::min(a.s0h * (1.0 - GUARD) - GUARD_ABS,
                                              0.25);
@@ -3627,7 +3631,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     const bool compact = s->layout == PD_LAYOUT_COMPACT;
     std::vector<int> nlow_h(compact ? N : 0);
     std::vector<long long> tile0_h(compact ? N : 0);
-    std::atomic<int> halo_mismatch{0};
+    std::atomic<int> halo_mismatch{0}, odd{0};
     run_parallel(ntiles, [&](int lo, int hi) {
         std::vector<int> lmap(N, -1);  // internal id -> halo position
         std::vector<int> hl;
@@ -3681,8 +3685,11 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
                     gidx[sl] = j;
                     pos[sl] = (unsigned short)p;
                     const size_t src = (size_t)i * K + p;
-                    if (s->has_corr)
+                    if (s->has_corr) {
                         corr[sl] = s->h_corr[src];
+                        if (!std::isfinite(corr[sl]))
+                            odd = 1;
+                    }
                     if (nlin)
                         state[sl] = (unsigned short)(
                             16 * (s->h_btypes[src] * nregimes +
@@ -3718,6 +3725,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     };
     s->ntiles = ntiles;
     s->nslots = S;
+    s->odd_corr = odd != 0;
     s->hstride = 1;
     for (const auto &t : tiles)
         s->hstride = std::max(s->hstride, t.halo);

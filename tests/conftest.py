@@ -25,3 +25,15 @@ def pytest_configure(config):
 @pytest.fixture(scope="session")
 def golden():
     return TESTS / "golden"
+
+
+@pytest.fixture(scope="session")
+def hip_device():
+    """Fails a GPU test where there is no device, instead of skipping it."""
+    from probabilistic_peridynamics_amd import _lib
+    try:
+        ok = _lib.device_count() > 0
+    except OSError:
+        ok = False
+    if not ok:
+        pytest.fail("no HIP device: the gpu tests need an MI355X")

@@ -1,0 +1,77 @@
+"""Broken and empty slots add nothing, whatever the correction, the damage
+tables or the node's own values hold: infinities and NaN reach only live
+bonds."""
+import numpy as np
+import pytest
+
+import oracle
+import pdcases as pc
+from probabilistic_peridynamics_amd import configs
+from probabilistic_peridynamics_amd import integrators as it
+
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("hip_device")]
+
+RTOL = 1e-10  # u against the oracle, relative L2; forces 1e-9
+BAD = [np.inf, -np.inf, np.nan]
+
+
+def _arrays(integ):
+    return integ.write(None, None, None, None, None, None, None, None)
+
+
+def _oracle_parity(integ, ref, steps):
+    d, f = 1e-8 * np.arange(1, steps + 1), np.linspace(0.5, 2, steps)
+    integ.run(steps, d, f)
+    for s in range(steps):
+        ref(d[s], f[s])
+    u, _, _, force, _, _, nl, _ = _arrays(integ)
+    assert np.all(np.isfinite(ref.force)) and np.any(ref.force != 0.0)
+    np.testing.assert_array_equal(nl, ref.nlist)
+    assert pc.rel_l2(u, ref.u) < RTOL
+    assert pc.rel_l2(force, ref.force) < 10 * RTOL
+
+
+@pytest.mark.parametrize("bad", BAD)
+@pytest.mark.parametrize("model", ["scalar", "tension", "field", "nlin"])
+def test_corrections_of_broken_bonds(model, bad):
+    """Every bond that breaks in the first step carries one that is not
+    finite."""
+    nlin, tension = model == "nlin", model == "tension"
+    w = (configs.composite_ec if nlin else configs.beam_vv)(shape=(13, 6, 5))
+    n, k = w.nlist.shape
+    rng = np.random.default_rng(6)
+    u = rng.normal(scale=(4e-3 if nlin else 2e-3) * w.extra["dx"],
+                   size=(n, 3))
+    corr = rng.uniform(0.5, 2.0, (n, k))
+    field = w.bond_stiffness * rng.uniform(0.5, 2, n) if model == "field" \
+        else None
+    # the n-linear bonds start in their last regime, so that some break at once
+    reg = np.full((n, k), 2, np.int32) if nlin else None
+    dens, bt = (w.densities, w.bond_types) if nlin else (None, None)
+
+    def reference():
+        return oracle.SlotStepper(
+            1 if nlin else 0, 1e-8 if nlin else 2e-15, w.coords, w.volume,
+            w.family, w.bc_types, w.bc_values, w.force_bc_types,
+            w.force_bc_values, w.nlist, w.bond_stiffness, w.critical_stretch,
+            damping=2.5e6 if nlin else 0.0, densities=dens,
+            stiffness_corrections=corr, bond_types=bt, regimes=reg,
+            plus_cs=w.plus_cs, nregimes=w.nregimes, cnode=field,
+            tension_only=tension, u=u)
+
+    first = reference()
+    first(1e-8, 0.5)
+    gone = (w.nlist >= 0) & (first.nlist < 0)
+    assert gone.sum() > 100
+    corr[gone] = bad
+    integ = (it.EulerCromerHIP(2.5e6, 1e-8) if nlin else it.EulerHIP(2e-15))
+    integ.build(n, 3, k, w.coords, w.volume, w.family, w.bc_types,
+                w.bc_values, w.force_bc_types, w.force_bc_values, corr, bt,
+                dens)
+    integ.set_node_stiffness(field)
+    integ.set_break_mode(tension)
+    for _ in range(2):  # as set up, and restarted on the same bonds
+        integ.create_buffers(w.nlist, w.n_neigh, w.bond_stiffness,
+                             w.critical_stretch, w.plus_cs, u, None, None,
+                             None, None, None, reg, w.nregimes, w.nbond_types)
+        _oracle_parity(integ, reference(), 4)
