@@ -2270,6 +2270,7 @@ struct pd_sim {
     size_t nslots = 0;  // bond slots of the tiles (loc holds LOC_SLACK more)
     bool coords_core = false;  // coordinates in bond_fast's range
     bool odd_corr = false;     // some bond's correction is not finite
+    bool odd_tables = false;   // set_tables
     bool retile_pending = false;  // tile_nodes changed since the tiling
     bool has_buffers = false, has_corr = false, has_btypes = false,
          has_cnode = false;
@@ -2468,9 +2469,9 @@ StepArgs make_args(pd_sim *s)
     a.damping = s->damping;
     a.s0h = s->s0 * 0.5;
     // coordinates outside the range that bond_fast relies on, or corrections
-    // whose product with a dead slot's zero force is not zero: every bond
-    // takes the exact path
-    a.lim = !s->coords_core || s->odd_corr ? -1.0
+    // or table values whose product with a dead slot's zeros is not zero:
+    // every bond takes the exact path
+    a.lim = !s->coords_core || s->odd_corr || s->odd_tables ? -1.0
             : dm_of(s) == DM_NLIN ? 1.0
                                   : std::min(a.s0h * (1.0 - GUARD) - GUARD_ABS,
                                              0.25);
@@ -2935,6 +2936,23 @@ void keep_plan(pd_sim *s, const int *nlist, const int *n_neigh, bool nlin,
     s->plan = true;
 }
 
+// The n-linear model's tables.  Values that are infinite or NaN, or become so
+// in the step's scaled form, are noted: a padding slot names row 0 of the
+// tables, whether or not a bond is of that type.
+hipError_t set_tables(pd_sim *s, const double *k, const double *crit,
+                      const double *pc)
+{
+    const size_t T = (size_t)s->nregimes * s->nbond_types;
+    s->odd_tables = false;
+    for (size_t t = 0; t < T; ++t)
+        s->odd_tables |= !std::isfinite(4.0 * k[t]) ||
+                         !std::isfinite(2.0 * pc[t]);
+    hipError_t e = upload(s->k_tab, k, T);
+    if (e == hipSuccess)
+        e = upload(s->s_tab, crit, T);
+    return e == hipSuccess ? upload(s->pc_tab, pc, T) : e;
+}
+
 // Whether the tiles and slots made by the last pd_create_buffers serve these
 // arguments too: the same bonds, launch shape and damage-model tables' shape
 // (node arrays, corrections, bond types and groups cannot have changed).
@@ -2973,10 +2991,7 @@ int restart(pd_sim *s, const double *bond_stiffness,
         HIPCHK(hipGetLastError());
     }
     if (s->plan_nlin) {
-        const size_t T = (size_t)s->nregimes * s->nbond_types;
-        HIPCHK(upload(s->k_tab, bond_stiffness, T));
-        HIPCHK(upload(s->s_tab, critical_stretch, T));
-        HIPCHK(upload(s->pc_tab, plus_cs, T));
+        HIPCHK(set_tables(s, bond_stiffness, critical_stretch, plus_cs));
     } else {
         s->k = bond_stiffness[0];
         s->s0 = critical_stretch[0];
@@ -3835,11 +3850,10 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         "nlist export");
     s->nregimes = nregimes;
     s->nbond_types = nbond_types;
+    s->odd_tables = false;
     if (nlin) {
-        const size_t T = (size_t)nregimes * nbond_types;
-        chk(upload(s->k_tab, bond_stiffness, T), "bond_stiffness");
-        chk(upload(s->s_tab, critical_stretch, T), "critical_stretch");
-        chk(upload(s->pc_tab, plus_cs, T), "plus_cs");
+        chk(set_tables(s, bond_stiffness, critical_stretch, plus_cs),
+            "damage model tables");
         s->k = 0.0;
         s->s0 = 0.0;
     } else {

@@ -75,3 +75,36 @@ def test_corrections_of_broken_bonds(model, bad):
                              w.critical_stretch, w.plus_cs, u, None, None,
                              None, None, None, reg, w.nregimes, w.nbond_types)
         _oracle_parity(integ, reference(), 4)
+
+
+@pytest.mark.parametrize("bad", BAD)
+@pytest.mark.parametrize("where", ["bond_stiffness", "plus_cs"])
+@pytest.mark.parametrize("given", ["at set-up", "at a restart"])
+def test_damage_tables_of_unused_types(given, where, bad):
+    """Type 0, whose row of the tables padding slots name, has no bond."""
+    w = configs.composite_ec(shape=(13, 6, 5))
+    n, k = w.nlist.shape
+    bt = np.where(w.nlist >= 0, w.bond_types + 1, 0).astype(np.int32)
+    tables = {name: np.vstack([t[:1], t]) for name, t in (
+        ("bond_stiffness", w.bond_stiffness), ("plus_cs", w.plus_cs),
+        ("critical_stretch", w.critical_stretch))}
+    u = np.random.default_rng(6).normal(scale=2e-3 * w.extra["dx"],
+                                        size=(n, 3))
+    integ = it.EulerCromerHIP(2.5e6, 1e-8)
+    integ.build(n, 3, k, w.coords, w.volume, w.family, w.bc_types,
+                w.bc_values, w.force_bc_types, w.force_bc_values, None, bt,
+                w.densities)
+    for finite in ([True, False, True] if given == "at a restart"
+                   else [False]):
+        t = {name: a.copy() for name, a in tables.items()}
+        if not finite:
+            t[where][0] = bad
+        integ.create_buffers(w.nlist, w.n_neigh, t["bond_stiffness"],
+                             t["critical_stretch"], t["plus_cs"], u, None,
+                             None, None, None, None, None, 3, 4)
+        ref = oracle.SlotStepper(
+            1, 1e-8, w.coords, w.volume, w.family, w.bc_types, w.bc_values,
+            w.force_bc_types, w.force_bc_values, w.nlist, t["bond_stiffness"],
+            t["critical_stretch"], damping=2.5e6, densities=w.densities,
+            bond_types=bt, plus_cs=t["plus_cs"], nregimes=3, u=u)
+        _oracle_parity(integ, ref, 6)
