@@ -2063,7 +2063,9 @@ struct AdjArgs {
 // of a node reads its neighbour from there.  LPN lanes per node take its
 // 4-bond chunks round-robin; a slot is live in step n if it broke at a step
 // > n (brk, -1 where it held no bond at the start of the recording), and
-// reads the far entry 0, whose terms are zero, otherwise.
+// reads the far entry 0, whose terms are zero, otherwise.  They are zero as
+// products with 0, so a node whose own values are infinite, NaN or so large
+// that they become infinite here skips its dead slots in a loop of its own.
 //
 // What bounds it: the chunks' streams (14 B a slot: loc0, brk, 1/l0) and the
 // latency of each, so they are requested two rounds ahead; the arithmetic is
@@ -2120,7 +2122,14 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     const double vm = own.a.w, cm = own.b.w;
     double jt[3] = {0.0, 0.0, 0.0};
     double gc = 0.0;
-    auto bond = [&](unsigned ev, int brk, double il0) {
+    // with r below half of the far entry's coordinate a dead slot's 1/l is at
+    // most 2^-299; 1/l0 is at most 2^537
+    bool plain = fabs(cm) < 0x1p400 && fabs(vm) < __builtin_inf();
+    for (int d = 0; d < 3; ++d)
+        plain &= fabs(rm[d]) < 0x1p299 && fabs(mum[d]) < __builtin_inf();
+    auto bond = [&](auto skip, unsigned ev, int brk, double il0) {
+        if (skip && brk <= a.step)
+            return;
         const char *pe = ldsb + (brk > a.step ? ev : (unsigned)LOC_DEAD);
         const double2 p0 = *reinterpret_cast<const double2 *>(pe);
         const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
@@ -2149,26 +2158,29 @@ __global__ __launch_bounds__(1024) void k_adj_tile(AdjArgs a)
     };
     // rounds as in k_step
     const int cmax = __builtin_amdgcn_readfirstlane(cnt);
-    auto round = [&](const Stream &v, int k) {
+    auto round = [&](auto skip, const Stream &v, int k) {
         if (sub + LPN * k > last)
             return;
-        bond(v.loc.x & 0xffffu, v.brk.x, v.ia.x);
-        bond(v.loc.x >> 16, v.brk.y, v.ia.y);
+        bond(skip, v.loc.x & 0xffffu, v.brk.x, v.ia.x);
+        bond(skip, v.loc.x >> 16, v.brk.y, v.ia.y);
         if (16 * (LPN * k / 4) + 8 < cmax) {
-            bond(v.loc.y & 0xffffu, v.brk.z, v.ib.x);
-            bond(v.loc.y >> 16, v.brk.w, v.ib.y);
+            bond(skip, v.loc.y & 0xffffu, v.brk.z, v.ib.x);
+            bond(skip, v.loc.y >> 16, v.brk.w, v.ib.y);
         }
     };
     const int rounds = (chunks_of(cmax) + LPN - 1) / LPN;
-    if (valid) {
+    if (valid && plain) {
         for (int k = 0; k < rounds; k += 2) {
-            round(qa, k);
+            round(std::false_type{}, qa, k);
             qa = stream_at(sub + LPN * (k + 2));
             if (k + 1 >= rounds)
                 break;
-            round(qb, k + 1);
+            round(std::false_type{}, qb, k + 1);
             qb = stream_at(sub + LPN * (k + 3));
         }
+    } else if (valid) {
+        for (int k = 0; k < rounds; ++k)
+            round(std::true_type{}, stream_at(sub + LPN * k), k);
     }
     gc *= -0.5;
     jt[0] = node_sum<LPN>(jt[0]);

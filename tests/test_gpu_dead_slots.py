@@ -108,3 +108,49 @@ def test_damage_tables_of_unused_types(given, where, bad):
             t["critical_stretch"], damping=2.5e6, densities=w.densities,
             bond_types=bt, plus_cs=t["plus_cs"], nregimes=3, u=u)
         _oracle_parity(integ, ref, 6)
+
+
+def _gradient(w, u, dL, c=None, volume=None, nlist=None, lanes=4, coords=None):
+    """dL/dc after six recorded steps, and the arrays they leave."""
+    n, k = w.nlist.shape
+    nl = w.nlist if nlist is None else nlist
+    integ = it.EulerHIP(2e-15)
+    integ.build(n, 3, k, w.coords if coords is None else coords,
+                w.volume if volume is None else volume, w.family,
+                np.zeros_like(w.bc_types), w.bc_values, w.force_bc_types,
+                w.force_bc_values, None, None, None)
+    integ.set_launch(lanes, 128)
+    integ.set_node_stiffness(c)
+    integ.create_buffers(nl, (nl >= 0).sum(axis=1).astype(np.int32),
+                         w.bond_stiffness, w.critical_stretch, None, u, None,
+                         None, None, None, None, None, 1, 1)
+    integ.adjoint_start(6, checkpoint_every=6)
+    integ.run(6, np.zeros(6), np.ones(6))
+    return integ.adjoint_backward(dL), _arrays(integ)
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+@pytest.mark.parametrize("what", ["c", "dL_du", "u", "volume"])
+def test_gradient_of_nodes_without_bonds(what, lanes):
+    """Their own values reach neither their own gradient nor a neighbour's."""
+    w = configs.beam_vv(shape=(13, 6, 5))
+    n = w.nnodes
+    alone = np.array([3, 140, n - 1])
+    nl = np.where(np.isin(w.nlist, alone), -1, w.nlist)
+    nl[alone] = -1
+    rng = np.random.default_rng(6)
+    args = dict(u=rng.normal(scale=2e-3 * w.extra["dx"], size=(n, 3)),
+                dL_du=rng.normal(size=(n, 3)), volume=w.volume,
+                c=w.bond_stiffness * rng.uniform(0.5, 2, n))
+    grads = []
+    for value in [1.0] + BAD:
+        a = {name: v.copy() for name, v in args.items()}
+        a[what][alone] = value
+        g, end = _gradient(w, a["u"], a["dL_du"], a["c"], a["volume"], nl,
+                           lanes)
+        assert end[7].sum() < (nl >= 0).sum()  # bonds break on the way
+        grads.append(g)
+    assert np.all(np.isfinite(grads[0])) and np.any(grads[0] != 0.0)
+    assert np.all(grads[0][alone] == 0.0)
+    for g in grads[1:]:
+        np.testing.assert_array_equal(g, grads[0])
