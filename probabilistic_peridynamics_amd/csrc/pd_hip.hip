@@ -1984,7 +1984,10 @@ __device__ __forceinline__ double rsqrt_cubic(double q)
 // of the same squared length as the backward kernel's 1/l, so that a bond
 // with l == l0 (bitwise, e.g. both ends at rest) gets 1/l0 - 1/l = 0 exactly,
 // as its stretch is 0 in the forward step: a one-ulp difference there, times
-// k dt, is not small.  Bound by the neighbours' coordinates (four scattered
+// k dt, is not small.  A squared length that is 0, infinite or NaN has no
+// reciprocal root; the forward step breaks such a bond before its first force,
+// and 0 takes the place of 1/l0, which a dead slot multiplies by its zeros.
+// Bound by the neighbours' coordinates (four scattered
 // reads per bond): 105 us on the 50,820-node bar with one lane per node, 61
 // with 4 lanes, 50 with 16.
 __global__ void __launch_bounds__(256)
@@ -2012,9 +2015,10 @@ __global__ void __launch_bounds__(256)
             const double ex = r0[bj] - x;
             const double ey = r0[bj + 1] - y;
             const double ez = r0[bj + 2] - z;
-            v[q] = lv[q] == LOC_DEAD
-                       ? 0.0
-                       : rsqrt_cubic(sq3<true>(ex, ey, ez));
+            const double q0 = sq3<true>(ex, ey, ez);
+            v[q] = lv[q] != LOC_DEAD && q0 > 0.0 && q0 < __builtin_inf()
+                       ? rsqrt_cubic(q0)
+                       : 0.0;
         }
         double2 *o = reinterpret_cast<double2 *>(il0) + 2 * k;
         o[0] = make_double2(v[0], v[1]);

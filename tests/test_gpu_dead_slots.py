@@ -154,3 +154,28 @@ def test_gradient_of_nodes_without_bonds(what, lanes):
     assert np.all(grads[0][alone] == 0.0)
     for g in grads[1:]:
         np.testing.assert_array_equal(g, grads[0])
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+def test_gradient_with_a_bond_of_no_length(lanes):
+    """Its stretch is NaN or infinite, so the first step breaks it: the
+    gradient is that of the body without it."""
+    w = configs.beam_vv(shape=(13, 6, 5))
+    n = w.nnodes
+    i = 140
+    j = int(w.nlist[i, 5])
+    coords = w.coords.copy()
+    coords[j] = coords[i]
+    without = w.nlist.copy()
+    for a, b in ((i, j), (j, i)):
+        without[a][without[a] == b] = -1
+    rng = np.random.default_rng(6)
+    u = rng.normal(scale=1e-3 * w.extra["dx"], size=(n, 3))
+    dL = rng.normal(size=(n, 3))
+    c = w.bond_stiffness * rng.uniform(0.5, 2, n)
+    got, end = _gradient(w, u, dL, c, lanes=lanes, coords=coords)
+    want, end2 = _gradient(w, u, dL, c, nlist=without, lanes=lanes,
+                           coords=coords)
+    np.testing.assert_array_equal(end[6], end2[6])
+    assert np.all(np.isfinite(want)) and np.any(want != 0.0)
+    assert pc.rel_l2(got, want) < RTOL
