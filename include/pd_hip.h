@@ -179,7 +179,9 @@ int pd_step(pd_sim *sim, double displacement_bc_magnitude,
             double force_bc_magnitude);
 
 /* nsteps calls of pd_step with magnitudes disp_mags[s], force_mags[s]
- * (either may be NULL for zeros). */
+ * (either may be NULL for zeros).  A run that fails after its first step
+ * leaves no whole state (u and the forces are stored by its last step):
+ * reading or stepping on is PD_E_STATE until pd_create_buffers. */
 int pd_run(pd_sim *sim, int nsteps, const double *disp_mags,
            const double *force_mags);
 
@@ -191,8 +193,10 @@ int pd_run_timed(pd_sim *sim, int nsteps, const double *disp_mags,
 
 /* pd_run captured as hipGraphs of a few steps, the device running one while
  * the next is captured (synchronous); if elapsed_ms is not NULL it receives
- * their run time, measured with events on the library's stream.  Replaces the step loop of Model.simulate
- * (model.py:1295-1301) when the magnitudes of all steps are known. */
+ * their run time, measured with events on the library's stream.  Replaces the
+ * step loop of Model.simulate (model.py:1295-1301) when the magnitudes of all
+ * steps are known.  Steps whose graph cannot be made are launched one by one;
+ * where the first graph cannot, nothing runs. */
 int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
                  const double *force_mags, float *elapsed_ms);
 

@@ -2290,6 +2290,7 @@ struct pd_sim {
     bool retile_pending = false;  // tile_nodes changed since the tiling
     bool has_buffers = false, has_corr = false, has_btypes = false,
          has_cnode = false;
+    bool lost = false;  // has_buffers was taken back by a run that failed
     int nregimes = 1, nbond_types = 1;
     double k = 0.0, s0 = 0.0;
     int cur = 0;
@@ -2460,6 +2461,15 @@ int check_sim(pd_sim *s)
         return fail(PD_E_ARG, "null simulation handle");
     HIPCHK(hipSetDevice(s->device));
     return PD_OK;
+}
+
+// What a call that needs the simulation's state says without it.
+int no_buffers(const pd_sim *s)
+{
+    return fail(PD_E_STATE,
+                s->lost ? "a run failed on its way and left no whole state: "
+                          "call pd_create_buffers"
+                        : "pd_create_buffers has not been called");
 }
 
 int dm_of(const pd_sim *s)
@@ -2775,6 +2785,16 @@ int launch_step(pd_sim *s, double dmag, double fmag, bool last)
     return after_step(s, dmag, fmag);
 }
 
+// After an error on the way of a run, some of whose steps have moved the
+// records and the bonds but stored neither u nor forces: without them there is
+// no state to read or to go on from.
+void run_failed(pd_sim *s)
+{
+    s->has_buffers = false;
+    s->lost = true;
+    adjoint_end(s);
+}
+
 // The tip entries as internal DOF indices 3p + d for the current tiling.
 int upload_tips(pd_sim *s)
 {
@@ -3018,6 +3038,7 @@ int restart(pd_sim *s, const double *bond_stiffness,
     if (rc)
         return rc;
     s->has_buffers = true;
+    s->lost = false;
     s->retile_pending = false;
     return PD_OK;
 }
@@ -3888,6 +3909,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     if (rc)
         return rc;
     s->has_buffers = true;
+    s->lost = false;
     s->retile_pending = false;
     keep_plan(s, nlist, n_neigh, nlin, given);
     return PD_OK;
@@ -3934,7 +3956,7 @@ int pd_monitor(pd_sim *s, double *model, double *tips)
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (!model)
         return fail(PD_E_ARG, "model (6 doubles) is required");
     const int ngroups =
@@ -4003,7 +4025,7 @@ int pd_monitor_noalloc(pd_sim *s, double *model, double *tips)
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (!model)
         return fail(PD_E_ARG, "model (6 doubles) is required");
     const int ngroups =
@@ -4178,7 +4200,7 @@ int pd_step(pd_sim *s, double dmag, double fmag)
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     return launch_step(s, dmag, fmag, true);
 }
 
@@ -4189,14 +4211,18 @@ int pd_run(pd_sim *s, int nsteps, const double *disp_mags,
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (nsteps < 0)
         return fail(PD_E_ARG, "nsteps < 0");
+    const int cur0 = s->cur;
     for (int t = 0; t < nsteps; ++t) {
         rc = launch_step(s, disp_mags ? disp_mags[t] : 0.0,
                          force_mags ? force_mags[t] : 0.0, t + 1 == nsteps);
-        if (rc)
+        if (rc) {
+            if (t > 0 || s->cur != cur0)
+                run_failed(s);
             return rc;
+        }
     }
     return PD_OK;
 }
@@ -4225,6 +4251,9 @@ int pd_run_timed(pd_sim *s, int nsteps, const double *disp_mags,
 // before the first step.  Wall clock of 25 steps, one graph / graphs of 4, 8
 // and 16: 1,280 nodes 363 / 244, 236, 238 us; 141,143 nodes 1162 / 1024, 1002,
 // 1019 (of 400: 18.3 / 16.0, 15.6, 15.6 ms).
+// All steps run or none: where the first graph cannot be made nothing has run,
+// and where a later one cannot, the steps from there on are launched one by
+// one.
 constexpr int GRAPH_STEPS = 8;
 
 int pd_run_graph(pd_sim *s, int nsteps, const double *disp_mags,
@@ -4234,7 +4263,7 @@ int pd_run_graph(pd_sim *s, int nsteps, const double *disp_mags,
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (nsteps < 0)
         return fail(PD_E_ARG, "nsteps < 0");
     if (nsteps == 0) {
@@ -4248,19 +4277,22 @@ int pd_run_graph(pd_sim *s, int nsteps, const double *disp_mags,
     HIPCHK(hipStreamSynchronize(s->stream));
     std::vector<hipGraphExec_t> execs;
     hipError_t e = hipSuccess;
-    for (int t0 = 0; t0 < nsteps && rc == PD_OK && e == hipSuccess;) {
+    const auto step = [&](int t) {
+        return launch_step(s, disp_mags ? disp_mags[t] : 0.0,
+                           force_mags ? force_mags[t] : 0.0, t + 1 == nsteps);
+    };
+    int t0 = 0;  // the steps before it are on their way
+    while (t0 < nsteps) {
         const int t1 = std::min(nsteps, t0 == 0 ? 2 : t0 + GRAPH_STEPS);
         const int cur0 = s->cur;
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess)
-            break;
-        for (int t = t0; t < t1 && rc == PD_OK; ++t)
-            rc = launch_step(s, disp_mags ? disp_mags[t] : 0.0,
-                             force_mags ? force_mags[t] : 0.0,
-                             t + 1 == nsteps);
-        e = hipStreamEndCapture(s->stream, &graph);
+        if (e == hipSuccess) {
+            for (int t = t0; t < t1 && rc == PD_OK; ++t)
+                rc = step(t);
+            e = hipStreamEndCapture(s->stream, &graph);
+        }
         if (rc == PD_OK && e == hipSuccess)
             e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
         if (graph)
@@ -4269,15 +4301,29 @@ int pd_run_graph(pd_sim *s, int nsteps, const double *disp_mags,
             execs.push_back(exec);
         if (rc == PD_OK && e == hipSuccess && t0 == 0 && elapsed_ms)
             e = hipEventRecord(s->ev0, s->stream);
-        if (rc == PD_OK && e == hipSuccess)
+        const bool made = rc == PD_OK && e == hipSuccess;
+        if (made)
             e = hipGraphLaunch(exec, s->stream);
-        if (rc != PD_OK || e != hipSuccess)
-            s->cur = cur0;  // these steps do not run
-        t0 = t1;
+        if (made && e == hipSuccess) {
+            t0 = t1;
+            continue;
+        }
+        s->cur = cur0;  // these steps do not run
+        (void)hipGetLastError();  // or the next launch would report it
+        if (made || t0 == 0)
+            break;
+        rc = PD_OK;
+        e = hipSuccess;
+        for (; t0 < nsteps && rc == PD_OK; ++t0)
+            rc = step(t0);
+        break;
     }
-    if (rc == PD_OK && e == hipSuccess && elapsed_ms)
+    const bool ran = rc == PD_OK && e == hipSuccess;
+    if (ran && elapsed_ms)
         e = hipEventRecord(s->ev1, s->stream);
     const hipError_t es = hipStreamSynchronize(s->stream);
+    if (t0 > 0 && !(ran && es == hipSuccess))
+        run_failed(s);
     for (hipGraphExec_t x : execs)
         (void)hipGraphExecDestroy(x);
     if (e == hipSuccess)
@@ -4328,7 +4374,7 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
     if (rc)
         return rc;
     if (!s->has_buffers || s->retile_pending)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (s->integrator != PD_EULER || s->layout != PD_LAYOUT_SLOT ||
         !s->has_cnode || s->nregimes > 1 || s->nbond_types > 1)
         return fail(PD_E_ARG, "the adjoint needs the Euler integrator, the "
@@ -4553,7 +4599,7 @@ int pd_write_device(pd_sim *s, double *u, double *damage)
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (damage) {
         HIPCHK(launch_export(s, 0, damage, u));
     } else if (u) {
@@ -4582,7 +4628,7 @@ int pd_write(pd_sim *s, double *u, double *ud, double *udd, double *force,
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     const int N = s->n;
     if (u)
         HIPCHK(s->wbuf.reserve(3 * (size_t)N));
@@ -4649,7 +4695,7 @@ int pd_get_regimes(pd_sim *s, int *regimes)
     if (rc)
         return rc;
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     if (!regimes)
         return fail(PD_E_ARG, "regimes is NULL");
     const size_t NK = (size_t)s->n * s->K;
@@ -4679,7 +4725,7 @@ int pd_live_bonds(pd_sim *s, long long *count)
     if (!count)
         return fail(PD_E_ARG, "count is NULL");
     if (!s->has_buffers)
-        return fail(PD_E_STATE, "pd_create_buffers has not been called");
+        return no_buffers(s);
     HIPCHK(hipMemsetAsync(s->counter.p, 0, sizeof(unsigned long long),
                           s->stream));
     hipLaunchKernelGGL(k_live, dim3(row_blocks(s->n, CHUNK_LANES)),

@@ -1,0 +1,157 @@
+"""Calls that fail on their way: what they leave is what was there before, or
+the whole result, or is refused until the buffers are made anew -- never a
+displacement of one step beside the bonds of another.
+
+Failures of HIP calls are made by a small library that stands before the HIP
+runtime in a process of its own and reports an error, without calling on, at
+the given call of the given function."""
+import json
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("hip_device")]
+
+SHIM = r"""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+typedef struct { unsigned x, y, z; } dim;
+static int left[3], pending;
+void shim_arm(int which, int calls) { left[which] = calls; pending = 0; }
+static int now(int which) { return left[which] > 0 && --left[which] == 0; }
+int hipGraphInstantiate(void *e, void *g, void *n, char *b, size_t s)
+{
+    if (now(0))
+        return 2;
+    int (*f)(void *, void *, void *, char *, size_t) =
+        dlsym(RTLD_NEXT, "hipGraphInstantiate");
+    return f(e, g, n, b, s);
+}
+int hipGraphLaunch(void *e, void *s)
+{
+    if (now(1))
+        return 2;
+    int (*f)(void *, void *) = dlsym(RTLD_NEXT, "hipGraphLaunch");
+    return f(e, s);
+}
+int hipLaunchKernel(const void *k, dim g, dim b, void **a, size_t m, void *s)
+{
+    if (now(2))
+        return pending = 2;
+    int (*f)(const void *, dim, dim, void **, size_t, void *) =
+        dlsym(RTLD_NEXT, "hipLaunchKernel");
+    return f(k, g, b, a, m, s);
+}
+int hipGetLastError(void)
+{
+    int (*f)(void) = dlsym(RTLD_NEXT, "hipGetLastError");
+    const int e = pending ? pending : f();
+    pending = 0;
+    return e;
+}
+"""
+
+CHILD = r"""
+import ctypes, json, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path[:0] = sys.argv[2:4]
+import numpy as np
+from probabilistic_peridynamics_amd import _lib
+from test_gpu_runs import _arrays, _make
+which, calls, method = json.loads(sys.argv[4])
+STEPS = 22
+d, f = 1e-6 * np.arange(1, STEPS + 1), np.linspace(0.5, 2, STEPS)
+integ = _make("euler")
+start = _arrays(integ)
+integ.run(STEPS, d, f)
+want = _arrays(integ)
+same = lambda a, b: all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def refused(call, *args):
+    try:
+        call(*args)
+    except _lib.PDError as e:
+        return e.code
+    return 0
+
+
+fresh = _make("euler")
+shim.shim_arm(which, calls)
+out = {"call": refused(getattr(fresh, method), STEPS, d, f)}
+shim.shim_arm(which, 0)
+out["write"] = refused(_arrays, fresh)
+if not out["write"]:
+    got = _arrays(fresh)
+    out["state"] = ("whole" if same(got, want) else
+                    "start" if same(got, start) else "neither")
+else:
+    out["others"] = [refused(call, *a) for call, a in (
+        (fresh.run, (1, d[:1], f[:1])), (fresh, (0.0, 0.0)),
+        (fresh.monitor, ()), (fresh.write_device, ()),
+        (fresh.adjoint_start, (2,)), (fresh.regimes, ()),
+        (fresh.live_bonds, ()))]
+w = __import__("test_gpu_runs").configs.beam_vv(shape=(23, 7, 6))
+n = fresh.nnodes
+rng = np.random.default_rng(5)
+rng.random(n), rng.normal(size=(n, 3))
+u = rng.normal(scale=2e-3 * w.extra["dx"], size=(n, 3))
+fresh.create_buffers(w.nlist, w.n_neigh, w.bond_stiffness,
+                     w.critical_stretch, w.plus_cs, u,
+                     rng.normal(scale=1e-2, size=(n, 3)), None, None, None,
+                     None, None, 1, 1)
+getattr(fresh, method)(STEPS, d, f)
+out["again"] = same(_arrays(fresh), want)
+print("RESULT", json.dumps(out), flush=True)
+"""
+
+INSTANTIATE, GRAPH, KERNEL = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shim")
+    (d / "shim.c").write_text(SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", str(d / "shim.so"),
+                    str(d / "shim.c"), "-Wl,--no-as-needed",
+                    "-L/opt/rocm/lib", "-lamdhip64", "-ldl"], check=True)
+    return d / "shim.so"
+
+
+def _after_failure(shim, which, calls, method):
+    from conftest import ROOT, TESTS
+    r = subprocess.run(
+        [sys.executable, "-c", CHILD, str(shim), str(ROOT), str(TESTS),
+         json.dumps([which, calls, method])],
+        capture_output=True, text=True, timeout=100)
+    line = [x for x in r.stdout.splitlines() if x.startswith("RESULT")]
+    assert r.returncode == 0 and line, r.stdout + r.stderr
+    out = json.loads(line[0][len("RESULT"):])
+    assert out["again"]  # new buffers, and all is well
+    return out
+
+
+@pytest.mark.parametrize("which,calls,method", [
+    (INSTANTIATE, 1, "run_graph"), (GRAPH, 1, "run_graph"),
+    (KERNEL, 1, "run_graph"), (KERNEL, 1, "run")])
+def test_a_run_that_fails_at_once_leaves_the_state(shim, which, calls,
+                                                   method):
+    out = _after_failure(shim, which, calls, method)
+    assert out["call"] == -2 and out["state"] == "start"
+
+
+@pytest.mark.parametrize("which,calls", [(INSTANTIATE, 3), (KERNEL, 6)])
+def test_a_graph_that_cannot_be_made_is_run_as_launches(shim, which, calls):
+    out = _after_failure(shim, which, calls, "run_graph")
+    assert out["call"] == 0 and out["state"] == "whole"
+
+
+@pytest.mark.parametrize("which,calls,method", [
+    (GRAPH, 3, "run_graph"), (KERNEL, 6, "run"), (KERNEL, 6, "timed_run")])
+def test_a_run_that_fails_on_its_way_is_not_read(shim, which, calls, method):
+    out = _after_failure(shim, which, calls, method)
+    assert out["call"] == -2 and out["write"] == -4
+    assert out["others"] == [-4] * 7
