@@ -2890,6 +2890,22 @@ void set_shape(pd_sim *s)
         --s->tile_cap;
 }
 
+// Keeps the shape of the current tiling while the next one is worked out: it
+// comes back unless the next tiling is taken.
+struct ShapeGuard {
+    pd_sim *s;
+    const int lanes = s->lanes, tile_cap = s->tile_cap, hmax = s->hmax;
+    bool taken = false;
+    ~ShapeGuard()
+    {
+        if (taken)
+            return;
+        s->lanes = lanes;
+        s->tile_cap = tile_cap;
+        s->hmax = hmax;
+    }
+};
+
 // Rows of w values given in the caller's order into tile order on the device
 // (through wbuf); null clears.  On the library's stream: h is read until the
 // next synchronization.
@@ -3553,6 +3569,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
         }
     });
 
+    ShapeGuard shape{s};
     // tiles, capped by tile_nodes and by the LDS halo capacity
     // entry 0 of a staged halo is the zero record of dead slots
     // the compact layout's tiles leave room for the exact step's windows
@@ -3767,6 +3784,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
     HIPCHK(hipStreamSynchronize(s->stream));
     // from here the device state is replaced: until it is whole again no
     // step may run (a failure below leaves the simulation without buffers)
+    shape.taken = true;
     s->has_buffers = false;
     s->plan = false;
     adjoint_release(s);

@@ -155,3 +155,39 @@ def test_a_run_that_fails_on_its_way_is_not_read(shim, which, calls, method):
     out = _after_failure(shim, which, calls, method)
     assert out["call"] == -2 and out["write"] == -4
     assert out["others"] == [-4] * 7
+
+
+def test_refused_lists_leave_the_tiles_and_their_shape():
+    """Bonds too many for a tile's halo are refused after the next tiling's
+    shape is known: the steps go on with the one that there is."""
+    from probabilistic_peridynamics_amd import _lib, configs
+    from probabilistic_peridynamics_amd import integrators as it
+    w = configs.beam_vv(shape=(14, 10, 10))
+    n, k = w.nnodes, 1408
+    nl = np.full((n, k), -1, np.int32)
+    nl[:, :w.nlist.shape[1]] = w.nlist
+    u = np.random.default_rng(1).normal(scale=2e-3 * w.extra["dx"],
+                                        size=(n, 3))
+    wide = nl.copy()
+    wide[0, :1300] = np.arange(1, 1301)
+    out = []
+    for refuse in (False, True):
+        integ = it.EulerHIP(2e-15)
+        integ.build(n, 3, k, w.coords, w.volume, w.family, w.bc_types,
+                    w.bc_values, w.force_bc_types, w.force_bc_values, None,
+                    None, None)
+        integ.set_launch(4, 64)
+        args = (w.bond_stiffness, w.critical_stretch, None, u, None, None,
+                None, None, None, None, 1, 1)
+        integ.create_buffers(nl, w.n_neigh, *args)
+        integ.set_launch(8, 64)
+        if refuse:
+            with pytest.raises(_lib.PDError) as e:
+                integ.create_buffers(wide, w.n_neigh, *args)
+            assert e.value.code == _lib.PD_E_LIMIT
+        integ.run(3, np.full(3, 1e-6), np.ones(3))
+        out.append(integ.write(None, None, None, None, None, None, None,
+                               None))
+    assert np.any(out[0][3] != 0.0)
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
