@@ -2713,12 +2713,17 @@ int after_step(pd_sim *s, double dmag, double fmag)
     return PD_OK;
 }
 
+int tiles_pending()
+{
+    return fail(PD_E_STATE, "tile_nodes changed: call pd_create_buffers "
+                            "to re-tile before stepping");
+}
+
 // One step; `last`: the last of its run, whose u and forces are stored.
 int launch_step(pd_sim *s, double dmag, double fmag, bool last)
 {
     if (s->retile_pending)
-        return fail(PD_E_STATE, "tile_nodes changed: call pd_create_buffers "
-                                "to re-tile before stepping");
+        return tiles_pending();
     if (s->ntiles == 0) {
         s->cur = 1 - s->cur;
         return PD_OK;
@@ -2786,8 +2791,8 @@ int launch_step(pd_sim *s, double dmag, double fmag, bool last)
 }
 
 // After an error on the way of a run, some of whose steps have moved the
-// records and the bonds but stored neither u nor forces: without them there is
-// no state to read or to go on from.
+// records and the bonds but stored neither u nor forces, or of a replay: there
+// is no state to read or to go on from.
 void run_failed(pd_sim *s)
 {
     s->has_buffers = false;
@@ -4501,6 +4506,8 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
     // with every u kept, the recording is one segment that needs no replay,
     // and the state is not touched
     const bool replay = !s->adj_all || s->adj_changed;
+    if (replay && s->retile_pending)
+        return tiles_pending();
     const int nsteps = s->adj_nsteps, every = replay ? s->adj_every : nsteps;
     const int nck = (nsteps + every - 1) / every;
     hipStream_t st = s->stream;
@@ -4543,6 +4550,16 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
     aa.loc0 = s->loc0.p;
     aa.il0 = s->il0.p;
     aa.gradc = s->gradc.p;
+    // from here on a replay takes the state back to earlier steps
+    struct StateGuard {
+        pd_sim *s;
+        bool away;
+        ~StateGuard()
+        {
+            if (away)
+                run_failed(s);
+        }
+    } state{s, replay};
     for (int k = nck - 1; k >= 0 && rc == PD_OK; --k) {
         const int n0 = k * every, n1 = std::min(n0 + every, nsteps);
         double *seg = s->seg.p + (s->adj_all ? (size_t)n0 * B : 0);
@@ -4588,6 +4605,7 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
         if (rc)
             return rc;
         s->step_counter = nsteps;
+        state.away = false;
     }
     if (device) {
         hipLaunchKernelGGL(k_unperm, dim3((s->n + 255) / 256), dim3(256), 0,

@@ -191,3 +191,20 @@ def test_refused_lists_leave_the_tiles_and_their_shape():
     assert np.any(out[0][3] != 0.0)
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("every", [3, 9])
+def test_a_backward_pass_that_is_refused_leaves_the_state(every):
+    """A tile size set after the recording, which a replay would need."""
+    from probabilistic_peridynamics_amd import _lib
+    from test_gpu_recording import _make, _state
+    integ, _ = _make(2e-3)
+    integ.adjoint_start(9, checkpoint_every=every)
+    integ.run(9, np.full(9, 1e-6), np.ones(9))
+    before = _state(integ)
+    integ.set_launch(4, 64)
+    with pytest.raises(_lib.PDError) as e:
+        integ.adjoint_backward(np.ones(before[0].shape))
+    assert e.value.code == _lib.PD_E_STATE
+    for a, b in zip(_state(integ), before):
+        np.testing.assert_array_equal(a, b)
