@@ -77,12 +77,11 @@
 // fixtures evaluated them.  The square roots use the correctly rounded
 // rsq-Goldschmidt sequence that the compiler emits for sqrt(double), without
 // its range scaling (taken only for q outside [2^-767, inf), where the
-// library sqrt is called); the step in plain order takes it with one
-// residual correction instead of two (sqrt_core<1>).  Its by-product h ~
-// 0.5/sqrt(q) (relative error ~5e-15) replaces the two divisions; a stretch
-// within a relative 1e-10 (and 2^-49) of any threshold it is compared with is
-// recomputed with the library's square roots and the IEEE division, so every
-// break and regime decision equals the one made with the correctly rounded s.
+// library sqrt is called).  Its by-product h ~ 0.5/sqrt(q) (relative error
+// ~5e-15) replaces the two divisions; a stretch within a relative 1e-10 of any
+// threshold it is compared with is recomputed with the library's square roots
+// and the IEEE division, so every break and regime decision equals the one
+// made with the correctly rounded s.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -133,8 +132,6 @@ constexpr uint32_t KEYM = 0x3FFFFFFFu;
 constexpr unsigned short LOC_DEAD = 0;  // loc of a broken or empty slot
 constexpr int MAX_NODES = 1 << 26;
 constexpr double GUARD = 1e-10;
-// and of s/2 itself, above what a root that is an ulp off does to it
-constexpr double GUARD_ABS = 0x1p-50;
 constexpr int MAX_TAB = 256;  // nbond_types * nregimes
 constexpr int MAX_LPN = 8;
 constexpr int XCDS = 8;
@@ -271,16 +268,12 @@ __device__ __forceinline__ void static_for(F f)
 // corrections of g -- the sequence LLVM emits for llvm.sqrt.f64 on gfx9,
 // minus the input scaling and the zero/infinity selects it needs outside
 // that range.
-// CORRECTIONS 1 leaves out the second one: the seed's relative error e is at
-// most 6.0e-8 (2^29 ulp), the step's d = 3/2 e^2 <= 5.4e-15, and the first
-// correction's 3/2 d^2 <= 4.4e-29 before its one rounding, so g is within
-// 0.5 + 4e-13 ulp of sqrt(q): the nearest double unless sqrt(q) lies within
-// 4e-13 ulp of the middle between two (of 4.3e9 random q none got another g).
-// The step kernel's fast evaluation, whose lengths need not be the Cython
-// code's to the bit, spends no instruction on the second: 4 of a bond's 51
-// issue slots, 255 -> 242 us a step on the 1,038,230-node beam, 37.1 -> 35.1 on
-// 141,143 nodes, 72.3 -> 69.1 with n-linear tables on 263,407.
-template <int CORRECTIONS = 2>
+// Both corrections are needed: before its rounding the first leaves up to
+// 3/2 d^2 = 4.4e-29 (the seed's e is at most 6e-8, the step's d = 3/2 e^2), so
+// that of roots within 4e-13 ulp of the middle between two doubles one in five
+// takes the wrong one.  The second costs the step 4 of a bond's 55 issue slots:
+// 233 -> 247 us on the 1,038,230-node beam, 38.4 -> 40.2 on 141,143 nodes, 72.6
+// -> 74.1 with n-linear tables on 263,407.
 __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
 {
     const double y = __builtin_amdgcn_rsq(q);
@@ -289,11 +282,10 @@ __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
     const double r = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, r, g);
     h = __builtin_fma(h, r, h);
-#pragma unroll
-    for (int c = 0; c < CORRECTIONS; ++c) {
-        const double d = __builtin_fma(-g, g, q);
-        g = __builtin_fma(d, h, g);
-    }
+    double d = __builtin_fma(-g, g, q);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, q);
+    g = __builtin_fma(d, h, g);
 }
 
 __device__ __forceinline__ bool core_range(double q)
@@ -670,10 +662,10 @@ struct Bond {
     double dx, dy, dz, sh, hl, w;
 };
 
-// The model's halved thresholds with margins of GUARD (relative) and
-// GUARD_ABS: a stretch strictly inside (lo, hi) is away from every threshold
-// and from lengths outside sqrt_core's range, so the bond neither breaks nor
-// changes its regime.  Anything else, NaN included, goes through bond_exact.
+// The model's halved thresholds with a margin of GUARD: a stretch strictly
+// inside (lo, hi) is away from every threshold and from lengths outside
+// sqrt_core's range, so the bond neither breaks nor changes its regime.
+// Anything else, NaN included, goes through bond_exact.
 //
 // Why the lengths need no test of their own: coordinates are zero or in
 // [2^-290, 2^300] (else the host sets hi so that every bond takes the exact
@@ -735,8 +727,8 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
     const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
     const double q0 = sq3<CLA>(ex, ey, ez);
     double l, l0, h0;
-    sqrt_core<1>(qq, l, o.hl);
-    sqrt_core<1>(q0, l0, h0);
+    sqrt_core(qq, l, o.hl);
+    sqrt_core(q0, l0, h0);
     o.sh = (l - l0) * h0;  // s/2, from h0 ~ 0.5/l0
     // k = (c_i + c_j)/2 for a field: s k/l V_j = (s/2)(0.5/l) w with
     // w = 2(c_i+c_j)V_j = c_i (2 V_j) + (2 c_j V_j), the staged pair
@@ -892,8 +884,8 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
 // Tiles by bisection and a leaner prologue gave 257 us on the beam, 74.5 and
 // 46.4 on the other two; what a run's inner steps store for nobody (force, the
 // slot layout's u, Euler-Cromer's udd) left out, 250, 72 and 45.5; tiles even
-// over the CUs 42.3 on the last, one correction of each square root less, 242,
-// 69 and 40.8; the narrow form 230 on the beam.
+// over the CUs 42.3 on the last; the narrow form takes 4 % off the beam
+// (narrow_fits).
 //
 // DM: DM_PMB, DM_NLIN or DM_FIELD.  One workgroup per tile, LPN lanes per
 // node taking its 4-bond chunks round-robin and reducing with cross-lane
@@ -1007,11 +999,10 @@ __global__ __launch_bounds__(NARROW ? 512 : 1024, NARROW ? 6 : 1) void k_step(
             double lo = -0.25;
             if (t % a.nregimes != 0) {
                 const double c = a.s_tab[t - 1] * 0.5;
-                lo = fmax(lo, c + (GUARD * fabs(c) + GUARD_ABS));
+                lo = fmax(lo, c + GUARD * fabs(c));
             }
             tsp[t] = make_double2(
-                lo, a.lim > 0.0 ? up - (GUARD * fabs(up) + GUARD_ABS)
-                                : -__DBL_MAX__);
+                lo, a.lim > 0.0 ? up - GUARD * fabs(up) : -__DBL_MAX__);
             tkp[t] = make_double2(4.0 * a.k_tab[t], 2.0 * a.pc_tab[t]);
         }
     }
@@ -2499,8 +2490,7 @@ StepArgs make_args(pd_sim *s)
     // every bond takes the exact path
     a.lim = !s->coords_core || s->odd_corr || s->odd_tables ? -1.0
             : dm_of(s) == DM_NLIN ? 1.0
-                                  : std::min(a.s0h * (1.0 - GUARD) - GUARD_ABS,
-                                             0.25);
+                                  : std::min(a.s0h * (1.0 - GUARD), 0.25);
     a.rec_old = s->rec[s->cur].p;
     a.rec_new = s->rec[1 - s->cur].p;
     a.tiles = s->tiles.p;
@@ -2551,8 +2541,9 @@ unsigned block_of(const pd_sim *s, int lanes)
 // Whether tiles of at most `halo` halo entries run the narrow form at four
 // lanes per node: it takes blocks of at most 512, and pays where a CU has
 // more than two tiles to run (us a step, wide / narrow: 1,038,230-node beam
-// 245 / 230, 93,433-node plate 11.5 / 11.0, bars of three to five tiles per CU
-// the same within the noise; with two or fewer the wide form's early reads of
+// 257 / 247, 263,407 nodes 72.7 / 70.1, 204,800 nodes 57.9 / 56.3, 141,143
+// nodes 43.1 / 42.4, 100 steps of a 93,433-node plate 1367 / 1307; with two or
+// fewer the wide form's early reads of
 // the node's state are worth more).
 bool narrow_fits(const pd_sim *s, int ntiles, int halo)
 {
