@@ -287,8 +287,9 @@ void pd_destroy(pd_sim *sim);
 #define PD_CHECK_TENSION 1 /* break on !(s < s0) instead of !(|s| < s0) */
 #define PD_CHECK_OPENCL 2  /* the slot layout's OpenCL stretch */
 
-/* Verification entry point: the step kernel's stretch pipeline on n bonds
- * (r_i, r_j, r0_i, r0_j each (n,3) f64), run on `device`.  Outputs per bond:
+/* Verification entry point: the scalar step kernel's own stretch evaluation
+ * (plain order) on n bonds (r_i, r_j, r0_i, r0_j each (n,3) f64), run on
+ * `device`.  Outputs per bond:
  * l = |r_j - r_i| and l0 = |r0_j - r0_i| (spatial.pyx:20-31, bitwise), the
  * kernel's working stretch s, the IEEE-division stretch (l - l0)/l0
  * (spatial.pyx:87-97) and the break decision !(|s| < s0)

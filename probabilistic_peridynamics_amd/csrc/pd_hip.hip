@@ -270,8 +270,9 @@ __device__ __forceinline__ void static_for(F f)
 // that range.
 // Both corrections are needed: before its rounding the first leaves up to
 // 3/2 d^2 = 4.4e-29 (the seed's e is at most 6e-8, the step's d = 3/2 e^2), so
-// that of roots within 4e-13 ulp of the middle between two doubles one in five
-// takes the wrong one.  The second costs the step 4 of a bond's 55 issue slots:
+// that a root within 4e-13 ulp of the middle between two doubles may take the
+// wrong one (8 of 4,023 squares built to lie 7e-15 to 5e-13 ulp off it did,
+// and none with the second).  The second costs the step 4 of a bond's 55 issue slots:
 // 233 -> 247 us on the 1,038,230-node beam, 38.4 -> 40.2 on 141,143 nodes, 72.6
 // -> 74.1 with n-linear tables on 263,407.
 __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
@@ -657,9 +658,10 @@ __device__ __forceinline__ T node_sum(T v)
     return v;
 }
 
-// A bond as the force needs it: the bond vector, s/2, 0.5/l and the weight.
+// A bond as the force needs it: the bond vector, s/2, 0.5/l and the weight;
+// and the lengths that s/2 came from (for k_bond_check).
 struct Bond {
-    double dx, dy, dz, sh, hl, w;
+    double dx, dy, dz, sh, hl, w, l, l0;
 };
 
 // The model's halved thresholds with a margin of GUARD: a stretch strictly
@@ -690,7 +692,7 @@ struct Bond {
 // (2^300, 2^300, 2^300) of weight 0, so that l == l0 and the force is zero.
 // lim: a.lim, or -1 where no bond of the node's may stand.
 template <int DM, bool TENS, bool CLA, bool NARROW>
-__device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
+__device__ __forceinline__ bool bond_fast(const char *ldsb,
                                           const double4 &r0i,
                                           const double4 &ri, double ci,
                                           double lim, unsigned ev, unsigned st,
@@ -726,10 +728,10 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
     }
     const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
     const double q0 = sq3<CLA>(ex, ey, ez);
-    double l, l0, h0;
-    sqrt_core(qq, l, o.hl);
-    sqrt_core(q0, l0, h0);
-    o.sh = (l - l0) * h0;  // s/2, from h0 ~ 0.5/l0
+    double h0;
+    sqrt_core(qq, o.l, o.hl);
+    sqrt_core(q0, o.l0, h0);
+    o.sh = (o.l - o.l0) * h0;  // s/2, from h0 ~ 0.5/l0
     // k = (c_i + c_j)/2 for a field: s k/l V_j = (s/2)(0.5/l) w with
     // w = 2(c_i+c_j)V_j = c_i (2 V_j) + (2 c_j V_j), the staged pair
     o.w = DM == DM_FIELD ? __builtin_fma(ci, p1.y, p3.y) : p1.y;
@@ -747,8 +749,38 @@ __device__ __forceinline__ bool bond_fast(const StepArgs &a, const char *ldsb,
     }
 }
 
-// The bond at slot `slot` with IEEE square roots and division
-// (spatial.pyx:87-97, cl/peridynamics.cl:72-74): decides whether it breaks or
+// The stretch of the bond to halo entry `ev` with IEEE square roots and
+// division (spatial.pyx:87-97, cl/peridynamics.cl:72-74), in place of
+// bond_fast's.
+template <int DM, bool CLA, bool NARROW>
+__device__ __forceinline__ void stretch_exact(const char *ldsb,
+                                              const double4 &r0i, unsigned ev,
+                                              Bond &o)
+{
+    constexpr unsigned PB = piece_bytes<DM, NARROW>();
+    const char *pe = ldsb + halo_base<DM>() + ev;
+    const double2 p0 = *reinterpret_cast<const double2 *>(pe);
+    const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
+    const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
+    const double ex = p0.x - r0i.x;
+    const double ey = p0.y - r0i.y;
+    const double ez = p1.x - r0i.z;
+    const double q0 = sq3<CLA>(ex, ey, ez);
+    o.l = sqrt(qq);
+    o.l0 = sqrt(q0);
+    if (!(core_range(qq) & core_range(q0)))
+        o.hl = 0.5 / o.l;
+    o.sh = ((o.l - o.l0) / o.l0) * 0.5;
+}
+
+// Whether a bond of that s/2 stays, by the scalar criterion.
+template <bool TENS>
+__device__ __forceinline__ bool stays(double sh, double s0h)
+{
+    return (TENS ? sh : fabs(sh)) < s0h;
+}
+
+// The bond at slot `slot` by stretch_exact: decides whether it breaks or
 // changes its regime, writes that, and leaves in `o` (and kb, pb for
 // DM_NLIN) what the force needs, zero for a broken or empty slot, whose
 // correction `cr` becomes zero too (it may be infinite or NaN).
@@ -760,23 +792,11 @@ __device__ __forceinline__ void bond_exact(const StepArgs &a,
                                            double &kb, double &pb, double &cr,
                                            int &nbroken)
 {
-    constexpr unsigned PB = piece_bytes<DM, NARROW>();
     bool live = ev != LOC_DEAD;
     if (live) {
-        const char *pe = ldsb + halo_base<DM>() + ev;
-        const double2 p0 = *reinterpret_cast<const double2 *>(pe);
-        const double2 p1 = *reinterpret_cast<const double2 *>(pe + PB);
-        const double qq = sq3<CLA>(o.dx, o.dy, o.dz);
-        const double ex = p0.x - r0i.x;
-        const double ey = p0.y - r0i.y;
-        const double ez = p1.x - r0i.z;
-        const double q0 = sq3<CLA>(ex, ey, ez);
-        const double l = sqrt(qq), l0 = sqrt(q0);
-        if (!(core_range(qq) & core_range(q0)))
-            o.hl = 0.5 / l;
-        o.sh = ((l - l0) / l0) * 0.5;
+        stretch_exact<DM, CLA, NARROW>(ldsb, r0i, ev, o);
         if constexpr (DM != DM_NLIN) {
-            live = (TENS ? o.sh : fabs(o.sh)) < a.s0h;
+            live = stays<TENS>(o.sh, a.s0h);
         } else {
             // cl/peridynamics.cl:326-378 (bond_force3/4), thresholds halved
             const int t = (int)(st >> 4) / a.nregimes;
@@ -844,9 +864,9 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
     const unsigned ev[2] = {lw & 0xffffu, lw >> 16};
     const unsigned st[2] = {sw & 0xffffu, sw >> 16};
     const bool ok0 = bond_fast<DM, TENS, CLA, NARROW>(
-        a, ldsb, r0i, ri, ci, lim, ev[0], st[0], o[0], kb[0], pb[0]);
+        ldsb, r0i, ri, ci, lim, ev[0], st[0], o[0], kb[0], pb[0]);
     const bool ok1 = bond_fast<DM, TENS, CLA, NARROW>(
-        a, ldsb, r0i, ri, ci, lim, ev[1], st[1], o[1], kb[1], pb[1]);
+        ldsb, r0i, ri, ci, lim, ev[1], st[1], o[1], kb[1], pb[1]);
     if (__builtin_expect(!(ok0 & ok1), 0)) {
         if (!ok0)
             bond_exact<DM, TENS, CLA, NARROW>(a, ldsb, r0i, ev[0], st[0], s0,
@@ -1124,73 +1144,69 @@ __global__ __launch_bounds__(NARROW ? 512 : 1024, NARROW ? 6 : 1) void k_step(
     }
 }
 
-// The stretch pipeline of bond<DM_PMB>, one bond per thread, for checking:
-// l, l0 (bitwise those of spatial.pyx, or of cl/peridynamics.cl:65-75 as
-// contracted with cla), the working s (2*sh), the exact s = (l - l0)/l0 and
-// the break decision.  With cla, ri and rj are the displacements u_i, u_j
-// (the OpenCL kernels form the bond from u); otherwise positions r0 + u.
-template <bool CLA>
-__device__ void bond_check_one(const double *ri, const double *rj,
-                               const double *r0i, const double *r0j,
-                               double s0, unsigned absmask, double &l,
-                               double &l0, double &s, double &se, int &brk)
+// Whether a coordinate is in the range that bond_fast relies on.
+__host__ __device__ __forceinline__ bool core_coord(double x)
 {
-    const double ex = r0j[0] - r0i[0];
-    const double ey = r0j[1] - r0i[1];
-    const double ez = r0j[2] - r0i[2];
-    double dx = rj[0] - ri[0], dy = rj[1] - ri[1], dz = rj[2] - ri[2];
-    if (CLA) {
-        dx = dx + ex;
-        dy = dy + ey;
-        dz = dz + ez;
-    }
-    const double q = sq3<CLA>(dx, dy, dz);
-    const double q0 = sq3<CLA>(ex, ey, ez);
-    double hl, h0;
-    sqrt_core(q, l, hl);
-    sqrt_core(q0, l0, h0);
-    double dl = l - l0;
-    double sh = dl * h0;
-    const bool fast = core_range(q) & core_range(q0);
-    const double s0h = s0 * 0.5;
-    double as = sign_mask(sh, absmask);
-    if (!fast || fabs(as - s0h) <= GUARD * s0h) {
-        if (!fast) {
-            l = sqrt(q);
-            l0 = sqrt(q0);
-            dl = l - l0;
-        }
-        sh = (dl / l0) * 0.5;
-        as = sign_mask(sh, absmask);
-    }
-    s = sh + sh;
-    se = dl / l0;
-    brk = !(as < s0h);
+    x = fabs(x);
+    return x == 0.0 || (x >= 0x1p-290 && x <= 0x1p300);
 }
 
-__global__ void k_bond_check(int n, int cla, const double *ri,
-                             const double *rj, const double *r0i,
-                             const double *r0j, double s0, unsigned absmask,
-                             double *l_out, double *l0_out, double *s_out,
-                             double *s_exact, int *broken)
+// bond_fast's limit for a halved critical stretch (scalar criterion).
+__host__ __device__ __forceinline__ double fast_limit(double s0h)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const double m = s0h * (1.0 - GUARD);
+    return 0.25 < m ? 0.25 : m;
+}
+
+// The stretch and break decision of the scalar step in plain order, one bond
+// per thread, for checking: the step's own bond_fast, and stretch_exact and
+// stays behind it, on a record that the thread puts into LDS.  Out come l and
+// l0 (bitwise those of spatial.pyx, or of cl/peridynamics.cl:65-75 as
+// contracted with CLA), the working s (2*sh), the exact s = (l - l0)/l0 and
+// the decision.  With CLA, ri and rj are the displacements u_i, u_j (the
+// OpenCL kernels form the bond from u); otherwise positions r0 + u.
+constexpr int CHECK_BLOCK = 256;
+
+template <bool TENS, bool CLA>
+__global__ __launch_bounds__(CHECK_BLOCK) void k_bond_check(
+    int n, const double *ri, const double *rj, const double *r0i,
+    const double *r0j, double s0, double *l_out, double *l0_out,
+    double *s_out, double *s_exact, int *broken)
+{
+    constexpr unsigned PB = piece_bytes<DM_PMB>();
+    static_assert(CHECK_BLOCK < LDS_CAP_PMB, "an entry per thread");
+    __shared__ double2 lds[LDS_BYTES / sizeof(double2)];
+    const int t = blockIdx.x * CHECK_BLOCK + threadIdx.x;
     if (t >= n)
         return;
     const size_t b = 3 * (size_t)t;
-    double l, l0, s, se;
-    int brk;
-    if (cla)
-        bond_check_one<true>(ri + b, rj + b, r0i + b, r0j + b, s0, absmask,
-                             l, l0, s, se, brk);
-    else
-        bond_check_one<false>(ri + b, rj + b, r0i + b, r0j + b, s0, absmask,
-                              l, l0, s, se, brk);
-    l_out[t] = l;
-    l0_out[t] = l0;
-    s_out[t] = s;
-    s_exact[t] = se;
-    broken[t] = brk;
+    const unsigned ev = 16u * (threadIdx.x + 1u);
+    char *ldsb = reinterpret_cast<char *>(lds);
+    const double e[8] = {r0j[b], r0j[b + 1], r0j[b + 2], 1.0,
+                         rj[b],  rj[b + 1],  rj[b + 2],  0.0};
+    bool core = true;
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<double2 *>(ldsb + q * PB + ev) =
+            make_double2(e[2 * q], e[2 * q + 1]);
+    for (int d = 0; d < 3; ++d)
+        core &= core_coord(r0i[b + d]) && core_coord(r0j[b + d]);
+    const double4 own0 = make_double4(r0i[b], r0i[b + 1], r0i[b + 2], 1.0);
+    const double4 own = make_double4(ri[b], ri[b + 1], ri[b + 2], 0.0);
+    const double s0h = s0 * 0.5;
+    Bond o;
+    double kb, pb;
+    bool live = true;
+    if (!bond_fast<DM_PMB, TENS, CLA, false>(ldsb, own0, own, 0.0,
+                                             core ? fast_limit(s0h) : -1.0, ev,
+                                             0u, o, kb, pb)) {
+        stretch_exact<DM_PMB, CLA, false>(ldsb, own0, ev, o);
+        live = stays<TENS>(o.sh, s0h);
+    }
+    l_out[t] = o.l;
+    l0_out[t] = o.l0;
+    s_out[t] = o.sh + o.sh;
+    s_exact[t] = (o.l - o.l0) / o.l0;
+    broken[t] = !live;
 }
 
 // Records of both ping-pong buffers from r0, V, u and c: a = (r0, wscale V),
@@ -2490,7 +2506,7 @@ StepArgs make_args(pd_sim *s)
     // every bond takes the exact path
     a.lim = !s->coords_core || s->odd_corr || s->odd_tables ? -1.0
             : dm_of(s) == DM_NLIN ? 1.0
-                                  : std::min(a.s0h * (1.0 - GUARD), 0.25);
+                                  : fast_limit(a.s0h);
     a.rec_old = s->rec[s->cur].p;
     a.rec_new = s->rec[1 - s->cur].p;
     a.tiles = s->tiles.p;
@@ -3375,10 +3391,8 @@ int pd_build(pd_sim **out, int device, int integrator, int layout, double dt,
     const size_t N = (size_t)nnodes;
     s->h_coords.assign(coords, coords + 3 * N);
     s->coords_core = true;
-    for (size_t q = 0; q < 3 * N && s->coords_core; ++q) {
-        const double x = std::fabs(coords[q]);
-        s->coords_core = x == 0.0 || (x >= 0x1p-290 && x <= 0x1p300);
-    }
+    for (size_t q = 0; q < 3 * N && s->coords_core; ++q)
+        s->coords_core = core_coord(coords[q]);
 
     std::vector<int> flags(N);
     for (size_t i = 0; i < N; ++i) {
@@ -4836,12 +4850,17 @@ int pd_bond_check(int device, int n, const double *ri, const double *rj,
     HIPCHK(d_s.alloc(N));
     HIPCHK(d_se.alloc(N));
     HIPCHK(d_b.alloc(N));
-    hipLaunchKernelGGL(k_bond_check, dim3((n + 255) / 256), dim3(256), 0, 0,
-                       n, (flags & PD_CHECK_OPENCL) ? 1 : 0, d_ri.p, d_rj.p,
-                       d_r0i.p, d_r0j.p, s0,
-                       (flags & PD_CHECK_TENSION) ? 0xffffffffu : 0x7fffffffu,
-                       d_l.p,
-                       d_l0.p, d_s.p, d_se.p, d_b.p);
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((n + CHECK_BLOCK - 1) / CHECK_BLOCK),
+                           dim3(CHECK_BLOCK), 0, 0, n, d_ri.p, d_rj.p,
+                           d_r0i.p, d_r0j.p, s0, d_l.p, d_l0.p, d_s.p, d_se.p,
+                           d_b.p);
+    };
+    const bool cla = (flags & PD_CHECK_OPENCL) != 0;
+    if (flags & PD_CHECK_TENSION)
+        cla ? go(k_bond_check<true, true>) : go(k_bond_check<true, false>);
+    else
+        cla ? go(k_bond_check<false, true>) : go(k_bond_check<false, false>);
     HIPCHK(hipGetLastError());
     HIPCHK(hipDeviceSynchronize());
     HIPCHK(hipMemcpy(l, d_l.p, N * sizeof(double), hipMemcpyDeviceToHost));

@@ -6,7 +6,10 @@ from fractions import Fraction
 import numpy as np
 import pytest
 
+import oracle
+from probabilistic_peridynamics_amd import _lib
 from probabilistic_peridynamics_amd import integrators as it
+from test_gpu_parity import _bond_batch
 
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("hip_device")]
 
@@ -88,3 +91,36 @@ def test_hard_lengths_are_rounded_correctly(layout):
     broken, force = _pairs(layout, False, 0.5, z, uj, z, r0j)
     assert not broken.any()
     np.testing.assert_array_equal(force, 0.0)
+
+
+@pytest.mark.parametrize("opencl", [False, True])
+@pytest.mark.parametrize("tension", [False, True])
+def test_bond_check_is_the_step(tension, opencl):
+    """pd_bond_check against steps of a body of such bonds and the oracle,
+    with stretches within ulps of the threshold; from the stretch on at which
+    the step divides (|s| >= 1/2), its working stretch is the divided one."""
+    for s0, far in ((0.005, 0.02), (10.0, 0.9), (1e-13, 3e-13)):
+        ri, rj, r0i, r0j = _bond_batch(seed=int(opencl), n=5000, s0=s0)
+        rng = np.random.default_rng(9)
+        target = rng.uniform(-far, far, len(ri))
+        near = rng.random(len(ri)) < 0.33
+        target[near] = rng.choice([-1, 1], near.sum()) * min(s0, far) * (
+            1 + rng.integers(-8, 9, near.sum()) * 2.0 ** -52)
+        d0 = r0j - r0i
+        ui = rng.normal(scale=1e-3 * min(1, s0), size=ri.shape)
+        uj = ui + d0 * target[:, None]
+        ri, rj = (ui, uj) if opencl else (r0i + ui, r0j + uj)
+        got = _lib.bond_check(ri, rj, r0i, r0j, s0, tension_only=tension,
+                              opencl=opencl)
+        s = np.array([oracle.cl_strain(*b)[0] if opencl else
+                      oracle.strain(*b) for b in zip(ri, rj, r0i, r0j)])
+        want = ~(s < s0) if tension else ~(np.abs(s) < s0)
+        np.testing.assert_array_equal(got["s_exact"], s)
+        np.testing.assert_array_equal(got["broken"].astype(bool), want)
+        divided = np.abs(s) >= 0.5
+        np.testing.assert_array_equal(got["s"][divided], s[divided])
+        broken, _ = _pairs("slot" if opencl else "compact", tension, s0, ui,
+                           uj, r0i, r0j)
+        np.testing.assert_array_equal(broken, want)
+        assert s0 == 10.0 or 0 < want.sum() < len(want)
+        assert s0 != 10.0 or divided.sum() > 100
