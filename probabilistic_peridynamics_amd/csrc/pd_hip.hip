@@ -52,7 +52,8 @@
 //     gidx  i32  j, with bit 31 DEAD and bit 30 NEW (broken in this step,
 //                compact layout) -- read only on breaks and exports
 //     pos   u16  reference column of the slot (exports)
-//     corr  f64, state u16 (16 * (bond type * nregimes + regime)): optional
+//     corr  f64, state u16 (16 * (bond type * nregimes + regime), of a broken
+//                bond regime 0): optional
 //   chunk0[N], stride[N]: node p's chunk 0 and its tile's node count, from
 //              which slot_of gives the slot of its k-th bond
 //   u, ud, udd, force, body_force (N,3) f64 in the reference's layout
@@ -810,9 +811,13 @@ __device__ __forceinline__ void bond_exact(const StepArgs &a,
                 nreg = reg + 1;
             }
             live = nreg < a.nregimes;
+            // a dead slot's s of 0 lies between the thresholds of regime 0
+            // (a later one's lower threshold would send it here in every
+            // step: a body without a live bond 11 % a step)
+            if (nreg != reg)
+                a.state[slot] =
+                    (unsigned short)((base + (live ? nreg : 0)) << 4);
             if (live) {
-                if (nreg != reg)
-                    a.state[slot] = (unsigned short)((base + nreg) << 4);
                 kb = 4.0 * a.k_tab[base + nreg];
                 pb = 2.0 * a.pc_tab[base + nreg];
             }

@@ -179,3 +179,32 @@ def test_gradient_with_a_bond_of_no_length(lanes):
     np.testing.assert_array_equal(end[6], end2[6])
     assert np.all(np.isfinite(want)) and np.any(want != 0.0)
     assert pc.rel_l2(got, want) < RTOL
+
+
+def test_broken_nlinear_bonds_cost_no_more_than_live_ones():
+    """A body all of whose bonds broke past their last regime against the
+    same body whole, timed in turn."""
+    w = configs.composite_ec(shape=(120, 24, 24))
+    n, k = w.nlist.shape
+    zeros = np.zeros((n, 3), np.int32)
+    sims = []
+    for torn in (False, True):
+        integ = it.EulerCromerHIP(2.5e6, 1e-14)
+        integ.build(n, 3, k, w.coords, w.volume, w.family, zeros, w.bc_values,
+                    zeros, w.force_bc_values, None, w.bond_types, w.densities)
+        u = (2.0 * w.coords if torn else
+             np.random.default_rng(1).normal(scale=1e-5 * w.extra["dx"],
+                                             size=(n, 3)))
+        integ.create_buffers(w.nlist, w.n_neigh, w.bond_stiffness,
+                             w.critical_stretch, w.plus_cs, u, None, None,
+                             None, None, None, None, 3, 3)
+        integ.run(6, np.zeros(6), np.zeros(6))
+        assert integ.live_bonds() == (0 if torn else w.n_neigh.sum())
+        sims.append(integ)
+    best = [1e9, 1e9]
+    for _ in range(15):
+        for q, integ in enumerate(sims):
+            best[q] = min(best[q], integ.timed_run(40, np.zeros(40),
+                                                   np.zeros(40)))
+    print("whole, torn:", best)
+    assert best[1] < 1.05 * best[0]
