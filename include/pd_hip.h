@@ -220,6 +220,11 @@ int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
  * pd_adjoint_stop, a pd_create_buffers that tiles anew, or pd_destroy. */
 int pd_adjoint_start(pd_sim *sim, int nsteps, int checkpoint_every);
 
+/* Whether later recordings may keep u of every step (1, the default) or are
+ * held to their checkpoints (0), so that checkpoint_every bounds their memory;
+ * gradients and states are bitwise the same. */
+int pd_adjoint_keep(pd_sim *sim, int every_step);
+
 /* dL_du (N,3) f64: dL/du after the recorded steps.  dL_dc (N) f64 receives
  * dL/dc for the node stiffness field c (k_ij = (c_i + c_j)/2).  Leaves the
  * state as it was at the end of the recording. */

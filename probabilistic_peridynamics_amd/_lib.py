@@ -53,6 +53,7 @@ SIGNATURES = {
     "pd_step": (ctypes.c_int, [_SIM, ctypes.c_double, ctypes.c_double]),
     "pd_run_graph": (ctypes.c_int, [_SIM, ctypes.c_int, _D, _D, _F]),
     "pd_adjoint_start": (ctypes.c_int, [_SIM, ctypes.c_int, ctypes.c_int]),
+    "pd_adjoint_keep": (ctypes.c_int, [_SIM, ctypes.c_int]),
     "pd_adjoint_backward": (ctypes.c_int, [_SIM, _D, _D]),
     "pd_adjoint_backward_device": (ctypes.c_int, [_SIM, ctypes.c_void_p,
                                                   ctypes.c_void_p]),

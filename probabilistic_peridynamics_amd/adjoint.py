@@ -4,9 +4,10 @@ The forward model is the Euler step of a :class:`~.configs.Workload` with a
 per-node stiffness field ``c = c0 exp(g)`` (bond stiffness ``(c_i + c_j)/2``)
 run on the GPU.  The backward pass is the library's hand-written adjoint
 (``pd_adjoint_*``): the forward pass records the step at which each bond
-broke and checkpoints ``u``; the backward pass replays each checkpoint
-segment with the step kernel and runs the adjoint kernel back through it,
-holding the recorded break mask fixed.  :class:`StiffnessField` wraps this
+broke and ``u`` of every step, or checkpoints of ``u`` where that takes much
+memory; the backward pass replays what lies between checkpoints with the step
+kernel and runs the adjoint kernel back through the steps, holding the
+recorded break mask fixed.  :class:`StiffnessField` wraps this
 as a ``torch.autograd.Function`` of the log-stiffness ``g``; a ``g`` on the
 GPU stays there (the field, u and the gradient pass to and from the library
 by device address), a ``g`` on the host goes through numpy.
@@ -17,11 +18,13 @@ from . import integrators as it
 
 
 class StiffnessAdjoint:
-    """Forward and adjoint solves of one workload for fields g."""
+    """Forward and adjoint solves of one workload for fields g.
+    ``keep_every_step`` False holds recordings to the memory of a checkpoint
+    every ``checkpoint_every`` steps (:meth:`.Integrator.adjoint_keep`)."""
 
     def __init__(self, w, steps, checkpoint_every=100, c0=None,
                  context=None, lanes_per_node=4, tile_nodes=128,
-                 tension_only=False):
+                 tension_only=False, keep_every_step=True):
         if w.integrator != "euler":
             raise ValueError("the adjoint is for the Euler integrator")
         self.w = w
@@ -35,6 +38,7 @@ class StiffnessAdjoint:
                               None, None)
         self.integrator.set_break_mode(tension_only)
         self.integrator.set_launch(lanes_per_node, tile_nodes)
+        self.integrator.adjoint_keep(keep_every_step)
         self.dmags, self.fmags = w.magnitudes(self.steps)
         self.c = None
         # incremented by every forward: the recording a backward uses is

@@ -2348,6 +2348,7 @@ struct pd_sim {
 
     // adjoint recording (Euler, node field): break steps, checkpoints
     bool adj_recording = false, adj_ready = false, adj_replay = false;
+    bool adj_keep = true;  // pd_adjoint_keep
     bool adj_all = false;  // u of every recorded step is in seg
     // the model or the launch shape was set anew since the recording began:
     // its steps are replayed with the new ones
@@ -4377,15 +4378,17 @@ namespace {
 // seg), where checkpoints and a segment take `slots` arrays: the backward
 // pass then replays nothing (a third of it and of the forward pass together:
 // 200 steps and their gradient on 50,820 nodes 12.3 -> 8.8 ms).  At most
-// KEEP_TIMES the memory that the caller's checkpoint interval asks for, a
-// 64th of the device's and a quarter of what is free (2000 steps of 50,820
-// nodes with checkpoints every 100: 17 times, 2.4 GB).
+// KEEP_TIMES the memory that the caller's checkpoint interval asks for (at an
+// interval of 100, recordings of up to 4,700 steps), a 64th of the device's and
+// a quarter of what is free (2000 steps of 50,820 nodes: 17 times, 2.4 GB);
+// never where the caller holds recordings to their checkpoints
+// (pd_adjoint_keep).
 constexpr size_t KEEP_TIMES = 32;
 
 bool keep_all(pd_sim *s, int nsteps, size_t slots)
 {
     const size_t count = (size_t)nsteps * 3 * s->n;
-    if ((size_t)nsteps > KEEP_TIMES * slots)
+    if (!s->adj_keep || (size_t)nsteps > KEEP_TIMES * slots)
         return false;
     if (s->seg.p && s->seg.n >= count)
         return true;
@@ -4400,6 +4403,15 @@ bool keep_all(pd_sim *s, int nsteps, size_t slots)
 }
 
 }  // namespace
+
+int pd_adjoint_keep(pd_sim *s, int every_step)
+{
+    int rc = check_sim(s);
+    if (rc)
+        return rc;
+    s->adj_keep = every_step != 0;
+    return PD_OK;
+}
 
 int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
 {
@@ -4431,6 +4443,11 @@ int pd_adjoint_start(pd_sim *s, int nsteps, int checkpoint_every)
     HIPCHK(s->loc0.reserve(S));
     s->adj_all = keep_all(s, nsteps, (size_t)nck + checkpoint_every);
     if (!s->adj_all) {
+        // held to the checkpoints, an earlier recording's room goes back
+        if (!s->adj_keep && s->seg.n > (size_t)checkpoint_every * B)
+            s->seg.release();
+        if (!s->adj_keep && s->ckpt.n > (size_t)nck * B)
+            s->ckpt.release();
         HIPCHK(s->ckpt.reserve((size_t)nck * B));
         HIPCHK(s->seg.reserve((size_t)checkpoint_every * B));
     }

@@ -289,6 +289,13 @@ class Integrator(ABC):
         check(_lib.lib().pd_adjoint_start(self._sim, int(steps),
                                           int(checkpoint_every)))
 
+    def adjoint_keep(self, every_step=True):
+        """Whether later recordings may keep u of every step (the default)
+        or are held to the memory of their checkpoints, from which the
+        backward pass then replays; the results are bitwise the same."""
+        self._need_sim()
+        check(_lib.lib().pd_adjoint_keep(self._sim, int(bool(every_step))))
+
     def adjoint_backward(self, dL_du):
         """dL/dc of the node stiffness field for dL/du (nnodes, 3) after the
         recorded steps (the break mask of the recording held fixed)."""
