@@ -179,9 +179,10 @@ int pd_step(pd_sim *sim, double displacement_bc_magnitude,
             double force_bc_magnitude);
 
 /* nsteps calls of pd_step with magnitudes disp_mags[s], force_mags[s]
- * (either may be NULL for zeros).  A run that fails after its first step
- * leaves no whole state (u and the forces are stored by its last step):
- * reading or stepping on is PD_E_STATE until pd_create_buffers. */
+ * (either may be NULL for zeros).  A run that fails once a step of it is on
+ * its way leaves no whole state (u and the forces are stored by its last step,
+ * a recording's copies are made after each): reading or stepping on is
+ * PD_E_STATE until pd_create_buffers. */
 int pd_run(pd_sim *sim, int nsteps, const double *disp_mags,
            const double *force_mags);
 

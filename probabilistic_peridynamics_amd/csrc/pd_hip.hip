@@ -4230,12 +4230,7 @@ int pd_set_groups(pd_sim *s, const int *group)
 
 int pd_step(pd_sim *s, double dmag, double fmag)
 {
-    int rc = check_sim(s);
-    if (rc)
-        return rc;
-    if (!s->has_buffers)
-        return no_buffers(s);
-    return launch_step(s, dmag, fmag, true);
+    return pd_run(s, 1, &dmag, &fmag);
 }
 
 int pd_run(pd_sim *s, int nsteps, const double *disp_mags,
@@ -4248,7 +4243,7 @@ int pd_run(pd_sim *s, int nsteps, const double *disp_mags,
         return no_buffers(s);
     if (nsteps < 0)
         return fail(PD_E_ARG, "nsteps < 0");
-    const int cur0 = s->cur;
+    const int cur0 = s->cur;  // of a first step that is not launched
     for (int t = 0; t < nsteps; ++t) {
         rc = launch_step(s, disp_mags ? disp_mags[t] : 0.0,
                          force_mags ? force_mags[t] : 0.0, t + 1 == nsteps);

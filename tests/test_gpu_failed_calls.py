@@ -19,7 +19,7 @@ SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 typedef struct { unsigned x, y, z; } dim;
-static int left[3], pending;
+static int left[4], pending;
 void shim_arm(int which, int calls) { left[which] = calls; pending = 0; }
 static int now(int which) { return left[which] > 0 && --left[which] == 0; }
 int hipGraphInstantiate(void *e, void *g, void *n, char *b, size_t s)
@@ -44,6 +44,14 @@ int hipLaunchKernel(const void *k, dim g, dim b, void **a, size_t m, void *s)
     int (*f)(const void *, dim, dim, void **, size_t, void *) =
         dlsym(RTLD_NEXT, "hipLaunchKernel");
     return f(k, g, b, a, m, s);
+}
+int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st)
+{
+    if (now(3))
+        return 2;
+    int (*f)(void *, const void *, size_t, int, void *) =
+        dlsym(RTLD_NEXT, "hipMemcpyAsync");
+    return f(d, s, n, kind, st);
 }
 int hipGetLastError(void)
 {
@@ -108,7 +116,38 @@ out["again"] = same(_arrays(fresh), want)
 print("RESULT", json.dumps(out), flush=True)
 """
 
-INSTANTIATE, GRAPH, KERNEL = 0, 1, 2
+INSTANTIATE, GRAPH, KERNEL, COPY = 0, 1, 2, 3
+
+HEAD = r"""
+import ctypes, json, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path[:0] = sys.argv[2:4]
+import numpy as np
+from probabilistic_peridynamics_amd import _lib
+from test_gpu_recording import _make, _state
+which, calls, what = json.loads(sys.argv[4])
+
+
+def refused(call, *args):
+    try:
+        call(*args)
+    except _lib.PDError as e:
+        return e.code
+    return 0
+
+
+"""
+
+RECORDED_STEP = HEAD + r"""
+integ, _ = _make(2e-3)
+integ.adjoint_keep(what)
+integ.adjoint_start(4, checkpoint_every=1)
+shim.shim_arm(which, calls)
+out = [refused(integ, 1e-6, 1.0) for _ in range(2)]
+shim.shim_arm(which, 0)
+out += [refused(_state, integ), refused(integ, 1e-6, 1.0)]
+print("RESULT", json.dumps(out), flush=True)
+"""
 
 
 @pytest.fixture(scope="module")
@@ -121,15 +160,19 @@ def shim(tmp_path_factory):
     return d / "shim.so"
 
 
-def _after_failure(shim, which, calls, method):
+def _child(shim, code, which, calls, what):
     from conftest import ROOT, TESTS
     r = subprocess.run(
-        [sys.executable, "-c", CHILD, str(shim), str(ROOT), str(TESTS),
-         json.dumps([which, calls, method])],
+        [sys.executable, "-c", code, str(shim), str(ROOT), str(TESTS),
+         json.dumps([which, calls, what])],
         capture_output=True, text=True, timeout=100)
     line = [x for x in r.stdout.splitlines() if x.startswith("RESULT")]
     assert r.returncode == 0 and line, r.stdout + r.stderr
-    out = json.loads(line[0][len("RESULT"):])
+    return json.loads(line[0][len("RESULT"):])
+
+
+def _after_failure(shim, which, calls, method):
+    out = _child(shim, CHILD, which, calls, method)
     assert out["again"]  # new buffers, and all is well
     return out
 
@@ -155,6 +198,14 @@ def test_a_run_that_fails_on_its_way_is_not_read(shim, which, calls, method):
     out = _after_failure(shim, which, calls, method)
     assert out["call"] == -2 and out["write"] == -4
     assert out["others"] == [-4] * 7
+
+
+@pytest.mark.parametrize("keep", [True, False])
+def test_a_step_whose_recording_fails_is_not_read(shim, keep):
+    """The copy of u that a recorded step makes after its launch, at the
+    second step."""
+    out = _child(shim, RECORDED_STEP, COPY, 2, keep)
+    assert out == [0, -2, -4, -4]
 
 
 def test_refused_lists_leave_the_tiles_and_their_shape():
