@@ -202,7 +202,9 @@ def test_broken_nlinear_bonds_cost_no_more_than_live_ones():
         assert integ.live_bonds() == (0 if torn else w.n_neigh.sum())
         sims.append(integ)
     best = [1e9, 1e9]
-    for _ in range(15):
+    for rep in range(60):  # fifteen times, and more on a noisy machine
+        if rep >= 15 and best[1] < 1.05 * best[0]:
+            break
         for q, integ in enumerate(sims):
             best[q] = min(best[q], integ.timed_run(40, np.zeros(40),
                                                    np.zeros(40)))
