@@ -2266,10 +2266,15 @@ struct DevBuf {
     hipError_t alloc(size_t count)
     {
         release();
-        n = count;
         if (count == 0)
             return hipSuccess;
-        return hipMalloc(reinterpret_cast<void **>(&p), count * sizeof(T));
+        const hipError_t e =
+            hipMalloc(reinterpret_cast<void **>(&p), count * sizeof(T));
+        if (e == hipSuccess)
+            n = count;
+        else
+            p = nullptr;  // n stays 0: a later call allocates again
+        return e;
     }
     // room for count values; what is there is kept if it suffices
     hipError_t reserve(size_t count)
@@ -2302,7 +2307,7 @@ struct pd_sim {
     bool retile_pending = false;  // tile_nodes changed since the tiling
     bool has_buffers = false, has_corr = false, has_btypes = false,
          has_cnode = false;
-    bool lost = false;  // has_buffers was taken back by a run that failed
+    bool lost = false;  // has_buffers was taken back (run_failed)
     int nregimes = 1, nbond_types = 1;
     double k = 0.0, s0 = 0.0;
     int cur = 0;
@@ -2480,7 +2485,7 @@ int check_sim(pd_sim *s)
 int no_buffers(const pd_sim *s)
 {
     return fail(PD_E_STATE,
-                s->lost ? "a run failed on its way and left no whole state: "
+                s->lost ? "a call failed on its way and left no whole state: "
                           "call pd_create_buffers"
                         : "pd_create_buffers has not been called");
 }
@@ -2804,14 +2809,26 @@ int launch_step(pd_sim *s, double dmag, double fmag, bool last)
 }
 
 // After an error on the way of a run, some of whose steps have moved the
-// records and the bonds but stored neither u nor forces, or of a replay: there
-// is no state to read or to go on from.
+// records and the bonds but stored neither u nor forces, of a replay, or of a
+// change of the model, whose records may be of both: there is no state to
+// read or to go on from.
 void run_failed(pd_sim *s)
 {
     s->has_buffers = false;
     s->lost = true;
     adjoint_end(s);
 }
+
+// run_failed for a call that leaves while its state is away.
+struct StateGuard {
+    pd_sim *s;
+    bool away;
+    ~StateGuard()
+    {
+        if (away)
+            run_failed(s);
+    }
+};
 
 // The tip entries as internal DOF indices 3p + d for the current tiling.
 int upload_tips(pd_sim *s)
@@ -4106,7 +4123,7 @@ int pd_set_node_stiffness(pd_sim *s, const double *c)
         return rc;
     HIPCHK(hipStreamSynchronize(s->stream));
     s->adj_changed = true;
-    s->cnode_caller.release();
+    StateGuard state{s, s->has_buffers};
     if (!c) {
         s->cnode.release();
         s->h_cnode.clear();
@@ -4118,12 +4135,14 @@ int pd_set_node_stiffness(pd_sim *s, const double *c)
         if (s->has_buffers)
             HIPCHK(upload_perm(s->cnode, s->perm, c, 1));
     }
+    s->cnode_caller.release();
     if (s->has_buffers) {
         // the records carry c: rewrite both from the device u
         rc = refresh_records(s);
         if (rc)
             return rc;
     }
+    state.away = false;
     return PD_OK;
 }
 
@@ -4137,18 +4156,21 @@ int pd_set_node_stiffness_device(pd_sim *s, const double *c)
     HIPCHK(hipStreamSynchronize(s->stream));
     s->adj_changed = true;
     const size_t N = (size_t)s->n;
-    HIPCHK(s->cnode_caller.alloc(N));
+    HIPCHK(s->cnode_caller.reserve(N));
+    StateGuard state{s, s->has_buffers};
     HIPCHK(hipMemcpyAsync(s->cnode_caller.p, c, N * sizeof(double),
                           hipMemcpyDeviceToDevice, s->stream));
     s->h_cnode.clear();
     s->has_cnode = true;
     if (s->has_buffers) {
-        HIPCHK(s->cnode.alloc(N));
+        HIPCHK(s->cnode.reserve(N));
         hipLaunchKernelGGL(k_perm, dim3((s->n + 255) / 256), dim3(256), 0,
                            s->stream, s->n, 1, s->tnode.p, s->cnode_caller.p,
                            s->cnode.p);
         HIPCHK(hipGetLastError());
-        return refresh_records(s);  // synchronizes the stream
+        rc = refresh_records(s);  // synchronizes the stream
+        state.away = rc != PD_OK;
+        return rc;
     }
     HIPCHK(hipStreamSynchronize(s->stream));
     return PD_OK;
@@ -4180,14 +4202,14 @@ int pd_set_exact_order(pd_sim *s, int on)
     // the records carry V (exact) or 4kV (default): rewrite them; the fast
     // step does not keep the fold lists
     if (s->has_buffers && was != s->exact) {
-        if (s->exact) {
-            const int rc2 = fold_lists(s);
-            if (rc2)
-                return rc2;
-        }
-        return refresh_records(s);
+        StateGuard state{s, true};
+        if (s->exact)
+            rc = fold_lists(s);
+        if (rc == PD_OK)
+            rc = refresh_records(s);
+        state.away = rc != PD_OK;
     }
-    return PD_OK;
+    return rc;
 }
 
 int pd_set_launch(pd_sim *s, int lanes_per_node, int tile_nodes)
@@ -4573,15 +4595,7 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
     aa.il0 = s->il0.p;
     aa.gradc = s->gradc.p;
     // from here on a replay takes the state back to earlier steps
-    struct StateGuard {
-        pd_sim *s;
-        bool away;
-        ~StateGuard()
-        {
-            if (away)
-                run_failed(s);
-        }
-    } state{s, replay};
+    StateGuard state{s, replay};
     for (int k = nck - 1; k >= 0 && rc == PD_OK; --k) {
         const int n0 = k * every, n1 = std::min(n0 + every, nsteps);
         double *seg = s->seg.p + (s->adj_all ? (size_t)n0 * B : 0);

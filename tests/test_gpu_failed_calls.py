@@ -19,7 +19,7 @@ SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 typedef struct { unsigned x, y, z; } dim;
-static int left[4], pending;
+static int left[5], pending;
 void shim_arm(int which, int calls) { left[which] = calls; pending = 0; }
 static int now(int which) { return left[which] > 0 && --left[which] == 0; }
 int hipGraphInstantiate(void *e, void *g, void *n, char *b, size_t s)
@@ -52,6 +52,13 @@ int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st)
     int (*f)(void *, const void *, size_t, int, void *) =
         dlsym(RTLD_NEXT, "hipMemcpyAsync");
     return f(d, s, n, kind, st);
+}
+int hipMalloc(void **p, size_t n)
+{
+    if (now(4))
+        return 2;
+    int (*f)(void **, size_t) = dlsym(RTLD_NEXT, "hipMalloc");
+    return f(p, n);
 }
 int hipGetLastError(void)
 {
@@ -116,7 +123,7 @@ out["again"] = same(_arrays(fresh), want)
 print("RESULT", json.dumps(out), flush=True)
 """
 
-INSTANTIATE, GRAPH, KERNEL, COPY = 0, 1, 2, 3
+INSTANTIATE, GRAPH, KERNEL, COPY, MALLOC = 0, 1, 2, 3, 4
 
 HEAD = r"""
 import ctypes, json, sys
@@ -146,6 +153,32 @@ shim.shim_arm(which, calls)
 out = [refused(integ, 1e-6, 1.0) for _ in range(2)]
 shim.shim_arm(which, 0)
 out += [refused(_state, integ), refused(integ, 1e-6, 1.0)]
+print("RESULT", json.dumps(out), flush=True)
+"""
+
+CHANGED_MODEL = HEAD + r"""
+if what == "order":
+    integ = __import__("test_gpu_runs")._make("cython")
+    call, args = integ.set_exact_order, (False,)
+else:
+    integ, cs = _make(2e-3)
+    call, args = integ.set_node_stiffness, (cs[1],)
+shim.shim_arm(which, calls)
+out = [refused(call, *args)]
+shim.shim_arm(which, 0)
+out += [refused(_state, integ), refused(integ, 0.0, 0.0)]
+print("RESULT", json.dumps(out), flush=True)
+"""
+
+MONITOR = HEAD + r"""
+integ, _ = _make(2e-3)
+integ(1e-6, 1.0)
+shim.shim_arm(which, calls)
+out = [refused(integ.monitor)]
+shim.shim_arm(which, 0)
+fresh, _ = _make(2e-3)
+fresh(1e-6, 1.0)
+out.append(integ.monitor() == fresh.monitor())
 print("RESULT", json.dumps(out), flush=True)
 """
 
@@ -206,6 +239,18 @@ def test_a_step_whose_recording_fails_is_not_read(shim, keep):
     second step."""
     out = _child(shim, RECORDED_STEP, COPY, 2, keep)
     assert out == [0, -2, -4, -4]
+
+
+@pytest.mark.parametrize("which,what", [(MALLOC, "field"), (KERNEL, "field"),
+                                        (KERNEL, "order")])
+def test_a_model_that_changed_half_is_not_stepped(shim, which, what):
+    out = _child(shim, CHANGED_MODEL, which, 1, what)
+    assert out == [-2, -4, -4]
+
+
+@pytest.mark.parametrize("calls", [1, 2])
+def test_memory_that_was_refused_is_asked_for_again(shim, calls):
+    assert _child(shim, MONITOR, MALLOC, calls, None) == [-2, True]
 
 
 def test_refused_lists_leave_the_tiles_and_their_shape():
