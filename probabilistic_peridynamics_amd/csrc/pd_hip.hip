@@ -44,8 +44,10 @@
 //              chunk_off + c*n + l and holds four bonds of its l-th node
 //              rows sorted ascending by j; a wavefront reads its nodes' c-th
 //              chunks contiguously.  A tile has as many chunk rows as its
-//              longest row needs (at least one); the kernel's look-ahead
-//              chunk loads are clamped to the last of them.
+//              longest row needs (at least one); the step kernel's look-ahead
+//              loads run past the last of them, into the next tile's rows or
+//              the LOC_SLACK slots that loc, state and corr have at their end
+//              (the adjoint kernel's stay at the last row).
 //     loc   u16  16 * (1 + halo-local index of j), the LDS offset of the
 //                record's first piece; 0: broken or empty (hot loop; entry 0
 //                of a staged halo is a far node of weight 0)
@@ -273,7 +275,7 @@ __device__ __forceinline__ void static_for(F f)
 // 3/2 d^2 = 4.4e-29 (the seed's e is at most 6e-8, the step's d = 3/2 e^2), so
 // that a root within 4e-13 ulp of the middle between two doubles may take the
 // wrong one (8 of 4,023 squares built to lie 7e-15 to 5e-13 ulp off it did,
-// and none with the second).  The second costs the step 4 of a bond's 55 issue slots:
+// and none with the second).  The second costs the step 4 of a bond's 51 issue slots:
 // 233 -> 247 us on the 1,038,230-node beam, 38.4 -> 40.2 on 141,143 nodes, 72.6
 // -> 74.1 with n-linear tables on 263,407.
 __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
@@ -897,10 +899,10 @@ __device__ __forceinline__ void bond_pair(const StepArgs &a, const char *ldsb,
     }
 }
 
-// What bounds it on large meshes: the VALU (busy 72 % of the cycles on the
-// 1,038,230-node beam in the wide form; 8.6e7 wave instructions per launch,
-// mostly FP64 at 4 cycles and more, where there were 1.16e8; the clock gives
-// way under that load) and the LDS (63 %).  So the bond loop has one
+// What bounds it on large meshes: the VALU (9.4e7 wave instructions per launch
+// on the 1,038,230-node beam, mostly FP64 at 4 cycles and more, where there were
+// 1.16e8: 81 % of the cycles at 4 each, 72 % in the wide form; the clock gives
+// way under that load) and the LDS (about 60 %).  So the bond loop has one
 // compare per bond for everything that is rare, dead slots cost no test, LDS
 // offsets come ready from loc, chunk loads step one 32-bit offset, and a row
 // runs half rounds: 305 -> 270 us a step there, 113 -> 77 on the 263k-node
