@@ -161,8 +161,9 @@ int pd_set_exact_order(pd_sim *sim, int on);
 int pd_set_launch(pd_sim *sim, int lanes_per_node, int tile_nodes);
 
 /* Tiling of the current state: number of tiles, halo capacity per tile
- * (from the device's LDS per workgroup), largest halo of any tile (sets the
- * LDS each workgroup requests), total halo entries, bond slots. */
+ * (from the device's LDS per workgroup), largest halo of any tile (below
+ * 960 entries the scalar model may run the narrow halo form), total halo
+ * entries, bond slots. */
 int pd_tile_stats(pd_sim *sim, int *ntiles, int *hmax, int *hstride,
                   long long *halo_total, long long *slots);
 

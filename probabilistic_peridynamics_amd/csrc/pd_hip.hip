@@ -38,10 +38,10 @@
 //   tiles[T]   TileInfo: node range [node_off, node_off + nodes) of p, halo
 //              range in halo[], first chunk of the tile's bond slots, chunk
 //              rows.
-//   tnode[N]   caller's node id of internal node p; halo: ascending internal
-//              ids per tile.
+//   tnode[N]   caller's node id of internal node p; halo: internal ids per
+//              tile, in the order of their LDS entries (HaloSpread).
 //   bond slots, in chunks of 4: chunk (c, l) of a tile with n nodes is
-//              chunk_off + c*n + l and holds four bonds of its l-th node
+//              chunk_off + c*n + l and holds four bonds of its l-th node,
 //              rows sorted ascending by j; a wavefront reads its nodes' c-th
 //              chunks contiguously.  A tile has as many chunk rows as its
 //              longest row needs (at least one); the step kernel's look-ahead
@@ -3105,7 +3105,7 @@ int restart(pd_sim *s, const double *bond_stiffness,
 // t = l * lpn + sub takes the chunks of four slots sub, sub + lpn, ...  Read
 // groups are (16 lanes, round, bond of the chunk).  Greedy: records in the
 // most groups first, each to the residue least loaded over its groups among
-// the entries left (entry 0 is the zero record).  Returns entry - 1 for each
+// the entries left (entry 0 is the far node).  Returns entry - 1 for each
 // halo index; the order changes no result.
 constexpr int HALO_BANK_GROUPS = 16;
 
@@ -3606,7 +3606,7 @@ int pd_create_buffers(pd_sim *s, const int *nlist, const int *n_neigh,
 
     ShapeGuard shape{s};
     // tiles, capped by tile_nodes and by the LDS halo capacity
-    // entry 0 of a staged halo is the zero record of dead slots
+    // entry 0 of a staged halo is the far node of dead slots
     // the compact layout's tiles leave room for the exact step's windows
     s->hmax = (nlin ? LDS_CAP_NLIN
                     : (s->layout == PD_LAYOUT_COMPACT ? EXACT_CAP
