@@ -819,9 +819,19 @@ __device__ __forceinline__ void bond_exact(const StepArgs &a,
             if (nreg != reg)
                 a.state[slot] =
                     (unsigned short)((base + (live ? nreg : 0)) << 4);
+            // the scale that the fast evaluation has in its tables stands
+            // with 0.5/l here, and where every bond comes this way (because
+            // of the tables' values, for one) a small V_j precedes it: 4 k or
+            // the force's quotient by l may be infinite where the term is not
             if (live) {
-                kb = 4.0 * a.k_tab[base + nreg];
-                pb = 2.0 * a.pc_tab[base + nreg];
+                kb = a.k_tab[base + nreg];
+                pb = 0.5 * a.pc_tab[base + nreg];
+                o.hl *= 4.0;
+                if (!(a.lim > 0.0) && fabs(o.w) <= 1.0) {
+                    const double w = o.w;
+                    o.w = o.hl;
+                    o.hl = w;
+                }
             }
         }
         if (!live) {
@@ -3025,17 +3035,17 @@ void keep_plan(pd_sim *s, const int *nlist, const int *n_neigh, bool nlin,
     s->plan = true;
 }
 
-// The n-linear model's tables.  Values that are infinite or NaN, or become so
-// in the step's scaled form, are noted: a padding slot names row 0 of the
-// tables, whether or not a bond is of that type.
+// The n-linear model's tables.  Values that are infinite or NaN, or so large
+// that the fast evaluation's scaled form might become so, are noted: a padding
+// slot names row 0 of the tables, whether or not a bond is of that type.
 hipError_t set_tables(pd_sim *s, const double *k, const double *crit,
                       const double *pc)
 {
     const size_t T = (size_t)s->nregimes * s->nbond_types;
     s->odd_tables = false;
+    const auto odd = [](double v) { return !(std::fabs(v) <= 0x1p1000); };
     for (size_t t = 0; t < T; ++t)
-        s->odd_tables |= !std::isfinite(4.0 * k[t]) ||
-                         !std::isfinite(2.0 * pc[t]);
+        s->odd_tables |= odd(k[t]) || odd(pc[t]);
     hipError_t e = upload(s->k_tab, k, T);
     if (e == hipSuccess)
         e = upload(s->s_tab, crit, T);
