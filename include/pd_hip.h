@@ -229,7 +229,8 @@ int pd_adjoint_keep(pd_sim *sim, int every_step);
 
 /* dL_du (N,3) f64: dL/du after the recorded steps.  dL_dc (N) f64 receives
  * dL/dc for the node stiffness field c (k_ij = (c_i + c_j)/2).  Leaves the
- * state as it was at the end of the recording. */
+ * state as it was at the end of the recording.  PD_E_STATE where the field was
+ * cleared after the recording. */
 int pd_adjoint_backward(pd_sim *sim, const double *dL_du, double *dL_dc);
 
 /* pd_adjoint_backward with dL_du and dL_dc in device memory of the

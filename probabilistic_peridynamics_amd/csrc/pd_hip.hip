@@ -4558,6 +4558,9 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
                                 "pd_adjoint_start and run its steps");
     if (!dL_du || !dL_dc)
         return fail(PD_E_ARG, "dL_du and dL_dc are required");
+    if (!s->has_cnode)
+        return fail(PD_E_STATE, "the node stiffness field was cleared after "
+                                "the recording: set it again");
     const size_t N = (size_t)s->n, B = 3 * N, BB = B * sizeof(double);
     // with every u kept, the recording is one segment that needs no replay,
     // and the state is not touched

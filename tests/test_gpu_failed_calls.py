@@ -304,3 +304,29 @@ def test_a_backward_pass_that_is_refused_leaves_the_state(every):
     assert e.value.code == _lib.PD_E_STATE
     for a, b in zip(_state(integ), before):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("every", [3, 9])
+def test_a_backward_pass_without_its_field_is_refused(every):
+    """The field cleared after the recording; set again, the pass is that of
+    a recording whose field was set anew."""
+    from probabilistic_peridynamics_amd import _lib
+    from test_gpu_recording import _make, _state
+    grads = []
+    for cleared in (False, True):
+        integ, cs = _make(2e-3)
+        integ.adjoint_start(9, checkpoint_every=every)
+        integ.run(9, np.full(9, 1e-6), np.ones(9))
+        before = _state(integ)
+        dL = np.random.default_rng(1).normal(size=before[0].shape)
+        if cleared:
+            integ.set_node_stiffness(None)
+            with pytest.raises(_lib.PDError) as e:
+                integ.adjoint_backward(dL)
+            assert e.value.code == _lib.PD_E_STATE
+            for a, b in zip(_state(integ), before):
+                np.testing.assert_array_equal(a, b)
+        integ.set_node_stiffness(cs[0])
+        grads.append(integ.adjoint_backward(dL))
+    assert np.any(grads[0] != 0.0)
+    np.testing.assert_array_equal(*grads)
