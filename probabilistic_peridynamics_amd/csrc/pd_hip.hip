@@ -4026,6 +4026,9 @@ int pd_monitor(pd_sim *s, double *model, double *tips)
         s->h_tip_off.empty() ? 0 : (int)s->h_tip_off.size() - 1;
     if (ngroups > 0 && !tips)
         return fail(PD_E_ARG, "tips (5 doubles per group) is required");
+    // where pd_set_tips got no memory for them
+    if (ngroups > 0 && !s->tip_off.p && (rc = upload_tips(s)) != PD_OK)
+        return rc;
     const int N = s->n;
     if (!s->mon_part.p) {
         HIPCHK(s->mon_part.alloc((size_t)MON_BLOCKS * MON_SUMS));
@@ -4098,6 +4101,9 @@ int pd_monitor_noalloc(pd_sim *s, double *model, double *tips)
                                 "groups (use pd_monitor)");
     if (ngroups > 0 && !tips)
         return fail(PD_E_ARG, "tips (5 doubles per group) is required");
+    // where pd_set_tips got no memory for them
+    if (ngroups > 0 && !s->tip_off.p && (rc = upload_tips(s)) != PD_OK)
+        return rc;
     double *sp = nullptr;
     rc = scratch_address(s->device, &sp);
     if (rc)

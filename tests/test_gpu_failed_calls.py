@@ -182,6 +182,20 @@ out.append(integ.monitor() == fresh.monitor())
 print("RESULT", json.dumps(out), flush=True)
 """
 
+TIPS = HEAD + r"""
+integ, _ = _make(2e-3)
+integ(1e-6, 1.0)
+tips = {"a": [(3, 0), (7, 2)], "b": [(0, 1)]}
+shim.shim_arm(which, calls)
+out = [refused(integ.set_tips, tips)]
+shim.shim_arm(which, 0)
+fresh, _ = _make(2e-3)
+fresh(1e-6, 1.0)
+fresh.set_tips(tips)
+out.append(integ.monitor() == fresh.monitor())
+print("RESULT", json.dumps(out), flush=True)
+"""
+
 
 @pytest.fixture(scope="module")
 def shim(tmp_path_factory):
@@ -251,6 +265,11 @@ def test_a_model_that_changed_half_is_not_stepped(shim, which, what):
 @pytest.mark.parametrize("calls", [1, 2])
 def test_memory_that_was_refused_is_asked_for_again(shim, calls):
     assert _child(shim, MONITOR, MALLOC, calls, None) == [-2, True]
+
+
+@pytest.mark.parametrize("calls", [1, 2])
+def test_tips_that_got_no_memory_are_asked_for_again(shim, calls):
+    assert _child(shim, TIPS, MALLOC, calls, None) == [-2, True]
 
 
 def test_refused_lists_leave_the_tiles_and_their_shape():
