@@ -105,7 +105,7 @@ int pd_build(pd_sim **sim, int device, int integrator, int layout, double dt,
  * the same nlist and n_neigh (compared value by value with a host copy, kept
  * while N*K is at most 2^28), launch shape and table shape, and no starting
  * regimes but zeros, the tiles and bond slots are kept and only the state is
- * set anew. */
+ * set anew.  force and body_force read as zeros until a step. */
 int pd_create_buffers(pd_sim *sim, const int *nlist, const int *n_neigh,
                       const double *bond_stiffness,
                       const double *critical_stretch, const double *plus_cs,

@@ -2973,8 +2973,9 @@ int upload_caller(pd_sim *s, DevBuf<double> &d, const double *h, int w)
     return PD_OK;
 }
 
-// The state of a (re)start once the bonds are set up: u, ud, udd, the fold
-// lists and the records.  Synchronizes.
+// The state of a (re)start once the bonds are set up: u, ud, udd, no force yet
+// (what is there is of the run before, in the order of the tiles before), the
+// fold lists and the records.  Synchronizes.
 int start_state(pd_sim *s, const double *u, const double *ud,
                 const double *udd)
 {
@@ -2983,6 +2984,10 @@ int start_state(pd_sim *s, const double *u, const double *ud,
         rc = upload_caller(s, s->ud, ud, 3);
     if (rc == PD_OK)
         rc = upload_caller(s, s->udd, udd, 3);
+    if (rc == PD_OK)
+        rc = upload_caller(s, s->force, nullptr, 3);
+    if (rc == PD_OK)
+        rc = upload_caller(s, s->body_force, nullptr, 3);
     if (rc == PD_OK)
         rc = fold_lists(s);
     return rc == PD_OK ? refresh_records(s) : rc;
@@ -3465,10 +3470,6 @@ int pd_build(pd_sim **out, int device, int integrator, int layout, double dt,
     chk(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "stream");
     chk(hipEventCreate(&s->ev0), "event");
     chk(hipEventCreate(&s->ev1), "event");
-    if (rc == PD_OK) {
-        chk(hipMemset(s->force.p, 0, 3 * N * sizeof(double)), "memset");
-        chk(hipMemset(s->body_force.p, 0, 3 * N * sizeof(double)), "memset");
-    }
     if (stiffness_corrections) {
         s->h_corr.assign(stiffness_corrections,
                          stiffness_corrections + N * max_neighbours);
