@@ -4572,9 +4572,10 @@ int adjoint_backward(pd_sim *s, const double *dL_du, double *dL_dc,
     // with every u kept, the recording is one segment that needs no replay,
     // and the state is not touched
     const bool replay = !s->adj_all || s->adj_changed;
-    if (replay && s->retile_pending)
-        return tiles_pending();
     const int nsteps = s->adj_nsteps, every = replay ? s->adj_every : nsteps;
+    // with a checkpoint of every step there is no step to run again
+    if (replay && s->retile_pending && std::min(every, nsteps) > 1)
+        return tiles_pending();
     const int nck = (nsteps + every - 1) / every;
     hipStream_t st = s->stream;
     HIPCHK(hipStreamSynchronize(st));

@@ -325,6 +325,27 @@ def test_a_backward_pass_that_is_refused_leaves_the_state(every):
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("steps,every", [(1, 1), (1, 5), (9, 1)])
+def test_a_backward_pass_that_replays_nothing_needs_no_tiles(steps, every):
+    from test_gpu_recording import _make, _state
+    grads = []
+    for later in (False, True):
+        integ, _ = _make(2e-3)
+        integ.adjoint_start(steps, checkpoint_every=every)
+        integ.run(steps, np.full(steps, 1e-6), np.ones(steps))
+        before = _state(integ)
+        if later:
+            integ.set_launch(4, 64)
+        dL = np.random.default_rng(1).normal(size=before[0].shape)
+        grads.append(integ.adjoint_backward(dL))
+        for a, b in zip(_state(integ), before):
+            np.testing.assert_array_equal(a, b)
+    assert np.any(grads[0] != 0.0)
+    # the lanes of the default shape may be others: the sums' order
+    np.testing.assert_allclose(grads[1], grads[0], rtol=0,
+                               atol=1e-10 * np.abs(grads[0]).max())
+
+
 @pytest.mark.parametrize("every", [3, 9])
 def test_a_backward_pass_without_its_field_is_refused(every):
     """The field cleared after the recording; set again, the pass is that of
