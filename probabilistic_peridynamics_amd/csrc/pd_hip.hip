@@ -275,9 +275,9 @@ __device__ __forceinline__ void static_for(F f)
 // 3/2 d^2 = 4.4e-29 (the seed's e is at most 6e-8, the step's d = 3/2 e^2), so
 // that a root within 4e-13 ulp of the middle between two doubles may take the
 // wrong one (8 of 4,023 squares built to lie 7e-15 to 5e-13 ulp off it did,
-// and none with the second).  The second costs the step 4 of a bond's 51 issue slots:
-// 233 -> 247 us on the 1,038,230-node beam, 38.4 -> 40.2 on 141,143 nodes, 72.6
-// -> 74.1 with n-linear tables on 263,407.
+// and none with the second).  The second costs the step 4 of a bond's 51 issue
+// slots: 233 -> 247 us on the 1,038,230-node beam, 38.4 -> 40.2 on 141,143
+// nodes, 72.6 -> 74.1 with n-linear tables on 263,407.
 __device__ __forceinline__ void sqrt_core(double q, double &g, double &h)
 {
     const double y = __builtin_amdgcn_rsq(q);
@@ -819,19 +819,9 @@ __device__ __forceinline__ void bond_exact(const StepArgs &a,
             if (nreg != reg)
                 a.state[slot] =
                     (unsigned short)((base + (live ? nreg : 0)) << 4);
-            // the scale that the fast evaluation has in its tables stands
-            // with 0.5/l here, and where every bond comes this way (because
-            // of the tables' values, for one) a small V_j precedes it: 4 k or
-            // the force's quotient by l may be infinite where the term is not
             if (live) {
-                kb = a.k_tab[base + nreg];
-                pb = 0.5 * a.pc_tab[base + nreg];
-                o.hl *= 4.0;
-                if (!(a.lim > 0.0) && fabs(o.w) <= 1.0) {
-                    const double w = o.w;
-                    o.w = o.hl;
-                    o.hl = w;
-                }
+                kb = 4.0 * a.k_tab[base + nreg];
+                pb = 2.0 * a.pc_tab[base + nreg];
             }
         }
         if (!live) {
@@ -1230,7 +1220,7 @@ __global__ __launch_bounds__(CHECK_BLOCK) void k_bond_check(
 // b = (r0 + u, v) -- (u, v) with ucla, the slot layout's OpenCL stretch --
 // with v = 2 c V for a field c, else 0.  The weights are the factors the
 // bond loop multiplies by: wscale = 4k for the scalar model, 2 for the field
-// model, 1 for the n-linear model.
+// model, 1 for the n-linear model (more where its tables are scaled).
 __global__ void k_records(int n, double wscale, int ucla, const double *r0,
                           const double *vol, const double *u, const double *c,
                           NodeRec *rec0, NodeRec *rec1)
@@ -2316,6 +2306,7 @@ struct pd_sim {
     bool coords_core = false;  // coordinates in bond_fast's range
     bool odd_corr = false;     // some bond's correction is not finite
     bool odd_tables = false;   // set_tables
+    double tab_scale = 1.0;    // set_tables
     bool retile_pending = false;  // tile_nodes changed since the tiling
     bool has_buffers = false, has_corr = false, has_btypes = false,
          has_cnode = false;
@@ -2865,8 +2856,10 @@ int refresh_records(pd_sim *s)
     const int dm = dm_of(s);
     // the exact-order step reads V itself
     const double wscale =
-        s->exact ? 1.0
-                 : (dm == DM_PMB ? 4.0 * s->k : (dm == DM_FIELD ? 2.0 : 1.0));
+        s->exact         ? 1.0
+        : dm == DM_PMB   ? 4.0 * s->k
+        : dm == DM_FIELD ? 2.0
+                         : 1.0 / s->tab_scale;
     hipLaunchKernelGGL(k_records, dim3(blocks), dim3(256), 0, s->stream, s->n,
                        wscale, s->layout == PD_LAYOUT_SLOT ? 1 : 0, s->r0.p,
                        s->vol.p, s->u.p,
@@ -3040,21 +3033,33 @@ void keep_plan(pd_sim *s, const int *nlist, const int *n_neigh, bool nlin,
     s->plan = true;
 }
 
-// The n-linear model's tables.  Values that are infinite or NaN, or so large
-// that the fast evaluation's scaled form might become so, are noted: a padding
-// slot names row 0 of the tables, whether or not a bond is of that type.
+// The n-linear model's tables.  Values that are infinite or NaN are noted: a
+// padding slot names row 0 of the tables, whether or not a bond is of that
+// type.  Values so large that four times them may be infinite are taken 2^-8
+// times, and the records' V_j 2^8 times (a quarter and four times beside volumes
+// as large).
 hipError_t set_tables(pd_sim *s, const double *k, const double *crit,
                       const double *pc)
 {
     const size_t T = (size_t)s->nregimes * s->nbond_types;
+    const auto large = [](double v) { return std::fabs(v) > 0x1p1000; };
+    s->tab_scale = 1.0;
+    if (std::any_of(k, k + T, large) || std::any_of(pc, pc + T, large))
+        s->tab_scale = std::any_of(s->h_vol.begin(), s->h_vol.end(), large)
+                           ? 0x1p-2
+                           : 0x1p-8;
+    std::vector<double> ks(k, k + T), ps(pc, pc + T);
     s->odd_tables = false;
-    const auto odd = [](double v) { return !(std::fabs(v) <= 0x1p1000); };
-    for (size_t t = 0; t < T; ++t)
-        s->odd_tables |= odd(k[t]) || odd(pc[t]);
-    hipError_t e = upload(s->k_tab, k, T);
+    for (size_t t = 0; t < T; ++t) {
+        ks[t] *= s->tab_scale;
+        ps[t] *= s->tab_scale;
+        s->odd_tables |= !std::isfinite(4.0 * ks[t]) ||
+                         !std::isfinite(2.0 * ps[t]);
+    }
+    hipError_t e = upload(s->k_tab, ks.data(), T);
     if (e == hipSuccess)
         e = upload(s->s_tab, crit, T);
-    return e == hipSuccess ? upload(s->pc_tab, pc, T) : e;
+    return e == hipSuccess ? upload(s->pc_tab, ps.data(), T) : e;
 }
 
 // Whether the tiles and slots made by the last pd_create_buffers serve these
