@@ -198,7 +198,10 @@ int pd_run_timed(pd_sim *sim, int nsteps, const double *disp_mags,
  * their run time, measured with events on the library's stream.  Replaces the
  * step loop of Model.simulate (model.py:1295-1301) when the magnitudes of all
  * steps are known.  Steps whose graph cannot be made are launched one by one;
- * where the first graph cannot, nothing runs. */
+ * where the first graph cannot, nothing runs.  While one thread captures, HIP
+ * refuses other threads' work on the legacy default stream, this library's
+ * synchronous copies too (PD_E_HIP): no other thread may call into the library
+ * during a graph run. */
 int pd_run_graph(pd_sim *sim, int nsteps, const double *disp_mags,
                  const double *force_mags, float *elapsed_ms);
 
