@@ -19,7 +19,7 @@ Prints one JSON line:
   batched        the UQ batch (256 jittered bars of 5k-60k nodes, per-node
                  stiffness fields, Euler dt 1e-5, 500 steps): sample-steps/s
                  of the whole batch in one simulation, its steps captured in
-                 one hipGraph, against the same samples run one after another
+                 hipGraphs, against the same samples run one after another
                  with plain per-step launches (GPU time of back-to-back
                  launches); the batch's launch shape from the autotuner, each
                  candidate timed as a graph run of the whole batch, the
